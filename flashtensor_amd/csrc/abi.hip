@@ -5,6 +5,7 @@
 // (python/asuka/backend/tensorrt/builder.py:104-111).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -18,6 +19,9 @@
 
 namespace ft {
 hipError_t launch_attn_fwd(const AttnKernelParams& p, int D, bool bf16, bool causal, bool emu, int kf, hipStream_t s);
+const SplitPlan& split_plan(int B, int H, int group, int Sq, int Skv, int D, bool causal, bool cap);
+hipError_t launch_attn_split(const AttnKernelParams& p, const SplitPlan& plan, float* part, int D, bool bf16, bool causal, bool emu, int kf,
+                             hipStream_t s);
 hipError_t launch_colstats(const ColstatsKernelParams& p, int D, bool bf16, bool causal, bool emu, int mode,
                            hipStream_t s);
 hipError_t launch_linattn(const FtAttnArgs& a, int kind, int normalize_q, int out_dtype, void* ws, hipStream_t s);
@@ -242,6 +246,21 @@ size_t colstats_bytes(const FtAttnArgs* a) {
   return lse_bytes(a) + (group_of(a) > 1 ? (size_t)a->B * a->H * a->Skv * sizeof(float) : 0);
 }
 
+size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
+const ft::SplitPlan& split_of(const FtAttnArgs* a, int kf) {
+  return ft::split_plan(a->B, a->H, group_of(a), a->Sq, a->Skv, a->D, a->flags & FT_CAUSAL, kf == ft::kKfSoftcap);
+}
+
+// The attention pass of the modes that have a split form (plain softmax, soft-cap): split where the plan says so and
+// the caller's workspace, of which `used` bytes are taken, has room for the shares' partial results.
+hipError_t run_attn(const FtAttnArgs* a, const ft::AttnKernelParams& p, int kf, void* ws, size_t used, size_t ws_bytes, void* stream) {
+  const bool emu = !(a->flags & FT_FAST_LOGITS), causal = a->flags & FT_CAUSAL, bf16 = a->dtype == FT_BF16;
+  const ft::SplitPlan& plan = split_of(a, kf);
+  char* part = ws ? static_cast<char*>(ws) + align256(used) : nullptr;
+  if (plan.chunk_tiles && (!plan.bytes || (part && aligned16(part) && align256(used) + plan.bytes <= ws_bytes)))
+    return ft::launch_attn_split(p, plan, reinterpret_cast<float*>(part), a->D, bf16, causal, emu, kf, (hipStream_t)stream);
+  return ft::launch_attn_fwd(p, a->D, bf16, causal, emu, kf, (hipStream_t)stream);
+}
 
 int validate_colstats(const FtAttnArgs* a, const float* colsum, const float* colsumsq) {
   if (int rc = validate_attn(a, true)) return rc;
@@ -253,8 +272,8 @@ int validate_colstats(const FtAttnArgs* a, const float* colsum, const float* col
 }
 
 // attention pass (writes the row normalisers to the scratch), column pass, group mean when grouped; `ws` holds
-// colstats_bytes(a) bytes.  Every scratch element that is read has been written earlier in the same call.
-int run_colstats(const FtAttnArgs* a, float* colsum, float* colsumsq, void* ws, void* stream) {
+// at least colstats_bytes(a) bytes.  Every scratch element that is read has been written earlier in the same call.
+int run_colstats(const FtAttnArgs* a, float* colsum, float* colsumsq, void* ws, size_t ws_bytes, void* stream) {
   const int group = group_of(a);
   const bool emu = !(a->flags & FT_FAST_LOGITS);
   const bool causal = a->flags & FT_CAUSAL;
@@ -262,7 +281,7 @@ int run_colstats(const FtAttnArgs* a, float* colsum, float* colsumsq, void* ws, 
   float* per_head = group > 1 ? lse + (size_t)a->B * a->H * a->Sq : colsum;
   ft::AttnKernelParams p = attn_params(a, emu);
   p.lse = lse;
-  hipError_t e = ft::launch_attn_fwd(p, a->D, a->dtype == FT_BF16, causal, emu, ft::kKfNone, (hipStream_t)stream);
+  hipError_t e = run_attn(a, p, ft::kKfNone, ws, colstats_bytes(a), ws_bytes, stream);
   if (e != hipSuccess) return hip_fail(e, "attn_fwd launch");
   ft::ColstatsKernelParams c = col_params(a, emu, lse, per_head, colsumsq);
   e = ft::launch_colstats(c, a->D, a->dtype == FT_BF16, causal, emu, colsumsq ? ft::kStatSumSq : ft::kStatSum,
@@ -330,12 +349,25 @@ size_t ft_workspace_bytes(int op, const FtAttnArgs* a) {
   }
 }
 
-int ft_attn_fwd(const FtAttnArgs* a, float* lse, void* stream) {
+size_t ft_workspace_bytes_split(int op, const FtAttnArgs* a) {
+  if (!a) return 0;
+  const size_t need = ft_workspace_bytes(op, a);
+  if (op != FT_OP_ATTN && op != FT_OP_COLSTATS && op != FT_OP_CORM) return need;
+  if (a->B < 1 || a->H < 1 || a->Sq < 1 || a->Skv < 1 || a->Hkv < 0 || a->Hkv > a->H || (a->Hkv > 0 && a->H % a->Hkv)) return need;
+  size_t split = split_of(a, ft::kKfNone).bytes;
+  if (op == FT_OP_ATTN) split = std::max(split, split_of(a, ft::kKfSoftcap).bytes);
+  return split ? align256(need) + split : need;
+}
+
+int ft_attn_fwd(const FtAttnArgs* a, float* lse, void* stream) { return ft_attn_fwd_ws(a, 0.f, lse, nullptr, 0, stream); }
+
+int ft_attn_fwd_ws(const FtAttnArgs* a, float softcap, float* lse, void* workspace, size_t workspace_bytes, void* stream) {
   if (int rc = validate_attn(a, true)) return rc;
-  const bool emu = !(a->flags & FT_FAST_LOGITS);
-  ft::AttnKernelParams p = attn_params(a, emu);
+  if (!(softcap >= 0.f) || !std::isfinite(softcap)) return fail(FT_EINVAL, "softcap must be positive and finite, or 0 for none (got %g)", (double)softcap);
+  ft::AttnKernelParams p = attn_params(a, !(a->flags & FT_FAST_LOGITS));
   p.lse = lse;
-  hipError_t e = ft::launch_attn_fwd(p, a->D, a->dtype == FT_BF16, a->flags & FT_CAUSAL, emu, ft::kKfNone, (hipStream_t)stream);
+  p.softcap = softcap;
+  hipError_t e = run_attn(a, p, softcap > 0.f ? ft::kKfSoftcap : ft::kKfNone, workspace, 0, workspace_bytes, stream);
   if (e != hipSuccess) return hip_fail(e, "attn_fwd launch");
   return FT_OK;
 }
@@ -347,7 +379,7 @@ int ft_attn_colstats_fwd(const FtAttnArgs* a, float* colsum, float* colsumsq, vo
   if (!workspace || workspace_bytes < need)
     return fail(FT_EWORKSPACE, "workspace of %zu bytes needed, got %zu", need, workspace ? workspace_bytes : (size_t)0);
   if (reinterpret_cast<uintptr_t>(workspace) & 3u) return fail(FT_EINVAL, "workspace must be 4-byte aligned");
-  return run_colstats(a, colsum, colsumsq, workspace, stream);
+  return run_colstats(a, colsum, colsumsq, workspace, workspace_bytes, stream);
 }
 
 int ft_attn_colstats_fwd_static(const FtAttnArgs* a, float* colsum, float* colsumsq, void* stream) {
@@ -358,7 +390,7 @@ int ft_attn_colstats_fwd_static(const FtAttnArgs* a, float* colsum, float* colsu
                 need, (size_t)FT_STATIC_SCRATCH_BYTES);
   void* ws = nullptr;
   if (int rc = static_scratch(&ws, (hipStream_t)stream)) return rc;
-  return run_colstats(a, colsum, colsumsq, ws, stream);
+  return run_colstats(a, colsum, colsumsq, ws, need, stream);
 }
 
 int ft_keyformer_fwd(const FtAttnArgs* a, const FtNoise* noise, float tau, float* kf_score, void* workspace,
@@ -424,13 +456,7 @@ int ft_keyformer_fwd(const FtAttnArgs* a, const FtNoise* noise, float tau, float
 int ft_attn_softcap_fwd(const FtAttnArgs* a, float softcap, float* lse, void* stream) {
   if (int rc = validate_attn(a, true)) return rc;
   if (!(softcap > 0.f) || !std::isfinite(softcap)) return fail(FT_EINVAL, "softcap must be positive and finite (got %g)", (double)softcap);
-  const bool emu = !(a->flags & FT_FAST_LOGITS);
-  ft::AttnKernelParams p = attn_params(a, emu);
-  p.lse = lse;
-  p.softcap = softcap;
-  hipError_t e = ft::launch_attn_fwd(p, a->D, a->dtype == FT_BF16, a->flags & FT_CAUSAL, emu, ft::kKfSoftcap, (hipStream_t)stream);
-  if (e != hipSuccess) return hip_fail(e, "attn_fwd (softcap) launch");
-  return FT_OK;
+  return ft_attn_fwd_ws(a, softcap, lse, nullptr, 0, stream);
 }
 
 int ft_corm_fwd(const FtAttnArgs* a, const float* corm_mask, int64_t mask_row_stride, uint8_t* corm_score, float* margin,
@@ -448,7 +474,7 @@ int ft_corm_fwd(const FtAttnArgs* a, const float* corm_mask, int64_t mask_row_st
   float* lse = static_cast<float*>(workspace);
   ft::AttnKernelParams p = attn_params(a, emu);
   p.lse = lse;
-  hipError_t e = ft::launch_attn_fwd(p, a->D, a->dtype == FT_BF16, causal, emu, ft::kKfNone, (hipStream_t)stream);
+  hipError_t e = run_attn(a, p, ft::kKfNone, workspace, lse_bytes(a), workspace_bytes, stream);
   if (e != hipSuccess) return hip_fail(e, "attn_fwd launch");
   ft::ColstatsKernelParams c = col_params(a, emu, lse, margin, nullptr);
   c.keep = corm_score;

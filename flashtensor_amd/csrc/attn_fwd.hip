@@ -36,6 +36,15 @@ int attn_form_override() {
   return form;
 }
 
+// The same variable for the split form: "s<n>" shares out n tiles at a time, any other override keeps blocks whole.
+int attn_split_override() {
+  const char* e = getenv("FT_ATTN_FORM");
+  if (!e || !*e) return 0;
+  if (e[0] != 's') return -1;
+  const int n = atoi(e + 1);
+  return n > 0 ? n : -1;
+}
+
 hipError_t launch_attn_f16_d64(const AttnKernelParams& p, bool causal, bool emu, int kf, hipStream_t s);
 hipError_t launch_attn_f16_d128(const AttnKernelParams& p, bool causal, bool emu, int kf, hipStream_t s);
 hipError_t launch_attn_bf16_d64(const AttnKernelParams& p, bool causal, bool emu, int kf, hipStream_t s);

@@ -33,7 +33,23 @@ constexpr bool kAttnTwoBlocks = true;
 // below 2^kRescaleSlack (exact in fp16/fp32; the final division uses the same maximum).
 constexpr float kRescaleSlack = 6.f;
 
-template <typename T, int D, bool CAUSAL, bool EMU, int KF, int WAVES>
+// One share's partial result of a row block in the workspace (SPLIT): per wave of 32 rows the accumulator registers of
+// its 64 lanes, row maxima and row sums.
+struct SplitPartial {
+  float *o, *m, *l;
+};
+__host__ __device__ constexpr int64_t split_wave_floats(int D) { return 32 * D + 64; }
+__device__ __forceinline__ SplitPartial split_partial(float* base, int D, int64_t slot) {
+  float* o = base + slot * split_wave_floats(D);
+  return SplitPartial{o, o + 32 * D, o + 32 * D + 32};
+}
+
+// SPLIT: the form for few query rows over many keys (see attn_split.hpp).  A workgroup's rows are the (query, head)
+// pairs of one k/v head, row r = query r / group of the group's head r % group, so that K and V are staged once for the
+// whole group, and it walks only its share of the row block's key tiles; where a block has several shares, each leaves
+// its accumulator, row maxima and row sums in the workspace and attn_combine_kernel folds them.  Built for the causal
+// instantiation only: without a mask `off` is set to Skv, which hides nothing.
+template <typename T, int D, bool CAUSAL, bool EMU, int KF, int WAVES, bool SPLIT = false>
 __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVES)) attn_fwd_kernel(const AttnKernelParams p) {
   constexpr int BM = 32 * WAVES, BN = kAttnBN, NT = 64 * WAVES;
   constexpr int KSTEPS = D / 16;
@@ -66,8 +82,10 @@ __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVE
   constexpr int kErWaveBytes = 32 * BN * 4;
   __shared__ __align__(16) char ldsEr[kErLds ? WAVES * kErWaveBytes : 16];
 
-  const int BH = p.B * p.H;
-  const int nMB = (p.Sq + BM - 1) / BM;
+  static_assert(!SPLIT || (CAUSAL && WAVES == 4 && (KF == kKfNone || KF == kKfSoftcap)), "the split form's instantiations");
+  const int rows = SPLIT ? p.Sq * p.group : p.Sq;  // rows of a (b, h) pair; SPLIT: of a (b, k/v head) pair
+  const int BH = SPLIT ? p.B * (p.H / p.group) : p.B * p.H;
+  const int nMB = (rows + BM - 1) / BM;
   // (b, h) pair and rank among that pair's workgroups.  Workgroups are dealt round-robin to the 8 XCDs and, inside
   // an XCD, start in index order.  head_major: the workgroups of an XCD walk through that XCD's pairs one after
   // the other (all ranks of a pair are neighbours in the XCD's order), so that the workgroups resident on an XCD
@@ -92,7 +110,13 @@ __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVE
     const int half = (nMB + 1) / 2;
     mb = rank < half ? nMB - 1 - rank : rank - half;
   }
-  const int b = bh / p.H, h = bh % p.H;
+  int chunk = 0;
+  if (SPLIT) {
+    mb = p.items[rank] >> 8;
+    chunk = p.items[rank] & 255;
+  }
+  const int b = SPLIT ? bh / (p.H / p.group) : bh / p.H;
+  const int h = SPLIT ? (bh % (p.H / p.group)) * p.group : bh % p.H;  // SPLIT: the group's first head
   const int lane = lane_id(), wave = wave_id();
   const int g = lane >> 5, n = lane & 31;
   // two_blocks (causal, set by the launcher when the pairs fill the chip evenly): the workgroup takes query
@@ -106,11 +130,14 @@ __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVE
   if (kTwoPass && p.two_blocks) mb = pass == 0 ? nMB - 1 - rank : rank;
   if (pass) __syncthreads();  // every wave has left the first block's K/V tiles
   const int m0 = mb * BM;
-  const int qi = m0 + wave * 32 + n;
-  const int qi_c = qi < p.Sq ? qi : p.Sq - 1;
+  const int qrow = m0 + wave * 32 + n;
+  const int qrow_c = qrow < rows ? qrow : rows - 1;
+  const int qi = SPLIT ? qrow_c / p.group : qrow;      // query position of the row
+  const int qi_c = SPLIT ? qi : qrow_c;
+  const int hq = SPLIT ? h + qrow_c % p.group : h;     // its head
   const float NEG_INF = -__builtin_inff();
 
-  const uint16_t* qptr = p.q + b * p.sq.b + (int64_t)qi_c * p.sq.s + h * p.sq.h;
+  const uint16_t* qptr = p.q + b * p.sq.b + (int64_t)qi_c * p.sq.s + hq * p.sq.h;
   vec8 qf[KSTEPS];
 #pragma unroll
   for (int t = 0; t < KSTEPS; ++t) qf[t] = *reinterpret_cast<const vec8*>(qptr + 16 * t + 8 * g);
@@ -120,13 +147,30 @@ __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVE
 
   // tiles of the workgroup, of this wave (not entirely above its diagonal), and of this wave's mask-free prefix
   const int wave_row0 = m0 + wave * 32;
-  int n_end = p.Skv;
-  if (CAUSAL) n_end = min(p.Skv, m0 + BM + p.off);
-  const int ntiles = (n_end + BN - 1) / BN;
-  int nw = ntiles, n_fast = p.Skv / BN;
-  if (CAUSAL) {
-    nw = min(ntiles, (wave_row0 + 31 + p.off) / BN + 1);
-    n_fast = min(n_fast, (wave_row0 + p.off + 1) / BN);  // tiles with n0 + BN - 1 <= wave_row0 + off
+  int Skv = p.Skv, off = p.off;  // SPLIT: counted from the first key of the workgroup's share
+  int n_end = Skv;
+  if (CAUSAL) n_end = min(Skv, (SPLIT ? (min(m0 + BM, rows) - 1) / p.group + 1 : m0 + BM) + off);
+  int ntiles = (n_end + BN - 1) / BN;
+  int nch = 1;  // shares of this row block
+  if (SPLIT) {
+    nch = (ntiles + p.chunk_tiles - 1) / p.chunk_tiles;
+    const int per = (ntiles + nch - 1) / nch, t0 = chunk * per, t1 = min(t0 + per, ntiles);
+    kbase += (int64_t)t0 * BN * p.sk.s;
+    vbase += (int64_t)t0 * BN * p.sv.s;
+    off -= t0 * BN;
+    Skv = min(Skv, t1 * BN) - t0 * BN;
+    ntiles = t1 - t0;  // >= 1: (nch - 1) per <= (nch - 1) chunk_tiles < tiles of the block
+  }
+  int nw = ntiles, n_fast = Skv / BN;
+  if (CAUSAL && !SPLIT) {
+    nw = min(ntiles, (wave_row0 + 31 + off) / BN + 1);
+    n_fast = min(n_fast, (wave_row0 + off + 1) / BN);  // tiles with n0 + BN - 1 <= wave_row0 + off
+  }
+  if (SPLIT) {
+    // the wave's first and last query position; a wave without rows, or whose rows see no key of the share, has no tiles
+    const int pos0 = min(wave_row0, rows - 1) / p.group, pos1 = min(wave_row0 + 31, rows - 1) / p.group;
+    nw = wave_row0 < rows ? min(ntiles, (max(pos1 + off, -BN) + BN) / BN) : 0;
+    n_fast = min(n_fast, max(pos0 + off + 1, 0) / BN);
   }
   n_fast = min(n_fast, nw);
   const int n_free = n_fast;             // leading tiles of which this wave sees every key
@@ -187,10 +231,10 @@ __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVE
   stK.init(kbase, p.sk.s);
   stV.init(vbase, p.sv.s);
   auto stage_k = [&](int t, char* dst) __attribute__((always_inline)) {
-    if (t < ntiles) stK.issue(t * BN, min(BN, p.Skv - t * BN), dst);
+    if (t < ntiles) stK.issue(t * BN, min(BN, Skv - t * BN), dst);
   };
   auto stage_v = [&](int t, char* dst) __attribute__((always_inline)) {
-    if (t < ntiles) stV.issue(t * BN, min(BN, p.Skv - t * BN), dst);
+    if (t < ntiles) stV.issue(t * BN, min(BN, Skv - t * BN), dst);
     if (kSeeded && t < ntiles && threadIdx.x < BN)
       ldsCol[(t & 1) * BN + threadIdx.x] = noise_col(nk, (uint32_t)(t * BN + threadIdx.x));
   };
@@ -260,7 +304,8 @@ __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVE
     const bool grow = rowmax > m_run + kRescaleSlack;  // identical in both lanes of a row
     if (__any(grow)) {
       const float m_new = grow ? rowmax : m_run;
-      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+      // (SPLIT: a row that has seen no key yet keeps -inf, whose difference with itself is no number)
+      const float alpha = SPLIT && !grow ? 1.f : __builtin_amdgcn_exp2f(m_run - m_new);
       if (KF == kKfSeededTau1) l_kf *= alpha;
       if (KF == kKfSeededFast) l_kf *= __builtin_amdgcn_exp2f((m_run - m_new) * p.inv_tau);
       m_run = m_new;
@@ -282,7 +327,7 @@ __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVE
   // row maximum of one tile's logits in the log2 domain (what rescale() compares with the running maximum)
   auto tile_max = [&](auto masked_tag, const float16v (&s)[2], int n0) __attribute__((always_inline)) -> float {
     constexpr bool MASKED = decltype(masked_tag)::value;
-    const int lim = (CAUSAL ? min(qi + p.off, p.Skv - 1) : p.Skv - 1) - n0 - 4 * g;
+    const int lim = (CAUSAL ? min(qi + off, Skv - 1) : Skv - 1) - n0 - 4 * g;
     auto at = [&](int mbk, int r) __attribute__((always_inline)) -> float {
       if (!MASKED) return s[mbk][r];
       const int jl = 32 * mbk + 8 * (r >> 2) + (r & 3);
@@ -321,7 +366,7 @@ __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVE
     const float neg_m = -m_run;
     const half2v pk_hi = __builtin_bit_cast(half2v, p.pk_hi2), pk_lo = __builtin_bit_cast(half2v, p.pk_lo2);
     // local key index of register r is 32 mbk + 8 (r / 4) + 4 g + r % 4; it is visible iff <= lim + 4 g
-    const int lim = (CAUSAL ? min(qi + p.off, p.Skv - 1) : p.Skv - 1) - n0 - 4 * g;
+    const int lim = (CAUSAL ? min(qi + off, Skv - 1) : Skv - 1) - n0 - 4 * g;
     uint4v pw[4];
     // Eight elements (one MFMA operand) at a time, stage by stage, so that consecutive instructions are
     // independent: every stage's result is needed only four instructions later.
@@ -599,7 +644,7 @@ __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVE
   int it = 0;
   // ---- mask-free tiles, two per trip so that the two score buffers swap roles without copies
   // pairs (it, it+1) of mask-free tiles whose staged tiles K[it+2], K[it+3], V[it+1], V[it+2] are whole tiles
-  const int nf2 = max(0, min(n_fast, p.Skv / BN - 2)) & ~1;
+  const int nf2 = max(0, min(n_fast, Skv / BN - 2)) & ~1;
   // tiles from nf2 on go through the masked instance (which is exact for a tile that needs no mask as well); so
   // does tile 0, which may be one of them.
   pend_max = tile_max(std::true_type{}, S0, 0);
@@ -742,9 +787,27 @@ __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVE
 
   // ---- epilogue
   l_run += xchg32(l_run);
+  if (SPLIT && nch > 1) {
+    // unnormalised: accumulator registers as they are, one 16-byte piece per lane and store (coalesced), rows that exist
+    const SplitPartial part = split_partial(p.part, D, ((int64_t)bh * p.nitems + rank) * p.part_waves + wave);
+    if (qrow < rows) {
+#pragma unroll
+      for (int db = 0; db < DB; ++db)
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4) {
+          const float4v w = {o_acc[db][4 * q4], o_acc[db][4 * q4 + 1], o_acc[db][4 * q4 + 2], o_acc[db][4 * q4 + 3]};
+          *reinterpret_cast<float4v*>(part.o + ((db * 4 + q4) * 64 + lane) * 4) = w;
+        }
+      if (g == 0) {
+        part.m[n] = m_run;
+        part.l[n] = l_run;
+      }
+    }
+    return;
+  }
   const float inv_l = 1.f / l_run;
-  if (qi < p.Sq) {
-    uint16_t* optr = p.o + b * p.so.b + (int64_t)qi * p.so.s + h * p.so.h;
+  if (qrow < rows) {
+    uint16_t* optr = p.o + b * p.so.b + (int64_t)qi * p.so.s + hq * p.so.h;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -758,7 +821,7 @@ __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVE
         pk.y = (uint32_t)w[2] | ((uint32_t)w[3] << 16);
         *reinterpret_cast<uint2*>(optr + d) = pk;
       }
-    if (g == 0 && p.lse) p.lse[(int64_t)bh * p.Sq + qi] = m_run + __builtin_amdgcn_logf(l_run);
+    if (g == 0 && p.lse) p.lse[(SPLIT ? (int64_t)b * p.H + hq : (int64_t)bh) * p.Sq + qi] = m_run + __builtin_amdgcn_logf(l_run);
   }
   if (kTensor || kSeeded) {
     l_kf += xchg32(l_kf);
@@ -774,6 +837,7 @@ __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVE
 // launch-shape selection (host)
 
 int device_cu_count();     // attn_fwd.hip
+int attn_split_override();  // attn_fwd.hip: 0, or -1: never split, n > 0: split into shares of n tiles
 int attn_form_override();  // attn_fwd.hip: 0, or (1: 4 waves, 2: 8 waves, 3: 8 waves and two blocks) | 8: head-major order
 
 template <typename T, int D, bool CAUSAL, bool EMU, int KF>

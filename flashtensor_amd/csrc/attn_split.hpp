@@ -1,0 +1,25 @@
+// Attention over few query rows and many keys (generation steps, a window of last queries, a chunk of a prompt): attn_fwd_kernel's SPLIT form, whose row blocks share their key tiles out between workgroups, and the
+// plan that says when.  Instantiated by attn_split_{f16,bf16}.hip; attn_split.hip holds the plan, the dispatcher and the
+// kernel that folds the shares.
+//
+// What bounds the unsplit form there: a row block is one workgroup that walks all of its tiles (1.1-1.3 us each), however
+// few blocks there are.  B4 Sq1 Skv4097 with 32 query heads on 8 k/v heads: 128 workgroups of which one wave of four has
+// one row, 65 tiles each, K and V staged four times over: 69 us for 67 MB.
+#pragma once
+#include "attn_fwd_kernel.hpp"
+
+namespace ft {
+
+template <typename T, int D>
+hipError_t launch_split_td(const AttnKernelParams& p, bool emu, int kf, unsigned grid, unsigned lds, hipStream_t s) {
+#define FT_CASE(E, K)                                                                                        \
+  if (emu == E && kf == K) {                                                                                 \
+    hipLaunchKernelGGL((attn_fwd_kernel<T, D, true, E, K, 4, true>), dim3(grid), dim3(256), lds, s, p);      \
+    return hipGetLastError();                                                                                \
+  }
+  FT_CASE(true, kKfNone) FT_CASE(false, kKfNone) FT_CASE(true, kKfSoftcap) FT_CASE(false, kKfSoftcap)
+#undef FT_CASE
+  return hipErrorInvalidValue;
+}
+
+}  // namespace ft

@@ -98,6 +98,14 @@ void init_ffi_kernels(py::module_&& m) {
   m.def("last_error", [] { return std::string(ft_last_error()); });
   m.def("workspace_bytes", [](int op, const FtAttnArgs& a) { return ft_workspace_bytes(op, &a); });
 
+  m.def("workspace_bytes_split", [](int op, const FtAttnArgs& a) { return ft_workspace_bytes_split(op, &a); });
+
+  m.def("attn_fwd_ws", [](const FtAttnArgs& a, float softcap, uintptr_t lse, uintptr_t ws, size_t ws_bytes, uintptr_t stream) {
+    py::gil_scoped_release nogil;
+    check(ft_attn_fwd_ws(&a, softcap, ptr<float>(lse), ptr<void>(ws), ws_bytes, ptr<void>(stream)));
+  }, py::arg("args"), py::arg("softcap") = 0.f, py::arg("lse") = 0, py::arg("workspace") = 0, py::arg("workspace_bytes") = 0,
+     py::arg("stream") = 0);
+
   m.def("attn_fwd", [](const FtAttnArgs& a, uintptr_t lse, uintptr_t stream) {
     py::gil_scoped_release nogil;
     check(ft_attn_fwd(&a, ptr<float>(lse), ptr<void>(stream)));

@@ -1,5 +1,6 @@
 // Launch-time parameter blocks shared by the host dispatcher and the kernels.
 #pragma once
+#include <stddef.h>
 #include <stdint.h>
 
 namespace ft {
@@ -7,6 +8,8 @@ namespace ft {
 struct Strides3 {
   int64_t b, s, h;
 };
+
+constexpr int kSplitMaxItems = 128, kSplitMaxBlocks = 64;  // of a (b, k/v head) pair
 
 struct AttnKernelParams {
   const uint16_t* q;
@@ -33,6 +36,25 @@ struct AttnKernelParams {
   int group;        // query heads per k/v head: query head h reads k/v head h / group
   int two_blocks;   // 256-row form: a workgroup takes query blocks nMB - 1 - slot and slot (set by the launcher)
   int head_major;   // workgroup order inside an XCD: all blocks of a (b, h) pair before the next pair's (launcher)
+  // split form (attn_split.hpp): a row block's key tiles are shared out between workgroups, at most chunk_tiles each
+  float* part;      // workspace of the shares' partial results (may be null where no block has more than one share)
+  int chunk_tiles;
+  int nitems;       // shares of all row blocks of a (b, k/v head) pair
+  int part_waves;   // waves of a row block that have rows
+  uint16_t items[kSplitMaxItems];       // row block << 8 | share; a block's shares are neighbours
+  uint8_t first_item[kSplitMaxBlocks];  // where they begin
+};
+
+// How attention shares the key tiles of its row blocks out between workgroups; chunk_tiles 0: it does not.
+struct SplitPlan {
+  int chunk_tiles;   // tiles of a share, at most
+  int items;         // shares of a (b, k/v head) pair
+  int first_shared;  // row blocks from this one on have more than one share
+  int nblocks, part_waves;
+  bool one_per_cu;   // no more workgroups than CUs: keep them from sharing one
+  size_t bytes;      // workspace of the shares' partial results
+  uint16_t list[kSplitMaxItems];
+  uint8_t first_item[kSplitMaxBlocks];
 };
 
 struct ColstatsKernelParams {

@@ -8,6 +8,8 @@ pybind11 module ft_ffi (csrc/ffi_kernels.cpp, the counterpart of the reference's
 raise ValueError, everything else RuntimeError, as std::invalid_argument / std::runtime_error do there
 (ffi/passes.cpp:81-83).
 """
+import math
+
 import torch
 
 from . import _lib
@@ -67,13 +69,24 @@ def _prep(q, k, v, dtypes=_DTYPES):
   return _dense_last(q), _dense_last(k), _dense_last(v)
 
 
+def _workspace(op, a, q):
+  nbytes = _k().workspace_bytes_split(op, a)
+  return torch.empty(nbytes, dtype=torch.uint8, device=q.device), nbytes
+
+
+def _attn_fwd(a, softcap, lse, q):
+  nbytes = _k().workspace_bytes_split(_lib.FT_OP_ATTN, a)
+  ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes else None
+  _k().attn_fwd_ws(a, softcap, lse.data_ptr() if lse is not None else 0, ws.data_ptr() if nbytes else 0, nbytes, _stream(q))
+
+
 def attn(q, k, v, causal=True, fast_logits=False, return_lse=False):
   """Attn.forward (cases/kernels/attn.py:18-34): q [B,S,H,D], k,v [B,Skv,Hkv,D] -> out [B,Sq,H,D].  With
   Hkv < H query head h attends to k/v head h // (H // Hkv), the grouping of cases/attn.py:29-31."""
   q, k, v = _prep(q, k, v)
   out = torch.empty_like(q, memory_format=torch.contiguous_format)
   lse = torch.empty(q.shape[0], q.shape[2], q.shape[1], dtype=torch.float32, device=q.device) if return_lse else None
-  _k().attn_fwd(_args(q, k, v, out, _flags(causal, fast_logits)), lse.data_ptr() if return_lse else 0, _stream(q))
+  _attn_fwd(_args(q, k, v, out, _flags(causal, fast_logits)), 0.0, lse, q)
   return (out, lse) if return_lse else out
 
 
@@ -86,8 +99,7 @@ def _colstats(q, k, v, want_sq, causal, fast_logits):
   s1 = torch.empty(B, k.shape[2], Skv, dtype=torch.float32, device=q.device)  # per k/v head (group mean when grouped)
   s2 = torch.empty(B, H, Skv, dtype=torch.float32, device=q.device) if want_sq else None
   a = _args(q, k, v, out, _flags(causal, fast_logits))
-  nbytes = ffi.workspace_bytes(_lib.FT_OP_COLSTATS, a)
-  ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
+  ws, nbytes = _workspace(_lib.FT_OP_COLSTATS, a, q)
   ffi.attn_colstats_fwd(a, s1.data_ptr(), s2.data_ptr() if want_sq else 0, ws.data_ptr(), nbytes, _stream(q))
   return (out, s1, s2) if want_sq else (out, s1)
 
@@ -157,8 +169,7 @@ def corm(q, k, v, corm_mask=None, causal=True, fast_logits=False, return_margin=
   keep = torch.empty(B, H, Skv, dtype=torch.uint8, device=q.device)
   margin = torch.empty(B, H, Skv, dtype=torch.float32, device=q.device) if return_margin else None
   a = _args(q, k, v, out, _flags(causal, fast_logits))
-  nbytes = ffi.workspace_bytes(_lib.FT_OP_CORM, a)
-  ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
+  ws, nbytes = _workspace(_lib.FT_OP_CORM, a, q)
   ffi.corm_fwd(a, mask_ptr, mask_stride, keep.data_ptr(), margin.data_ptr() if return_margin else 0, ws.data_ptr(), nbytes,
                _stream(q))
   keep = keep.view(torch.bool)
@@ -169,7 +180,9 @@ def gemma2(q, k, v, softcap=50.0, causal=True, fast_logits=False):
   """Gemma2.forward (cases/kernels/gemma2.py:19-39): attention with logits softcap * tanh(logit / softcap)."""
   q, k, v = _prep(q, k, v)
   out = torch.empty_like(q, memory_format=torch.contiguous_format)
-  _k().attn_softcap_fwd(_args(q, k, v, out, _flags(causal, fast_logits)), float(softcap), 0, _stream(q))
+  if not (softcap > 0 and math.isfinite(softcap)):
+    raise ValueError(f"softcap need a positive finite number but got {softcap}")
+  _attn_fwd(_args(q, k, v, out, _flags(causal, fast_logits)), float(softcap), None, q)
   return out
 
 

@@ -84,9 +84,19 @@ const char* ft_last_error(void);
 /* Bytes of device scratch the op needs for this problem (0 if none).  The caller owns the buffer. */
 size_t ft_workspace_bytes(int op, const FtAttnArgs* a);
 
+/* The same plus room for the partial results of the shares into which FT_OP_ATTN, FT_OP_COLSTATS and FT_OP_CORM divide
+ * the keys where there are too few query rows to fill the chip (generation steps, a window of last queries, chunks of a
+ * prompt).  With a workspace of this size those calls are faster; with one of
+ * ft_workspace_bytes() they run undivided.  The number of shares depends on the device, so ask with it current. */
+size_t ft_workspace_bytes_split(int op, const FtAttnArgs* a);
+
 /* Causal (or full) softmax attention: replaces the fused kernel of Attn.forward (cases/kernels/attn.py:18-34).
  * lse: optional [B,H,Sq] fp32 output, log2-domain row normaliser max + log2(sum). */
 int ft_attn_fwd(const FtAttnArgs* a, float* lse, void* stream);
+
+/* ft_attn_fwd (softcap == 0) or ft_attn_softcap_fwd (softcap > 0) with an optional workspace of
+ * ft_workspace_bytes_split(FT_OP_ATTN, a) bytes, 16-byte aligned. */
+int ft_attn_fwd_ws(const FtAttnArgs* a, float softcap, float* lse, void* workspace, size_t workspace_bytes, void* stream);
 
 /* Attention + per-key column statistics: H2O.forward (cases/kernels/h2o.py:18-38; colsumsq == NULL) and
  * RoCo.forward (cases/kernels/roco.py:18-48).  colsum, colsumsq: [B,H,Skv] fp32.

@@ -1,0 +1,50 @@
+"""The split form of the attention pass (a row block's keys shared out between workgroups) against the CPU oracle: rows of
+one wave and of several, shares of one tile, keys one off a tile, rows that see no key of a share."""
+import pytest
+import torch
+
+import oracle
+from flashtensor_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("tiles", [1, 3])
+@pytest.mark.parametrize("Sq,Skv,H,Hkv,D,dtype", [
+    (1, 65, 8, 2, 128, torch.float16), (1, 1000, 4, 4, 64, torch.bfloat16), (8, 449, 8, 2, 64, torch.float16), (33, 129, 4, 1, 128, torch.float16),
+    (130, 1090, 4, 2, 64, torch.float16), (300, 300, 2, 2, 128, torch.float16), (257, 640, 2, 1, 128, torch.bfloat16)])
+def test_shares_of_the_keys(gpu, monkeypatch, tiles, Sq, Skv, H, Hkv, D, dtype):
+  monkeypatch.setenv("FT_ATTN_FORM", f"s{tiles}")
+  g = torch.Generator().manual_seed(Sq + Skv)
+  q, k, v = (torch.randn(s, h * D, dtype=dtype, generator=g) for s, h in ((Sq, H), (Skv, Hkv), (Skv, Hkv)))
+  dev = [t.to(gpu).view(1, t.shape[0], -1, D) for t in (q, k, v)]
+  tol = 1e-2 if dtype is torch.bfloat16 else 2e-3
+  for causal in (True, False):
+    ref_o, ref_s = oracle.attn_h2o2d_forward(q, k, v, Hkv, H, D, masked=causal)
+    out, lse = ops.attn(*dev, causal=causal, return_lse=True)
+    out2, score = ops.h2o(*dev, causal=causal)
+    assert torch.isfinite(lse).all() and torch.equal(out, out2)
+    ref = ref_o.float().view(1, Sq, H, D)
+    assert (out.float().cpu() - ref).norm() <= tol * ref.norm()
+    assert (score.cpu()[0] - ref_s).norm() <= tol * ref_s.norm()
+  if H == Hkv:
+    q4, k4, v4 = (t.view(1, t.shape[0], -1, D) for t in (q, k, v))
+    ref = oracle.gemma2_forward(q4, k4, v4, 5.0).float()
+    assert (ops.gemma2(*dev, softcap=5.0).float().cpu() - ref).norm() <= tol * ref.norm()
+
+
+def test_a_workspace_without_room_for_the_shares_keeps_blocks_whole(gpu, monkeypatch):
+  """The C ABI takes any workspace of at least ft_workspace_bytes(); only one of ft_workspace_bytes_split() lets it split."""
+  monkeypatch.setenv("FT_ATTN_FORM", "s1")
+  q, k, v = (torch.randn(1, s, 2, 64, dtype=torch.float16, device=gpu) for s in (4, 500, 500))
+  k_ = ops._k()
+  a = ops._args(q, k, v, torch.empty_like(q), ops._flags(True, False))
+  need, more = (f(k_.OP_COLSTATS, a) for f in (k_.workspace_bytes, k_.workspace_bytes_split))
+  assert more > need == 2 * 4 * 4
+  ref = ops.h2o(q, k, v)
+  for nbytes in (need, more - 1, more):
+    out = torch.empty_like(q)
+    score = torch.empty(1, 2, 500, device=gpu)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=gpu)
+    k_.attn_colstats_fwd(ops._args(q, k, v, out, ops._flags(True, False)), score.data_ptr(), 0, ws.data_ptr(), nbytes, ops._stream(q))
+    assert (out.float() - ref[0].float()).norm() <= 1e-3 * ref[0].float().norm() and torch.allclose(score, ref[1], rtol=1e-4)
