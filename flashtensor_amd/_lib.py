@@ -1,5 +1,5 @@
-"""Loaders of the native code: `ffi()` imports the pybind11 module ft_ffi (csrc/ffi_kernels.cpp) the operators
-call through, `load()` binds libflashtensor_hip.so (the C ABI of include/ft_abi.h) directly with ctypes for
+"""Loaders of the native code: `native()` imports ft_ops (csrc/ops_torch.cpp), the operators on torch tensors, `ffi()`
+the pybind11 module ft_ffi (csrc/ffi_kernels.cpp) over the C ABI, `load()` binds libflashtensor_hip.so (the C ABI of include/ft_abi.h) directly with ctypes for
 callers and tests that work at the level of the C ABI, `load_diag()` the diagnostics library.
 
 The library is the product: if it is missing or fails to load these raise, there is no fallback.
@@ -160,3 +160,19 @@ def ffi():
                         f"binding {ABI_VERSION}")
     _ffi = ft_ffi
   return _ffi
+
+
+_native = None
+
+
+def native():
+  """The module of the operators on torch tensors."""
+  global _native
+  if _native is None:
+    ffi()  # the library is there and of this version
+    try:
+      from . import ft_ops
+    except ImportError as e:
+      raise ImportError(f"the module ft_ops is not built: run `python -m flashtensor_amd.build` ({e})") from e
+    _native = ft_ops
+  return _native

@@ -19,6 +19,7 @@ SOURCES = ["abi.hip", "attn_fwd.hip", "attn_fwd_f16_d128.hip", "attn_fwd_f16_d64
            "attn_split.hip", "attn_split_f16.hip", "attn_split_bf16.hip", "colstats.hip", "linattn.hip", "aux.hip", "linblock.hip", "linblock_small.hip"]
 DIAG_SOURCES = ["diag.hip"]
 FFI_SOURCE = "ffi_kernels.cpp"  # pybind11 module ft_ffi over the C ABI (plain C++: no device code, no torch headers)
+OPS_SOURCE = "ops_torch.cpp"    # module ft_ops: the operators on torch tensors (plain C++ over torch's headers and the C ABI)
 HEADERS = ["device_common.hpp", "kernel_params.h", "noise.h", "attn_fwd_kernel.hpp", "attn_split.hpp", os.path.join("..", "..", "include", "ft_abi.h"),
            os.path.join("..", "..", "include", "ft_diag.h")]
 # packed fp32 VALU ops are disabled on purpose: some forms have produced wrong results on this hardware
@@ -89,9 +90,13 @@ def _link(lib_path, objs, force):
       raise RuntimeError(f"link failed:\n{res.stdout}\n{res.stderr}")
 
 
-def ffi_path():
+def module_path(name):
   import sysconfig
-  return os.path.join(HERE, "ft_ffi" + sysconfig.get_config_var("EXT_SUFFIX"))
+  return os.path.join(HERE, name + sysconfig.get_config_var("EXT_SUFFIX"))
+
+
+def ffi_path():
+  return module_path("ft_ffi")
 
 
 def _build_ffi(force):
@@ -104,12 +109,29 @@ def _build_ffi(force):
   deps = [src, os.path.join(HERE, "..", "include", "ft_abi.h"), LIB_PATH]
   if not force and not _stale(out, deps):
     return out
-  cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
-         "-I" + pybind11.get_include(), "-I" + sysconfig.get_paths()["include"], src, "-o", out,
-         "-L" + HERE, "-lflashtensor_hip", "-Wl,-rpath,$ORIGIN"]
+  _module(src, out, ["-I" + pybind11.get_include(), "-I" + sysconfig.get_paths()["include"]], [])
+  return out
+
+
+def _module(src, out, includes, libs):
+  cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden"] + includes + [
+      src, "-o", out, "-L" + HERE, "-lflashtensor_hip", "-Wl,-rpath,$ORIGIN"] + libs
   res = subprocess.run(cmd, capture_output=True, text=True)
   if res.returncode != 0:
-    raise RuntimeError(f"building ft_ffi failed:\n{res.stdout}\n{res.stderr}")
+    raise RuntimeError(f"building {os.path.basename(out)} failed:\n{res.stdout}\n{res.stderr}")
+
+
+def _build_ops(force):
+  """g++ on csrc/ops_torch.cpp against torch's headers; torch's libraries are loaded by the time the module is imported."""
+  import sysconfig
+  import torch
+  from torch.utils import cpp_extension
+  out = module_path("ft_ops")
+  src = os.path.join(CSRC, OPS_SOURCE)
+  if force or _stale(out, [src, os.path.join(HERE, "..", "include", "ft_abi.h"), LIB_PATH]):
+    includes = ["-isystem" + p for p in cpp_extension.include_paths()] + ["-I" + sysconfig.get_paths()["include"]]
+    libs = ["-L" + p for p in cpp_extension.library_paths()] + ["-lc10", "-ltorch_cpu", "-ltorch", "-ltorch_python"]
+    _module(src, out, includes + [f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"], libs)
   return out
 
 
@@ -121,9 +143,9 @@ def build(force=False, verbose=True):
   objs = [o for o, _ in results]
   _link(LIB_PATH, objs[:len(SOURCES)], force)
   _link(DIAG_LIB_PATH, objs[len(SOURCES):], force)
-  ffi = _build_ffi(force)
+  ffi, ops = _build_ffi(force), _build_ops(force)
   if verbose:
-    print(f"built {LIB_PATH}, {DIAG_LIB_PATH} and {ffi}")
+    print(f"built {LIB_PATH}, {DIAG_LIB_PATH}, {ffi} and {ops}")
   return LIB_PATH
 
 

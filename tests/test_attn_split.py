@@ -4,7 +4,7 @@ import pytest
 import torch
 
 import oracle
-from flashtensor_amd import ops
+from flashtensor_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -37,8 +37,13 @@ def test_a_workspace_without_room_for_the_shares_keeps_blocks_whole(gpu, monkeyp
   """The C ABI takes any workspace of at least ft_workspace_bytes(); only one of ft_workspace_bytes_split() lets it split."""
   monkeypatch.setenv("FT_ATTN_FORM", "s1")
   q, k, v = (torch.randn(1, s, 2, 64, dtype=torch.float16, device=gpu) for s in (4, 500, 500))
-  k_ = ops._k()
-  a = ops._args(q, k, v, torch.empty_like(q), ops._flags(True, False))
+  k_ = _lib.ffi().kernels
+
+  def args(o):
+    return k_.AttnArgs(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), *(t.stride()[:3] for t in (q, k, v, o)), 1, 2, 4, 500, 64,
+                       k_.F16, k_.CAUSAL, 2)
+
+  a = args(torch.empty_like(q))
   need, more = (f(k_.OP_COLSTATS, a) for f in (k_.workspace_bytes, k_.workspace_bytes_split))
   assert more > need == 2 * 4 * 4
   ref = ops.h2o(q, k, v)
@@ -46,5 +51,5 @@ def test_a_workspace_without_room_for_the_shares_keeps_blocks_whole(gpu, monkeyp
     out = torch.empty_like(q)
     score = torch.empty(1, 2, 500, device=gpu)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=gpu)
-    k_.attn_colstats_fwd(ops._args(q, k, v, out, ops._flags(True, False)), score.data_ptr(), 0, ws.data_ptr(), nbytes, ops._stream(q))
+    k_.attn_colstats_fwd(args(out), score.data_ptr(), 0, ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream)
     assert (out.float() - ref[0].float()).norm() <= 1e-3 * ref[0].float().norm() and torch.allclose(score, ref[1], rtol=1e-4)
