@@ -14,12 +14,12 @@ DIAG_LIB_PATH = os.path.join(_HERE, "libflashtensor_diag.so")  # include/ft_diag
 FT_OK, FT_EINVAL, FT_EUNSUPPORTED, FT_ELAUNCH, FT_EWORKSPACE = 0, -1, -2, -3, -4
 FT_F16, FT_BF16, FT_F32 = 0, 1, 2
 FT_CAUSAL, FT_FAST_LOGITS = 1, 2
-FT_OP_ATTN, FT_OP_COLSTATS, FT_OP_KEYFORMER, FT_OP_EA, FT_OP_SIMA, FT_OP_CORM = 0, 1, 2, 3, 4, 5
+FT_OP_ATTN, FT_OP_COLSTATS, FT_OP_KEYFORMER, FT_OP_EA, FT_OP_SIMA, FT_OP_CORM, FT_OP_SNAPKV = 0, 1, 2, 3, 4, 5, 6
 ABI_VERSION = 5
 
 # every symbol include/ft_abi.h declares
 EXPORTS = ("ft_abi_version", "ft_last_error", "ft_workspace_bytes", "ft_workspace_bytes_split", "ft_attn_fwd", "ft_attn_fwd_ws", "ft_attn_colstats_fwd", "ft_attn_colstats_fwd_static",
-           "ft_keyformer_fwd", "ft_attn_softcap_fwd", "ft_corm_fwd", "ft_avgpool1d", "ft_linattn_fwd", "ft_topk",
+           "ft_keyformer_fwd", "ft_attn_softcap_fwd", "ft_corm_fwd", "ft_snapkv_fwd", "ft_avgpool1d", "ft_linattn_fwd", "ft_topk",
            "ft_noise_exp_fill", "ft_noise_exp_fill_host", "ft_linattn_block_workspace_bytes", "ft_linattn_block_fwd")
 
 
@@ -90,6 +90,8 @@ def load():
   lib.ft_attn_softcap_fwd.argtypes = [args_p, ctypes.c_float, f32p, vp]
   lib.ft_corm_fwd.restype = ctypes.c_int
   lib.ft_corm_fwd.argtypes = [args_p, f32p, ctypes.c_int64, vp, f32p, vp, ctypes.c_size_t, vp]
+  lib.ft_snapkv_fwd.restype = ctypes.c_int
+  lib.ft_snapkv_fwd.argtypes = [args_p, ctypes.c_int32, f32p, vp, ctypes.c_size_t, vp]
   lib.ft_avgpool1d.restype = ctypes.c_int
   lib.ft_avgpool1d.argtypes = [f32p, ctypes.c_int64, ctypes.c_int32, ctypes.c_int32, f32p, vp]
   lib.ft_linattn_fwd.restype = ctypes.c_int

@@ -19,9 +19,9 @@
 
 namespace ft {
 hipError_t launch_attn_fwd(const AttnKernelParams& p, int D, bool bf16, bool causal, bool emu, int kf, hipStream_t s);
-const SplitPlan& split_plan(int B, int H, int group, int Sq, int Skv, int D, bool causal, bool cap);
-hipError_t launch_attn_split(const AttnKernelParams& p, const SplitPlan& plan, float* part, int D, bool bf16, bool causal, bool emu, int kf,
-                             hipStream_t s);
+const SplitPlan& split_plan(int B, int H, int group, int Sq, int Skv, int D, bool causal, bool cap, bool stats);
+hipError_t launch_attn_split(const AttnKernelParams& p, const SplitPlan& plan, char* ws, const SplitStats* stats, int D, bool bf16, bool causal,
+                             bool emu, int kf, hipStream_t s);
 hipError_t launch_colstats(const ColstatsKernelParams& p, int D, bool bf16, bool causal, bool emu, int mode,
                            hipStream_t s);
 hipError_t launch_linattn(const FtAttnArgs& a, int kind, int normalize_q, int out_dtype, void* ws, hipStream_t s);
@@ -246,9 +246,13 @@ size_t colstats_bytes(const FtAttnArgs* a) {
   return lse_bytes(a) + (group_of(a) > 1 ? (size_t)a->B * a->H * a->Skv * sizeof(float) : 0);
 }
 
+// SnapKV: the sums in front of their window means, behind the column sums' own scratch
+size_t snapkv_bytes(const FtAttnArgs* a) { return colstats_bytes(a) + (size_t)a->B * (a->H / group_of(a)) * a->Skv * sizeof(float); }
+
 size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
-const ft::SplitPlan& split_of(const FtAttnArgs* a, int kf) {
-  return ft::split_plan(a->B, a->H, group_of(a), a->Sq, a->Skv, a->D, a->flags & FT_CAUSAL, kf == ft::kKfSoftcap);
+const ft::SplitPlan& split_of(const FtAttnArgs* a, int kf, bool stats = false) {
+  return ft::split_plan(a->B, a->H, group_of(a), a->Sq, a->Skv, a->D, a->flags & FT_CAUSAL, kf == ft::kKfSoftcap,
+                        stats && !(a->flags & FT_FAST_LOGITS));
 }
 
 // The attention pass of the modes that have a split form (plain softmax, soft-cap): split where the plan says so and
@@ -258,7 +262,7 @@ hipError_t run_attn(const FtAttnArgs* a, const ft::AttnKernelParams& p, int kf, 
   const ft::SplitPlan& plan = split_of(a, kf);
   char* part = ws ? static_cast<char*>(ws) + align256(used) : nullptr;
   if (plan.chunk_tiles && (!plan.bytes || (part && aligned16(part) && align256(used) + plan.bytes <= ws_bytes)))
-    return ft::launch_attn_split(p, plan, reinterpret_cast<float*>(part), a->D, bf16, causal, emu, kf, (hipStream_t)stream);
+    return ft::launch_attn_split(p, plan, part, nullptr, a->D, bf16, causal, emu, kf, (hipStream_t)stream);
   return ft::launch_attn_fwd(p, a->D, bf16, causal, emu, kf, (hipStream_t)stream);
 }
 
@@ -272,24 +276,36 @@ int validate_colstats(const FtAttnArgs* a, const float* colsum, const float* col
 }
 
 // attention pass (writes the row normalisers to the scratch), column pass, group mean when grouped; `ws` holds
-// at least colstats_bytes(a) bytes.  Every scratch element that is read has been written earlier in the same call.
-int run_colstats(const FtAttnArgs* a, float* colsum, float* colsumsq, void* ws, size_t ws_bytes, void* stream) {
+// at least `used` >= colstats_bytes(a) bytes.  pool: the sums go to `raw` and their window means to colsum.  Every scratch element that is read has been written earlier in the same call.
+int run_colstats(const FtAttnArgs* a, float* colsum, float* colsumsq, int pool, float* raw, void* ws, size_t used, size_t ws_bytes, void* stream) {
   const int group = group_of(a);
   const bool emu = !(a->flags & FT_FAST_LOGITS);
   const bool causal = a->flags & FT_CAUSAL;
   float* lse = static_cast<float*>(ws);
-  float* per_head = group > 1 ? lse + (size_t)a->B * a->H * a->Sq : colsum;
+  float* sums = pool ? raw : colsum;
+  float* per_head = group > 1 ? lse + (size_t)a->B * a->H * a->Sq : sums;
   ft::AttnKernelParams p = attn_params(a, emu);
   p.lse = lse;
-  hipError_t e = run_attn(a, p, ft::kKfNone, ws, colstats_bytes(a), ws_bytes, stream);
+  const ft::SplitPlan& plan = split_of(a, ft::kKfNone, true);
+  char* rest = static_cast<char*>(ws) + align256(used);
+  if (plan.logit_tiles && pool <= ft::kSplitMaxPool && aligned16(rest) && align256(used) + plan.bytes <= ws_bytes) {
+    const ft::SplitStats stats{colsum, colsumsq, pool};
+    hipError_t e = ft::launch_attn_split(p, plan, rest, &stats, a->D, a->dtype == FT_BF16, causal, emu, ft::kKfNone, (hipStream_t)stream);
+    return e == hipSuccess ? (int)FT_OK : hip_fail(e, "attn with column sums launch");
+  }
+  hipError_t e = run_attn(a, p, ft::kKfNone, ws, used, ws_bytes, stream);
   if (e != hipSuccess) return hip_fail(e, "attn_fwd launch");
   ft::ColstatsKernelParams c = col_params(a, emu, lse, per_head, colsumsq);
   e = ft::launch_colstats(c, a->D, a->dtype == FT_BF16, causal, emu, colsumsq ? ft::kStatSumSq : ft::kStatSum,
                           (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(e, "colstats launch");
   if (group > 1) {
-    e = ft::launch_group_mean(per_head, (int64_t)a->B * a->Hkv, group, a->Skv, colsum, (hipStream_t)stream);
+    e = ft::launch_group_mean(per_head, (int64_t)a->B * a->Hkv, group, a->Skv, sums, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "group mean launch");
+  }
+  if (pool) {
+    e = ft::launch_avgpool1d(raw, (int64_t)a->B * (a->H / group), a->Skv, pool, colsum, (hipStream_t)stream);
+    if (e != hipSuccess) return hip_fail(e, "avgpool1d launch");
   }
   return FT_OK;
 }
@@ -338,6 +354,8 @@ size_t ft_workspace_bytes(int op, const FtAttnArgs* a) {
       return 0;
     case FT_OP_COLSTATS:
       return colstats_bytes(a);
+    case FT_OP_SNAPKV:
+      return snapkv_bytes(a);
     case FT_OP_KEYFORMER:
     case FT_OP_CORM:
       return lse_bytes(a);
@@ -352,9 +370,10 @@ size_t ft_workspace_bytes(int op, const FtAttnArgs* a) {
 size_t ft_workspace_bytes_split(int op, const FtAttnArgs* a) {
   if (!a) return 0;
   const size_t need = ft_workspace_bytes(op, a);
-  if (op != FT_OP_ATTN && op != FT_OP_COLSTATS && op != FT_OP_CORM) return need;
+  if (op != FT_OP_ATTN && op != FT_OP_COLSTATS && op != FT_OP_CORM && op != FT_OP_SNAPKV) return need;
   if (a->B < 1 || a->H < 1 || a->Sq < 1 || a->Skv < 1 || a->Hkv < 0 || a->Hkv > a->H || (a->Hkv > 0 && a->H % a->Hkv)) return need;
   size_t split = split_of(a, ft::kKfNone).bytes;
+  if (op == FT_OP_COLSTATS || op == FT_OP_SNAPKV) split = std::max(split, split_of(a, ft::kKfNone, true).bytes);
   if (op == FT_OP_ATTN) split = std::max(split, split_of(a, ft::kKfSoftcap).bytes);
   return split ? align256(need) + split : need;
 }
@@ -379,7 +398,7 @@ int ft_attn_colstats_fwd(const FtAttnArgs* a, float* colsum, float* colsumsq, vo
   if (!workspace || workspace_bytes < need)
     return fail(FT_EWORKSPACE, "workspace of %zu bytes needed, got %zu", need, workspace ? workspace_bytes : (size_t)0);
   if (reinterpret_cast<uintptr_t>(workspace) & 3u) return fail(FT_EINVAL, "workspace must be 4-byte aligned");
-  return run_colstats(a, colsum, colsumsq, workspace, workspace_bytes, stream);
+  return run_colstats(a, colsum, colsumsq, 0, nullptr, workspace, need, workspace_bytes, stream);
 }
 
 int ft_attn_colstats_fwd_static(const FtAttnArgs* a, float* colsum, float* colsumsq, void* stream) {
@@ -390,7 +409,19 @@ int ft_attn_colstats_fwd_static(const FtAttnArgs* a, float* colsum, float* colsu
                 need, (size_t)FT_STATIC_SCRATCH_BYTES);
   void* ws = nullptr;
   if (int rc = static_scratch(&ws, (hipStream_t)stream)) return rc;
-  return run_colstats(a, colsum, colsumsq, ws, need, stream);
+  return run_colstats(a, colsum, colsumsq, 0, nullptr, ws, need, need, stream);
+}
+
+int ft_snapkv_fwd(const FtAttnArgs* a, int32_t kernel, float* pooled, void* workspace, size_t workspace_bytes, void* stream) {
+  if (int rc = validate_colstats(a, pooled, nullptr)) return rc;
+  if (kernel < 1 || (kernel & 1) == 0) return fail(FT_EINVAL, "kernel must be odd and positive (got %d): only then is the output as long as the input", kernel);
+  if ((int64_t)a->B * (a->H / group_of(a)) > 65535) return fail(FT_EUNSUPPORTED, "too many rows");
+  const size_t need = snapkv_bytes(a);
+  if (!workspace || workspace_bytes < need)
+    return fail(FT_EWORKSPACE, "workspace of %zu bytes needed, got %zu", need, workspace ? workspace_bytes : (size_t)0);
+  if (reinterpret_cast<uintptr_t>(workspace) & 3u) return fail(FT_EINVAL, "workspace must be 4-byte aligned");
+  float* raw = reinterpret_cast<float*>(static_cast<char*>(workspace) + colstats_bytes(a));
+  return run_colstats(a, pooled, nullptr, kernel, raw, workspace, need, workspace_bytes, stream);
 }
 
 int ft_keyformer_fwd(const FtAttnArgs* a, const FtNoise* noise, float tau, float* kf_score, void* workspace,

@@ -49,7 +49,8 @@ __device__ __forceinline__ SplitPartial split_partial(float* base, int D, int64_
 // whole group, and it walks only its share of the row block's key tiles; where a block has several shares, each leaves
 // its accumulator, row maxima and row sums in the workspace and attn_combine_kernel folds them.  Built for the causal
 // instantiation only: without a mask `off` is set to Skv, which hides nothing.
-template <typename T, int D, bool CAUSAL, bool EMU, int KF, int WAVES, bool SPLIT = false>
+// STORE: the 16-bit logits of the rows go to the workspace as well, for the column sums (attn_split.hip).
+template <typename T, int D, bool CAUSAL, bool EMU, int KF, int WAVES, bool SPLIT = false, bool STORE = false>
 __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVES)) attn_fwd_kernel(const AttnKernelParams p) {
   constexpr int BM = 32 * WAVES, BN = kAttnBN, NT = 64 * WAVES;
   constexpr int KSTEPS = D / 16;
@@ -83,6 +84,7 @@ __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVE
   __shared__ __align__(16) char ldsEr[kErLds ? WAVES * kErWaveBytes : 16];
 
   static_assert(!SPLIT || (CAUSAL && WAVES == 4 && (KF == kKfNone || KF == kKfSoftcap)), "the split form's instantiations");
+  static_assert(!STORE || (SPLIT && EMU && KF == kKfNone), "logits are kept where they are 16-bit values");
   const int rows = SPLIT ? p.Sq * p.group : p.Sq;  // rows of a (b, h) pair; SPLIT: of a (b, k/v head) pair
   const int BH = SPLIT ? p.B * (p.H / p.group) : p.B * p.H;
   const int nMB = (rows + BM - 1) / BM;
@@ -147,6 +149,15 @@ __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVE
 
   // tiles of the workgroup, of this wave (not entirely above its diagonal), and of this wave's mask-free prefix
   const int wave_row0 = m0 + wave * 32;
+  // STORE: logits [pair][row][key].  A lane has keys 16 b + 4 g + [0..3] and + 8 of its row; the halves of the wave swap
+  // four keys each, so that a lane stores eight neighbours
+  uint16_t* logit_row = STORE ? p.logits + ((int64_t)bh * rows + qrow_c) * (p.logit_tiles * BN) + 8 * g : nullptr;
+  auto store_logits = [&](int b16, uint32_t a0, uint32_t a1, uint32_t b0, uint32_t b1) __attribute__((always_inline)) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const auto s0 = __builtin_amdgcn_permlane32_swap(a0, b0, false, false), s1 = __builtin_amdgcn_permlane32_swap(a1, b1, false, false);
+    if (qrow < rows) *reinterpret_cast<uint4v*>(logit_row + 16 * b16) = uint4v{s0[0], s1[0], s0[1], s1[1]};
+#endif
+  };
   int Skv = p.Skv, off = p.off;  // SPLIT: counted from the first key of the workgroup's share
   int n_end = Skv;
   if (CAUSAL) n_end = min(Skv, (SPLIT ? (min(m0 + BM, rows) - 1) / p.group + 1 : m0 + BM) + off);
@@ -158,6 +169,7 @@ __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVE
     kbase += (int64_t)t0 * BN * p.sk.s;
     vbase += (int64_t)t0 * BN * p.sv.s;
     off -= t0 * BN;
+    if (STORE) logit_row += t0 * BN;
     Skv = min(Skv, t1 * BN) - t0 * BN;
     ntiles = t1 - t0;  // >= 1: (nch - 1) per <= (nch - 1) chunk_tiles < tiles of the block
   }
@@ -361,7 +373,7 @@ __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVE
     return amax * p.logit_mul;  // logit_mul = log2e / sqrt(D) when the logits stay in fp32
   };
   // MASKED: key j of the tile is hidden from this lane's query when j > qi + off or j >= Skv.
-  auto fast_exp = [&](auto masked_tag, const float16v (&s)[2], vec8 (&pb)[4], int n0, int buf) __attribute__((always_inline)) {
+  auto fast_exp = [&](auto masked_tag, const float16v (&s)[2], vec8 (&pb)[4], int n0, int it) __attribute__((always_inline)) {
     constexpr bool MASKED = decltype(masked_tag)::value;
     const float neg_m = -m_run;
     const half2v pk_hi = __builtin_bit_cast(half2v, p.pk_hi2), pk_lo = __builtin_bit_cast(half2v, p.pk_lo2);
@@ -383,6 +395,9 @@ __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVE
           // ... divided by sqrt(D) in fp16: t2 = 8 * f16(h / sqrt(D)), exact for D = 64, two packed ops for D = 128
           t2[i] = D == 64 ? h2 : __builtin_elementwise_fma(h2, pk_hi, h2 * pk_lo);
         }
+        if (STORE)
+          store_logits(it * 4 + blk, __builtin_bit_cast(uint32_t, t2[0]), __builtin_bit_cast(uint32_t, t2[1]),
+                       __builtin_bit_cast(uint32_t, t2[2]), __builtin_bit_cast(uint32_t, t2[3]));
 #pragma unroll
         for (int i = 0; i < 8; ++i)
           x[i] = kCap ? (float)t2[i >> 1][i & 1] * (rcp_cap * 0.125f)  // logit / cap, rounded below
@@ -390,13 +405,16 @@ __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVE
       } else if constexpr (EMU) {
         // bf16: round QK^T, multiply by the tuned constant (== dividing by sqrt(D) in bf16), round again; the
         // conversions handle two elements each, unpacking a half is a shift or a mask
+        uint32_t tw[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const uint32_t h2 = T::pack2(s[mbk][rb + 2 * i], s[mbk][rb + 2 * i + 1]);
           const uint32_t t2 = T::pack2(T::lo(h2) * p.logit_mul, T::hi(h2) * p.logit_mul);
+          tw[i] = t2;
           x[2 * i] = kCap ? T::lo(t2) * rcp_cap : __builtin_fmaf(T::lo(t2), kLog2e, neg_m);
           x[2 * i + 1] = kCap ? T::hi(t2) * rcp_cap : __builtin_fmaf(T::hi(t2), kLog2e, neg_m);
         }
+        if (STORE) store_logits(it * 4 + blk, tw[0], tw[1], tw[2], tw[3]);
       } else {
 #pragma unroll
         for (int i = 0; i < 8; ++i)
@@ -435,7 +453,7 @@ __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVE
       // 32 mbk + 8 (rb / 4 [+ 1]) + 4 g + [0..3] are two aligned groups of four in LDS
       float ee[8];
       if constexpr (kKfFast) {
-        const uint32_t* col = ldsCol + buf * BN + 32 * mbk + 2 * rb + 4 * g;
+        const uint32_t* col = ldsCol + (it & 1) * BN + 32 * mbk + 2 * rb + 4 * g;
         const uint4v c0 = *reinterpret_cast<const uint4v*>(col), c1 = *reinterpret_cast<const uint4v*>(col + 8);
 #pragma unroll
         for (int i = 0; i < 8; ++i)  // log2 u = -E / ln 2 (negative): the constant factor is applied once, at the end
@@ -602,7 +620,7 @@ __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVE
     qk(s_next, tk_next);
     if (kKfFast && STAGE && threadIdx.x < BN)  // column terms of tile it + 1 (the other half of ldsCol)
       ldsCol[((it + 1) & 1) * BN + threadIdx.x] = noise_col(nk, (uint32_t)((it + 1) * BN + threadIdx.x));
-    fast_exp(masked_tag, s_cur, pb, n0, it & 1);
+    fast_exp(masked_tag, s_cur, pb, n0, it);
     pv(pb, tv);
     pend_max = tile_max(next_masked_tag, s_next, n0 + BN);
     __builtin_amdgcn_sched_group_barrier(0x100, 6, 2);

@@ -16,9 +16,9 @@ namespace {
 
 struct SplitShape {
   int B, H, group, Sq, Skv, D, forced, cus;
-  bool causal, cap;
+  bool causal, cap, stats;
   bool operator==(const SplitShape& o) const {
-    return B == o.B && H == o.H && group == o.group && Sq == o.Sq && Skv == o.Skv && D == o.D && forced == o.forced && cus == o.cus && causal == o.causal && cap == o.cap;
+    return B == o.B && H == o.H && group == o.group && Sq == o.Sq && Skv == o.Skv && D == o.D && forced == o.forced && cus == o.cus && causal == o.causal && cap == o.cap && stats == o.stats;
   }
 };
 
@@ -70,9 +70,11 @@ SplitPlan make_plan(const SplitShape& a) {
                                          : std::max(longest * alone, sum * shared_cu / (2.0 * cus) + 0.25 * longest * alone);
     return kLaunch + std::max(work, kv_us) + 0.25 * std::min(work, kv_us);
   };
-  double best;
+  // few rows: the column sums come from kept logits (2 bytes a pair each way against K once more and another launch)
+  const bool keep = a.stats && rows <= kSplitStatRows;
+  double best = 1e30;
   int best_chunk = 0;
-  {  // the unsplit form: a workgroup per 128 queries of a head
+  if (!keep) {  // the unsplit form: a workgroup per 128 queries of a head
     const int nq = (a.Sq + 127) / 128;
     int64_t sum = 0;
     for (int i = 0; i < nq; ++i) sum += (std::min(a.Skv, std::min(i * 128 + 128, a.Sq) + off) + 63) / 64;
@@ -119,34 +121,80 @@ SplitPlan make_plan(const SplitShape& a) {
   }
   plan.one_per_cu = plan.items * pairs <= cus;
   if (plan.first_shared < nMB) plan.bytes = (size_t)(pairs * plan.items * part_waves * split_wave_floats(a.D)) * sizeof(float);
+  if (keep) {
+    plan.logit_tiles = (a.Skv + 63) / 64;
+    plan.logits_at = plan.bytes;
+    plan.bytes += (size_t)(pairs * rows * plan.logit_tiles) * 64 * sizeof(uint16_t);
+  }
   return plan;
 }
 
 }  // namespace
 
 // The plan of a shape costs some microseconds and a program calls with few shapes: each thread keeps its last ones.
-const SplitPlan& split_plan(int B, int H, int group, int Sq, int Skv, int D, bool causal, bool cap) {
+// stats: column sums of rounded logits are wanted too
+const SplitPlan& split_plan(int B, int H, int group, int Sq, int Skv, int D, bool causal, bool cap, bool stats) {
   struct Entry {
     SplitShape shape{};
     SplitPlan plan{};
   };
   constexpr int kEntries = 16;
   static thread_local Entry kept[kEntries];
-  const SplitShape shape{B, H, group, Sq, Skv, D, attn_split_override(), device_cu_count(), causal, cap};
-  Entry& e = kept[(unsigned)(B * 31 + H * 7 + group * 3 + Sq * 5 + Skv + D + cap) % kEntries];
+  const SplitShape shape{B, H, group, Sq, Skv, D, attn_split_override(), device_cu_count(), causal, cap, stats};
+  Entry& e = kept[(unsigned)(B * 31 + H * 7 + group * 3 + Sq * 5 + Skv + D + cap + 2 * stats) % kEntries];
   if (!(e.shape == shape)) e = Entry{shape, make_plan(shape)};
   return e.plan;
 }
 
-// One workgroup per (wave of 32 rows of a shared block, 32 channels), a wave per four of a lane's 16 channels: weights of
+namespace {
+
+__device__ __forceinline__ int shares_of_block(const AttnKernelParams& p, int mb) {
+  const int n_end = min(p.Skv, (min(mb * 128 + 128, p.Sq * p.group) - 1) / p.group + 1 + p.off);
+  return ((n_end + kAttnBN - 1) / kAttnBN + p.chunk_tiles - 1) / p.chunk_tiles;
+}
+
+// Folds the shares of a row, eight loads at a time: running maximum and sum, and what `f(share, weight)` adds up;
+// `scale` multiplies that when the maximum moves.  slot0: the row's wave in the first share, n: the row in the wave; every
+// `step`-th share is taken.  A part whose shares hide every key from the row leaves M = -inf, sum = 0.
+template <typename L, typename F, typename S>
+__device__ __forceinline__ void fold_shares(const AttnKernelParams& p, int D, int64_t slot0, int n, int nch, int step, float& M, float& sum, L load, F f, S scale) {
+  constexpr int U = 8;
+  M = -__builtin_inff(), sum = 0.f;
+  for (int c0 = 0; c0 < nch; c0 += U) {
+    float m[U], l[U];
+    float4v o[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {  // shares past the last one re-read it, with weight 0
+      const SplitPartial s = split_partial(p.part, D, slot0 + (int64_t)min(c0 + u, nch - 1) * step * p.part_waves);
+      m[u] = s.m[n];
+      l[u] = s.l[n];
+      load(s, o[u]);
+    }
+    float M1 = M;
+#pragma unroll
+    for (int u = 0; u < U; ++u) M1 = fmaxf(M1, m[u]);
+    const float base = M1 == -__builtin_inff() ? 0.f : M1;
+    const float move = __builtin_amdgcn_exp2f(M - base);
+    sum *= move;
+    scale(move);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const float w = c0 + u < nch ? __builtin_amdgcn_exp2f(m[u] - base) : 0.f;  // 0 too for a share that hides every key from the row
+      sum = __builtin_fmaf(w, l[u], sum);
+      f(o[u], w);
+    }
+    M = M1;
+  }
+}
+
+// One workgroup per (wave of 32 rows of a shared block, 32 channels), a wave for four of a lane's 16 channels: weights of
 // the shares from their row maxima, then the shares' accumulators in their own register layout (every load is 1 KB
-// contiguous).  Bound by the latency of its loads, so eight shares are requested at a time.
+// contiguous).  Bound by the latency of its loads.
 template <typename T, int D>
-__global__ void __launch_bounds__(256) attn_combine_kernel(const AttnKernelParams p, int first_shared) {
-  constexpr int DB = D / 32, U = 8;
+__device__ __forceinline__ void combine_rows(const AttnKernelParams& p, int first_shared, int i) {
+  constexpr int DB = D / 32;
   const int rows = p.Sq * p.group, Hkv = p.H / p.group;
-  const int nMB = (rows + 127) / 128, nshared = nMB - first_shared;
-  int i = blockIdx.x;
+  const int nshared = (rows + 127) / 128 - first_shared;
   const int db = i % DB;
   i /= DB;
   const int wv = i % p.part_waves;
@@ -155,37 +203,19 @@ __global__ void __launch_bounds__(256) attn_combine_kernel(const AttnKernelParam
   const int lane = lane_id(), q4 = wave_id(), g = lane >> 5, n = lane & 31;
   const int row = mb * 128 + wv * 32 + n;
   if (row >= rows) return;
-  const int n_end = min(p.Skv, (min(mb * 128 + 128, rows) - 1) / p.group + 1 + p.off);
-  const int nch = ((n_end + kAttnBN - 1) / kAttnBN + p.chunk_tiles - 1) / p.chunk_tiles;
   const int64_t slot0 = ((int64_t)bh * p.nitems + p.first_item[mb]) * p.part_waves + wv;
-  float M = -__builtin_inff(), L = 0.f;
+  float M, L;
   float4v acc = {0.f, 0.f, 0.f, 0.f};
-  for (int c0 = 0; c0 < nch; c0 += U) {
-    float m[U], l[U];
-    float4v o[U];
+  fold_shares(p, D, slot0, n, shares_of_block(p, mb), 1, M, L,
+              [&](const SplitPartial& s, float4v& o) { o = *reinterpret_cast<const float4v*>(s.o + ((db * 4 + q4) * 64 + lane) * 4); },
+              [&](const float4v& o, float w) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) {  // shares past the last one re-read it, with weight 0
-      const SplitPartial s = split_partial(p.part, D, slot0 + (int64_t)min(c0 + u, nch - 1) * p.part_waves);
-      m[u] = s.m[n];
-      l[u] = s.l[n];
-      o[u] = *reinterpret_cast<const float4v*>(s.o + ((db * 4 + q4) * 64 + lane) * 4);
-    }
-    float M1 = M;
+                for (int e = 0; e < 4; ++e) acc[e] = __builtin_fmaf(w, o[e], acc[e]);
+              },
+              [&](float move) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) M1 = fmaxf(M1, m[u]);
-    const float f = __builtin_amdgcn_exp2f(M - M1);  // share 0 sees every row's first key: M1 is finite
-    L *= f;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) acc[e] *= f;
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const float w = c0 + u < nch ? __builtin_amdgcn_exp2f(m[u] - M1) : 0.f;  // 0 too for a share that hides every key from the row
-      L = __builtin_fmaf(w, l[u], L);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) acc[e] = __builtin_fmaf(w, o[u][e], acc[e]);
-    }
-    M = M1;
-  }
+                for (int e = 0; e < 4; ++e) acc[e] *= move;
+              });
   const float inv = 1.f / L;
   const int b = bh / Hkv, h = (bh % Hkv) * p.group + row % p.group, qi = row / p.group;
   uint16_t* optr = p.o + b * p.so.b + (int64_t)qi * p.so.s + h * p.so.h;
@@ -193,14 +223,140 @@ __global__ void __launch_bounds__(256) attn_combine_kernel(const AttnKernelParam
   if (db == 0 && q4 == 0 && g == 0 && p.lse) p.lse[((int64_t)b * p.H + h) * p.Sq + qi] = M + __builtin_amdgcn_logf(L);
 }
 
-hipError_t launch_attn_split(const AttnKernelParams& p0, const SplitPlan& plan, float* part, int D, bool bf16, bool causal, bool emu, int kf,
-                             hipStream_t s) {
+template <typename T, int D>
+__global__ void __launch_bounds__(256) attn_combine_kernel(const AttnKernelParams p, int first_shared) {
+  combine_rows<T, D>(p, first_shared, blockIdx.x);
+}
+
+// The column sums of few rows from their kept logits, and (the last `gridDim.x - ncol` workgroups) the folding of the
+// shares: one launch where the column pass would read K a second time, per query head, behind the launch that folds.
+// B4 H32/8 Sq1 Skv4097: 31 + 5 us (column pass, group mean) -> under 2 on top of the folding's 4.
+// A workgroup takes 512 keys of one (b, k/v head), eight of them per lane; its waves share out the rows and meet in LDS.
+// A wave requests all of its rows (1 KB each) before the row normalisers are folded.
+constexpr int kStatTiles = 8;
+__host__ __device__ constexpr int stat_step(int pool) { return pool ? kStatTiles - 1 : kStatTiles; }  // half a tile on either side for the window
+
+template <typename T, int D, bool SQ>
+__global__ void __launch_bounds__(256) split_stats_kernel(const AttnKernelParams p, const SplitStats st, int ncol) {
+  if ((int)blockIdx.x >= ncol) {
+    combine_rows<T, D>(p, 0, blockIdx.x - ncol);
+    return;
+  }
+  constexpr int KT = kStatTiles * kAttnBN;
+  constexpr bool kF16 = __is_same(typename T::elem, _Float16);
+  __shared__ float s_nlse[kSplitStatRows];
+  __shared__ __align__(16) float s_sum[4][KT];
+  __shared__ __align__(16) float s_sq[SQ ? 4 : 1][SQ ? KT : 4];
+  const int rows = p.Sq * p.group, Hkv = p.H / p.group, pairs = p.B * Hkv;
+  const int bh = blockIdx.x % pairs, tile = blockIdx.x / pairs;
+  const int t = threadIdx.x, lane = lane_id(), wave = wave_id();
+  const int tile0 = tile * stat_step(st.pool) - (st.pool ? 1 : 0);
+  const int k0 = 8 * lane, j0 = tile0 * kAttnBN + k0;  // the lane's first key, of the workgroup's and of the row
+  const int stride = p.logit_tiles * kAttnBN;
+  const uint16_t* col = p.logits + (int64_t)bh * rows * stride + max(0, min(j0, stride - 8));
+  const int per = (rows + 3) >> 2;  // rows of a wave, the last ones past the end
+  float sum[8] = {}, sq[8] = {};
+  auto rows_of_wave = [&](auto n_tag) __attribute__((always_inline)) {
+    constexpr int N = decltype(n_tag)::value;
+    uint4v w[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int r = min(wave * per + min(i, per - 1), rows - 1);
+      w[i] = *reinterpret_cast<const uint4v*>(col + (int64_t)r * stride);
+    }
+    // eight threads a row for its shares: one round of loads up to 64 shares
+    const int row = t & 31, part = t >> 5, rc = min(row, rows - 1);
+    const int nch = shares_of_block(p, 0);
+    if (nch > 1) {
+      float M = -__builtin_inff(), L = 0.f;
+      if (part < nch)
+        fold_shares(p, D, (int64_t)bh * p.nitems + part, rc, (nch - part + 7) >> 3, 8, M, L, [](const SplitPartial&, float4v&) {},
+                    [](const float4v&, float) {}, [](float) {});
+      s_sum[0][t] = M;
+      s_sum[1][t] = L;
+      __syncthreads();
+      if (t < 32) {
+#pragma unroll
+        for (int u = 1; u < 8; ++u) M = fmaxf(M, s_sum[0][32 * u + t]);
+        L = 0.f;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) L = __builtin_fmaf(__builtin_amdgcn_exp2f(s_sum[0][32 * u + t] - M), s_sum[1][32 * u + t], L);
+        s_nlse[t] = -(M + __builtin_amdgcn_logf(L));
+      }
+    } else if (t < 32) {
+      s_nlse[t] = -p.lse[((int64_t)(bh / Hkv) * p.H + (bh % Hkv) * p.group + rc % p.group) * p.Sq + rc / p.group];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int r = wave * per + i;
+      const float nlse = s_nlse[min(r, rows - 1)];
+      const int last = i < per && r < rows ? min(r / p.group + p.off, p.Skv - 1) : -1;  // the row's last visible key
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float x = e & 1 ? T::hi(w[i][e >> 1]) : T::lo(w[i][e >> 1]);
+        const float pr = __builtin_amdgcn_exp2f(__builtin_fmaf(x, kF16 ? kLog2e / 8.f : kLog2e, nlse));  // fp16 logits are kept times 8
+        const int j = j0 + e;
+        const float v = j >= 0 && j <= last ? pr : 0.f;  // hidden, or outside the row (what is kept there is not defined)
+        sum[e] += v;
+        if (SQ) sq[e] = __builtin_fmaf(v, v, sq[e]);
+      }
+    }
+  };
+  if (per <= 1)
+    rows_of_wave(std::integral_constant<int, 1>{});
+  else if (per <= 3)
+    rows_of_wave(std::integral_constant<int, 3>{});
+  else
+    rows_of_wave(std::integral_constant<int, kSplitStatRows / 4>{});
+#pragma unroll
+  for (int hf = 0; hf < 2; ++hf) {
+    *reinterpret_cast<float4v*>(&s_sum[wave][k0 + 4 * hf]) = float4v{sum[4 * hf], sum[4 * hf + 1], sum[4 * hf + 2], sum[4 * hf + 3]};
+    if constexpr (SQ) *reinterpret_cast<float4v*>(&s_sq[wave][k0 + 4 * hf]) = float4v{sq[4 * hf], sq[4 * hf + 1], sq[4 * hf + 2], sq[4 * hf + 3]};
+  }
+  __syncthreads();
+  float tot[KT / 256];
+#pragma unroll
+  for (int i = 0; i < KT / 256; ++i) {
+    const int k = t + 256 * i;
+    tot[i] = ((s_sum[0][k] + s_sum[1][k]) + (s_sum[2][k] + s_sum[3][k])) / (float)p.group;
+  }
+  if (st.pool) {
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < KT / 256; ++i) s_sum[0][t + 256 * i] = tot[i];
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < KT / 256; ++i) {
+    const int k = t + 256 * i, j = tile0 * kAttnBN + k;
+    if (j < 0 || j >= p.Skv) continue;
+    if (st.pool) {
+      if (k < 32 || k >= KT - 32) continue;
+      float s = 0.f;
+      for (int u = -(st.pool / 2); u <= st.pool / 2; ++u) s += s_sum[0][k + u];
+      tot[i] = s / (float)st.pool;
+    }
+    st.colsum[(int64_t)bh * p.Skv + j] = tot[i];
+    if constexpr (SQ) st.colsumsq[(int64_t)bh * p.Skv + j] = (s_sq[0][k] + s_sq[1][k]) + (s_sq[2][k] + s_sq[3][k]);
+  }
+}
+
+}  // namespace
+
+// `stats`: column sums of the rows wanted (plan.logit_tiles > 0), else null
+hipError_t launch_attn_split(const AttnKernelParams& p0, const SplitPlan& plan, char* ws, const SplitStats* stats, int D, bool bf16, bool causal,
+                             bool emu, int kf, hipStream_t s) {
   AttnKernelParams p = p0;
   p.pair_order = p.two_blocks = p.head_major = 0;
-  p.part = part;
+  p.part = reinterpret_cast<float*>(ws);
   p.chunk_tiles = plan.chunk_tiles;
   p.nitems = plan.items;
   p.part_waves = plan.part_waves;
+  if (stats) {
+    p.logits = reinterpret_cast<uint16_t*>(ws + plan.logits_at);
+    p.logit_tiles = plan.logit_tiles;
+  }
   std::copy(plan.list, plan.list + plan.items, p.items);
   std::copy(plan.first_item, plan.first_item + plan.nblocks, p.first_item);
   if (!causal) p.off = p.Skv;
@@ -209,8 +365,30 @@ hipError_t launch_attn_split(const AttnKernelParams& p0, const SplitPlan& plan, 
   // what a workgroup lacks to more than half of a CU's LDS
   const unsigned pad = plan.one_per_cu ? 88 * 1024 - 4 * kAttnBN * 2 * D : 0;
   hipError_t e = bf16 ? launch_attn_split_bf16(p, D, emu, kf, grid, pad, s) : launch_attn_split_f16(p, D, emu, kf, grid, pad, s);
-  if (e != hipSuccess || plan.first_shared == plan.nblocks) return e;
-  const dim3 cgrid((unsigned)(pairs * (plan.nblocks - plan.first_shared) * plan.part_waves * (D / 32))), cblk(256);
+  const int nshared = plan.nblocks - plan.first_shared;
+  if (e != hipSuccess || (nshared == 0 && !stats)) return e;
+  const int64_t ncomb = pairs * nshared * plan.part_waves * (D / 32);
+  if (stats) {
+    // (with a window the outputs of workgroup c end half a tile short of its keys)
+    const int step = stat_step(stats->pool) * kAttnBN;
+    const int64_t ncol = pairs * ((p.Skv + (stats->pool ? kAttnBN / 2 : 0) + step - 1) / step);
+    const dim3 g((unsigned)(ncol + ncomb)), blk(256);
+#define FT_CASE(T, DD, SQ) hipLaunchKernelGGL((split_stats_kernel<T, DD, SQ>), g, blk, 0, s, p, *stats, (int)ncol)
+    if (stats->colsumsq) {
+      if (D == 128 && bf16) FT_CASE(BF16, 128, true);
+      else if (D == 128) FT_CASE(F16, 128, true);
+      else if (bf16) FT_CASE(BF16, 64, true);
+      else FT_CASE(F16, 64, true);
+    } else {
+      if (D == 128 && bf16) FT_CASE(BF16, 128, false);
+      else if (D == 128) FT_CASE(F16, 128, false);
+      else if (bf16) FT_CASE(BF16, 64, false);
+      else FT_CASE(F16, 64, false);
+    }
+#undef FT_CASE
+    return hipGetLastError();
+  }
+  const dim3 cgrid((unsigned)ncomb), cblk(256);
   if (D == 128 && bf16) hipLaunchKernelGGL((attn_combine_kernel<BF16, 128>), cgrid, cblk, 0, s, p, plan.first_shared);
   else if (D == 128) hipLaunchKernelGGL((attn_combine_kernel<F16, 128>), cgrid, cblk, 0, s, p, plan.first_shared);
   else if (bf16) hipLaunchKernelGGL((attn_combine_kernel<BF16, 64>), cgrid, cblk, 0, s, p, plan.first_shared);

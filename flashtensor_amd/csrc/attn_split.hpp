@@ -17,6 +17,10 @@ hipError_t launch_split_td(const AttnKernelParams& p, bool emu, int kf, unsigned
     hipLaunchKernelGGL((attn_fwd_kernel<T, D, true, E, K, 4, true>), dim3(grid), dim3(256), lds, s, p);      \
     return hipGetLastError();                                                                                \
   }
+  if (p.logits && emu && kf == kKfNone) {
+    hipLaunchKernelGGL((attn_fwd_kernel<T, D, true, true, kKfNone, 4, true, true>), dim3(grid), dim3(256), lds, s, p);
+    return hipGetLastError();
+  }
   FT_CASE(true, kKfNone) FT_CASE(false, kKfNone) FT_CASE(true, kKfSoftcap) FT_CASE(false, kKfSoftcap)
 #undef FT_CASE
   return hipErrorInvalidValue;

@@ -59,6 +59,7 @@ void init_ffi_kernels(py::module_&& m) {
   m.attr("OP_EA") = (int)FT_OP_EA;
   m.attr("OP_SIMA") = (int)FT_OP_SIMA;
   m.attr("OP_CORM") = (int)FT_OP_CORM;
+  m.attr("OP_SNAPKV") = (int)FT_OP_SNAPKV;
   m.attr("STATIC_SCRATCH_BYTES") = (size_t)FT_STATIC_SCRATCH_BYTES;
 
   py::class_<FtAttnArgs>(m, "AttnArgs", py::module_local())
@@ -140,6 +141,11 @@ void init_ffi_kernels(py::module_&& m) {
                       ws_bytes, ptr<void>(stream)));
   }, py::arg("args"), py::arg("corm_mask"), py::arg("mask_row_stride"), py::arg("corm_score"), py::arg("margin"), py::arg("workspace"),
      py::arg("workspace_bytes"), py::arg("stream") = 0);
+
+  m.def("snapkv_fwd", [](const FtAttnArgs& a, int32_t kernel, uintptr_t pooled, uintptr_t ws, size_t ws_bytes, uintptr_t stream) {
+    py::gil_scoped_release nogil;
+    check(ft_snapkv_fwd(&a, kernel, ptr<float>(pooled), ptr<void>(ws), ws_bytes, ptr<void>(stream)));
+  }, py::arg("args"), py::arg("kernel"), py::arg("pooled"), py::arg("workspace"), py::arg("workspace_bytes"), py::arg("stream") = 0);
 
   m.def("avgpool1d", [](uintptr_t src, int64_t rows, int32_t S, int32_t kernel, uintptr_t dst, uintptr_t stream) {
     py::gil_scoped_release nogil;

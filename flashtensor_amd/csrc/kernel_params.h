@@ -37,6 +37,8 @@ struct AttnKernelParams {
   int two_blocks;   // 256-row form: a workgroup takes query blocks nMB - 1 - slot and slot (set by the launcher)
   int head_major;   // workgroup order inside an XCD: all blocks of a (b, h) pair before the next pair's (launcher)
   // split form (attn_split.hpp): a row block's key tiles are shared out between workgroups, at most chunk_tiles each
+  uint16_t* logits; // 16-bit logits of every row, kept for the column sums
+  int logit_tiles;
   float* part;      // workspace of the shares' partial results (may be null where no block has more than one share)
   int chunk_tiles;
   int nitems;       // shares of all row blocks of a (b, k/v head) pair
@@ -51,11 +53,21 @@ struct SplitPlan {
   int items;         // shares of a (b, k/v head) pair
   int first_shared;  // row blocks from this one on have more than one share
   int nblocks, part_waves;
+  int logit_tiles;   // logits are kept for the column sums: key tiles of a row, else 0
   bool one_per_cu;   // no more workgroups than CUs: keep them from sharing one
-  size_t bytes;      // workspace of the shares' partial results
+  size_t bytes;      // workspace of the shares' partial results and of the logits
+  size_t logits_at;  // where in it the logits begin
   uint16_t list[kSplitMaxItems];
   uint8_t first_item[kSplitMaxBlocks];
 };
+
+// What the column sums of few rows are wanted for: sums [B, Hkv, Skv] (means over a group's heads), sums of squares (no
+// groups) or null, and the odd width of SnapKV's window over the sums or 0.
+struct SplitStats {
+  float *colsum, *colsumsq;
+  int pool;
+};
+constexpr int kSplitMaxPool = 65, kSplitStatRows = 32;
 
 struct ColstatsKernelParams {
   const uint16_t* q;

@@ -216,10 +216,12 @@ PyObject* snapkv(PyObject* const* o) {
   const Qkv x(o);
   void* s = stream_of(x.q);
   const int kernel = (int)int_arg(o[3]);
-  const Stats r = run_colstats(x, false, flags_of(o[4], o[5]), s);
-  const at::Tensor pooled = at::empty_like(r.s1);
-  launch([&] { return ft_avgpool1d(r.s1.const_data_ptr<float>(), x.B * x.Hkv, (int32_t)x.Skv, kernel, pooled.data_ptr<float>(), s); });
-  return result(r.out, pooled);
+  const at::Tensor out = x.out(), pooled = x.f32({x.B, x.Hkv, x.Skv});
+  const FtAttnArgs a = x.args(out, flags_of(o[4], o[5]));
+  const size_t bytes = ft_workspace_bytes_split(FT_OP_SNAPKV, &a);
+  const at::Tensor ws = workspace(x.q, bytes);
+  launch([&] { return ft_snapkv_fwd(&a, kernel, pooled.data_ptr<float>(), ptr(ws), bytes, s); });
+  return result(out, pooled);
 }
 
 void check_f32(const at::Tensor& t, const at::Tensor& like, at::IntArrayRef shape, const char* arg) {

@@ -42,7 +42,7 @@ enum FtFlags {
                           of the logits (cases/kernels/attn.py:29); faster, ~1e-3 relative on probabilities */
 };
 
-enum FtOp { FT_OP_ATTN = 0, FT_OP_COLSTATS = 1, FT_OP_KEYFORMER = 2, FT_OP_EA = 3, FT_OP_SIMA = 4, FT_OP_CORM = 5 };
+enum FtOp { FT_OP_ATTN = 0, FT_OP_COLSTATS = 1, FT_OP_KEYFORMER = 2, FT_OP_EA = 3, FT_OP_SIMA = 4, FT_OP_CORM = 5, FT_OP_SNAPKV = 6 };
 
 /* Element strides of a logical [B, S, H, D] tensor; the D axis must be contiguous (stride 1). */
 typedef struct FtStrides {
@@ -84,7 +84,7 @@ const char* ft_last_error(void);
 /* Bytes of device scratch the op needs for this problem (0 if none).  The caller owns the buffer. */
 size_t ft_workspace_bytes(int op, const FtAttnArgs* a);
 
-/* The same plus room for the partial results of the shares into which FT_OP_ATTN, FT_OP_COLSTATS and FT_OP_CORM divide
+/* The same plus room for the partial results of the shares into which FT_OP_ATTN, FT_OP_COLSTATS, FT_OP_SNAPKV and FT_OP_CORM divide
  * the keys where there are too few query rows to fill the chip (generation steps, a window of last queries, chunks of a
  * prompt).  With a workspace of this size those calls are faster; with one of
  * ft_workspace_bytes() they run undivided.  The number of shares depends on the device, so ask with it current. */
@@ -136,6 +136,10 @@ int ft_attn_softcap_fwd(const FtAttnArgs* a, float softcap, float* lse, void* st
  * max_i (p_ij - (1 - 1e-6) mask_ij) for a tensor. */
 int ft_corm_fwd(const FtAttnArgs* a, const float* corm_mask, int64_t mask_row_stride, uint8_t* corm_score, float* margin,
                 void* workspace, size_t workspace_bytes, void* stream);
+
+/* SnapKV.forward (cases/kernels/snapkv.py:19-43): attention + ft_attn_colstats_fwd's colsum smoothed as by ft_avgpool1d,
+ * `kernel` odd.  pooled: [B,H,Skv] fp32, [B,Hkv,Skv] under grouped queries. */
+int ft_snapkv_fwd(const FtAttnArgs* a, int32_t kernel, float* pooled, void* workspace, size_t workspace_bytes, void* stream);
 
 /* SnapKV's smoothing of the per-key scores (cases/kernels/snapkv.py:39): dst[r, j] = (1 / kernel) * sum of
  * src[r, j - kernel/2 .. j + kernel/2] with zeros outside the row, kernel odd; src, dst: [rows, S] fp32. */

@@ -53,3 +53,23 @@ def test_a_workspace_without_room_for_the_shares_keeps_blocks_whole(gpu, monkeyp
     ws = torch.empty(nbytes, dtype=torch.uint8, device=gpu)
     k_.attn_colstats_fwd(args(out), score.data_ptr(), 0, ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream)
     assert (out.float() - ref[0].float()).norm() <= 1e-3 * ref[0].float().norm() and torch.allclose(score, ref[1], rtol=1e-4)
+
+
+@pytest.mark.parametrize("tiles", [0, 1])
+@pytest.mark.parametrize("Sq,Skv,H,D,dtype", [(1, 2, 1, 128, torch.float16), (3, 447, 4, 64, torch.float16), (8, 448, 2, 128, torch.bfloat16),
+                                              (17, 513, 2, 128, torch.float16), (32, 1025, 3, 64, torch.float16), (33, 600, 2, 64, torch.float16)])
+def test_column_sums_of_few_rows(gpu, monkeypatch, tiles, Sq, Skv, H, D, dtype):
+  """Up to 32 rows keep their logits for the column sums (key counts around the 448 and 512 keys of a workgroup, windows
+  up to the widest that is taken in the same launch and one beyond), 33 go through the column pass."""
+  if tiles:
+    monkeypatch.setenv("FT_ATTN_FORM", f"s{tiles}")
+  (q, k, v) = oracle.prepare_inputs(2, Sq, H, D, seed=Skv, dtype=dtype, kv_len=Skv)
+  dev = [t.to(gpu) for t in (q, k, v)]
+  tol = 1e-2 if dtype is torch.bfloat16 else 2e-3
+  ref_o, ref_s, ref_sq = oracle.roco_forward(q, k, v)
+  out, s, sq = ops.roco(*dev)
+  assert (out.float().cpu() - ref_o.float()).norm() <= tol * ref_o.float().norm()
+  assert (s.cpu() - ref_s).norm() <= tol * ref_s.norm() and (sq.cpu() - ref_sq).norm() <= 2 * tol * ref_sq.norm()
+  for width in (1, 5, 65, 67):
+    ref = torch.nn.functional.avg_pool1d(ref_s, width, 1, width // 2)
+    assert (ops.snapkv(*dev, kernel_size=width)[1].cpu() - ref).norm() <= tol * ref.norm()
