@@ -33,6 +33,8 @@
 // multi-strip prefetch at each step; plain loads into registers are tracked exactly.
 #include "device_common.hpp"
 #include "kernel_params.h"
+#include <algorithm>
+#include <cstdlib>
 #include <type_traits>
 #include "../../include/ft_abi.h"
 
@@ -61,6 +63,7 @@ struct LinParams {
   int out_tiles_per_chunk;
   int half_heads;           // every 64-channel "head" is two adjacent heads of 32 channels (head_dim 32)
   int out_wave_heads;       // output pass: a workgroup takes four adjacent heads, one per wave
+  int normalize_q;          // SimA: the queries' norms go into the matrix too (output pass that merges for itself)
 };
 
 // Splits the sequence of every (b, h) into chunks so that about `workgroups` workgroups exist.  The K/V pass
@@ -68,7 +71,7 @@ struct LinParams {
 // workgroup, so it wants one round of them (512); the output pass runs more workgroups per CU and has no
 // epilogue, so more, shorter ones balance better (measured in one process at B8 H16 S8192, EA / SimA:
 // 1024 + 1024 workgroups 148 / 147 us, 512 + 1024 136 / 139, 512 + 2048 135 / 137, 512 + 4096 143 / 141).
-constexpr int kKvWorkgroups = 512, kOutWorkgroups = 2048;
+constexpr int kKvWorkgroups = 512, kOutWorkgroups = 2048, kFusedWorkgroups = 512;
 
 static void lin_plan(const FtAttnArgs& a, int workgroups, int* nch, int* tpc) {
   const int ntiles = (a.Sq + kLinTile - 1) / kLinTile;
@@ -641,7 +644,83 @@ __global__ void __launch_bounds__(kLinThreads) linattn_merge_kernel(const LinPar
 }
 
 // ---------------------------------------------------------------------------------------------------
-template <typename T, bool IN32, bool EA, bool F32OUT>
+// The merge step of one (b, h) inside a workgroup of the output pass, for calls with few chunks and few workgroups: what a
+// launch costs (4 us and the gap in front of it) is more than every workgroup reading its head's few partials (17 KB a
+// chunk, from L2) and folding them again.  Thread t takes row d = t / 4 and 16 columns, one output-channel block: its
+// chunks' statistics are those of one channel.  The operand pair lands in LDS rows w[hi / lo][e][d], the blocks' inverse
+// scales in s_winv.
+constexpr int kFusedChunks = 8, kFusedRow = kLinD + 8;
+
+template <typename T, bool EA, bool LO>
+__device__ __forceinline__ void merge_in_lds(const LinParams& p, int bh, uint16_t (*s_w)[kLinD][kFusedRow], float* s_winv, float* s_max) {
+  constexpr int D = kLinD;
+  const int t = threadIdx.x, d = t >> 2, qr = t & 3;
+  const float* part = p.part + (int64_t)bh * p.nch * kPartStride;
+  // every load at once: chunks past the last one re-read it, with weight 0
+  float a[kFusedChunks], b[kFusedChunks];
+  float4v m[kFusedChunks][4];
+#pragma unroll
+  for (int c = 0; c < kFusedChunks; ++c) {
+    const float* pc = part + (int64_t)min(c, p.nch - 1) * kPartStride;
+    a[c] = pc[D * D + d];
+    b[c] = pc[D * D + D + d];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) m[c][i] = *reinterpret_cast<const float4v*>(pc + d * D + 16 * qr + 4 * i);
+  }
+  float w[kFusedChunks], scale;
+  if (EA) {
+    float M = a[0], L = 0.f;
+#pragma unroll
+    for (int c = 1; c < kFusedChunks; ++c) M = fmaxf(M, a[c]);
+#pragma unroll
+    for (int c = 0; c < kFusedChunks; ++c) {
+      w[c] = c < p.nch ? __builtin_amdgcn_exp2f((a[c] - M) * kLog2e) : 0.f;
+      L += w[c] * b[c];
+    }
+    scale = 1.f / L;
+  } else {
+    float nk = 0.f, nq = 0.f;
+#pragma unroll
+    for (int c = 0; c < kFusedChunks; ++c) {
+      w[c] = c < p.nch ? 1.f : 0.f;
+      nk += w[c] * a[c];
+      nq += w[c] * b[c];
+    }
+    scale = 1.f / (p.normalize_q ? nk * nq : nk);
+  }
+  float x[16], gmax = 0.f;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    float s = 0.f;
+#pragma unroll
+    for (int c = 0; c < kFusedChunks; ++c) s += w[c] * m[c][i >> 2][i & 3];
+    if (p.half_heads && (d >> 5) != (qr >> 1)) s = 0.f;  // two heads of 32 channels: no products across them
+    x[i] = s * scale;
+    gmax = fmaxf(gmax, __builtin_fabsf(x[i]));
+  }
+  // the maximum of each 16-channel block: lanes that share t % 4, then the waves
+#pragma unroll
+  for (int o = 32; o >= 4; o >>= 1) gmax = fmaxf(gmax, __shfl_xor(gmax, o));
+  if ((t & 63) < 4) s_max[(t >> 6) * 4 + qr] = gmax;
+  __syncthreads();
+  gmax = fmaxf(fmaxf(s_max[qr], s_max[4 + qr]), fmaxf(s_max[8 + qr], s_max[12 + qr]));
+  int ex = 0;
+  if (gmax > 0.f && gmax < __builtin_inff()) ex = 13 - (int)__builtin_floorf(__builtin_log2f(gmax));
+  ex = max(-100, min(100, ex));
+  const float up = __builtin_ldexpf(1.f, ex);
+  if (d == 0) s_winv[qr] = __builtin_ldexpf(1.f, -ex);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const float y = x[i] * up;
+    const uint16_t hi = T::from_float(y);
+    s_w[0][16 * qr + i][d] = hi;
+    if (LO) s_w[LO ? 1 : 0][16 * qr + i][d] = T::from_float((y - T::to_float(hi)) * (float)(1 << kLoShift<T>));
+  }
+  __syncthreads();
+}
+
+// MERGE: the workgroup folds its head's partials itself (merge_in_lds), one head per workgroup.
+template <typename T, bool IN32, bool EA, bool F32OUT, bool MERGE = false>
 __global__ void __launch_bounds__(kLinThreads, 2) linattn_out_kernel(const LinParams p) {
   static_assert(!IN32 || __is_same(typename T::elem, _Float16), "fp32 tensors are rounded to fp16 operands");
   typedef typename T::vec8 vec8;
@@ -653,6 +732,8 @@ __global__ void __launch_bounds__(kLinThreads, 2) linattn_out_kernel(const LinPa
   constexpr int SL = SUB * D * (F32OUT ? 4 : 2) / 1024;  // 16-byte row stores per strip and lane
   __shared__ __align__(16) char s_q[kLinWaves][STRIP];       // wave-private Q strip
   __shared__ __align__(16) char otr[kLinWaves * SUB * OROW]; // wave-private output transpose buffers
+  __shared__ __align__(16) uint16_t s_w[MERGE && F32OUT ? 2 : 1][MERGE ? kLinD : 1][kFusedRow];
+  __shared__ float s_winv[4], s_max[16];
 
   const int lane = lane_id(), wave = wave_id();
   const int g = lane >> 5, n = lane & 31;
@@ -665,7 +746,7 @@ __global__ void __launch_bounds__(kLinThreads, 2) linattn_out_kernel(const LinPa
   // touched by one workgroup at one time, not by sixteen at sixteen times).  Otherwise one head per
   // workgroup, the strips of the chunk dealt round-robin to the waves.
   int bh, ch, strip0, strip_step;
-  if (p.out_wave_heads) {
+  if (!MERGE && p.out_wave_heads) {
     const int hq = p.H / kLinWaves, groups = p.B * hq;
     const int bg = blockIdx.x % groups;
     ch = blockIdx.x / groups;
@@ -686,9 +767,25 @@ __global__ void __launch_bounds__(kLinThreads, 2) linattn_out_kernel(const LinPa
   const int nsub = (tok_end - tok_begin + SUB - 1) / SUB;
   const int nmine = nsub > strip0 ? (nsub - strip0 + strip_step - 1) / strip_step : 0;
 
+  StripMover<SUB, kRowSwizzle, IN32> mvQ;
+  mvQ.init(p.q + (b * p.sq.b + h * p.sq.h) * (IN32 ? 2 : 1), p.sq.s, p.S);
+  constexpr int RL = IN32 ? 2 * R : R;
+  uint4v rq[P][RL];  // strips in flight, indexed by compile-time slot
+  auto strip_row0 = [&](int i) { return tok_begin + (strip0 + strip_step * i) * SUB; };
+  mvQ.limit_rows(nmine > 0 ? strip_row0(nmine - 1) + SUB - 1 : tok_begin);
+  auto load_strips = [&]() {
+    __builtin_amdgcn_sched_barrier(0);  // strip 0, then strip 1: loads complete in the order they are issued
+    mvQ.load(strip_row0(0), rq[0]);
+    __builtin_amdgcn_sched_barrier(0);
+    mvQ.load(strip_row0(1), rq[1]);
+  };
+  if constexpr (MERGE) {
+    load_strips();  // in flight during the merge
+    merge_in_lds<T, EA, F32OUT>(p, bh, s_w, s_winv, s_max);
+  }
   float winv[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) winv[i] = p.winv[bh * 4 + i];
+  for (int i = 0; i < 4; ++i) winv[i] = MERGE ? s_winv[i] : p.winv[bh * 4 + i];
   // A operand: W^T[e][d], hi and lo, rows e = 32 eb + n, contraction slots d = 16 t + 8 g + [0..7]
   const uint16_t* w = p.w + (int64_t)bh * 2 * D * D;
   vec8 whi[2][4], wlo[2][4];
@@ -696,25 +793,22 @@ __global__ void __launch_bounds__(kLinThreads, 2) linattn_out_kernel(const LinPa
   for (int eb = 0; eb < 2; ++eb)
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      whi[eb][t] = *reinterpret_cast<const vec8*>(w + (32 * eb + n) * D + 16 * t + 8 * g);
-      if (F32OUT) wlo[eb][t] = *reinterpret_cast<const vec8*>(w + D * D + (32 * eb + n) * D + 16 * t + 8 * g);
+      if constexpr (MERGE) {
+        whi[eb][t] = *reinterpret_cast<const vec8*>(&s_w[0][32 * eb + n][16 * t + 8 * g]);
+        if constexpr (F32OUT) wlo[eb][t] = *reinterpret_cast<const vec8*>(&s_w[1][32 * eb + n][16 * t + 8 * g]);
+      } else {
+        whi[eb][t] = *reinterpret_cast<const vec8*>(w + (32 * eb + n) * D + 16 * t + 8 * g);
+        if (F32OUT) wlo[eb][t] = *reinterpret_cast<const vec8*>(w + D * D + (32 * eb + n) * D + 16 * t + 8 * g);
+      }
     }
-
-  StripMover<SUB, kRowSwizzle, IN32> mvQ;
-  mvQ.init(p.q + (b * p.sq.b + h * p.sq.h) * (IN32 ? 2 : 1), p.sq.s, p.S);
-  constexpr int RL = IN32 ? 2 * R : R;
-  uint4v rq[P][RL];  // strips in flight, indexed by compile-time slot
-  auto strip_row0 = [&](int i) { return tok_begin + (strip0 + strip_step * i) * SUB; };
-  mvQ.limit_rows(nmine > 0 ? strip_row0(nmine - 1) + SUB - 1 : tok_begin);
-  __builtin_amdgcn_sched_barrier(0);  // scales and W, then strip 0, then strip 1: loads complete in the order they are issued
-  mvQ.load(strip_row0(0), rq[0]);
-  __builtin_amdgcn_sched_barrier(0);
-  mvQ.load(strip_row0(1), rq[1]);
+  if (!MERGE) load_strips();  // scales and W, then the strips
   // W has landed before the loop starts, the two strips (the 2 R loads issued after it) stay in flight.  Left to
   // the compiler, the wait for W sits inside the loop, in front of the MFMAs, where on every later trip it
   // waits for the strip requested a few instructions earlier instead.
   static_assert(P * R == 8, "the wait below counts the loads of the two strips");
-  if (IN32)
+  if (MERGE)
+    ;  // everything has landed with the merge
+  else if (IN32)
     __builtin_amdgcn_s_waitcnt(0x4F70);  // vmcnt(16): fp32 strips take twice the loads
   else
     __builtin_amdgcn_s_waitcnt(0x0F78);  // vmcnt(8), every other counter at its maximum
@@ -831,6 +925,12 @@ __global__ void __launch_bounds__(kLinThreads, 2) linattn_out_kernel(const LinPa
   }
 }
 
+// Test hook: FT_LINATTN_MERGE=fused or =launch in the environment forces where the chunks are folded.
+static int lin_merge_override() {
+  const char* e = getenv("FT_LINATTN_MERGE");
+  return !e ? 0 : e[0] == 'f' ? 1 : e[0] == 'l' ? 2 : 0;
+}
+
 template <typename T>
 struct TypeTag {
   typedef T type;
@@ -859,6 +959,18 @@ hipError_t launch_linattn(const FtAttnArgs& a0, int kind, int normalize_q, int o
   // 127.4 -> 121.2 us per call.  SimA with normalised queries has just read Q in its K/V pass and finds much of it
   // in the memory-side cache; there the one-head form is the faster by 1 us (126.6 vs 127.7) and stays.
   p.out_wave_heads = a.H % kLinWaves == 0 && !nq;
+  p.normalize_q = nq;
+  // Short calls fold the partials in the output pass (merge_in_lds), with chunks of up to four tiles where single tiles
+  // would make more than eight chunks.  Per call, fp16 EA: B1 H4 S64 16.8 -> 12.3 us, B2 H8 S1000 20.9 -> 13.9, B4 H16
+  // S1000 (512 workgroups in the output pass) 26.1 -> 20.4; at 1024 the same or slower, B8 H16 S1000 26.8 and 29.5.
+  const int forced = lin_merge_override();
+  const int ntiles = (a.Sq + kLinTile - 1) / kLinTile;
+  const bool fused = ntiles <= 4 * kFusedChunks && (forced ? forced == 1 : (int64_t)a.B * a.H * p.out_nch <= kFusedWorkgroups);
+  if (fused) {
+    p.out_wave_heads = 0;
+    p.tiles_per_chunk = std::max(p.tiles_per_chunk, (ntiles + kFusedChunks - 1) / kFusedChunks);
+    p.nch = (ntiles + p.tiles_per_chunk - 1) / p.tiles_per_chunk;  // no more than the workspace has room for
+  }
   if (p.out_wave_heads) {  // the same number of workgroups over a quarter as many (b, head group) pairs
     FtAttnArgs quarter = a;
     quarter.H = a.H / kLinWaves;
@@ -888,28 +1000,25 @@ hipError_t launch_linattn(const FtAttnArgs& a0, int kind, int normalize_q, int o
       hipLaunchKernelGGL((linattn_kv_kernel<T, IN32, false, false>), grid1, blk, 0, s, p);
     e = hipGetLastError();
     if (e != hipSuccess) return;
-    if (ea)
-      hipLaunchKernelGGL((linattn_merge_kernel<T, true>), grid2, blk, 0, s, p, 0);
-    else
-      hipLaunchKernelGGL((linattn_merge_kernel<T, false>), grid2, blk, 0, s, p, nq ? 1 : 0);
-    e = hipGetLastError();
-    if (e != hipSuccess) return;
-    if constexpr (IN32) {
+    if (!fused) {
       if (ea)
-        hipLaunchKernelGGL((linattn_out_kernel<T, true, true, true>), grid3, blk, 0, s, p);
+        hipLaunchKernelGGL((linattn_merge_kernel<T, true>), grid2, blk, 0, s, p, 0);
       else
-        hipLaunchKernelGGL((linattn_out_kernel<T, true, false, true>), grid3, blk, 0, s, p);
-    } else if (ea) {
-      if (f32)
-        hipLaunchKernelGGL((linattn_out_kernel<T, false, true, true>), grid3, blk, 0, s, p);
-      else
-        hipLaunchKernelGGL((linattn_out_kernel<T, false, true, false>), grid3, blk, 0, s, p);
-    } else {
-      if (f32)
-        hipLaunchKernelGGL((linattn_out_kernel<T, false, false, true>), grid3, blk, 0, s, p);
-      else
-        hipLaunchKernelGGL((linattn_out_kernel<T, false, false, false>), grid3, blk, 0, s, p);
+        hipLaunchKernelGGL((linattn_merge_kernel<T, false>), grid2, blk, 0, s, p, nq ? 1 : 0);
+      e = hipGetLastError();
+      if (e != hipSuccess) return;
     }
+    auto out = [&](auto ea_tag, auto f32_tag) {
+      constexpr bool EA = decltype(ea_tag)::value, F32OUT = IN32 || decltype(f32_tag)::value;
+      if (fused)
+        hipLaunchKernelGGL((linattn_out_kernel<T, IN32, EA, F32OUT, true>), grid3, blk, 0, s, p);
+      else
+        hipLaunchKernelGGL((linattn_out_kernel<T, IN32, EA, F32OUT, false>), grid3, blk, 0, s, p);
+    };
+    if (ea)
+      f32 ? out(std::true_type{}, std::true_type{}) : out(std::true_type{}, std::false_type{});
+    else
+      f32 ? out(std::false_type{}, std::true_type{}) : out(std::false_type{}, std::false_type{});
     e = hipGetLastError();
   };
   if (a.dtype == FT_F32)
