@@ -71,7 +71,8 @@ struct LinParams {
 // workgroup, so it wants one round of them (512); the output pass runs more workgroups per CU and has no
 // epilogue, so more, shorter ones balance better (measured in one process at B8 H16 S8192, EA / SimA:
 // 1024 + 1024 workgroups 148 / 147 us, 512 + 1024 136 / 139, 512 + 2048 135 / 137, 512 + 4096 143 / 141).
-constexpr int kKvWorkgroups = 512, kOutWorkgroups = 2048, kFusedWorkgroups = 512;
+constexpr int kKvWorkgroups = 512, kOutWorkgroups = 2048, kFusedWorkgroups = 256;
+constexpr int64_t kFusedTokens = 1 << 19;
 
 static void lin_plan(const FtAttnArgs& a, int workgroups, int* nch, int* tpc) {
   const int ntiles = (a.Sq + kLinTile - 1) / kLinTile;
@@ -576,7 +577,7 @@ __global__ void __launch_bounds__(kLinThreads) linattn_merge_kernel(const LinPar
     }
     __syncthreads();
   }
-  // weighted sum of the chunk matrices, four chunks (16 independent loads per thread) at a time
+  // weighted sum of the chunk matrices, eight chunks (32 independent loads per thread) at a time
   for (int c0 = 0; c0 < p.nch; c0 += 16) {
     const int cn = min(16, p.nch - c0);
     if (EA) {
@@ -586,16 +587,16 @@ __global__ void __launch_bounds__(kLinThreads) linattn_merge_kernel(const LinPar
       }
       __syncthreads();
     }
-    for (int c = 0; c < cn; c += 4) {
-      float v[4][4];
+    for (int c = 0; c < cn; c += 8) {
+      float v[8][4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < 8; ++u) {
         const int cc = c0 + min(c + u, cn - 1);
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[u][i] = part[cc * kPartStride + pidx[i]];
       }
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
+      for (int u = 0; u < 8; ++u)
         if (c + u < cn) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) accv[i] += (EA ? s_w[c + u][drow[i]] : 1.f) * v[u][i];
@@ -644,9 +645,8 @@ __global__ void __launch_bounds__(kLinThreads) linattn_merge_kernel(const LinPar
 }
 
 // ---------------------------------------------------------------------------------------------------
-// The merge step of one (b, h) inside a workgroup of the output pass, for calls with few chunks and few workgroups: what a
-// launch costs (4 us and the gap in front of it) is more than every workgroup reading its head's few partials (17 KB a
-// chunk, from L2) and folding them again.  Thread t takes row d = t / 4 and 16 columns, one output-channel block: its
+// The merge step of one (b, h) inside a workgroup of the output pass: what a launch costs (4 us and the gap in front of it)
+// is more than every workgroup reading its head's partials (17 KB a chunk, from L2) and folding them again.  Thread t takes row d = t / 4 and 16 columns, one output-channel block: its
 // chunks' statistics are those of one channel.  The operand pair lands in LDS rows w[hi / lo][e][d], the blocks' inverse
 // scales in s_winv.
 constexpr int kFusedChunks = 8, kFusedRow = kLinD + 8;
@@ -656,46 +656,45 @@ __device__ __forceinline__ void merge_in_lds(const LinParams& p, int bh, uint16_
   constexpr int D = kLinD;
   const int t = threadIdx.x, d = t >> 2, qr = t & 3;
   const float* part = p.part + (int64_t)bh * p.nch * kPartStride;
-  // every load at once: chunks past the last one re-read it, with weight 0
-  float a[kFusedChunks], b[kFusedChunks];
-  float4v m[kFusedChunks][4];
-#pragma unroll
-  for (int c = 0; c < kFusedChunks; ++c) {
-    const float* pc = part + (int64_t)min(c, p.nch - 1) * kPartStride;
-    a[c] = pc[D * D + d];
-    b[c] = pc[D * D + D + d];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) m[c][i] = *reinterpret_cast<const float4v*>(pc + d * D + 16 * qr + 4 * i);
-  }
-  float w[kFusedChunks], scale;
-  if (EA) {
-    float M = a[0], L = 0.f;
-#pragma unroll
-    for (int c = 1; c < kFusedChunks; ++c) M = fmaxf(M, a[c]);
+  float x[16] = {}, M = -__builtin_inff(), L = 0.f, nq = 0.f;
+#pragma unroll 1
+  for (int c0 = 0; c0 < p.nch; c0 += kFusedChunks) {
+    // eight chunks' loads at once: chunks past the last one re-read it, with weight 0
+    float a[kFusedChunks], b[kFusedChunks];
+    float4v m[kFusedChunks][4];
 #pragma unroll
     for (int c = 0; c < kFusedChunks; ++c) {
-      w[c] = c < p.nch ? __builtin_amdgcn_exp2f((a[c] - M) * kLog2e) : 0.f;
-      L += w[c] * b[c];
+      const float* pc = part + (int64_t)min(c0 + c, p.nch - 1) * kPartStride;
+      a[c] = pc[D * D + d];
+      b[c] = pc[D * D + D + d];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) m[c][i] = *reinterpret_cast<const float4v*>(pc + d * D + 16 * qr + 4 * i);
     }
-    scale = 1.f / L;
-  } else {
-    float nk = 0.f, nq = 0.f;
+    if (EA) {  // a: maximum, b: sum of exponentials
+      float M1 = M;
+#pragma unroll
+      for (int c = 0; c < kFusedChunks; ++c) M1 = fmaxf(M1, a[c]);
+      const float move = __builtin_amdgcn_exp2f((M - M1) * kLog2e);
+      M = M1;
+      L *= move;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) x[i] *= move;
+    }
 #pragma unroll
     for (int c = 0; c < kFusedChunks; ++c) {
-      w[c] = c < p.nch ? 1.f : 0.f;
-      nk += w[c] * a[c];
-      nq += w[c] * b[c];
+      const float w = c0 + c < p.nch ? (EA ? __builtin_amdgcn_exp2f((a[c] - M) * kLog2e) : 1.f) : 0.f;
+      L = __builtin_fmaf(w, EA ? b[c] : a[c], L);  // SimA: a, b are the norms of K and Q
+      nq = __builtin_fmaf(w, b[c], nq);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) x[i] = __builtin_fmaf(w, m[c][i >> 2][i & 3], x[i]);
     }
-    scale = 1.f / (p.normalize_q ? nk * nq : nk);
   }
-  float x[16], gmax = 0.f;
+  const float scale = 1.f / (!EA && p.normalize_q ? L * nq : L);
+  float gmax = 0.f;
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
-    float s = 0.f;
-#pragma unroll
-    for (int c = 0; c < kFusedChunks; ++c) s += w[c] * m[c][i >> 2][i & 3];
-    if (p.half_heads && (d >> 5) != (qr >> 1)) s = 0.f;  // two heads of 32 channels: no products across them
-    x[i] = s * scale;
+    if (p.half_heads && (d >> 5) != (qr >> 1)) x[i] = 0.f;  // two heads of 32 channels: no products across them
+    x[i] *= scale;
     gmax = fmaxf(gmax, __builtin_fabsf(x[i]));
   }
   // the maximum of each 16-channel block: lanes that share t % 4, then the waves
@@ -960,21 +959,21 @@ hipError_t launch_linattn(const FtAttnArgs& a0, int kind, int normalize_q, int o
   // in the memory-side cache; there the one-head form is the faster by 1 us (126.6 vs 127.7) and stays.
   p.out_wave_heads = a.H % kLinWaves == 0 && !nq;
   p.normalize_q = nq;
-  // Short calls fold the partials in the output pass (merge_in_lds), with chunks of up to four tiles where single tiles
-  // would make more than eight chunks.  Per call, fp16 EA: B1 H4 S64 16.8 -> 12.3 us, B2 H8 S1000 20.9 -> 13.9, B4 H16
-  // S1000 (512 workgroups in the output pass) 26.1 -> 20.4; at 1024 the same or slower, B8 H16 S1000 26.8 and 29.5.
+  // Calls of up to 2^19 tokens (times heads) fold the partials in the output pass (merge_in_lds), with fewer,
+  // longer chunks and one workgroup per CU in the output pass, so that each folds
+  // once.  Per call, fp16 EA: B1 H4 S64 16.8 -> 12.3 us, B2 H8 S1000 20.9 -> 13.9, B1 H16 S4000 32.9 -> 19.6, B8 H16 S1000
+  // 27.5 -> 23.9, B8 H16 S4000 67.8 -> 64.7 (with 512 workgroups 25.3 and 64.8, with 1024 29.4 and 70.0); at S8192 121 and
+  // 134: there many short workgroups that only stream are worth the launch.
   const int forced = lin_merge_override();
-  const int ntiles = (a.Sq + kLinTile - 1) / kLinTile;
-  const bool fused = ntiles <= 4 * kFusedChunks && (forced ? forced == 1 : (int64_t)a.B * a.H * p.out_nch <= kFusedWorkgroups);
+  const bool fused = forced ? forced == 1 : (int64_t)a.B * a.H * a.Sq <= kFusedTokens;
   if (fused) {
+    const int ntiles = (a.Sq + kLinTile - 1) / kLinTile;
     p.out_wave_heads = 0;
-    p.tiles_per_chunk = std::max(p.tiles_per_chunk, (ntiles + kFusedChunks - 1) / kFusedChunks);
+    lin_plan(a, kFusedWorkgroups, &p.out_nch, &p.out_tiles_per_chunk);
+    // eight chunks to a round of folding; more of up to four tiles where eight would leave CUs idle in the K/V pass
+    const int eighth = (ntiles + kFusedChunks - 1) / kFusedChunks;
+    p.tiles_per_chunk = std::max(p.tiles_per_chunk, (int64_t)a.B * a.H * kFusedChunks >= kFusedWorkgroups ? eighth : std::min(4, eighth));
     p.nch = (ntiles + p.tiles_per_chunk - 1) / p.tiles_per_chunk;  // no more than the workspace has room for
-  }
-  if (p.out_wave_heads) {  // the same number of workgroups over a quarter as many (b, head group) pairs
-    FtAttnArgs quarter = a;
-    quarter.H = a.H / kLinWaves;
-    lin_plan(quarter, kOutWorkgroups, &p.out_nch, &p.out_tiles_per_chunk);
   }
   const bool f32 = out_dtype == FT_F32;
   const size_t bh = (size_t)a.B * a.H;
