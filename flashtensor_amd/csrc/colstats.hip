@@ -1,4 +1,4 @@
-// Dispatcher of the column-statistics pass (colstats_kernel.hpp) and its 128-key instantiations; colstats_narrow.hip holds
+// Dispatcher of the column-statistics pass (colstats_kernel.hpp) and its 128-key instantiations; colstats_{narrow,teams}.hip hold
 // the 64-key ones.
 #include <cstdlib>
 
@@ -7,11 +7,14 @@
 namespace ft {
 
 hipError_t launch_colstats_narrow(const ColstatsKernelParams& p, int D, bool bf16, bool causal, int mode, hipStream_t s);
+hipError_t launch_colstats_teams(const ColstatsKernelParams& p, int D, bool bf16, bool causal, int mode, hipStream_t s);
 
-// Test hook: FT_COLSTATS_KEYS=1 or 2 in the environment forces 64 or 128 keys per workgroup.
-int colstats_keys_override() {
+// Test hook: FT_COLSTATS_KEYS=1 or 2 in the environment forces 64 or 128 keys per workgroup, 1t 64 and two teams of waves.
+enum { kFormAuto = 0, kFormNarrow = 1, kFormWide = 2, kFormTeams = 3 };
+static int form_override() {
   const char* e = getenv("FT_COLSTATS_KEYS");
-  return e && (e[0] == '1' || e[0] == '2') ? e[0] - '0' : 0;
+  if (!e || (e[0] != '1' && e[0] != '2')) return kFormAuto;
+  return e[0] == '2' ? kFormWide : e[1] == 't' ? kFormTeams : kFormNarrow;
 }
 
 template <typename T, int D>
@@ -35,12 +38,18 @@ static hipError_t launch_td(const ColstatsKernelParams& p, bool causal, bool emu
 
 hipError_t launch_colstats(const ColstatsKernelParams& p, int D, bool bf16, bool causal, bool emu, int mode, hipStream_t s) {
   const bool tensor = mode == kStatKfTensor || mode == kStatCormTensor;
-  const int forced = colstats_keys_override();
-  // 64 keys per workgroup where there are fewer than two workgroups of 128 per CU (h2o calls, same process: B1 H8 S1500
-  // 49.8 -> 43.5 us, B1 H32 S1024 38.3 -> 34.0, keyformer B1 H16 S2048 102.5 -> 87.6; at two per CU the same or slower,
-  // 77.8 and 78.2 at B1 H32 S2048, and at eight 62.0 and 66.7)
-  const int64_t wgs = (int64_t)p.B * p.H * ((p.Skv + 127) / 128);
-  if (!tensor && emu && (forced ? forced == 1 : wgs < 2 * device_cu_count())) return launch_colstats_narrow(p, D, bf16, causal, mode, s);
+  if (!tensor && emu) {
+    int form = form_override();
+    // 64 keys per workgroup where there are fewer than two workgroups of 128 per CU (h2o calls, same process: B1 H8 S1500
+    // 49.6 -> 43.7 us, B1 H32 S1000 38.0 -> 34.7, keyformer B1 H16 S2048 101.7 -> 86.6; at two per CU the same or slower,
+    // 77.4 and 78.7 at B1 H32 S2048, and at eight 62.0 and 66.7); and two teams of waves below one per CU, where a
+    // workgroup of 64 keys often has its CU to itself (B1 H8 S1500 43.7 -> 41.0, S3000 76.4 -> 70.4, roco B1 H8 S2048 D64 39.4 ->
+    // 37.1; at one per CU 56.3 and 56.1 at B1 H16 S2048, 34.7 and 35.3 at B1 H32 S1000, above it slower: 52.3 and 57.6 at B1 H32 S1500)
+    const int64_t wgs = (int64_t)p.B * p.H * ((p.Skv + 127) / 128), cus = device_cu_count();
+    if (!form) form = wgs < cus ? kFormTeams : wgs < 2 * cus ? kFormNarrow : kFormWide;
+    if (form == kFormTeams) return launch_colstats_teams(p, D, bf16, causal, mode, s);
+    if (form == kFormNarrow) return launch_colstats_narrow(p, D, bf16, causal, mode, s);
+  }
   if (D == 128) return bf16 ? launch_td<BF16, 128>(p, causal, emu, mode, s) : launch_td<F16, 128>(p, causal, emu, mode, s);
   if (D == 64) return bf16 ? launch_td<BF16, 64>(p, causal, emu, mode, s) : launch_td<F16, 64>(p, causal, emu, mode, s);
   return hipErrorInvalidValue;

@@ -20,6 +20,11 @@
 // NKEYS: 16-key columns per lane of the 16x16 form.  Two: 128 keys per workgroup, every Q operand read from LDS feeds two
 // MFMAs.  One: 64 keys per workgroup, for launches that leave CUs idle: twice the workgroups with half the vector work per
 // tile each; a key's sum is taken over the same rows in the same order.
+//
+// TEAMS = 2: eight waves per workgroup, two sets of four that take the workgroup's row tiles in turn, each with LDS buffers of
+// its own, and meet at the end: half as many tiles in the chain that bounds a launch of few workgroups, for nothing in
+// memory.  Its second set fills the SIMDs where the first would have been alone (D128 h2o, column pass: B1 H8 S4096 36 -> 31 us,
+// S3000 28 -> 22); where CUs hold two workgroups of 64 keys anyway it gains nothing, above that it costs a third.
 #pragma once
 #include "device_common.hpp"
 #include "kernel_params.h"
@@ -39,9 +44,11 @@ constexpr int colstats_waves_per_simd() {
   return (MODE == kStatSum || MODE == kStatSumSq) ? 3 : 2;
 }
 
-template <typename T, int D, bool CAUSAL, bool EMU, int MODE, int NKEYS = 2>
-__global__ void __launch_bounds__(kColThreads, (colstats_waves_per_simd<T, CAUSAL, EMU, MODE>())) colstats_kernel(const ColstatsKernelParams p) {
+template <typename T, int D, bool CAUSAL, bool EMU, int MODE, int NKEYS = 2, int TEAMS = 1>
+__global__ void __launch_bounds__(kColThreads * TEAMS, (TEAMS == 1 ? colstats_waves_per_simd<T, CAUSAL, EMU, MODE>() : 2))
+    colstats_kernel(const ColstatsKernelParams p) {
   constexpr int BK = 64 * NKEYS, BQ = kColBQ, NT = kColThreads;
+  constexpr int BS = TEAMS * BQ;  // rows from one tile of a team to its next
   constexpr int KSTEPS = D / 16;
   typedef TileGeom<D> G;
   typedef typename T::vec8 vec8;
@@ -54,17 +61,18 @@ __global__ void __launch_bounds__(kColThreads, (colstats_waves_per_simd<T, CAUSA
   constexpr bool kPlainF32 = !EMU;                                        // logits stay in fp32: one fma per element
   constexpr bool kTensor = MODE == kStatKfTensor || MODE == kStatCormTensor;
   constexpr bool k16 = !kTensor;            // 16x16x32 blocks; the tensor modes stay on 32x32x16
-  static_assert(k16 || NKEYS == 2, "32 keys per wave");
+  static_assert(k16 || (NKEYS == 2 && TEAMS == 1), "32 keys per wave");
   constexpr int NKEY = k16 ? NKEYS : 1;     // key columns per lane
   constexpr int WK = BK / 4;                // keys per wave
   constexpr int NBLK = k16 ? 4 : 8;         // groups of 4 query rows per lane and key in a tile
   constexpr int KS16 = D / 32;
   // one LDS object per buffer: reads of one do not wait for the direct-to-LDS loads in flight into the other
-  __shared__ __align__(16) char ldsQ0[TILE_BYTES];
-  __shared__ __align__(16) char ldsQ1[TILE_BYTES];
-  __shared__ __align__(16) char ldsQ2[TILE_BYTES];  // tile t lives in buffer t % 3: two tiles in flight behind the one being read
-  __shared__ __align__(16) float ldsLse[2 * BQ];     // row normalisers of the current / next tile
-  __shared__ __align__(16) uint32_t ldsRow[2 * BQ];  // noise row terms (seeded KeyFormer)
+  __shared__ __align__(16) char s_q0[TEAMS * TILE_BYTES];
+  __shared__ __align__(16) char s_q1[TEAMS * TILE_BYTES];
+  __shared__ __align__(16) char s_q2[TEAMS * TILE_BYTES];  // tile t lives in buffer t % 3: two tiles in flight behind the one being read
+  __shared__ __align__(16) float s_lse[TEAMS * 2 * BQ];     // row normalisers of the current / next tile
+  __shared__ __align__(16) uint32_t s_row[TEAMS * 2 * BQ];  // noise row terms (seeded KeyFormer)
+  __shared__ float s_fold[TEAMS > 1 ? 2 * BK : 1];          // the second team's results
 
   const int BH = p.B * p.H;
   // Low key blocks see the most rows under the causal mask: heaviest first, every (b, h) pair's block 0 before any
@@ -82,7 +90,13 @@ __global__ void __launch_bounds__(kColThreads, (colstats_waves_per_simd<T, CAUSA
   }
   const int b = bh / p.H, h = bh % p.H;
   const int j0 = jb * BK;
-  const int lane = lane_id(), wave = wave_id();
+  const int lane = lane_id(), wave = wave_id() & 3;
+  const int team = TEAMS > 1 ? wave_id() >> 2 : 0, tid = TEAMS > 1 ? threadIdx.x & (NT - 1) : threadIdx.x;
+  char* const ldsQ0 = s_q0 + team * TILE_BYTES;
+  char* const ldsQ1 = s_q1 + team * TILE_BYTES;
+  char* const ldsQ2 = s_q2 + team * TILE_BYTES;
+  float* const ldsLse = s_lse + team * 2 * BQ;
+  uint32_t* const ldsRow = s_row + team * 2 * BQ;
   const int g = lane >> 5, n = lane & 31;      // 32x32 blocks: half and column
   const int q4l = lane >> 4, n16 = lane & 15;  // 16x16 blocks: quarter and column
   const int rsub = k16 ? 4 * q4l : 4 * g;      // first of the lane's 4 rows inside a group of 16 (8) rows
@@ -118,11 +132,14 @@ __global__ void __launch_bounds__(kColThreads, (colstats_waves_per_simd<T, CAUSA
   // first query row that can see key j0 is j0 - off
   int i_begin = 0;
   if (CAUSAL) i_begin = max(0, j0 - p.off) / BQ * BQ;
-  const int ntiles = (p.Sq - i_begin + BQ - 1) / BQ;  // <= 0 when no row sees this block
+  // trips of the loops below, the same in every wave: each holds one barrier.  The first team has them all.
+  const int ntrips = (p.Sq - i_begin + BS - 1) / BS;  // <= 0 when no row sees this block
+  i_begin += team * BQ;
+  const int ntiles = TEAMS == 1 ? ntrips : max(0, (p.Sq - i_begin + BS - 1) / BS);
   // leading tiles in which some (row, key) pair of this wave is above the diagonal
   const int wave_key0 = j0 + wave * WK;
   int n_masked = 0;
-  if (CAUSAL) n_masked = max(0, min(ntiles, (wave_key0 + WK - 1 - p.off - i_begin + BQ - 1) / BQ));
+  if (CAUSAL) n_masked = max(0, min(ntiles, (wave_key0 + WK - 1 - p.off - i_begin + BS - 1) / BS));
 
   NoiseKeys nk = {0, 0};
   uint32_t b_j[NKEY] = {};
@@ -156,7 +173,7 @@ __global__ void __launch_bounds__(kColThreads, (colstats_waves_per_simd<T, CAUSA
     for (int e = 0; e < 4; ++e) best[key][e] = NEG_INF;
 
   auto stage_q = [&](int t, char* dst) {
-    if (t < ntiles) stQ.issue(i_begin + t * BQ, min(BQ, p.Sq - (i_begin + t * BQ)), dst);
+    if (t < ntiles) stQ.issue(i_begin + t * BS, min(BQ, p.Sq - (i_begin + t * BS)), dst);
   };
   // Tensor modes: this lane's slice of the S x S noise / threshold tensor for one tile (its key column, the rows
   // of its score registers; 32 lanes read 128 contiguous bytes of a row), fetched one tile ahead of its use:
@@ -165,7 +182,7 @@ __global__ void __launch_bounds__(kColThreads, (colstats_waves_per_simd<T, CAUSA
   // wave are not read, and the loads carry the non-temporal hint: the tensor is read once and should not evict Q.
   float er[2][16], er_nx[2][16];
   auto load_er = [&](float (&dst)[2][16], int t) {
-    const int i0 = i_begin + t * BQ;
+    const int i0 = i_begin + t * BS;
     // nothing to fetch past the last tile, or when no row of the tile sees a key of this wave
     if (t >= ntiles || (CAUSAL && wave_key0 > i0 + BQ - 1 + p.off)) return;
     const float* row0 = er_col + (int64_t)(i0 + 4 * g) * p.er_sr;
@@ -195,18 +212,18 @@ __global__ void __launch_bounds__(kColThreads, (colstats_waves_per_simd<T, CAUSA
   // row term.  The normaliser is fetched one iteration before it is parked in LDS, so that no wave sits
   // out a global-memory round trip inside the loop.
   auto load_rows = [&](int t) -> float {
-    const int i = i_begin + t * BQ + threadIdx.x;
-    return (t < ntiles && threadIdx.x < BQ && i < p.Sq) ? lse_bh[i] : POS_INF;
+    const int i = i_begin + t * BS + tid;
+    return (t < ntiles && tid < BQ && i < p.Sq) ? lse_bh[i] : POS_INF;
   };
   auto store_rows = [&](int t, float lse_i) {
-    if (t < ntiles && threadIdx.x < BQ) {
-      const int i = i_begin + t * BQ + threadIdx.x;
+    if (t < ntiles && tid < BQ) {
+      const int i = i_begin + t * BS + tid;
       float nl = -lse_i;  // negated: one fma per logit
       // CoRM rule: p_ij >= 1 / (i + 1)  <=>  log2 p_ij + log2(i + 1) >= 0, so no exponential is needed
       if (MODE == kStatCormRule) nl += __builtin_amdgcn_logf((float)(i + 1));
       if (MODE == kStatKfSeededFast) nl -= kLog2Ln2 * p.inv_tau;  // the constant part of -log2(E) / tau
-      ldsLse[(t & 1) * BQ + threadIdx.x] = nl;
-      if (kSeeded) ldsRow[(t & 1) * BQ + threadIdx.x] = noise_row(nk, (uint32_t)i);
+      ldsLse[(t & 1) * BQ + tid] = nl;
+      if (kSeeded) ldsRow[(t & 1) * BQ + tid] = noise_row(nk, (uint32_t)i);
     }
   };
 
@@ -273,7 +290,7 @@ __global__ void __launch_bounds__(kColThreads, (colstats_waves_per_simd<T, CAUSA
   auto block_row0 = [&](int blk) __attribute__((always_inline)) -> int { return (k16 ? 16 * blk : 32 * (blk >> 2) + 8 * (blk & 3)) + rsub; };
   auto reduce_block = [&](auto masked_tag, const STile& s, int t, int blk, const float4v nlse4, const uint4v row4) __attribute__((always_inline)) {
     constexpr bool MASKED = decltype(masked_tag)::value;
-    const int i0 = i_begin + t * BQ;
+    const int i0 = i_begin + t * BS;
     const half2v pk_hi = __builtin_bit_cast(half2v, p.pk_hi2), pk_lo = __builtin_bit_cast(half2v, p.pk_lo2);
     // key kj is hidden from row i0 + il when kj > i0 + il + off, i.e. il < kj - i0 - off; il = il0 + rsub + e
     int lim[NKEY];
@@ -431,7 +448,7 @@ __global__ void __launch_bounds__(kColThreads, (colstats_waves_per_simd<T, CAUSA
       }
   };
   STile S0;
-  if (ntiles > 0) {
+  if (ntrips > 0) {
     // ---- prologue: Q[0], Q[1], Q[2] in flight; rows of tile 0; scores of tile 0
     if (kTensor) load_er(er, 0);
     stage_q(0, ldsQ0);
@@ -482,7 +499,7 @@ __global__ void __launch_bounds__(kColThreads, (colstats_waves_per_simd<T, CAUSA
       lse_next = load_rows(t + 2);
       stage_q(t + 3, b0);
       // every row of this tile above the diagonal for all 32 keys of the wave: nothing to add
-      const bool skip = CAUSAL && (wave_key0 > i_begin + t * BQ + BQ - 1 + p.off);
+      const bool skip = CAUSAL && (wave_key0 > i_begin + t * BS + BQ - 1 + p.off);
       if (!skip) reduce_tile(std::true_type{}, S0, t);
       qk(S0, b1);
       if (kTensor) take_next_er();
@@ -508,23 +525,23 @@ __global__ void __launch_bounds__(kColThreads, (colstats_waves_per_simd<T, CAUSA
       // While tile t + 3 is a whole tile every load of an iteration is issued unconditionally, so that the waits
       // can be counted: kStageLoads staging loads (Q[t+2]) stay in flight across the barrier.  A clean start
       // (nothing outstanding) keeps the compiler's own wait for the row normalisers at that count as well.
-      const int nfull = (p.Sq - i_begin) / BQ;  // whole tiles
+      const int nfull = (p.Sq - i_begin + BS - BQ) / BS;  // whole tiles
       if (t + 3 < nfull) wait_vmem();
       for (; t + 3 < nfull; ++t) {
         // vmcnt(kStageLoads) lgkmcnt(0), then a bare barrier: __syncthreads() carries a fence that drains every load
         __builtin_amdgcn_s_waitcnt(kStageLoads == 4 ? 0x0074 : 0x0072);
         __builtin_amdgcn_s_barrier();
-        if (threadIdx.x < BQ) {
-          const int i = i_begin + (t + 1) * BQ + threadIdx.x;
+        if (tid < BQ) {
+          const int i = i_begin + (t + 1) * BS + tid;
           float nl = -lse_next;
           if (MODE == kStatCormRule) nl += __builtin_amdgcn_logf((float)(i + 1));
           if (MODE == kStatKfSeededFast) nl -= kLog2Ln2 * p.inv_tau;
-          ldsLse[((t + 1) & 1) * BQ + threadIdx.x] = nl;
-          if (kSeeded) ldsRow[((t + 1) & 1) * BQ + threadIdx.x] = noise_row(nk, (uint32_t)i);
+          ldsLse[((t + 1) & 1) * BQ + tid] = nl;
+          if (kSeeded) ldsRow[((t + 1) & 1) * BQ + tid] = noise_row(nk, (uint32_t)i);
         }
-        lse_next = lse_bh[i_begin + (t + 2) * BQ + (threadIdx.x & (BQ - 1))];
+        lse_next = lse_bh[i_begin + (t + 2) * BS + (tid & (BQ - 1))];
         __builtin_amdgcn_sched_barrier(0);  // the normalisers first: their wait must not reach into the staging loads
-        stQ.issue_full(i_begin + (t + 3) * BQ, b0);
+        stQ.issue_full(i_begin + (t + 3) * BS, b0);
         reduce_qk(S0, b1, t);
         rotate();
       }
@@ -535,6 +552,10 @@ __global__ void __launch_bounds__(kColThreads, (colstats_waves_per_simd<T, CAUSA
         stage_q(t + 3, b0);
         reduce_qk(S0, b1, t);  // scores of tile t + 1: past the last tile they come from stale LDS and are discarded
         rotate();
+      }
+      if (TEAMS > 1 && t < ntrips) {  // (one at most)
+        wait_vmem();
+        __syncthreads();
       }
     }
   }
@@ -547,6 +568,7 @@ __global__ void __launch_bounds__(kColThreads, (colstats_waves_per_simd<T, CAUSA
   auto add = [](float a, float c) { return a + c; };
   auto mx = [](float a, float c) { return fmaxf(a, c); };
   const bool writer = k16 ? q4l == 0 : g == 0;
+  float tots[NKEY], totsqs[NKEY], tops[NKEY];
 #pragma unroll
   for (int key = 0; key < NKEY; ++key) {
     float tot = across((sum[key][0] + sum[key][1]) + (sum[key][2] + sum[key][3]), add);
@@ -555,6 +577,25 @@ __global__ void __launch_bounds__(kColThreads, (colstats_waves_per_simd<T, CAUSA
     if (MODE == kStatSumSq) totsq = across(totsq, add);
     float top = fmaxf(fmaxf(best[key][0], best[key][1]), fmaxf(best[key][2], best[key][3]));
     if (CORM) top = across(top, mx);
+    tots[key] = tot, totsqs[key] = totsq, tops[key] = top;
+    if (TEAMS > 1 && team == 1 && writer) {
+      s_fold[kjs[key] - j0] = CORM ? top : tot;
+      if (MODE == kStatSumSq) s_fold[BK + kjs[key] - j0] = totsq;
+    }
+  }
+  if (TEAMS > 1) {
+    __syncthreads();
+    if (team == 1) return;
+  }
+#pragma unroll
+  for (int key = 0; key < NKEY; ++key) {
+    float tot = tots[key], totsq = totsqs[key], top = tops[key];
+    if (TEAMS > 1 && writer) {
+      const float other = s_fold[kjs[key] - j0];
+      tot += other;
+      top = fmaxf(top, other);
+      if (MODE == kStatSumSq) totsq += s_fold[BK + kjs[key] - j0];
+    }
     if (writer && kjs[key] < p.Skv) {
       const int64_t idx = (int64_t)bh * p.Skv + kjs[key];
       if (CORM) {
@@ -572,16 +613,14 @@ __global__ void __launch_bounds__(kColThreads, (colstats_waves_per_simd<T, CAUSA
 
 int device_cu_count();  // attn_fwd.hip
 
-int colstats_keys_override();  // colstats.hip: 0, or the 16-key columns per lane that FT_COLSTATS_KEYS asks for
-
-template <typename T, int D, bool CAUSAL, bool EMU, int MODE, int NKEYS>
+template <typename T, int D, bool CAUSAL, bool EMU, int MODE, int NKEYS, int TEAMS = 1>
 hipError_t launch_colstats_one(const ColstatsKernelParams& p, hipStream_t stream) {
   const int nJB = (p.Skv + 64 * NKEYS - 1) / (64 * NKEYS);
   dim3 grid((unsigned)(nJB * p.B * p.H));
   ColstatsKernelParams pp = p;
   const int64_t cus = device_cu_count();
-  pp.pair_order = CAUSAL && (int64_t)grid.x > cus && (int64_t)grid.x <= 2 * cus;
-  hipLaunchKernelGGL((colstats_kernel<T, D, CAUSAL, EMU, MODE, NKEYS>), grid, dim3(kColThreads), 0, stream, pp);
+  pp.pair_order = CAUSAL && TEAMS == 1 && (int64_t)grid.x > cus && (int64_t)grid.x <= 2 * cus;
+  hipLaunchKernelGGL((colstats_kernel<T, D, CAUSAL, EMU, MODE, NKEYS, TEAMS>), grid, dim3(kColThreads * TEAMS), 0, stream, pp);
   return hipGetLastError();
 }
 

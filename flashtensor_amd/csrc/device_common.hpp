@@ -190,7 +190,7 @@ struct TileStager {
     rsrc = make_rsrc(base);
     row_bytes = (uint32_t)(row_stride * 2);
     const int lane = lane_id();
-    const int wave = wave_id();
+    const int wave = wave_id() & (NT / 64 - 1);
 #pragma unroll
     for (int it = 0; it < ROUNDS; ++it) {
       const int slot = it * NT + wave * 64 + lane;
@@ -204,7 +204,7 @@ struct TileStager {
   // A tile known to lie entirely inside the operand: straight-line code (one load per round) that a
   // caller can spread between other instructions.
   __device__ __forceinline__ void issue_full(int row0, char* lds_tile) const {
-    const int wave = wave_id();
+    const int wave = wave_id() & (NT / 64 - 1);
     const uint32_t tile_off = (uint32_t)row0 * row_bytes;  // wave-uniform
 #pragma unroll
     for (int it = 0; it < ROUNDS; ++it) {
@@ -215,7 +215,7 @@ struct TileStager {
 
   // Tile whose row 0 is row `row0` of the operand.
   __device__ __forceinline__ void issue(int row0, int rows_valid, char* lds_tile) const {
-    const int wave = wave_id();
+    const int wave = wave_id() & (NT / 64 - 1);
     const uint32_t tile_off = (uint32_t)row0 * row_bytes;  // wave-uniform
     if (rows_valid >= ROWS) {
       issue_full(row0, lds_tile);
