@@ -23,7 +23,7 @@ int device_cu_count() {
 
 // Test hook: FT_ATTN_FORM in the environment overrides the launch shape the dispatcher would pick for the
 // problem size ("4": 128-row workgroups; "8": 256-row workgroups, one query block each; "8x2": 256-row workgroups
-// that take the heaviest and the lightest remaining block; an "h" appended: head-major workgroup order), so that
+// that take the heaviest and the lightest remaining block; an "h" appended: head-major workgroup order; "t": two teams of waves), so that
 // every form can be checked on every shape whatever the CU count of the device.  Read on every launch.
 int attn_form_override() {
   const char* e = getenv("FT_ATTN_FORM");
@@ -31,6 +31,7 @@ int attn_form_override() {
   int form = 0;
   if (e[0] == '4') form = 1;
   else if (e[0] == '8') form = (e[1] == 'x' && e[2] == '2') ? 3 : 2;
+  else if (e[0] == 't') form = 16;
   for (const char* c = e; *c; ++c)
     if (*c == 'h') form |= 8;
   return form;
@@ -50,7 +51,38 @@ hipError_t launch_attn_f16_d128(const AttnKernelParams& p, bool causal, bool emu
 hipError_t launch_attn_bf16_d64(const AttnKernelParams& p, bool causal, bool emu, int kf, hipStream_t s);
 hipError_t launch_attn_bf16_d128(const AttnKernelParams& p, bool causal, bool emu, int kf, hipStream_t s);
 
+hipError_t launch_attn_teams_f16(const AttnKernelParams& p, int D, bool emu, int kf, unsigned grid, hipStream_t s);
+hipError_t launch_attn_teams_bf16(const AttnKernelParams& p, int D, bool emu, int kf, unsigned grid, hipStream_t s);
+
+// Two teams of waves on blocks of 64 rows (attn_split.hpp) instead of four waves on 128: half the rows and half the chain of
+// key tiles per workgroup.  Taken where the chain is the launch: with a workgroup of this form for every CU at most, from
+// ten key tiles on (attention calls, same process: B1 H8 D128 S1000 21.1 -> 18.1 us, S2048 35.6 -> 29.3; D64, of whose
+// workgroups a CU holds two, from five tiles on: H8 S1000 14.9 -> 12.0).  Shorter plain calls have 2 us at most to gain
+// (S500 14.0 -> 12.3) and keep to the forms whose results agree bit for bit; soft-capped ones, whose waves are slow
+// enough alone, take it from four tiles on (S300 13.4 -> 12.2, S500 19.4 -> 14.9, S130 9.6 -> 9.8).
+// With up to two workgroups for every CU: D64 gains under the causal mask, whose blocks differ in length (B1 H16 S2048
+// 25.2 -> 22.8; without the mask 28.6 -> 30.5; plain prompts beyond 32 tiles again keep to the bit-equal forms); D128 does not
+// (128 KB of LDS, and two in turn: H16 S2048 37.1 -> 38.7) but for soft-capped logits over twelve tiles or more (H16 S2048
+// 59.2 -> 47.8, H32 S777 26.8 -> 24.6, but B2 H32 S500 20.5 -> 23.0).
+static bool use_teams(const AttnKernelParams& p, int D, bool causal, bool cap, int64_t grid) {
+  const int forced = attn_form_override();
+  if (forced || attn_split_override()) return (forced & 16) != 0;
+  const int64_t cus = device_cu_count();
+  const int tiles = (p.Skv + 63) / 64;
+  if (tiles <= (cap ? 3 : D == 64 ? 5 : 10) || grid > 2 * cus) return false;
+  if (grid <= cus) return true;
+  return causal && (D == 64 ? cap || tiles <= 32 : cap && tiles > 11);
+}
+
 hipError_t launch_attn_fwd(const AttnKernelParams& p, int D, bool bf16, bool causal, bool emu, int kf, hipStream_t s) {
+  const int64_t rows = (int64_t)p.Sq * p.group, grid = (rows + 63) / 64 * p.B * (p.H / p.group);
+  if ((kf == kKfNone || kf == kKfSoftcap) && rows < 0x7fffffff - 64 && grid < 0x7fffffff && use_teams(p, D, causal, kf == kKfSoftcap, grid)) {
+    AttnKernelParams pp = p;
+    if (!causal) pp.off = p.Skv;
+    // (D = 64: two workgroups per CU; see the kernel)
+    pp.pair_order = causal && D == 64 && grid > device_cu_count() && grid <= 2 * device_cu_count();
+    return bf16 ? launch_attn_teams_bf16(pp, D, emu, kf, (unsigned)grid, s) : launch_attn_teams_f16(pp, D, emu, kf, (unsigned)grid, s);
+  }
   if (D == 128) return bf16 ? launch_attn_bf16_d128(p, causal, emu, kf, s) : launch_attn_f16_d128(p, causal, emu, kf, s);
   if (D == 64) return bf16 ? launch_attn_bf16_d64(p, causal, emu, kf, s) : launch_attn_f16_d64(p, causal, emu, kf, s);
   return hipErrorInvalidValue;

@@ -50,8 +50,12 @@ __device__ __forceinline__ SplitPartial split_partial(float* base, int D, int64_
 // its accumulator, row maxima and row sums in the workspace and attn_combine_kernel folds them.  Built for the causal
 // instantiation only: without a mask `off` is set to Skv, which hides nothing.
 // STORE: the 16-bit logits of the rows go to the workspace as well, for the column sums (attn_split.hip).
-template <typename T, int D, bool CAUSAL, bool EMU, int KF, int WAVES, bool SPLIT = false, bool STORE = false>
-__global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVES)) attn_fwd_kernel(const AttnKernelParams p) {
+// TEAMS = 2 (SPLIT): the two shares of a block of 64 rows are taken by two pairs of waves of one workgroup, each with LDS
+// buffers of its own, and fold in LDS: each wave has its SIMD to itself, as in a launch of fewer 128-row blocks than CUs, which
+// is bound by the chain of its longest block (0.9 us a tile at D128, whatever the other CUs do), and the chain is half as
+// long.  B1 H8 S2048 D128 36 -> 29 us, soft-capped 58 -> 39; D64 25 -> 20 (when it is taken: attn_fwd.hip).
+template <typename T, int D, bool CAUSAL, bool EMU, int KF, int WAVES, bool SPLIT = false, bool STORE = false, int TEAMS = 1>
+__global__ void __launch_bounds__(64 * WAVES * TEAMS, (KF == kKfTensorLds ? 1 : 8 / (WAVES * TEAMS))) attn_fwd_kernel(const AttnKernelParams p) {
   constexpr int BM = 32 * WAVES, BN = kAttnBN, NT = 64 * WAVES;
   constexpr int KSTEPS = D / 16;
   constexpr int DB = D / 32;
@@ -73,17 +77,23 @@ __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVE
   // K therefore runs one tile ahead of V in LDS.
   // One LDS object per buffer: the compiler tracks outstanding direct-to-LDS loads per object, so reads
   // of one buffer do not wait for the loads in flight into the others.
-  __shared__ __align__(16) char ldsK0[TILE_BYTES];
-  __shared__ __align__(16) char ldsK1[TILE_BYTES];
-  __shared__ __align__(16) char ldsV0[TILE_BYTES];
-  __shared__ __align__(16) char ldsV1[TILE_BYTES];
+  __shared__ __align__(16) char s_k0[TEAMS * TILE_BYTES];
+  __shared__ __align__(16) char s_k1[TEAMS * TILE_BYTES];
+  __shared__ __align__(16) char s_v0[TEAMS * TILE_BYTES];
+  __shared__ __align__(16) char s_v1[TEAMS * TILE_BYTES];
+  const int team = TEAMS > 1 ? wave_id() / WAVES : 0;
+  char* const ldsK0 = s_k0 + team * TILE_BYTES;
+  char* const ldsK1 = s_k1 + team * TILE_BYTES;
+  char* const ldsV0 = s_v0 + team * TILE_BYTES;
+  char* const ldsV1 = s_v1 + team * TILE_BYTES;
   __shared__ __align__(16) uint32_t ldsCol[2 * BN];  // noise column terms of the current / next tile
   // kKfTensorLds: every wave's slice of the next noise tile (32 rows x 64 keys fp32), one 16-byte slot per lane and
   // load instruction: a lane reads back exactly the slots it filled
   constexpr int kErWaveBytes = 32 * BN * 4;
   __shared__ __align__(16) char ldsEr[kErLds ? WAVES * kErWaveBytes : 16];
 
-  static_assert(!SPLIT || (CAUSAL && WAVES == 4 && (KF == kKfNone || KF == kKfSoftcap)), "the split form's instantiations");
+  static_assert(TEAMS == 1 || (SPLIT && !STORE && WAVES == 2 && TEAMS == 2), "the teams' instantiations");
+  static_assert(!SPLIT || (CAUSAL && WAVES * TEAMS == 4 && (KF == kKfNone || KF == kKfSoftcap)), "the split form's instantiations");
   static_assert(!STORE || (SPLIT && EMU && KF == kKfNone), "logits are kept where they are 16-bit values");
   const int rows = SPLIT ? p.Sq * p.group : p.Sq;  // rows of a (b, h) pair; SPLIT: of a (b, k/v head) pair
   const int BH = SPLIT ? p.B * (p.H / p.group) : p.B * p.H;
@@ -113,13 +123,15 @@ __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVE
     mb = rank < half ? nMB - 1 - rank : rank - half;
   }
   int chunk = 0;
-  if (SPLIT) {
+  if (TEAMS > 1) {
+    chunk = team;
+  } else if (SPLIT) {
     mb = p.items[rank] >> 8;
     chunk = p.items[rank] & 255;
   }
   const int b = SPLIT ? bh / (p.H / p.group) : bh / p.H;
   const int h = SPLIT ? (bh % (p.H / p.group)) * p.group : bh % p.H;  // SPLIT: the group's first head
-  const int lane = lane_id(), wave = wave_id();
+  const int lane = lane_id(), wave = TEAMS > 1 ? wave_id() % WAVES : wave_id();
   const int g = lane >> 5, n = lane & 31;
   // two_blocks (causal, set by the launcher when the pairs fill the chip evenly): the workgroup takes query
   // block nMB - 1 - slot and then block slot, the heaviest with the lightest, so that every workgroup walks the
@@ -163,15 +175,17 @@ __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVE
   if (CAUSAL) n_end = min(Skv, (SPLIT ? (min(m0 + BM, rows) - 1) / p.group + 1 : m0 + BM) + off);
   int ntiles = (n_end + BN - 1) / BN;
   int nch = 1;  // shares of this row block
+  int ntrips = 0;  // TEAMS: barriers that every wave takes part in, whatever its own share
   if (SPLIT) {
-    nch = (ntiles + p.chunk_tiles - 1) / p.chunk_tiles;
+    nch = TEAMS > 1 ? TEAMS : (ntiles + p.chunk_tiles - 1) / p.chunk_tiles;
     const int per = (ntiles + nch - 1) / nch, t0 = chunk * per, t1 = min(t0 + per, ntiles);
+    ntrips = per;
     kbase += (int64_t)t0 * BN * p.sk.s;
     vbase += (int64_t)t0 * BN * p.sv.s;
     off -= t0 * BN;
     if (STORE) logit_row += t0 * BN;
     Skv = min(Skv, t1 * BN) - t0 * BN;
-    ntiles = t1 - t0;  // >= 1: (nch - 1) per <= (nch - 1) chunk_tiles < tiles of the block
+    ntiles = t1 - t0;  // >= 1: (nch - 1) per <= (nch - 1) chunk_tiles < tiles of the block (TEAMS: the second team may have none)
   }
   int nw = ntiles, n_fast = Skv / BN;
   if (CAUSAL && !SPLIT) {
@@ -623,19 +637,20 @@ __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVE
     fast_exp(masked_tag, s_cur, pb, n0, it);
     pv(pb, tv);
     pend_max = tile_max(next_masked_tag, s_next, n0 + BN);
+    constexpr int kStageEvery = TEAMS > 1 ? 2 : 4;  // (the loads of a tile fall to fewer waves)
     __builtin_amdgcn_sched_group_barrier(0x100, 6, 2);
 #pragma unroll
     for (int i = 0; i < 2 * KSTEPS; ++i) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 2);
       __builtin_amdgcn_sched_group_barrier(0x100, 2, 2);
-      if (STAGE && (i & 3) == 1) __builtin_amdgcn_sched_group_barrier(0x020, 1, 2);
+      if (STAGE && i % kStageEvery == 1) __builtin_amdgcn_sched_group_barrier(0x020, 1, 2);
       __builtin_amdgcn_sched_group_barrier(0x002, kValuGroup, 2);
     }
 #pragma unroll
     for (int i = 0; i < 4 * DB; ++i) {
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 2);
       __builtin_amdgcn_sched_group_barrier(0x100, 2, 2);
-      if (STAGE && (i & 3) == 1) __builtin_amdgcn_sched_group_barrier(0x020, 1, 2);
+      if (STAGE && i % kStageEvery == 1) __builtin_amdgcn_sched_group_barrier(0x020, 1, 2);
       __builtin_amdgcn_sched_group_barrier(0x002, kValuGroup, 2);
     }
   };
@@ -713,7 +728,7 @@ __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVE
     for (int mbk = 0; mbk < 2; ++mbk) S0[mbk] = S1[mbk];
   }
   // ---- tiles entirely above this wave's diagonal: keep the workgroup's barriers and staging in step
-  for (; it < ntiles; ++it) sync_and_stage(it, (it & 1) ? ldsK1 : ldsK0, (it & 1) ? ldsV0 : ldsV1);
+  for (; it < (TEAMS > 1 ? ntrips : ntiles); ++it) sync_and_stage(it, (it & 1) ? ldsK1 : ldsK0, (it & 1) ? ldsV0 : ldsV1);
   } else {
   // ---- generic path: not pipelined across tiles.  K and V of tile it are read while those of tile it + 1 are
   // loaded; a tile is worked on as two halves of 32 keys (8 + 8 MFMAs each), every key masked by comparison.
@@ -805,7 +820,35 @@ __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVE
 
   // ---- epilogue
   l_run += xchg32(l_run);
-  if (SPLIT && nch > 1) {
+  if constexpr (TEAMS > 1) {
+    // the second team's accumulators, row maxima and row sums through LDS (the tiles' buffers) to the first team
+    float4v* fold_o = reinterpret_cast<float4v*>(s_k0) + wave * (DB * 4 * 64) + lane;
+    float* fold_ml = reinterpret_cast<float*>(s_v0) + wave * 128 + lane;
+    static_assert(WAVES * DB * 4 * 64 * 16 <= TEAMS * TILE_BYTES && WAVES * 128 * 4 <= TEAMS * TILE_BYTES, "room of the fold");
+    wait_vmem();
+    __syncthreads();
+    if (team == 1) {
+#pragma unroll
+      for (int i = 0; i < DB * 4; ++i)
+        fold_o[i * 64] = float4v{o_acc[i >> 2][4 * (i & 3)], o_acc[i >> 2][4 * (i & 3) + 1], o_acc[i >> 2][4 * (i & 3) + 2], o_acc[i >> 2][4 * (i & 3) + 3]};
+      fold_ml[0] = m_run;
+      fold_ml[64] = l_run;
+    }
+    __syncthreads();
+    if (team == 1) return;
+    const float m1 = fold_ml[0], l1 = fold_ml[64];
+    const float m_new = fmaxf(m_run, m1);  // (the first team has seen key 0)
+    const float w0 = __builtin_amdgcn_exp2f(m_run - m_new), w1 = __builtin_amdgcn_exp2f(m1 - m_new);
+    m_run = m_new;
+    l_run = __builtin_fmaf(l1, w1, l_run * w0);
+#pragma unroll
+    for (int i = 0; i < DB * 4; ++i) {
+      const float4v o1 = fold_o[i * 64];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o_acc[i >> 2][4 * (i & 3) + e] = __builtin_fmaf(o1[e], w1, o_acc[i >> 2][4 * (i & 3) + e] * w0);
+    }
+  }
+  if (SPLIT && TEAMS == 1 && nch > 1) {
     // unnormalised: accumulator registers as they are, one 16-byte piece per lane and store (coalesced), rows that exist
     const SplitPartial part = split_partial(p.part, D, ((int64_t)bh * p.nitems + rank) * p.part_waves + wave);
     if (qrow < rows) {
@@ -856,7 +899,7 @@ __global__ void __launch_bounds__(64 * WAVES, (KF == kKfTensorLds ? 1 : 8 / WAVE
 
 int device_cu_count();     // attn_fwd.hip
 int attn_split_override();  // attn_fwd.hip: 0, or -1: never split, n > 0: split into shares of n tiles
-int attn_form_override();  // attn_fwd.hip: 0, or (1: 4 waves, 2: 8 waves, 3: 8 waves and two blocks) | 8: head-major order
+int attn_form_override();  // attn_fwd.hip: 0, or (1: 4 waves, 2: 8 waves, 3: 8 waves and two blocks) | 8: head-major order, or 16: two teams of waves
 
 template <typename T, int D, bool CAUSAL, bool EMU, int KF>
 hipError_t launch_one(const AttnKernelParams& p0, hipStream_t stream) {

@@ -26,4 +26,17 @@ hipError_t launch_split_td(const AttnKernelParams& p, bool emu, int kf, unsigned
   return hipErrorInvalidValue;
 }
 
+// Blocks of 64 rows, a workgroup of two teams for each (heaviest first).
+template <typename T, int D>
+hipError_t launch_teams_td(const AttnKernelParams& p, bool emu, int kf, unsigned grid, hipStream_t s) {
+#define FT_CASE(E, K)                                                                                                    \
+  if (emu == E && kf == K) {                                                                                             \
+    hipLaunchKernelGGL((attn_fwd_kernel<T, D, true, E, K, 2, true, false, 2>), dim3(grid), dim3(256), 0, s, p);          \
+    return hipGetLastError();                                                                                            \
+  }
+  FT_CASE(true, kKfNone) FT_CASE(false, kKfNone) FT_CASE(true, kKfSoftcap) FT_CASE(false, kKfSoftcap)
+#undef FT_CASE
+  return hipErrorInvalidValue;
+}
+
 }  // namespace ft

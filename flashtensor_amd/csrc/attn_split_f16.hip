@@ -5,4 +5,8 @@ namespace ft {
 hipError_t launch_attn_split_f16(const AttnKernelParams& p, int D, bool emu, int kf, unsigned grid, unsigned lds, hipStream_t s) {
   return D == 128 ? launch_split_td<F16, 128>(p, emu, kf, grid, lds, s) : launch_split_td<F16, 64>(p, emu, kf, grid, lds, s);
 }
+hipError_t launch_attn_teams_f16(const AttnKernelParams& p, int D, bool emu, int kf, unsigned grid, hipStream_t s) {
+  return D == 128 ? launch_teams_td<F16, 128>(p, emu, kf, grid, s) : launch_teams_td<F16, 64>(p, emu, kf, grid, s);
+}
+
 }  // namespace ft

@@ -1,5 +1,6 @@
-"""The split form of the attention pass (a row block's keys shared out between workgroups) against the CPU oracle: rows of
-one wave and of several, shares of one tile, keys one off a tile, rows that see no key of a share."""
+"""The forms of the attention pass that share out a row block's keys, between workgroups ("s") and between the two teams of
+waves of one ("t"), against the CPU oracle: rows of one wave and of several, one off a block, shares of one tile or none,
+keys one off a tile, rows that see no key of a share."""
 import pytest
 import torch
 
@@ -9,12 +10,13 @@ from flashtensor_amd import _lib, ops
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("tiles", [1, 3])
+@pytest.mark.parametrize("form", ["s1", "s3", "t"])
 @pytest.mark.parametrize("Sq,Skv,H,Hkv,D,dtype", [
     (1, 65, 8, 2, 128, torch.float16), (1, 1000, 4, 4, 64, torch.bfloat16), (8, 449, 8, 2, 64, torch.float16), (33, 129, 4, 1, 128, torch.float16),
-    (130, 1090, 4, 2, 64, torch.float16), (300, 300, 2, 2, 128, torch.float16), (257, 640, 2, 1, 128, torch.bfloat16)])
-def test_shares_of_the_keys(gpu, monkeypatch, tiles, Sq, Skv, H, Hkv, D, dtype):
-  monkeypatch.setenv("FT_ATTN_FORM", f"s{tiles}")
+    (130, 1090, 4, 2, 64, torch.float16), (300, 300, 2, 2, 128, torch.float16), (257, 640, 2, 1, 128, torch.bfloat16),
+    (1, 1, 1, 1, 128, torch.float16), (64, 64, 2, 2, 64, torch.bfloat16), (65, 65, 3, 3, 128, torch.float16), (63, 129, 2, 2, 64, torch.float16)])
+def test_shares_of_the_keys(gpu, monkeypatch, form, Sq, Skv, H, Hkv, D, dtype):
+  monkeypatch.setenv("FT_ATTN_FORM", form)
   g = torch.Generator().manual_seed(Sq + Skv)
   q, k, v = (torch.randn(s, h * D, dtype=dtype, generator=g) for s, h in ((Sq, H), (Skv, Hkv), (Skv, Hkv)))
   dev = [t.to(gpu).view(1, t.shape[0], -1, D) for t in (q, k, v)]
