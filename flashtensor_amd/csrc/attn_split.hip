@@ -27,7 +27,9 @@ struct SplitShape {
 // and the launch, then 0.9 per tile where it has its CU to itself and 2.2 where two share one: the second wave of a
 // SIMD hides little of the first one's work (soft-capped logits: 1.9 and 3.5; there it does).  Partial results are
 // written at 10 MB/us and folded at 7, by a kernel that takes 5.5 us to begin with, its launch included; K and V come from HBM at 5.
-constexpr double kLaunch = 7.0, kCombine = 5.5, kPartWrite = 10e6, kPartRead = 7e6, kKvBytes = 5e6;
+// In a launch of more workgroups than fit at once each further one in a slot takes 1 us until its first tile has landed (left
+// out of account, B5 H32 Sq3 Skv3329 soft-capped bf16 became 8480 workgroups of one tile: 126 us against 100 unsplit).
+constexpr double kLaunch = 7.0, kCombine = 5.5, kNext = 1.0, kPartWrite = 10e6, kPartRead = 7e6, kKvBytes = 5e6;
 
 SplitPlan make_plan(const SplitShape& a) {
   SplitPlan plan{};
@@ -57,7 +59,7 @@ SplitPlan make_plan(const SplitShape& a) {
     for (int i = 0; i < items; ++i)
       for (int64_t j = 0; j < per_xcd; ++j) {
         std::pop_heap(free_at.begin(), free_at.end(), std::greater<double>());
-        free_at.back() += len[i] * shared_cu;
+        free_at.back() += len[i] * shared_cu + kNext;
         end = std::max(end, free_at.back());
         std::push_heap(free_at.begin(), free_at.end(), std::greater<double>());
       }
