@@ -32,6 +32,10 @@ constexpr bool kAttnTwoBlocks = true;
 // rescaled) while the new row maximum exceeds it by less than this, so unnormalised probabilities stay
 // below 2^kRescaleSlack (exact in fp16/fp32; the final division uses the same maximum).
 constexpr float kRescaleSlack = 6.f;
+// Where the running maximum begins: the lowest finite value.  Visible logits may be -inf (a QK^T below the range of the
+// tensor type); a tile that shows a row nothing else leaves the maximum here, and its exponentials are exp2(-inf - kNoMax) = 0,
+// where a maximum of -inf would make them NaN.  A row that ends here has seen no finite logit: its sum is 0.
+constexpr float kNoMax = -__FLT_MAX__;
 
 // One share's partial result of a row block in the workspace (SPLIT): per wave of 32 rows the accumulator registers of
 // its 64 lanes, row maxima and row sums.
@@ -270,8 +274,8 @@ __global__ void __launch_bounds__(64 * WAVES * TEAMS, (KF == kKfTensorLds ? 1 : 
   for (int i = 0; i < DB; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) o_acc[i][r] = 0.f;
-  float m_run = NEG_INF, l_run = 0.f;  // running max (log2 domain) and this lane's share of the row sum
-  float m_kf = NEG_INF, l_kf = 0.f;
+  float m_run = kNoMax, l_run = 0.f;  // running max (log2 domain) and this lane's share of the row sum
+  float m_kf = kNoMax, l_kf = 0.f;
   float16v S0[2], S1[2];  // score accumulators of the current / next tile (they swap every tile)
 
   // Per-lane LDS byte offsets of the MFMA operand reads inside a tile (the XOR swizzles make them
@@ -330,8 +334,7 @@ __global__ void __launch_bounds__(64 * WAVES * TEAMS, (KF == kKfTensorLds ? 1 : 
     const bool grow = rowmax > m_run + kRescaleSlack;  // identical in both lanes of a row
     if (__any(grow)) {
       const float m_new = grow ? rowmax : m_run;
-      // (SPLIT: a row that has seen no key yet keeps -inf, whose difference with itself is no number)
-      const float alpha = SPLIT && !grow ? 1.f : __builtin_amdgcn_exp2f(m_run - m_new);
+      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
       if (KF == kKfSeededTau1) l_kf *= alpha;
       if (KF == kKfSeededFast) l_kf *= __builtin_amdgcn_exp2f((m_run - m_new) * p.inv_tau);
       m_run = m_new;
@@ -560,8 +563,7 @@ __global__ void __launch_bounds__(64 * WAVES * TEAMS, (KF == kKfTensorLds ? 1 : 
       for (int r = 3; r < 15; r += 2) zmax = max3(zmax, z[r], z[r + 1]);
       zmax = fmaxf(zmax, z[15]);
       zmax = fmaxf(zmax, xchg32(zmax));
-      // finite from the first half on: key 0 is visible to every row, so a later half that is hidden
-      // entirely (zmax = -inf) adds exp2(-inf) = 0
+      // (finite: a half that is hidden entirely, zmax = -inf, adds exp2(-inf) = 0)
       const float mk_new = fmaxf(m_kf, zmax);
       float zs = 0.f;
 #pragma unroll
@@ -837,7 +839,7 @@ __global__ void __launch_bounds__(64 * WAVES * TEAMS, (KF == kKfTensorLds ? 1 : 
     __syncthreads();
     if (team == 1) return;
     const float m1 = fold_ml[0], l1 = fold_ml[64];
-    const float m_new = fmaxf(m_run, m1);  // (the first team has seen key 0)
+    const float m_new = fmaxf(m_run, m1);
     const float w0 = __builtin_amdgcn_exp2f(m_run - m_new), w1 = __builtin_amdgcn_exp2f(m1 - m_new);
     m_run = m_new;
     l_run = __builtin_fmaf(l1, w1, l_run * w0);

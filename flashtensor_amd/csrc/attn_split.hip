@@ -157,11 +157,11 @@ __device__ __forceinline__ int shares_of_block(const AttnKernelParams& p, int mb
 
 // Folds the shares of a row, eight loads at a time: running maximum and sum, and what `f(share, weight)` adds up;
 // `scale` multiplies that when the maximum moves.  slot0: the row's wave in the first share, n: the row in the wave; every
-// `step`-th share is taken.  A part whose shares hide every key from the row leaves M = -inf, sum = 0.
+// `step`-th share is taken.  A share that shows the row no finite logit has m = kNoMax, l = 0.
 template <typename L, typename F, typename S>
 __device__ __forceinline__ void fold_shares(const AttnKernelParams& p, int D, int64_t slot0, int n, int nch, int step, float& M, float& sum, L load, F f, S scale) {
   constexpr int U = 8;
-  M = -__builtin_inff(), sum = 0.f;
+  M = kNoMax, sum = 0.f;
   for (int c0 = 0; c0 < nch; c0 += U) {
     float m[U], l[U];
     float4v o[U];
@@ -175,13 +175,12 @@ __device__ __forceinline__ void fold_shares(const AttnKernelParams& p, int D, in
     float M1 = M;
 #pragma unroll
     for (int u = 0; u < U; ++u) M1 = fmaxf(M1, m[u]);
-    const float base = M1 == -__builtin_inff() ? 0.f : M1;
-    const float move = __builtin_amdgcn_exp2f(M - base);
+    const float move = __builtin_amdgcn_exp2f(M - M1);
     sum *= move;
     scale(move);
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const float w = c0 + u < nch ? __builtin_amdgcn_exp2f(m[u] - base) : 0.f;  // 0 too for a share that hides every key from the row
+      const float w = c0 + u < nch ? __builtin_amdgcn_exp2f(m[u] - M1) : 0.f;
       sum = __builtin_fmaf(w, l[u], sum);
       f(o[u], w);
     }
@@ -270,7 +269,7 @@ __global__ void __launch_bounds__(256) split_stats_kernel(const AttnKernelParams
     const int row = t & 31, part = t >> 5, rc = min(row, rows - 1);
     const int nch = shares_of_block(p, 0);
     if (nch > 1) {
-      float M = -__builtin_inff(), L = 0.f;
+      float M = kNoMax, L = 0.f;
       if (part < nch)
         fold_shares(p, D, (int64_t)bh * p.nitems + part, rc, (nch - part + 7) >> 3, 8, M, L, [](const SplitPartial&, float4v&) {},
                     [](const float4v&, float) {}, [](float) {});
