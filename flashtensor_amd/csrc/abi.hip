@@ -126,11 +126,12 @@ float tuned_logit_multiplier(int D, bool bf16) {
   return best;
 }
 
-// Packed-fp16 form of the division by sqrt(128) used by the fp16 fast paths: with hi = 0.70751953125 and
-// lo = -0.0004127025604248047 (both fp16), fma16(h, hi, mul16(h, lo)) == 8 * f16(h / sqrt(128)) for every finite
-// fp16 h whose quotient is at least 2.5e-3 in magnitude, and is within 2e-6 * 8 of it below (checked here over
-// all 65536 inputs on first use; a logit that small moves a probability by 2e-6 relative).  D = 64 needs no
-// constants: h / 8 is exact.
+// Packed-fp16 form of the division by sqrt(128) used by the fp16 fast paths: with hi = 0.7001953125 and
+// lo = 0.0069122314453125 (both fp16), fma16(h, hi, mul16(h, lo)) == 8 * f16(h / sqrt(128)) for every finite
+// fp16 h whose quotient is at least 7e-4 in magnitude, and is within 5e-7 of it (times 8) below (checked here over
+// all 65536 inputs on first use; a logit that small moves a probability by 5e-7 relative).  Both constants are
+// positive, so that an infinite h keeps its sign (with one of either sign inf * hi + inf * lo is NaN).  Of all pairs of a
+// positive lo and a hi in [0.61, 0.7071] this one is exact furthest down.  D = 64 needs no constants: h / 8 is exact.
 struct PackedLogitConstants {
   uint32_t hi2, lo2;  // the constant in both halves of a 32-bit word
   bool good;          // the exhaustive check passed
@@ -138,7 +139,7 @@ struct PackedLogitConstants {
 const PackedLogitConstants& packed_logit_constants() {
   // a function-local static is initialised exactly once per process, by whichever thread gets here first
   static const PackedLogitConstants consts = [] {
-    const _Float16 hi = (_Float16)0.70751953125f, lo = (_Float16)-0.0004127025604248047f;
+    const _Float16 hi = (_Float16)0.7001953125f, lo = (_Float16)0.0069122314453125f;
     bool ok = true;
     const float c = (float)std::sqrt(128.0);
     for (uint32_t bits = 0; bits < 65536 && ok; ++bits) {
@@ -147,7 +148,7 @@ const PackedLogitConstants& packed_logit_constants() {
       const double want = (double)(float)(_Float16)(x / c);
       const double cterm = (double)(float)(_Float16)((double)x * (double)(float)lo);
       const double got = (double)(float)(_Float16)((double)x * (double)(float)hi + cterm) / 8.0;
-      if (got != want && (std::fabs(want) >= 2.5e-3 || std::fabs(got - want) > 2e-6)) ok = false;
+      if (got != want && (std::fabs(want) >= 7e-4 || std::fabs(got - want) > 5e-7)) ok = false;
     }
     const uint16_t hb = float_to_half_bits((float)hi), lb = float_to_half_bits((float)lo);
     return PackedLogitConstants{(uint32_t)hb | ((uint32_t)hb << 16), (uint32_t)lb | ((uint32_t)lb << 16), ok};

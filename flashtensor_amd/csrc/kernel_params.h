@@ -29,7 +29,7 @@ struct AttnKernelParams {
   float inv_tau;
   // packed fp16 form of the same division for D = 128 (two packed ops on element pairs instead of one
   // mixed-precision multiply per element): t8 = fma(h, pk_hi, h * pk_lo) is 8 * f16(h / sqrt(D)) for every
-  // fp16 h except where |h / sqrt(D)| < 2.5e-3, and there within 2e-6 of it; both halves hold the constant
+  // fp16 h except where |h / sqrt(D)| < 7e-4, and there within 5e-7 of it; both halves hold the constant
   uint32_t pk_hi2, pk_lo2;
   float softcap;    // kKfSoftcap: logits become softcap * tanh(logit / softcap)
   int pair_order;   // block order of the causal attention kernel: heavy half descending, light half ascending

@@ -1057,10 +1057,10 @@ def test_logit_rounding_flips_explain_the_relaxed_bars(gpu, S, D, seed):
   flipped = a != b
   n_flip = int(flipped.sum())
   # One ulp of the fp16 QK^T, carried through the division by sqrt(D): a relative step in (2^-11, 2^-10], i.e.
-  # one or two ulps of the quotient (fp16 spacing 2^-10 * 2^floor(log2 |x|)).  Quotients below 2.5e-3 may also
-  # differ by 2e-6 (the packed form of the division by sqrt(128) is exact above that only).
+  # one or two ulps of the quotient (fp16 spacing 2^-10 * 2^floor(log2 |x|)).  Quotients below 7e-4 may also
+  # differ by 5e-7 (the packed form of the division by sqrt(128) is exact above that only).
   ulp = torch.maximum(a.abs(), b.abs()).clamp_min(2.0 ** -14).log2().floor().exp2() * 2.0 ** -10
-  assert ((a - b).abs() <= 2.001 * ulp + 2e-6).all()
+  assert ((a - b).abs() <= 2.001 * ulp + 5e-7).all()
   assert n_flip <= 4e-3 * a.numel(), f"{n_flip} of {a.numel()} logits differ"
   _, s1, s2 = ops.roco(qd, kd, vd)
   _, r1, r2 = oracle.roco_forward(q, k, v)

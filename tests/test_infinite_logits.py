@@ -38,7 +38,7 @@ def _close(got, ref, tol, what):
     (65, 65, [(64, 65)]),                             # the second team's only key
     (300, 300, [(64, 193)]), (300, 300, [(0, 40)]),   # rows with nothing left: NaN
     (130, 1090, [(0, 70), (500, 600), (1088, 1090)])])
-@pytest.mark.parametrize("D,dtype", [(64, torch.float16), (64, torch.bfloat16), (128, torch.bfloat16)])
+@pytest.mark.parametrize("D,dtype", [(64, torch.float16), (128, torch.float16), (64, torch.bfloat16), (128, torch.bfloat16)])
 def test_keys_below_the_range(gpu, monkeypatch, form, Sq, Skv, lost, D, dtype):
   monkeypatch.setenv("FT_ATTN_FORM", form)
   q, k, v = _inputs(Sq, Skv, 2, D, dtype, lost)
@@ -53,7 +53,7 @@ def test_keys_below_the_range(gpu, monkeypatch, form, Sq, Skv, lost, D, dtype):
   _close(ops.attn(*dev), ref_o, tol, "attn")
 
 
-@pytest.mark.parametrize("D,dtype", [(64, torch.float16), (64, torch.bfloat16)])
+@pytest.mark.parametrize("D,dtype", [(64, torch.float16), (128, torch.float16), (64, torch.bfloat16)])
 @pytest.mark.parametrize("tau", [1.0, 1.5, 0.2])
 def test_keys_below_the_range_under_noise(gpu, D, dtype, tau):
   """The perturbed softmax's own maximum, and the plain one's that the packed forms share."""
