@@ -88,10 +88,18 @@ double float_arg(PyObject* o) {
   if (v == -1.0 && PyErr_Occurred()) throw python_error();
   return v;
 }
-int64_t int_arg(PyObject* o) {
-  const long long v = PyLong_AsLongLong(o);
+// Counts and sizes cross the C ABI as int32: what does not fit is refused, here and nowhere else cut.
+int32_t int32_arg(PyObject* o, const char* what) {
+  int over = 0;
+  const long long v = PyLong_AsLongLongAndOverflow(o, &over);
   if (v == -1 && PyErr_Occurred()) throw python_error();
-  return v;
+  if (over || v != (int32_t)v) bad_value(std::string(what) + " does not fit 32 bits");
+  return (int32_t)v;
+}
+int32_t size32(const at::Tensor& t, int64_t dim) {
+  const int64_t n = t.size(dim);
+  if (n != (int32_t)n) bad_value("need sizes that fit 32 bits but got shape " + str_of(t));
+  return (int32_t)n;
 }
 
 int ft_dtype(at::ScalarType t, bool linear) {
@@ -109,7 +117,7 @@ FtStrides strides_of(const at::Tensor& t) { return FtStrides{t.stride(0), t.stri
 
 struct Qkv {
   const at::Tensor &q, &k, &v;
-  int64_t B, Sq, H, D, Skv, Hkv;
+  int32_t B, Sq, H, D, Skv, Hkv;
   int dtype;
 
   Qkv(PyObject* const* args, bool linear = false) : q(tensor_arg(args[0], 0)), k(tensor_arg(args[1], 1)), v(tensor_arg(args[2], 2)) {
@@ -124,8 +132,8 @@ struct Qkv {
     }
     dtype = ft_dtype(q.scalar_type(), linear);
     if (dtype < 0) bad_call(std::string("arg 0 need dtype float16 or bfloat16") + (linear ? " or float32" : "") + " but got " + str_of(q.scalar_type()));
-    B = q.size(0), Sq = q.size(1), H = q.size(2), D = q.size(3);
-    Skv = k.size(1), Hkv = k.size(2);
+    B = size32(q, 0), Sq = size32(q, 1), H = size32(q, 2), D = size32(q, 3);
+    Skv = size32(k, 1), Hkv = size32(k, 2);
     if (k.size(0) != B || k.size(3) != D || Hkv < 1 || H % Hkv != 0)
       bad_call("arg 1 need shape (" + std::to_string(B) + ", " + std::to_string(Skv) + ", 'a divisor of " + std::to_string(H) + "', " + std::to_string(D) +
                ") but got " + str_of(k));
@@ -134,7 +142,7 @@ struct Qkv {
   }
   FtAttnArgs args(const at::Tensor& o, unsigned flags) const {
     return FtAttnArgs{q.const_data_ptr(), k.const_data_ptr(), v.const_data_ptr(), o.data_ptr(), strides_of(q), strides_of(k), strides_of(v), strides_of(o),
-                      (int32_t)B, (int32_t)H, (int32_t)Sq, (int32_t)Skv, (int32_t)D, dtype, flags, (int32_t)Hkv};
+                      B, H, Sq, Skv, D, dtype, flags, Hkv};
   }
   at::Tensor out() const { return at::empty({B, Sq, H, D}, q.options()); }
   at::Tensor f32(at::IntArrayRef shape) const { return at::empty(shape, q.options().dtype(at::kFloat)); }
@@ -215,7 +223,7 @@ PyObject* roco(PyObject* const* o) {
 PyObject* snapkv(PyObject* const* o) {
   const Qkv x(o);
   void* s = stream_of(x.q);
-  const int kernel = (int)int_arg(o[3]);
+  const int32_t kernel = int32_arg(o[3], "kernel_size");
   const at::Tensor out = x.out(), pooled = x.f32({x.B, x.Hkv, x.Skv});
   const FtAttnArgs a = x.args(out, flags_of(o[4], o[5]));
   const size_t bytes = ft_workspace_bytes_split(FT_OP_SNAPKV, &a);
@@ -283,7 +291,7 @@ PyObject* linattn(PyObject* const* o) {
       if (all[i]->stride(2) != 32)
         bad_value("arg " + std::to_string(i) + " with head_dim 32 need heads stored 32 elements apart but got head stride " + std::to_string(all[i]->stride(2)));
   }
-  const int kind = (int)int_arg(o[3]);
+  const int kind = int32_arg(o[3], "kind");
   const bool normalize_q = flag_arg(o[4]);
   at::ScalarType out_type = x.q.scalar_type();
   if (o[5] != Py_None) {
@@ -314,10 +322,11 @@ PyObject* linattn_block(PyObject* const* o) {
     if (t[i]->scalar_type() != t[0]->scalar_type()) bad_call(arg + " need " + str_of(t[0]->scalar_type()) + " but got " + str_of(t[i]->scalar_type()));
   }
   const at::Tensor& x = *t[0];
-  const int64_t heads = int_arg(o[5]);
+  const int32_t heads = int32_arg(o[5], "head_num");
   if (x.dim() != 3 || heads < 1 || x.size(2) % heads)
     bad_value("x need [B,S,C] with C a multiple of head_num=" + std::to_string(heads) + " but got " + str_of(x));
-  const int64_t B = x.size(0), S = x.size(1), C = x.size(2);
+  const int32_t B = size32(x, 0), S = size32(x, 1);
+  const int64_t C = x.size(2);
   if (t[1]->sizes() != at::IntArrayRef{3 * C, C} || t[3]->sizes() != at::IntArrayRef{C, C})
     bad_value("weights need [" + std::to_string(3 * C) + "," + std::to_string(C) + "] and [" + std::to_string(C) + "," + std::to_string(C) + "] but got " +
               str_of(*t[1]) + " and " + str_of(*t[3]));
@@ -328,11 +337,11 @@ PyObject* linattn_block(PyObject* const* o) {
       bad_value("arg " + std::to_string(i) + " (" + names[i] + ") need a contiguous tensor but got strides " + str_of(t[i]->strides()));
   const int dtype = ft_dtype(x.scalar_type(), true);
   if (dtype < 0) bad_call("arg 0 (x) need float16, bfloat16 or float32 but got " + str_of(x.scalar_type()));
-  const int kind = (int)int_arg(o[6]);
+  const int kind = int32_arg(o[6], "kind");
   const bool normalize_q = flag_arg(o[7]);
   const at::Tensor y = at::empty({B, S, C}, x.options());
   auto data = [&](int i) -> const void* { return t[i] ? t[i]->const_data_ptr() : nullptr; };
-  const FtLinBlockArgs a{data(0), data(1), data(2), data(3), data(4), y.data_ptr(), (int32_t)B, (int32_t)S, (int32_t)heads, (int32_t)(C / heads), dtype};
+  const FtLinBlockArgs a{data(0), data(1), data(2), data(3), data(4), y.data_ptr(), B, S, heads, size32(x, 2) / heads, dtype};
   const size_t bytes = ft_linattn_block_workspace_bytes(&a, kind);
   if (bytes == 0) bad_call(std::string("libflashtensor_hip: ") + ft_last_error());
   const at::Tensor ws = workspace(x, bytes);
@@ -348,12 +357,13 @@ PyObject* topk(PyObject* const* o) {
     bad_call("arg 0 need a float32 GPU tensor but got " + str_of(score.scalar_type()) + " on " + score.device().str());
   if (!score.is_contiguous()) bad_value("arg 0 need a contiguous tensor but got strides " + str_of(score.strides()));
   if (score.dim() < 1 || score.size(-1) < 1) bad_value("arg 0 need a last axis with entries but got " + str_of(score));
-  const int64_t S = score.size(-1), rows = score.numel() / S, k = int_arg(o[1]);
+  const int32_t S = size32(score, -1), k = int32_arg(o[1], "k");
+  const int64_t rows = score.numel() / S;
   std::vector<int64_t> shape = score.sizes().vec();
   shape.back() = k;
   const at::Tensor idx = at::empty(shape, score.options().dtype(at::kLong));
   void* s = stream_of(score);
-  launch([&] { return ft_topk(score.const_data_ptr<float>(), rows, (int32_t)S, (int32_t)k, idx.data_ptr<int64_t>(), s); });
+  launch([&] { return ft_topk(score.const_data_ptr<float>(), rows, S, k, idx.data_ptr<int64_t>(), s); });
   return result(idx);
 }
 
