@@ -2,8 +2,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <functional>
-#include <vector>
+#include <cstdint>
 
 #include "attn_split.hpp"
 
@@ -31,14 +30,53 @@ struct SplitShape {
 // out of account, B5 H32 Sq3 Skv3329 soft-capped bf16 became 8480 workgroups of one tile: 126 us against 100 unsplit).
 constexpr double kLaunch = 7.0, kCombine = 5.5, kNext = 1.0, kPartWrite = 10e6, kPartRead = 7e6, kKvBytes = 5e6;
 
+// `count` shares of `len` tiles.
+struct ShareRun {
+  int len, count;
+};
+
+// When the last workgroup of a launch ends that has more of them than slots: `copies` of every share, longest first, each
+// to the slot that is free first.  Slots that come free together are one entry (there are few: a run adds at most one), so
+// that a round of equal workgroups is one step, and a run on slots that are all free together none at all.
+double rounds_us(const ShareRun* runs, int nruns, int64_t copies, int slots, double tile_us) {
+  struct Free {
+    double at;
+    int64_t n;
+  } f[kSplitMaxBlocks + 2];
+  int nf = 1;
+  f[0] = {0.0, slots};
+  for (int r = 0; r < nruns; ++r) {
+    const double us = runs[r].len * tile_us + kNext;
+    int64_t left = runs[r].count * copies;
+    while (left > 0) {
+      if (nf == 1 && left >= f[0].n) {
+        f[0].at += us * (double)(left / f[0].n);
+        left %= f[0].n;
+        continue;
+      }
+      const int64_t n = std::min(left, f[0].n);
+      const double at = f[0].at + us;
+      left -= n;
+      f[0].n -= n;
+      if (f[0].n == 0) std::copy(f + 1, f + nf--, f);
+      int i = nf;
+      while (i > 0 && f[i - 1].at > at) --i;
+      if (i > 0 && f[i - 1].at == at) {
+        f[i - 1].n += n;
+      } else {
+        std::copy_backward(f + i, f + nf, f + nf + 1);
+        f[i] = {at, n};
+        ++nf;
+      }
+    }
+  }
+  return f[nf - 1].at;
+}
+
 SplitPlan make_plan(const SplitShape& a) {
   SplitPlan plan{};
-  const int64_t pairs = (int64_t)a.B * (a.H / a.group), rows64 = (int64_t)a.Sq * a.group;
-  if (rows64 > 128 * kSplitMaxBlocks || pairs * ((rows64 + 127) / 128) > 4 * a.cus || a.forced < 0) return plan;
-  // A whole prompt (more than half as many queries as keys) keeps its blocks whole: at most a sixth is to be gained there (B1 H8 S2048:
-  // 35 against 29 us), and its results are those of every launch form of the unsplit kernel, bit for bit.
-  if (a.Skv < 2 * (int64_t)a.Sq && a.forced == 0) return plan;
-  const int rows = (int)rows64, nMB = (rows + 127) / 128, off = a.causal ? a.Skv - a.Sq : a.Skv;
+  const int64_t pairs = (int64_t)a.B * (a.H / a.group);
+  const int rows = a.Sq * a.group, nMB = (rows + 127) / 128, off = a.causal ? a.Skv - a.Sq : a.Skv;
   const int cus = a.cus;
   int tiles[kSplitMaxBlocks];
   int64_t total = 0;
@@ -49,31 +87,16 @@ SplitPlan make_plan(const SplitShape& a) {
   const int most = tiles[nMB - 1], part_waves = std::min(4, (rows + 31) / 32);
   const double size = a.D == 128 ? 1.0 : 0.6, alone = (a.cap ? 1.9 : 0.9) * size, shared_cu = (a.cap ? 3.5 : 2.2) * size;
   const double kv_us = pairs * (double)a.Skv * a.D * 4 / kKvBytes;
+  auto launch_us = [&](double work) { return kLaunch + std::max(work, kv_us) + 0.25 * std::min(work, kv_us); };
   // second: tiles of the workgroup that shares a CU with the longest one, where all of them are resident at once
+  auto resident_us = [&](int64_t wgs, int longest, int second) {
+    return wgs <= cus ? longest * alone : second * shared_cu + (longest - second) * alone;
+  };
   // more than that: handed out in order (longest first) to the slots of an XCD as they become free
-  auto rounds_us = [&](const int* len, int items) {
-    const int slots = std::max(1, 2 * cus / 8);
-    const int64_t per_xcd = (pairs + 7) / 8;
-    std::vector<double> free_at(slots, 0.0);  // a heap whose front is the earliest
-    double end = 0;
-    for (int i = 0; i < items; ++i)
-      for (int64_t j = 0; j < per_xcd; ++j) {
-        std::pop_heap(free_at.begin(), free_at.end(), std::greater<double>());
-        free_at.back() += len[i] * shared_cu + kNext;
-        end = std::max(end, free_at.back());
-        std::push_heap(free_at.begin(), free_at.end(), std::greater<double>());
-      }
-    return end;
-  };
-  auto kernel_us = [&](int64_t wgs, const int* len, int items, int longest, int second, double sum) {
-    const double work = wgs <= cus       ? longest * alone
-                        : wgs <= 2 * cus ? second * shared_cu + (longest - second) * alone
-                        : len            ? rounds_us(len, items)
-                                         : std::max(longest * alone, sum * shared_cu / (2.0 * cus) + 0.25 * longest * alone);
-    return kLaunch + std::max(work, kv_us) + 0.25 * std::min(work, kv_us);
-  };
+  const int slots = std::max(1, 2 * cus / 8);
+  const int64_t per_xcd = (pairs + 7) / 8;
   // few rows: the column sums come from kept logits (2 bytes a pair each way against K once more and another launch)
-  const bool keep = a.stats && rows <= kSplitStatRows;
+  const bool keep = a.stats;
   double best = 1e30;
   int best_chunk = 0;
   if (!keep) {  // the unsplit form: a workgroup per 128 queries of a head
@@ -82,22 +105,37 @@ SplitPlan make_plan(const SplitShape& a) {
     for (int i = 0; i < nq; ++i) sum += (std::min(a.Skv, std::min(i * 128 + 128, a.Sq) + off) + 63) / 64;
     const int64_t wgs = (int64_t)a.B * a.H * nq;
     // heavy and light blocks share a CU: the average makes up the longest block's company
-    best = kernel_us(wgs, nullptr, 0, most, (int)std::max<int64_t>(0, std::min<int64_t>(most, 2 * sum / nq - most)), (double)sum * a.B * a.H);
+    best = launch_us(wgs <= 2 * cus ? resident_us(wgs, most, (int)std::max<int64_t>(0, std::min<int64_t>(most, 2 * sum / nq - most)))
+                                    : std::max(most * alone, (double)sum * a.B * a.H * shared_cu / (2.0 * cus) + 0.25 * most * alone));
   }
   for (int parts = 1; parts <= kSplitMaxItems; ++parts) {
     const int chunk = a.forced > 0 ? a.forced : (most + parts - 1) / parts;
-    if (chunk < 1 || (parts > 1 && chunk == (most + parts - 2) / (parts - 1) && !a.forced)) continue;
-    int items = 0, shared = 0, len[kSplitMaxItems];
-    for (int mb = 0; mb < nMB && items <= kSplitMaxItems; ++mb) {
-      const int nch = (tiles[mb] + chunk - 1) / chunk;
-      for (int c = 0; c < nch && items + c < kSplitMaxItems; ++c) len[items + c] = (tiles[mb] + nch - 1) / nch;
+    if (parts > 1 && chunk == (most + parts - 2) / (parts - 1) && !a.forced) continue;
+    int items = 0, shared = 0, nruns = 0;
+    ShareRun runs[kSplitMaxBlocks];  // longest first
+    for (int mb = nMB - 1; mb >= 0 && items <= kSplitMaxItems; --mb) {
+      const int nch = (tiles[mb] + chunk - 1) / chunk, len = (tiles[mb] + nch - 1) / nch;
       items += nch;
       shared += nch > 1 ? nch : 0;
+      int at = nruns;
+      while (at > 0 && runs[at - 1].len < len) --at;
+      if (at > 0 && runs[at - 1].len == len) {
+        runs[at - 1].count += nch;
+      } else {
+        for (int j = nruns++; j > at; --j) runs[j] = runs[j - 1];
+        runs[at] = {len, nch};
+      }
     }
     if (items > kSplitMaxItems) break;
-    std::sort(len, len + items, std::greater<int>());
-    double us = kernel_us(items * pairs, len, items, len[0], len[std::min<int64_t>(items - 1, cus / pairs)], (double)total * pairs);
-    if (shared) us += kCombine + (double)shared * pairs * std::min(rows, 128) * a.D * 4 * (1 / kPartWrite + 1 / kPartRead);
+    const int64_t wgs = items * pairs;
+    const double fold = shared ? kCombine + (double)shared * pairs * std::min(rows, 128) * a.D * 4 * (1 / kPartWrite + 1 / kPartRead) : 0;
+    // The search ends where no further cut can win: smaller shares mean more of them, so the folding, and in a launch of
+    // several rounds the least that the slots' work adds up to, only grow.
+    const double least = wgs > 2 * cus ? (total * shared_cu + items * kNext) * per_xcd / slots : 0;
+    if (a.forced <= 0 && launch_us(least) + fold >= best) break;
+    int second = 0;  // the share at place cus / pairs
+    for (int64_t i = 0, left = std::min<int64_t>(items - 1, cus / pairs); i < nruns && left >= 0; left -= runs[i++].count) second = runs[i].len;
+    const double us = launch_us(wgs <= 2 * cus ? resident_us(wgs, runs[0].len, second) : rounds_us(runs, nruns, per_xcd, slots, shared_cu)) + fold;
     if (a.forced > 0 || us < best) {
       best = us;
       best_chunk = chunk;
@@ -133,17 +171,29 @@ SplitPlan make_plan(const SplitShape& a) {
 
 }  // namespace
 
-// The plan of a shape costs some microseconds and a program calls with few shapes: each thread keeps its last ones.
-// stats: column sums of rounded logits are wanted too
+// stats: column sums of rounded logits are wanted too.  The reference holds until the thread's next call.
+// A plan costs 0.1 to 2.4 us of host time (a whole search by simulated launches: 9 to 280) and is asked for several times per
+// operator call: each thread keeps its last ones.
 const SplitPlan& split_plan(int B, int H, int group, int Sq, int Skv, int D, bool causal, bool cap, bool stats) {
   struct Entry {
     SplitShape shape{};
     SplitPlan plan{};
   };
   constexpr int kEntries = 16;
+  static const SplitPlan whole{};
   static thread_local Entry kept[kEntries];
-  const SplitShape shape{B, H, group, Sq, Skv, D, attn_split_override(), device_cu_count(), causal, cap, stats};
-  Entry& e = kept[(unsigned)(B * 31 + H * 7 + group * 3 + Sq * 5 + Skv + D + cap + 2 * stats) % kEntries];
+  const int forced = attn_split_override(), cus = device_cu_count();
+  const int64_t pairs = (int64_t)B * (H / group), rows = (int64_t)Sq * group;
+  if (forced < 0 || rows > 128 * kSplitMaxBlocks || pairs * ((rows + 127) / 128) > 4 * cus) return whole;
+  if (Skv > INT32_MAX - 64 || (causal && Skv < Sq)) return whole;  // refused by every entry point
+  // A whole prompt (more than half as many queries as keys) keeps its blocks whole: at most a sixth is to be gained there (B1 H8 S2048:
+  // 35 against 29 us), and its results are those of every launch form of the unsplit kernel, bit for bit.
+  if (Skv < 2 * (int64_t)Sq && forced == 0) return whole;
+  // One row block: Skv matters through its tiles only, and a generation loop, whose Skv grows with every step, makes a plan
+  // once in 64 steps.
+  if (rows <= 128) Skv = (Skv + 63) / 64 * 64;
+  const SplitShape shape{B, H, group, Sq, Skv, D, forced, cus, causal, cap, stats && rows <= kSplitStatRows};
+  Entry& e = kept[(unsigned)(B * 31 + H * 7 + group * 3 + Sq * 5 + Skv / 64 + D + cap + 2 * shape.stats) % kEntries];
   if (!(e.shape == shape)) e = Entry{shape, make_plan(shape)};
   return e.plan;
 }
