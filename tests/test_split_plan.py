@@ -26,12 +26,12 @@ def test_new_shapes_are_planned_in_microseconds(op, B, H, Hkv, Sq, Skv, D):
   """A search that simulates a launch for every number of shares takes 10 to 300 us a shape here."""
   f = _lib.load().ft_workspace_bytes_split
   best = float("inf")
-  for rep in range(8):
-    args = [ctypes.byref(_args(B, H, Hkv, Sq, Skv + 64 * (i + 20 * rep), D)) for i in range(20)]
-    t = time.perf_counter()
+  for rep in range(60):  # the quietest of many short spells: other processes may be busy
+    args = [ctypes.byref(_args(B, H, Hkv, Sq, Skv + 64 * (i + 10 * rep), D)) for i in range(10)]
+    t = time.thread_time()
     for a in args:
       f(op, a)
-    best = min(best, (time.perf_counter() - t) / len(args))
+    best = min(best, (time.thread_time() - t) / len(args))
   assert best < 8e-6, f"{best * 1e6:.1f} us a shape"
 
 
