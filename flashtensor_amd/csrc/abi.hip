@@ -256,6 +256,11 @@ const ft::SplitPlan& split_of(const FtAttnArgs* a, int kf, bool stats = false) {
                         stats && !(a->flags & FT_FAST_LOGITS));
 }
 
+// shapes a plan can be asked for (the entry points refuse the others)
+bool splittable(const FtAttnArgs* a) {
+  return a->B >= 1 && a->H >= 1 && a->Sq >= 1 && a->Skv >= 1 && a->Hkv >= 0 && a->Hkv <= a->H && (a->Hkv == 0 || a->H % a->Hkv == 0);
+}
+
 // The attention pass of the modes that have a split form (plain softmax, soft-cap): split where the plan says so and
 // the caller's workspace, of which `used` bytes are taken, has room for the shares' partial results.
 hipError_t run_attn(const FtAttnArgs* a, const ft::AttnKernelParams& p, int kf, void* ws, size_t used, size_t ws_bytes, void* stream) {
@@ -371,12 +376,27 @@ size_t ft_workspace_bytes(int op, const FtAttnArgs* a) {
 size_t ft_workspace_bytes_split(int op, const FtAttnArgs* a) {
   if (!a) return 0;
   const size_t need = ft_workspace_bytes(op, a);
-  if (op != FT_OP_ATTN && op != FT_OP_COLSTATS && op != FT_OP_CORM && op != FT_OP_SNAPKV) return need;
-  if (a->B < 1 || a->H < 1 || a->Sq < 1 || a->Skv < 1 || a->Hkv < 0 || a->Hkv > a->H || (a->Hkv > 0 && a->H % a->Hkv)) return need;
-  size_t split = split_of(a, ft::kKfNone).bytes;
-  if (op == FT_OP_COLSTATS || op == FT_OP_SNAPKV) split = std::max(split, split_of(a, ft::kKfNone, true).bytes);
-  if (op == FT_OP_ATTN) split = std::max(split, split_of(a, ft::kKfSoftcap).bytes);
+  if (!splittable(a)) return need;
+  size_t split = 0;
+  switch (op) {
+    case FT_OP_ATTN:
+      split = std::max(split_of(a, ft::kKfNone).bytes, split_of(a, ft::kKfSoftcap).bytes);
+      break;
+    case FT_OP_COLSTATS:
+      split = split_of(a, ft::kKfNone, true).bytes;
+      break;
+    case FT_OP_SNAPKV:  // windows wider than kSplitMaxPool go without the kept logits
+      split = std::max(split_of(a, ft::kKfNone).bytes, split_of(a, ft::kKfNone, true).bytes);
+      break;
+    case FT_OP_CORM:
+      split = split_of(a, ft::kKfNone).bytes;
+      break;
+  }
   return split ? align256(need) + split : need;
+}
+
+size_t ft_attn_workspace_bytes(const FtAttnArgs* a, float softcap) {
+  return a && splittable(a) ? split_of(a, softcap > 0.f ? ft::kKfSoftcap : ft::kKfNone).bytes : 0;
 }
 
 int ft_attn_fwd(const FtAttnArgs* a, float* lse, void* stream) { return ft_attn_fwd_ws(a, 0.f, lse, nullptr, 0, stream); }

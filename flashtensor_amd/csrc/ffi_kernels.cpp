@@ -101,6 +101,9 @@ void init_ffi_kernels(py::module_&& m) {
 
   m.def("workspace_bytes_split", [](int op, const FtAttnArgs& a) { return ft_workspace_bytes_split(op, &a); });
 
+  m.def("attn_workspace_bytes", [](const FtAttnArgs& a, float softcap) { return ft_attn_workspace_bytes(&a, softcap); }, py::arg("args"),
+        py::arg("softcap") = 0.f);
+
   m.def("attn_fwd_ws", [](const FtAttnArgs& a, float softcap, uintptr_t lse, uintptr_t ws, size_t ws_bytes, uintptr_t stream) {
     py::gil_scoped_release nogil;
     check(ft_attn_fwd_ws(&a, softcap, ptr<float>(lse), ptr<void>(ws), ws_bytes, ptr<void>(stream)));

@@ -171,7 +171,7 @@ PyObject* result(const at::Tensor& a, const Ts&... more) {
 at::Tensor run_attn(const Qkv& x, unsigned flags, float softcap, const at::Tensor& lse) {
   at::Tensor out = x.out();
   const FtAttnArgs a = x.args(out, flags);
-  const size_t bytes = ft_workspace_bytes_split(FT_OP_ATTN, &a);
+  const size_t bytes = ft_attn_workspace_bytes(&a, softcap);
   const at::Tensor ws = workspace(x.q, bytes);
   void* s = stream_of(x.q);
   launch([&] { return ft_attn_fwd_ws(&a, softcap, static_cast<float*>(ptr(lse)), ptr(ws), bytes, s); });

@@ -90,12 +90,16 @@ size_t ft_workspace_bytes(int op, const FtAttnArgs* a);
  * ft_workspace_bytes() they run undivided.  The number of shares depends on the device, so ask with it current. */
 size_t ft_workspace_bytes_split(int op, const FtAttnArgs* a);
 
+/* What ft_attn_fwd_ws takes for this problem and softcap alone.  (FT_OP_ATTN above is room enough for either form: they
+ * divide differently, and one may be left whole where the other takes tens of megabytes.) */
+size_t ft_attn_workspace_bytes(const FtAttnArgs* a, float softcap);
+
 /* Causal (or full) softmax attention: replaces the fused kernel of Attn.forward (cases/kernels/attn.py:18-34).
  * lse: optional [B,H,Sq] fp32 output, log2-domain row normaliser max + log2(sum). */
 int ft_attn_fwd(const FtAttnArgs* a, float* lse, void* stream);
 
 /* ft_attn_fwd (softcap == 0) or ft_attn_softcap_fwd (softcap > 0) with an optional workspace of
- * ft_workspace_bytes_split(FT_OP_ATTN, a) bytes, 16-byte aligned. */
+ * ft_attn_workspace_bytes(a, softcap) bytes, 16-byte aligned. */
 int ft_attn_fwd_ws(const FtAttnArgs* a, float softcap, float* lse, void* workspace, size_t workspace_bytes, void* stream);
 
 /* Attention + per-key column statistics: H2O.forward (cases/kernels/h2o.py:18-38; colsumsq == NULL) and

@@ -75,3 +75,16 @@ def test_column_sums_of_few_rows(gpu, monkeypatch, tiles, Sq, Skv, H, D, dtype):
   for width in (1, 5, 65, 67):
     ref = torch.nn.functional.avg_pool1d(ref_s, width, 1, width // 2)
     assert (ops.snapkv(*dev, kernel_size=width)[1].cpu() - ref).norm() <= tol * ref.norm()
+
+
+def test_undivided_attention_allocates_its_result_only(gpu):
+  """Plain attention over a chunk that only the soft-capped form divides."""
+  q, k, v = (torch.randn(1, s, h, 128, dtype=torch.bfloat16, device=gpu) for s, h in ((777, 32), (3000, 8), (3000, 8)))
+  for op, room in ((ops.attn, 0), (ops.gemma2, 50 << 20)):
+    op(q, k, v)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    out = op(q, k, v)
+    extra = torch.cuda.max_memory_allocated() - before - out.numel() * 2
+    assert room <= extra < room + (20 << 20), extra

@@ -42,3 +42,15 @@ def test_one_plan_for_all_lengths_of_as_many_tiles(op, B, H, Hkv, Sq, D):
   pad = lambda n: -(-n // 256) * 256
   parts = {_bytes(op, B, H, Hkv, Sq, Skv, D) - pad(need(op, ctypes.byref(_args(B, H, Hkv, Sq, Skv, D)))) for Skv in range(64 * 63 + 1, 64 * 64 + 1, 7)}
   assert len(parts) == 1 and parts.pop() > 0
+
+
+def test_each_form_of_attention_asks_for_its_own_workspace():
+  """A chunk that only the soft-capped form divides (61 MB): the plain one needs nothing."""
+  lib = _lib.load()
+  a = _args(1, 32, 8, 777, 3000, 128)
+  plain, capped = (lib.ft_attn_workspace_bytes(ctypes.byref(a), cap) for cap in (0.0, 50.0))
+  assert plain == 0 and capped > 50 << 20 and lib.ft_workspace_bytes_split(_lib.FT_OP_ATTN, ctypes.byref(a)) == capped
+  assert lib.ft_attn_workspace_bytes(ctypes.byref(_args(4, 32, 8, 1, 4097, 128)), 0.0) > 0
+  for bad in (_args(1, 32, 5, 777, 3000, 128), _args(1, 32, 8, 0, 3000, 128), _args(0, 32, 8, 1, 3000, 128)):
+    assert lib.ft_attn_workspace_bytes(ctypes.byref(bad), 0.0) == 0
+  assert lib.ft_attn_workspace_bytes(None, 0.0) == 0
