@@ -77,6 +77,69 @@ def test_column_sums_of_few_rows(gpu, monkeypatch, tiles, Sq, Skv, H, D, dtype):
     assert (ops.snapkv(*dev, kernel_size=width)[1].cpu() - ref).norm() <= tol * ref.norm()
 
 
+def _stored(t, layout):
+  """The same values as views that programs hold: rows of a longer cache, heads of a packed tensor, [B, H, S, D] storage."""
+  B, S, H, D = t.shape
+  if layout == "cache":
+    return torch.cat([t, t.new_full((B, 70, H, D), 9.0)], 1)[:, :S]
+  if layout == "packed":
+    return torch.cat([t.new_full((B, S, 1, D), 9.0), t, t.new_full((B, S, 2, D), 9.0)], 2)[:, :, 1:1 + H]
+  return t.transpose(1, 2).contiguous().transpose(1, 2)
+
+
+def _near(got, ref, tol):
+  got, ref = got.float().cpu(), ref.float()
+  assert (got - ref).norm() <= tol * ref.norm(), ((got - ref).norm() / ref.norm()).item()
+
+
+@pytest.mark.parametrize("form", ["s1", "s3", "t", ""])
+@pytest.mark.parametrize("layout", [("packed", "cache"), ("bhsd", "bhsd"), ("plain", "packed")])
+@pytest.mark.parametrize("B,Sq,Skv,H,Hkv,D,dtype", [
+    (3, 1, 321, 8, 2, 128, torch.float16), (2, 5, 450, 4, 1, 64, torch.bfloat16), (2, 40, 300, 6, 2, 64, torch.float16),
+    (2, 33, 200, 3, 3, 128, torch.float16), (3, 2, 640, 2, 2, 64, torch.bfloat16), (2, 150, 513, 2, 2, 128, torch.float16)])
+def test_shares_over_views_batches_and_groups(gpu, monkeypatch, form, layout, B, Sq, Skv, H, Hkv, D, dtype):
+  monkeypatch.setenv("FT_ATTN_FORM", form)
+  q, k, v = oracle.prepare_inputs(B, Sq, H, D, seed=Skv, dtype=dtype, kv_len=Skv)
+  k, v = k[:, :, :Hkv].contiguous(), v[:, :, :Hkv].contiguous()
+  dq, dk, dv = (t if lay == "plain" else _stored(t, lay) for t, lay in zip((q.to(gpu), k.to(gpu), v.to(gpu)), (layout[0], layout[1], layout[1])))
+  group, tol = H // Hkv, 1e-2 if dtype is torch.bfloat16 else 2e-3
+  kr, vr = (t.repeat_interleave(group, 2) for t in (k, v))  # query head h reads k/v head h // group
+  ref_o, ref_s, ref_sq = oracle.roco_forward(q, kr, vr)
+  ref_s = ref_s.view(B, Hkv, group, Skv).mean(2)
+  out, lse = ops.attn(dq, dk, dv, return_lse=True)
+  _near(out, ref_o, tol)
+  logits = torch.matmul(q.transpose(1, 2).float(), kr.permute(0, 2, 3, 1).float()) / D**0.5
+  logits += torch.full((Sq, Skv), -torch.inf).triu(Skv - Sq + 1)
+  assert (lse.cpu() * 0.6931471805599453 - logits.logsumexp(-1)).abs().max() <= tol * logits.abs().where(logits.isfinite(), 0).max()
+  out2, score = ops.h2o(dq, dk, dv)
+  _near(out2, ref_o, tol)
+  _near(score, ref_s, tol)
+  _near(ops.gemma2(dq, dk, dv, softcap=5.0), oracle.gemma2_forward(q, kr, vr, 5.0), tol)
+  _near(ops.snapkv(dq, dk, dv, kernel_size=7)[1], torch.nn.functional.avg_pool1d(ref_s, 7, 1, 3), tol)
+  # logits kept in fp32: against the fp32 definition
+  probs = logits.softmax(-1)
+  fast_o = torch.matmul(probs.to(dtype).float(), vr.transpose(1, 2).float()).transpose(1, 2)
+  out3, score3 = ops.h2o(dq, dk, dv, fast_logits=True)
+  _near(out3, fast_o, tol)
+  _near(ops.attn(dq, dk, dv, fast_logits=True), fast_o, tol)
+  _near(score3, probs.sum(2).view(B, Hkv, group, Skv).mean(2), tol)
+  if group == 1:
+    out4, s1, s2 = ops.roco(dq, dk, dv)
+    _near(out4, ref_o, tol)
+    _near(s1, ref_s, tol)
+    _near(s2, ref_sq, 2 * tol)
+    out5, keep = ops.corm(dq, dk, dv)
+    _near(out5, ref_o, tol)
+    ratio = oracle.corm_margin(q, k, oracle.corm_mask_rule(Sq, Skv))  # a key is kept from 1 on; nearer than tol either way goes
+    sure = (ratio - 1).abs() > tol
+    assert torch.equal(keep.cpu()[sure], (ratio >= 1)[sure]) and sure.float().mean() > 0.9
+  # no mask: every row sees every key of every share
+  full_o, full_s = zip(*(oracle.attn_h2o2d_forward(*(t[b].reshape(t.shape[1], -1) for t in (q, k, v)), Hkv, H, D, masked=False) for b in range(B)))
+  out6, score6 = ops.h2o(dq, dk, dv, causal=False)
+  _near(out6, torch.stack(full_o).view(B, Sq, H, D), tol)
+  _near(score6, torch.stack(full_s), tol)
+
+
 def test_undivided_attention_allocates_its_result_only(gpu):
   """Plain attention over a chunk that only the soft-capped form divides."""
   q, k, v = (torch.randn(1, s, h, 128, dtype=torch.bfloat16, device=gpu) for s, h in ((777, 32), (3000, 8), (3000, 8)))

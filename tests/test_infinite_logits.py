@@ -65,3 +65,22 @@ def test_keys_below_the_range_under_noise(gpu, D, dtype, tau):
     out, s = ops.keyformer(*dev, er.to(gpu) if seed is None else None, tau=tau, seed=seed or 0)
     _close(out, ref_o, tol, "out")
     _close(s, ref_s, tol, "score")
+
+
+@pytest.mark.parametrize("form", ["", "s1", "s2", "t", "4"])
+@pytest.mark.parametrize("Sq,Skv,D,dtype", [(1, 200, 128, torch.float16), (6, 333, 64, torch.float16), (40, 260, 128, torch.float16), (3, 300, 64, torch.bfloat16)])
+def test_keys_below_the_range_under_groups(gpu, monkeypatch, form, Sq, Skv, D, dtype):
+  """Two batches, four query heads on each of two k/v heads; the two k/v heads lose different keys."""
+  monkeypatch.setenv("FT_ATTN_FORM", form)
+  B, H, Hkv = 2, 8, 2
+  q, k, v = oracle.prepare_inputs(B, Sq, H, D, seed=Skv, dtype=dtype, kv_len=Skv)
+  k, v = k[:, :, :Hkv].contiguous(), v[:, :, :Hkv].contiguous()
+  big = 2e19 if dtype is torch.bfloat16 else 200.0
+  q[..., :4], k[..., :4] = big, 0
+  k[:, :65, 0, :4], k[:, 128:192, 1, :4], k[1, Skv - 1, 1, :4] = -big, -big, -big
+  kr, vr = (t.repeat_interleave(H // Hkv, 2) for t in (k, v))
+  tol = 1e-2 if dtype is torch.bfloat16 else 2e-3
+  ref_o, ref_s = oracle.h2o_forward(q, kr, vr)
+  out, score = ops.h2o(*(t.to(gpu) for t in (q, k, v)))
+  _close(out, ref_o, tol, "out")
+  _close(score, ref_s.view(B, Hkv, H // Hkv, Skv).mean(2), tol, "sums")
