@@ -46,6 +46,9 @@ constexpr int kLinThreads = 256;
 constexpr int kLinWaves = kLinThreads / 64;
 constexpr int kPartStride = kLinD * kLinD + 2 * kLinD;  // floats per (bh, chunk) partial
 constexpr int kNoSwizzle = 2;
+// Where EA's running maxima begin: finite, and so times log2 e, so that tokens whose K is -inf (padding masked that way, or an
+// fp32 value below fp16's range) come to exp2(-inf) = 0 also where nothing else has been seen.
+constexpr float kNoMax = -2.3e38f;
 
 struct LinParams {
   const uint16_t* q;
@@ -232,7 +235,7 @@ __global__ void __launch_bounds__(kLinThreads, (IN32 && NQ) ? 1 : 2) linattn_kv_
   for (int i = 0; i < 4; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[i >> 1][i & 1][r] = 0.f;
-  float m_run[2] = {NEG_INF, NEG_INF};  // EA: running max of K[:, d], d = 32 db + n
+  float m_run[2] = {kNoMax, kNoMax};  // EA: running max of K[:, d], d = 32 db + n
   float l_run[2] = {0.f, 0.f};          // EA: sum of exp; SimA: sum |K|   (this lane's token slots only)
   float qabs[8];
 #pragma unroll
@@ -545,7 +548,7 @@ __global__ void __launch_bounds__(kLinThreads) linattn_merge_kernel(const LinPar
   const int sd = t & (D - 1), cg = t >> 6;
   const float* stat = part + D * D + sd;
   if (EA) {
-    float M = -__builtin_inff();
+    float M = kNoMax;
     for (int c = cg; c < p.nch; c += 4) M = fmaxf(M, stat[c * kPartStride]);
     s_red[t] = M;
     __syncthreads();
@@ -656,7 +659,7 @@ __device__ __forceinline__ void merge_in_lds(const LinParams& p, int bh, uint16_
   constexpr int D = kLinD;
   const int t = threadIdx.x, d = t >> 2, qr = t & 3;
   const float* part = p.part + (int64_t)bh * p.nch * kPartStride;
-  float x[16] = {}, M = -__builtin_inff(), L = 0.f, nq = 0.f;
+  float x[16] = {}, M = kNoMax, L = 0.f, nq = 0.f;
 #pragma unroll 1
   for (int c0 = 0; c0 < p.nch; c0 += kFusedChunks) {
     // eight chunks' loads at once: chunks past the last one re-read it, with weight 0

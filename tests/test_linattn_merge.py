@@ -46,3 +46,20 @@ def test_views(gpu, monkeypatch, form, layout, B, S, H, dtype):
   assert (ops.ea(*dev).float().cpu() - ref).norm() <= tol * ref.norm()
   ref = oracle.sima_forward(q, k, v, out_dtype=torch.float32)
   assert (ops.sima(*dev, out_dtype=torch.float32).cpu() - ref).norm() <= tol * ref.norm()
+
+
+@pytest.mark.parametrize("form", ["fused", "launch"])
+@pytest.mark.parametrize("S,lost", [(40, [(0, 20)]), (700, [(0, 300), (512, 640)]), (4200, [(0, 1500), (2100, 2101), (4000, 4200)])])
+@pytest.mark.parametrize("D,dtype,low", [(64, torch.float16, -torch.inf), (32, torch.float16, -60000.0), (64, torch.bfloat16, -torch.inf),
+                                         (64, torch.float32, -torch.inf), (64, torch.float32, torch.finfo(torch.float32).min)])
+def test_tokens_masked_in_k(gpu, monkeypatch, form, S, lost, D, dtype, low):
+  """Padding masked with -inf or the type's lowest value in K (fp32 beyond fp16's range becomes -inf as it is loaded): whole strips,
+  waves and chunks of it, in one channel only in the second head."""
+  monkeypatch.setenv("FT_LINATTN_MERGE", form)
+  q, k, v = oracle.prepare_inputs(1, S, 2, D, seed=S, dtype=dtype)
+  for a, b in lost:
+    k[:, a:b, 0], k[:, a:b, 1, 3] = low, low
+  tol = 1e-2 if dtype is torch.bfloat16 else 2e-3
+  ref = oracle.ea_forward(q, k, v).float()
+  out = ops.ea(q.to(gpu), k.to(gpu), v.to(gpu)).float().cpu()
+  assert ref.isfinite().all() and (out - ref).norm() <= tol * ref.norm()
