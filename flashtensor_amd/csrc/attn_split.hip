@@ -26,8 +26,8 @@ struct SplitShape {
 // and the launch, then 0.9 per tile where it has its CU to itself and 2.2 where two share one: the second wave of a
 // SIMD hides little of the first one's work (soft-capped logits: 1.9 and 3.5; there it does).  Partial results are
 // written at 10 MB/us and folded at 7, by a kernel that takes 5.5 us to begin with, its launch included; K and V come from HBM at 5.
-// In a launch of more workgroups than fit at once each further one in a slot takes 1 us until its first tile has landed (left
-// out of account, B5 H32 Sq3 Skv3329 soft-capped bf16 became 8480 workgroups of one tile: 126 us against 100 unsplit).
+// In a launch of more workgroups than fit at once each further one in a slot takes 1 us until its first tile has landed (set
+// from four generation shapes; left out of account, B5 H32 Sq3 Skv3329 soft-capped bf16 became 8480 workgroups of one tile: 126 us against 100 unsplit).
 constexpr double kLaunch = 7.0, kCombine = 5.5, kNext = 1.0, kPartWrite = 10e6, kPartRead = 7e6, kKvBytes = 5e6;
 
 // `count` shares of `len` tiles.
@@ -281,7 +281,7 @@ __global__ void __launch_bounds__(256) attn_combine_kernel(const AttnKernelParam
 
 // The column sums of few rows from their kept logits, and (the last `gridDim.x - ncol` workgroups) the folding of the
 // shares: one launch where the column pass would read K a second time, per query head, behind the launch that folds.
-// B4 H32/8 Sq1 Skv4097: 31 + 5 us (column pass, group mean) -> under 2 on top of the folding's 4.
+// B4 H32/8 Sq1 Skv4097: 31 + 5 us (column pass, group mean) and 4 for the folding -> 4.1 for all of it.
 // A workgroup takes 512 keys of one (b, k/v head), eight of them per lane; its waves share out the rows and meet in LDS.
 // A wave requests all of its rows (1 KB each) before the row normalisers are folded.
 constexpr int kStatTiles = 8;

@@ -2,8 +2,8 @@
 // plan that says when.  Instantiated by attn_split_{f16,bf16}.hip; attn_split.hip holds the plan, the dispatcher and the
 // kernel that folds the shares.
 //
-// What bounds the unsplit form there: a row block is one workgroup that walks all of its tiles (1.1-1.3 us each), however
-// few blocks there are.  B4 Sq1 Skv4097 with 32 query heads on 8 k/v heads: 128 workgroups of which one wave of four has
+// What bounds the unsplit form there: a row block is one workgroup that walks all of its tiles (0.9 us each where it has a CU to
+// itself, D = 128), however few blocks there are.  B4 Sq1 Skv4097 with 32 query heads on 8 k/v heads: 128 workgroups of which one wave of four has
 // one row, 65 tiles each, K and V staged four times over: 69 us for 67 MB.
 #pragma once
 #include "attn_fwd_kernel.hpp"
