@@ -16,7 +16,8 @@ OBJ_DIR = os.path.join(CSRC, "build")
 LIB_PATH = os.path.join(HERE, "libflashtensor_hip.so")
 DIAG_LIB_PATH = os.path.join(HERE, "libflashtensor_diag.so")  # include/ft_diag.h: probes for the benchmark, not product
 SOURCES = ["abi.hip", "attn_fwd.hip", "attn_fwd_f16_d128.hip", "attn_fwd_f16_d64.hip", "attn_fwd_bf16_d128.hip", "attn_fwd_bf16_d64.hip",
-           "attn_split.hip", "attn_split_f16.hip", "attn_split_bf16.hip", "colstats.hip", "colstats_narrow.hip", "colstats_teams.hip", "linattn.hip", "aux.hip", "linblock.hip", "linblock_small.hip"]
+           "attn_split.hip", "attn_split_f16.hip", "attn_split_bf16.hip", "attn_teams_kf_f16.hip", "attn_teams_kf_bf16.hip",
+           "colstats.hip", "colstats_narrow.hip", "colstats_teams.hip", "linattn.hip", "aux.hip", "linblock.hip", "linblock_small.hip"]
 DIAG_SOURCES = ["diag.hip"]
 FFI_SOURCE = "ffi_kernels.cpp"  # pybind11 module ft_ffi over the C ABI (plain C++: no device code, no torch headers)
 OPS_SOURCE = "ops_torch.cpp"    # module ft_ops: the operators on torch tensors (plain C++ over torch's headers and the C ABI)
@@ -31,7 +32,7 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Xclang", "-tar
 # The attention kernels take row maxima of MFMA results with plain fmaxf chains: without NaN honouring they become
 # v_max3_f32 with no quieting moves, and stay visible to the compiler's hazard handling (no kernel relies on NaNs)
 EXTRA_FLAGS = {src: ["-fno-honor-nans"] for src in ("attn_fwd_f16_d128.hip", "attn_fwd_f16_d64.hip", "attn_fwd_bf16_d128.hip", "attn_fwd_bf16_d64.hip",
-                                                    "attn_split.hip", "attn_split_f16.hip", "attn_split_bf16.hip")}
+                                                    "attn_split.hip", "attn_split_f16.hip", "attn_split_bf16.hip", "attn_teams_kf_f16.hip", "attn_teams_kf_bf16.hip")}
 
 
 def _hipcc():

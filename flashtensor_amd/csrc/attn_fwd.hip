@@ -53,6 +53,8 @@ hipError_t launch_attn_bf16_d128(const AttnKernelParams& p, bool causal, bool em
 
 hipError_t launch_attn_teams_f16(const AttnKernelParams& p, int D, bool emu, int kf, unsigned grid, hipStream_t s);
 hipError_t launch_attn_teams_bf16(const AttnKernelParams& p, int D, bool emu, int kf, unsigned grid, hipStream_t s);
+hipError_t launch_attn_teams_kf_f16(const AttnKernelParams& p, int D, int kf, unsigned grid, hipStream_t s);
+hipError_t launch_attn_teams_kf_bf16(const AttnKernelParams& p, int D, int kf, unsigned grid, hipStream_t s);
 
 // Two teams of waves on blocks of 64 rows (attn_split.hpp) instead of four waves on 128: half the rows and half the chain of
 // key tiles per workgroup.  Taken where the chain is the launch: with a workgroup of this form for every CU at most, from
@@ -74,6 +76,21 @@ static bool use_teams(const AttnKernelParams& p, int D, bool causal, bool cap, i
   return causal && (D == 64 ? cap || tiles <= 32 : cap && tiles > 11);
 }
 
+// KeyFormer's passes do two to four times the vector work per tile, so the chain of a block's tiles bounds launches of more
+// workgroups still, and half the chain pays from two key tiles on (whole calls, same process, four waves on 128 rows against the
+// teams).  Noise from a tensor, D128: B1 H8 S100 16.9 -> 15.5 us (S64 12.5 -> 14.0), S2091 165 -> 118, H16 S3543 328 -> 297, and at
+// more than 3.5 workgroups for every CU slower, H32 S2091 214 -> 224; D64 H16 S2527 169 -> 146, H32 S1501 107 -> 107, S2091 166 -> 182.
+// From a seed, D128: H8 S391 28.5 -> 25.0, S1003 51.8 -> 40.5, H16 S2091 109 -> 96, S2527 (2.5 for every CU) 146 -> 146 or, bf16,
+// 176 -> 168, H32 S1501 92 -> 105; D64 H16 S3543 142 -> 127, H32 S2091 100 -> 95, S2527 128 -> 129.
+static bool use_kf_teams(const AttnKernelParams& p, int D, int kf, int64_t grid) {
+  const int forced = attn_form_override();
+  if (forced) return (forced & 16) != 0;
+  const int64_t cus = device_cu_count();
+  if (p.Skv <= 64) return false;
+  if (kf == kKfTensor || kf == kKfTensorLds) return grid <= (D == 128 ? 7 * cus / 2 : 3 * cus);
+  return grid <= (D == 128 ? 5 * cus / 2 : 9 * cus / 2);
+}
+
 hipError_t launch_attn_fwd(const AttnKernelParams& p, int D, bool bf16, bool causal, bool emu, int kf, hipStream_t s) {
   const int64_t rows = (int64_t)p.Sq * p.group, grid = (rows + 63) / 64 * p.B * (p.H / p.group);
   if ((kf == kKfNone || kf == kKfSoftcap) && rows < 0x7fffffff - 64 && grid < 0x7fffffff && use_teams(p, D, causal, kf == kKfSoftcap, grid)) {
@@ -82,6 +99,12 @@ hipError_t launch_attn_fwd(const AttnKernelParams& p, int D, bool bf16, bool cau
     // (D = 64: two workgroups per CU; see the kernel)
     pp.pair_order = causal && D == 64 && grid > device_cu_count() && grid <= 2 * device_cu_count();
     return bf16 ? launch_attn_teams_bf16(pp, D, emu, kf, (unsigned)grid, s) : launch_attn_teams_f16(pp, D, emu, kf, (unsigned)grid, s);
+  }
+  if (emu && (kf == kKfTensor || kf == kKfTensorLds || kf == kKfSeeded || kf == kKfSeededTau1 || kf == kKfSeededFast) && grid < 0x7fffffff && use_kf_teams(p, D, kf, grid)) {
+    AttnKernelParams pp = p;
+    if (!causal) pp.off = p.Skv;
+    pp.pair_order = pp.two_blocks = pp.head_major = 0;
+    return bf16 ? launch_attn_teams_kf_bf16(pp, D, kf, (unsigned)grid, s) : launch_attn_teams_kf_f16(pp, D, kf, (unsigned)grid, s);
   }
   if (D == 128) return bf16 ? launch_attn_bf16_d128(p, causal, emu, kf, s) : launch_attn_f16_d128(p, causal, emu, kf, s);
   if (D == 64) return bf16 ? launch_attn_bf16_d64(p, causal, emu, kf, s) : launch_attn_f16_d64(p, causal, emu, kf, s);

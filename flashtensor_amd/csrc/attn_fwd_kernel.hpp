@@ -57,9 +57,11 @@ __device__ __forceinline__ SplitPartial split_partial(float* base, int D, int64_
 // TEAMS = 2 (SPLIT): the two shares of a block of 64 rows are taken by two pairs of waves of one workgroup, each with LDS
 // buffers of its own, and fold in LDS: each wave has its SIMD to itself, as in a launch of fewer 128-row blocks than CUs, which
 // is bound by the chain of its longest block (0.9 us a tile at D128, whatever the other CUs do), and the chain is half as
-// long.  B1 H8 S2048 D128 36 -> 29 us, soft-capped 58 -> 39; D64 25 -> 20 (when it is taken: attn_fwd.hip).
+// long.  B1 H8 S2048 D128 36 -> 29 us, soft-capped 58 -> 39; D64 25 -> 20 (when it is taken: attn_fwd.hip).  The KeyFormer modes
+// have it too (B1 H16 S697, whole call, noise from a tensor 63 -> 50 us, from a seed 40 -> 33): their running sums of the perturbed
+// softmax fold beside the plain ones.
 template <typename T, int D, bool CAUSAL, bool EMU, int KF, int WAVES, bool SPLIT = false, bool STORE = false, int TEAMS = 1>
-__global__ void __launch_bounds__(64 * WAVES * TEAMS, (KF == kKfTensorLds ? 1 : 8 / (WAVES * TEAMS))) attn_fwd_kernel(const AttnKernelParams p) {
+__global__ void __launch_bounds__(64 * WAVES * TEAMS, ((KF == kKfTensor || KF == kKfTensorLds) && D == 128 ? 1 : 8 / (WAVES * TEAMS))) attn_fwd_kernel(const AttnKernelParams p) {
   constexpr int BM = 32 * WAVES, BN = kAttnBN, NT = 64 * WAVES;
   constexpr int KSTEPS = D / 16;
   constexpr int DB = D / 32;
@@ -73,8 +75,7 @@ __global__ void __launch_bounds__(64 * WAVES * TEAMS, (KF == kKfTensorLds ? 1 : 
   // logits, and the packed seeded KeyFormer modes (fp16)
   constexpr bool kFastMasked = (kIsF16 && EMU && kKfFast) || KF == kKfNone || KF == kKfSoftcap;
   constexpr bool kCap = KF == kKfSoftcap;
-  constexpr bool kErLds = KF == kKfTensorLds;               // noise tensor staged through LDS
-  constexpr bool kTensor = KF == kKfTensor || kErLds;
+  constexpr bool kTensor = KF == kKfTensor || KF == kKfTensorLds;  // noise tensor staged through LDS
   static_assert(!kKfFast || (kIsF16 && EMU), "the packed KeyFormer modes exist for fp16 with reference rounding only");
   // Software pipeline across tiles: the QK^T MFMAs of tile it+1 are issued in the same iteration as the
   // softmax (VALU) and PV MFMAs of tile it, so the matrix and vector pipes overlap inside one wave.
@@ -90,14 +91,16 @@ __global__ void __launch_bounds__(64 * WAVES * TEAMS, (KF == kKfTensorLds ? 1 : 
   char* const ldsK1 = s_k1 + team * TILE_BYTES;
   char* const ldsV0 = s_v0 + team * TILE_BYTES;
   char* const ldsV1 = s_v1 + team * TILE_BYTES;
-  __shared__ __align__(16) uint32_t ldsCol[2 * BN];  // noise column terms of the current / next tile
+  __shared__ __align__(16) uint32_t s_col[TEAMS * 2 * BN];
+  uint32_t* const ldsCol = s_col + team * 2 * BN;  // noise column terms of the current / next tile
+  const int tid = TEAMS > 1 ? threadIdx.x % NT : threadIdx.x;
   // kKfTensorLds: every wave's slice of the next noise tile (32 rows x 64 keys fp32), one 16-byte slot per lane and
   // load instruction: a lane reads back exactly the slots it filled
   constexpr int kErWaveBytes = 32 * BN * 4;
-  __shared__ __align__(16) char ldsEr[kErLds ? WAVES * kErWaveBytes : 16];
+  __shared__ __align__(16) char ldsEr[kTensor ? TEAMS * WAVES * kErWaveBytes : 16];
 
   static_assert(TEAMS == 1 || (SPLIT && !STORE && WAVES == 2 && TEAMS == 2), "the teams' instantiations");
-  static_assert(!SPLIT || (CAUSAL && WAVES * TEAMS == 4 && (KF == kKfNone || KF == kKfSoftcap)), "the split form's instantiations");
+  static_assert(!SPLIT || (CAUSAL && WAVES * TEAMS == 4 && (TEAMS > 1 || KF == kKfNone || KF == kKfSoftcap)), "the split form's instantiations");
   static_assert(!STORE || (SPLIT && EMU && KF == kKfNone), "logits are kept where they are 16-bit values");
   const int rows = SPLIT ? p.Sq * p.group : p.Sq;  // rows of a (b, h) pair; SPLIT: of a (b, k/v head) pair
   const int BH = SPLIT ? p.B * (p.H / p.group) : p.B * p.H;
@@ -174,7 +177,8 @@ __global__ void __launch_bounds__(64 * WAVES * TEAMS, (KF == kKfTensorLds ? 1 : 
     if (qrow < rows) *reinterpret_cast<uint4v*>(logit_row + 16 * b16) = uint4v{s0[0], s1[0], s0[1], s1[1]};
 #endif
   };
-  int Skv = p.Skv, off = p.off;  // SPLIT: counted from the first key of the workgroup's share
+  int Skv = p.Skv, off = p.off;  // SPLIT: counted from the first key of the workgroup's share,
+  int tile0 = 0;                 // which is that of this tile of the row
   int n_end = Skv;
   if (CAUSAL) n_end = min(Skv, (SPLIT ? (min(m0 + BM, rows) - 1) / p.group + 1 : m0 + BM) + off);
   int ntiles = (n_end + BN - 1) / BN;
@@ -184,6 +188,7 @@ __global__ void __launch_bounds__(64 * WAVES * TEAMS, (KF == kKfTensorLds ? 1 : 
     nch = TEAMS > 1 ? TEAMS : (ntiles + p.chunk_tiles - 1) / p.chunk_tiles;
     const int per = (ntiles + nch - 1) / nch, t0 = chunk * per, t1 = min(t0 + per, ntiles);
     ntrips = per;
+    tile0 = t0;
     kbase += (int64_t)t0 * BN * p.sk.s;
     vbase += (int64_t)t0 * BN * p.sv.s;
     off -= t0 * BN;
@@ -208,36 +213,60 @@ __global__ void __launch_bounds__(64 * WAVES * TEAMS, (KF == kKfTensorLds ? 1 : 
 
   NoiseKeys nk = {0, 0};
   uint32_t a_i = 0;
-  const float* er_row = nullptr;
   if (kSeeded) {
     nk = noise_keys(p.seed, (uint32_t)bh);
     a_i = noise_row(nk, (uint32_t)qi);
   }
-  if (KF == kKfTensor) er_row = p.exp_rand + b * p.er_sb + h * p.er_sh + (int64_t)qi_c * p.er_sr;
-  // kKfTensorLds: the wave's slice of a noise tile is 32 rows x 256 bytes.  Load r8 of a tile brings rows
+  // Noise from a tensor: the wave's slice of a tile is 32 rows x 256 bytes.  kKfTensorLds: load r8 of a tile brings rows
   // 4 r8 + [0..3] whole (a load instruction then touches 8 cache lines; with a lane fetching its own row's chunks
   // it touched 32, and the address path, not HBM, bounded the pass): lane l fills slot l % 16 of row 4 r8 + l / 16
   // with global chunk (l % 16) ^ (row % 16), the XOR placement that lets 32 rows be read back one chunk column at
   // a time without bank conflicts.  Chunks past the end of a row re-read its last chunk (those keys are masked),
   // rows past Sq the last row.
-  rsrc_t er_rsrc = make_rsrc(kErLds ? p.exp_rand + b * p.er_sb + h * p.er_sh : nullptr);
-  char* er_lds = ldsEr + (kErLds ? wave * kErWaveBytes : 0);
+  // kKfTensor, for rows that do not begin at multiples of 16 bytes or do not hold whole chunks (and slices of 2 GiB and
+  // more): one row and 4 bytes a lane per load, into the same slots.  Four times the loads, but 16-byte ones at odd addresses
+  // take the address path as long as four and do not coalesce (B1 H32 S3543 D128, whole call, noise read into registers
+  // 618 us, by 16 bytes 615, by 4 bytes 480; rows of 3544 450).  Keys past the end of a row re-read its last one.
+  // (kKfTensor: from the wave's first row on, so that 32-bit offsets reach its rows unless they are 128 MiB apart)
+  constexpr int64_t kNearRow = 1 << 25;
+  const int er_row0 = KF == kKfTensor ? min(wave_row0, p.Sq - 1) : 0, er_rows = p.Sq - er_row0;
+  const float* er_slice = kTensor ? p.exp_rand + b * p.er_sb + h * p.er_sh + er_row0 * p.er_sr : nullptr;
+  rsrc_t er_rsrc = make_rsrc(er_slice);
+  char* er_lds = ldsEr + (kTensor ? (team * WAVES + wave) * kErWaveBytes : 0);
   // per-lane state of those loads: two registers (the offsets of the eight loads are rebuilt from them for every
   // tile: kept in registers across the loop they would cost eight, and this path has none to spare)
   const int er_cs = (lane & 15) ^ (lane >> 4);  // slot ^ (row % 4); the row's bits 2..3 are those of r8
   const uint32_t er_row_bytes = (uint32_t)p.er_sr * 4u;
-  const uint32_t er_off0 = kErLds ? (uint32_t)(m0 + wave * 32 + (lane >> 4)) * er_row_bytes : 0u;
-  const uint32_t er_off_last = kErLds ? (uint32_t)(p.Sq - 1) * er_row_bytes : 0u;
+  const uint32_t er_off0 = kTensor ? (uint32_t)(m0 + wave * 32 + (lane >> 4)) * er_row_bytes : 0u;
+  const uint32_t er_off_last = kTensor ? (uint32_t)(p.Sq - 1) * er_row_bytes : 0u;
   auto issue_er = [&](int t) __attribute__((always_inline)) {
-    const int last_chunk = p.Skv / 4 - 1;
-    int cs = er_cs;
-    uint32_t off0 = er_off0;
-    asm volatile("" : "+v"(cs), "+v"(off0));  // not loop-invariant as far as the compiler can tell
+    if constexpr (KF == kKfTensorLds) {
+      const int last_chunk = p.Skv / 4 - 1;
+      int cs = er_cs;
+      uint32_t off0 = er_off0;
+      asm volatile("" : "+v"(cs), "+v"(off0));  // not loop-invariant as far as the compiler can tell
 #pragma unroll
-    for (int r8 = 0; r8 < 8; ++r8) {
-      const int c = min(t * (BN / 4) + (cs ^ (4 * (r8 & 3))), last_chunk);
-      const uint32_t row_off = min(off0 + (uint32_t)(4 * r8) * er_row_bytes, er_off_last);
-      load_lds16(er_rsrc, er_lds + r8 * 1024, row_off + (uint32_t)c * 16u, 0);
+      for (int r8 = 0; r8 < 8; ++r8) {
+        const int c = min((tile0 + t) * (BN / 4) + (cs ^ (4 * (r8 & 3))), last_chunk);
+        const uint32_t row_off = min(off0 + (uint32_t)(4 * r8) * er_row_bytes, er_off_last);
+        load_lds16(er_rsrc, er_lds + r8 * 1024, row_off + (uint32_t)c * 16u, 0);
+      }
+    } else {
+      const uint32_t last = (uint32_t)(p.Skv - 1) * 4u, tile_byte = (uint32_t)(tile0 + t) * (BN * 4u);
+      uint32_t d0 = (uint32_t)lane * 4u;
+      asm volatile("" : "+v"(d0));
+      // (row offsets are wave-uniform)
+      if (p.er_sr < kNearRow) {
+#pragma unroll
+        for (int r = 0; r < 32; ++r)
+          load_lds4(er_rsrc, er_lds + r * 256, min((d0 ^ (uint32_t)((r & 15) << 4)) + tile_byte, last), (uint32_t)min(r, er_rows - 1) * er_row_bytes);
+      } else {
+#pragma unroll 1
+        for (int r = 0; r < 32; ++r) {
+          const rsrc_t row = make_rsrc(er_slice + (int64_t)min(r, er_rows - 1) * p.er_sr);
+          load_lds4(row, er_lds + r * 256, min((d0 ^ (uint32_t)((r & 15) << 4)) + tile_byte, last), 0);
+        }
+      }
     }
   };
   // the lane's query row n, chunks 2 k8 + g (keys 8 k8 + 4 g + [0..3] of the tile: score registers 4 (k8 % 4) + [0..3]
@@ -265,8 +294,7 @@ __global__ void __launch_bounds__(64 * WAVES * TEAMS, (KF == kKfTensorLds ? 1 : 
   };
   auto stage_v = [&](int t, char* dst) __attribute__((always_inline)) {
     if (t < ntiles) stV.issue(t * BN, min(BN, Skv - t * BN), dst);
-    if (kSeeded && t < ntiles && threadIdx.x < BN)
-      ldsCol[(t & 1) * BN + threadIdx.x] = noise_col(nk, (uint32_t)(t * BN + threadIdx.x));
+    if (kSeeded && t < ntiles && tid < BN) ldsCol[(t & 1) * BN + tid] = noise_col(nk, (uint32_t)((tile0 + t) * BN + tid));
   };
 
   float16v o_acc[DB];
@@ -533,7 +561,7 @@ __global__ void __launch_bounds__(64 * WAVES * TEAMS, (KF == kKfTensorLds ? 1 : 
     }
     if (MASKED) {
       // local key index of register r is 8 (r / 4) + 4 g + r % 4; it is visible iff <= lim + 4 g
-      const int lim = (CAUSAL ? min(qi + p.off, p.Skv - 1) : p.Skv - 1) - n0h - 4 * g;
+      const int lim = (CAUSAL ? min(qi + off, Skv - 1) : Skv - 1) - n0h - 4 * g;
 #pragma unroll
       for (int r = 0; r < 16; ++r) x[r] = (8 * (r >> 2) + (r & 3) > lim) ? NEG_INF : x[r];
     }
@@ -634,8 +662,8 @@ __global__ void __launch_bounds__(64 * WAVES * TEAMS, (KF == kKfTensorLds ? 1 : 
       stV.issue_full((it + 1) * BN, v_dst);
     }
     qk(s_next, tk_next);
-    if (kKfFast && STAGE && threadIdx.x < BN)  // column terms of tile it + 1 (the other half of ldsCol)
-      ldsCol[((it + 1) & 1) * BN + threadIdx.x] = noise_col(nk, (uint32_t)((it + 1) * BN + threadIdx.x));
+    if (kKfFast && STAGE && tid < BN)  // column terms of tile it + 1 (the other half of ldsCol)
+      ldsCol[((it + 1) & 1) * BN + tid] = noise_col(nk, (uint32_t)((tile0 + it + 1) * BN + tid));
     fast_exp(masked_tag, s_cur, pb, n0, it);
     pv(pb, tv);
     pend_max = tile_max(next_masked_tag, s_next, n0 + BN);
@@ -737,27 +765,9 @@ __global__ void __launch_bounds__(64 * WAVES * TEAMS, (KF == kKfTensorLds ? 1 : 
   // Two tiles per trip, so that every LDS buffer is named at compile time: with a buffer chosen at run time
   // the compiler cannot tell the tile being read from the tile being loaded, and drains every load in flight
   // before the first LDS read of the tile.
-  // KeyFormer, tensor mode: er[mbk] is this lane's slice of the noise tile (its query row, the 16 keys of its
-  // score registers in half mbk).  The S x S tensor is the one operand that comes from HBM every time, so the
-  // slice of the next tile is requested as soon as the softmax has consumed this tile's (same registers) and is
-  // in flight for the rest of the tile: a load consumed in the iteration that issues it leaves the memory
-  // system idle while the tile is worked on.  (Ordinary loads: the four 16-byte pieces a lane pair takes from
-  // one 128-byte line arrive in four instructions, and with the non-temporal hint each went to HBM.)
+  // Noise from a tensor: er[mbk] is this lane's slice of the noise tile (its query row, the 16 keys of its score registers
+  // in half mbk), read from LDS at the top of the tile.  The S x S tensor is the one operand that comes from HBM every time.
   float er[2][16];
-  auto load_er_half = [&](float (&dst)[16], int it, int mbk) __attribute__((always_inline)) {
-    const int c0 = it * BN + 32 * mbk;
-    if (p.er_vec4 && c0 + 32 <= p.Skv) {  // the whole half lies inside the tensor: four 16-byte loads
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        const float4v e4 = *reinterpret_cast<const float4v*>(er_row + c0 + 8 * q4 + 4 * g);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) dst[4 * q4 + e] = e4[e];
-      }
-    } else {  // keys past the end read the last one instead (no branches); they are masked
-#pragma unroll
-      for (int r = 0; r < 16; ++r) dst[r] = er_row[min(c0 + 8 * (r >> 2) + 4 * g + (r & 3), p.Skv - 1)];
-    }
-  };
   auto qk_half = [&](float16v& s, const char* tk, int mbk) __attribute__((always_inline)) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) s[r] = 0.f;
@@ -775,7 +785,7 @@ __global__ void __launch_bounds__(64 * WAVES * TEAMS, (KF == kKfTensorLds ? 1 : 
     constexpr bool odd = decltype(odd_tag)::value;
     wait_vmem();
     __syncthreads();
-    if (kErLds && it < nw) {
+    if (kTensor && it < nw) {
       // this tile's slice from LDS to registers; the next tile's is requested into the same slots further down.  The
       // reads must have returned before those loads may overwrite their slots (nothing in the hardware orders an LDS
       // read against a later direct-to-LDS load).
@@ -794,39 +804,36 @@ __global__ void __launch_bounds__(64 * WAVES * TEAMS, (KF == kKfTensorLds ? 1 : 
           softmax_half(std::false_type{}, s, pb, it * BN + 32 * mbk, odd ? 1 : 0, mbk, er[mbk]);
         else
           softmax_half(std::true_type{}, s, pb, it * BN + 32 * mbk, odd ? 1 : 0, mbk, er[mbk]);
-        if (KF == kKfTensor && it + 1 < nw) load_er_half(er[mbk], it + 1, mbk);
         // The next tile's noise, in flight for the rest of the tile without holding a register.  Requested here, behind
         // the first half's contraction and softmax, rather than at the top of the tile in front of the K / V staging
         // loads: the eight loads no longer queue up with the staging at the moment every wave leaves the barrier
         // (B1 H32 S4096, same process: 538 -> 512 us per call; before the softmax 523, after the first half's PV 516,
         // four loads behind each half's softmax 524).
-        if (kErLds && mbk == 0 && it + 1 < nw) issue_er(it + 1);
+        if (kTensor && mbk == 0 && it + 1 < nw) issue_er(it + 1);
         pv_half(pb, odd ? ldsV1 : ldsV0, mbk);
       }
     }
   };
-  if (KF == kKfTensor) {
-    load_er_half(er[0], 0, 0);
-    load_er_half(er[1], 0, 1);
-  }
-  if (kErLds && nw > 0) issue_er(0);
+  if (kTensor && nw > 0) issue_er(0);
   stage_k(0, ldsK0);
   stage_v(0, ldsV0);
   int it = 0;
-  for (; it + 1 < ntiles; it += 2) {
+  const int trips = TEAMS > 1 ? ntrips : ntiles;
+  for (; it + 1 < trips; it += 2) {
     slow_tile(it, std::false_type{});
     slow_tile(it + 1, std::true_type{});
   }
-  if (it < ntiles) slow_tile(it, std::false_type{});
+  if (it < trips) slow_tile(it, std::false_type{});
   }
 
   // ---- epilogue
   l_run += xchg32(l_run);
+  if (kTensor || kSeeded) l_kf += xchg32(l_kf);
   if constexpr (TEAMS > 1) {
     // the second team's accumulators, row maxima and row sums through LDS (the tiles' buffers) to the first team
     float4v* fold_o = reinterpret_cast<float4v*>(s_k0) + wave * (DB * 4 * 64) + lane;
-    float* fold_ml = reinterpret_cast<float*>(s_v0) + wave * 128 + lane;
-    static_assert(WAVES * DB * 4 * 64 * 16 <= TEAMS * TILE_BYTES && WAVES * 128 * 4 <= TEAMS * TILE_BYTES, "room of the fold");
+    float* fold_ml = reinterpret_cast<float*>(s_v0) + wave * 256 + lane;
+    static_assert(WAVES * DB * 4 * 64 * 16 <= TEAMS * TILE_BYTES && WAVES * 256 * 4 <= TEAMS * TILE_BYTES, "room of the fold");
     wait_vmem();
     __syncthreads();
     if (team == 1) {
@@ -835,12 +842,28 @@ __global__ void __launch_bounds__(64 * WAVES * TEAMS, (KF == kKfTensorLds ? 1 : 
         fold_o[i * 64] = float4v{o_acc[i >> 2][4 * (i & 3)], o_acc[i >> 2][4 * (i & 3) + 1], o_acc[i >> 2][4 * (i & 3) + 2], o_acc[i >> 2][4 * (i & 3) + 3]};
       fold_ml[0] = m_run;
       fold_ml[64] = l_run;
+      if (kTensor || kSeeded) {
+        fold_ml[128] = m_kf;
+        fold_ml[192] = l_kf;
+      }
     }
     __syncthreads();
     if (team == 1) return;
     const float m1 = fold_ml[0], l1 = fold_ml[64];
     const float m_new = fmaxf(m_run, m1);
     const float w0 = __builtin_amdgcn_exp2f(m_run - m_new), w1 = __builtin_amdgcn_exp2f(m1 - m_new);
+    if (kTensor || kSeeded) {
+      const float lk1 = fold_ml[192];
+      if constexpr (KF == kKfSeededTau1) {
+        l_kf = __builtin_fmaf(lk1, w1, l_kf * w0);
+      } else if constexpr (KF == kKfSeededFast) {
+        l_kf = __builtin_fmaf(lk1, __builtin_amdgcn_exp2f((m1 - m_new) * p.inv_tau), l_kf * __builtin_amdgcn_exp2f((m_run - m_new) * p.inv_tau));
+      } else {
+        const float mk1 = fold_ml[128], mk = fmaxf(m_kf, mk1);
+        l_kf = __builtin_fmaf(lk1, __builtin_amdgcn_exp2f(mk1 - mk), l_kf * __builtin_amdgcn_exp2f(m_kf - mk));
+        m_kf = mk;
+      }
+    }
     m_run = m_new;
     l_run = __builtin_fmaf(l1, w1, l_run * w0);
 #pragma unroll
@@ -887,11 +910,10 @@ __global__ void __launch_bounds__(64 * WAVES * TEAMS, (KF == kKfTensorLds ? 1 : 
     if (g == 0 && p.lse) p.lse[(SPLIT ? (int64_t)b * p.H + hq : (int64_t)bh) * p.Sq + qi] = m_run + __builtin_amdgcn_logf(l_run);
   }
   if (kTensor || kSeeded) {
-    l_kf += xchg32(l_kf);
     if (KF == kKfSeededTau1) l_kf *= -kLog2e;  // the sum was taken over 1 / log2 u = -ln2 / E
     // packed modes: the perturbed sum shares the plain softmax's stabiliser, scaled by 1 / tau
     const float base = KF == kKfSeededTau1 ? m_run : KF == kKfSeededFast ? m_run * p.inv_tau : m_kf;
-    if (qi < p.Sq && g == 0) p.lse_kf[(int64_t)bh * p.Sq + qi] = base + __builtin_amdgcn_logf(l_kf);
+    if (qrow < rows && g == 0) p.lse_kf[(int64_t)bh * p.Sq + qi] = base + __builtin_amdgcn_logf(l_kf);
   }
   }  // pass
 }
@@ -913,14 +935,16 @@ hipError_t launch_one(const AttnKernelParams& p0, hipStream_t stream) {
   const int64_t BH = (int64_t)p.B * p.H;
   // 256-row workgroups (8 waves) halve the K/V staging per row (measured 148 vs 158 us at B1 H32 S4096), but
   // there are half as many of them: used on the pipelined paths once they still fill the chip twice
-  // (kKfTensorLds: the noise slices in flight through LDS leave room for one workgroup per CU in either form, so the
-  // 256-row one is used as soon as there is a workgroup for every CU)
-  constexpr bool kHas8 = KF == kKfNone || KF == kKfSoftcap || KF == kKfSeededTau1 || KF == kKfSeededFast || KF == kKfTensorLds;
+  // (noise from a tensor: its slices in flight through LDS leave a CU room for one workgroup of either form at D = 128, and the
+  // 256-row one is used from five for every four CUs on, H32 S2527 315 -> 297 us, S2091 214 -> 222; at D = 64 two of the 128-row
+  // form fit, and it takes seven for four, H32 S3543 423 -> 408, S2527 226 -> 253)
+  constexpr bool kNoiseTensor = KF == kKfTensor || KF == kKfTensorLds;
+  constexpr bool kHas8 = KF == kKfNone || KF == kKfSoftcap || KF == kKfSeededTau1 || KF == kKfSeededFast || kNoiseTensor;
   if constexpr (kHas8) {
     const int nMB8 = (p.Sq + 255) / 256;
     const int64_t n8 = (int64_t)nMB8 * BH;
     const int64_t cus = device_cu_count();
-    if ((forced & 7) ? (forced & 7) >= 2 : n8 >= (KF == kKfTensorLds ? cus : 2 * cus)) {
+    if ((forced & 7) ? (forced & 7) >= 2 : n8 >= (kNoiseTensor ? (D == 128 ? 5 : 7) * cus / 4 : 2 * cus)) {
       // causal: pair the heaviest block with the lightest inside one workgroup when the pairs come out as whole
       // rounds of the chip (or as many rounds that a ragged last one does not matter)
       const int64_t pairs = (int64_t)((nMB8 + 1) / 2) * BH;

@@ -39,4 +39,20 @@ hipError_t launch_teams_td(const AttnKernelParams& p, bool emu, int kf, unsigned
   return hipErrorInvalidValue;
 }
 
+// The same for KeyFormer with the reference's rounding of the logits (attn_teams_kf_{f16,bf16}.hip).
+template <typename T, int D>
+hipError_t launch_teams_kf_td(const AttnKernelParams& p, int kf, unsigned grid, hipStream_t s) {
+#define FT_CASE(K)                                                                                                       \
+  if (kf == K) {                                                                                                         \
+    hipLaunchKernelGGL((attn_fwd_kernel<T, D, true, true, K, 2, true, false, 2>), dim3(grid), dim3(256), 0, s, p);       \
+    return hipGetLastError();                                                                                            \
+  }
+  FT_CASE(kKfTensor) FT_CASE(kKfTensorLds) FT_CASE(kKfSeeded)
+  if constexpr (std::is_same<T, F16>::value) {
+    FT_CASE(kKfSeededTau1) FT_CASE(kKfSeededFast)
+  }
+#undef FT_CASE
+  return hipErrorInvalidValue;
+}
+
 }  // namespace ft

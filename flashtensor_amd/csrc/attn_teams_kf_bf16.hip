@@ -1,0 +1,8 @@
+// attn_split.hpp's KeyFormer form with two teams of waves, instantiated for bf16, head sizes 64 and 128.
+#include "attn_split.hpp"
+
+namespace ft {
+hipError_t launch_attn_teams_kf_bf16(const AttnKernelParams& p, int D, int kf, unsigned grid, hipStream_t s) {
+  return D == 128 ? launch_teams_kf_td<BF16, 128>(p, kf, grid, s) : launch_teams_kf_td<BF16, 64>(p, kf, grid, s);
+}
+}  // namespace ft

@@ -38,6 +38,14 @@ static hipError_t launch_td(const ColstatsKernelParams& p, bool causal, bool emu
 
 hipError_t launch_colstats(const ColstatsKernelParams& p, int D, bool bf16, bool causal, bool emu, int mode, hipStream_t s) {
   const bool tensor = mode == kStatKfTensor || mode == kStatCormTensor;
+  const int64_t wgs = (int64_t)p.B * p.H * ((p.Skv + 127) / 128), cus = device_cu_count();
+  if (tensor && emu) {
+    // Two teams of waves on 128 keys where a lane's loads of the tensor, one tile ahead, are what a tile waits for: twice the
+    // loads in flight (keyformer calls, same process: B1 H8 S1003 83 -> 80 us, S2091 177 -> 169, H16 S2527 247 -> 227, H32 S1501
+    // 166 -> 154; D64 H32 S2091 237 -> 226; even at two and a half workgroups per CU, 368 and 370 at H32 S2527)
+    const int forced = form_override();
+    if (forced ? forced == kFormTeams : wgs <= 9 * cus / 4) return launch_colstats_teams(p, D, bf16, causal, mode, s);
+  }
   if (!tensor && emu) {
     int form = form_override();
     // 64 keys per workgroup where there are fewer than two workgroups of 128 per CU (h2o calls, same process: B1 H8 S1500
@@ -45,7 +53,6 @@ hipError_t launch_colstats(const ColstatsKernelParams& p, int D, bool bf16, bool
     // 77.4 and 78.7 at B1 H32 S2048, and at eight 62.0 and 66.7); and two teams of waves below one per CU, where a
     // workgroup of 64 keys often has its CU to itself (B1 H8 S1500 43.7 -> 41.0, S3000 76.4 -> 70.4, roco B1 H8 S2048 D64 39.4 ->
     // 37.1; at one per CU 56.3 and 56.1 at B1 H16 S2048, 34.7 and 35.3 at B1 H32 S1000, above it slower: 52.3 and 57.6 at B1 H32 S1500)
-    const int64_t wgs = (int64_t)p.B * p.H * ((p.Skv + 127) / 128), cus = device_cu_count();
     if (!form) form = wgs < cus ? kFormTeams : wgs < 2 * cus ? kFormNarrow : kFormWide;
     if (form == kFormTeams) return launch_colstats_teams(p, D, bf16, causal, mode, s);
     if (form == kFormNarrow) return launch_colstats_narrow(p, D, bf16, causal, mode, s);

@@ -61,7 +61,7 @@ __global__ void __launch_bounds__(kColThreads * TEAMS, (TEAMS == 1 ? colstats_wa
   constexpr bool kPlainF32 = !EMU;                                        // logits stay in fp32: one fma per element
   constexpr bool kTensor = MODE == kStatKfTensor || MODE == kStatCormTensor;
   constexpr bool k16 = !kTensor;            // 16x16x32 blocks; the tensor modes stay on 32x32x16
-  static_assert(k16 || (NKEYS == 2 && TEAMS == 1), "32 keys per wave");
+  static_assert(k16 || NKEYS == 2, "32 keys per wave");
   constexpr int NKEY = k16 ? NKEYS : 1;     // key columns per lane
   constexpr int WK = BK / 4;                // keys per wave
   constexpr int NBLK = k16 ? 4 : 8;         // groups of 4 query rows per lane and key in a tile
@@ -553,10 +553,10 @@ __global__ void __launch_bounds__(kColThreads * TEAMS, (TEAMS == 1 ? colstats_wa
         reduce_qk(S0, b1, t);  // scores of tile t + 1: past the last tile they come from stale LDS and are discarded
         rotate();
       }
-      if (TEAMS > 1 && t < ntrips) {  // (one at most)
-        wait_vmem();
-        __syncthreads();
-      }
+    }
+    if (TEAMS > 1 && t < ntrips) {  // (one at most)
+      wait_vmem();
+      __syncthreads();
     }
   }
 

@@ -1,4 +1,5 @@
-// colstats_kernel.hpp with 64 keys and two teams of waves per workgroup: the modes with the reference's rounding of the logits.
+// colstats_kernel.hpp with 64 keys (128 in the modes that read a tensor) and two teams of waves per workgroup: the modes with the
+// reference's rounding of the logits.
 #include "colstats_kernel.hpp"
 
 namespace ft {
@@ -8,6 +9,13 @@ static hipError_t launch_teams_td(const ColstatsKernelParams& p, bool causal, in
 #define FT_CASE(M) \
   if (mode == M) return causal ? launch_colstats_one<T, D, true, true, M, 1, 2>(p, s) : launch_colstats_one<T, D, false, true, M, 1, 2>(p, s);
   FT_CASE(kStatSum) FT_CASE(kStatSumSq) FT_CASE(kStatKfSeeded) FT_CASE(kStatCormRule)
+#undef FT_CASE
+#define FT_CASE(M) \
+  if (mode == M) return causal ? launch_colstats_one<T, D, true, true, M, 2, 2>(p, s) : launch_colstats_one<T, D, false, true, M, 2, 2>(p, s);
+  FT_CASE(kStatKfTensor) FT_CASE(kStatCormTensor)
+#undef FT_CASE
+#define FT_CASE(M) \
+  if (mode == M) return causal ? launch_colstats_one<T, D, true, true, M, 1, 2>(p, s) : launch_colstats_one<T, D, false, true, M, 1, 2>(p, s);
   if constexpr (std::is_same<T, F16>::value) {
     FT_CASE(kStatKfSeededTau1) FT_CASE(kStatKfSeededFast)
   }

@@ -171,10 +171,15 @@ __device__ __forceinline__ rsrc_t make_rsrc(const void* base) {
 __device__ __forceinline__ void load_lds16(rsrc_t rsrc, char* lds_dst, uint32_t voff, uint32_t soff) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, FT_LDS(void, lds_dst), 16, voff, soff, 0, 0);
 }
+// the same for 4 bytes a lane (LDS address = wave-uniform base + lane * 4)
+__device__ __forceinline__ void load_lds4(rsrc_t rsrc, char* lds_dst, uint32_t voff, uint32_t soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, FT_LDS(void, lds_dst), 4, voff, soff, 0, 0);
+}
 #else
 typedef int rsrc_t;
 __device__ inline rsrc_t make_rsrc(const void*) { return 0; }
 __device__ inline void load_lds16(rsrc_t, char*, uint32_t, uint32_t) {}
+__device__ inline void load_lds4(rsrc_t, char*, uint32_t, uint32_t) {}
 #endif
 
 template <int D, int ROWS, int NT, int SWZ>

@@ -21,7 +21,6 @@ struct AttnKernelParams {
   float* lse_kf;  // [B,H,Sq] normaliser of the perturbed softmax (KeyFormer modes)
   const float* exp_rand;
   int64_t er_sb, er_sh, er_sr;
-  int er_vec4;  // exp_rand rows can be read as aligned float4
   uint64_t seed;
   int B, H, Sq, Skv;
   int off;          // Skv - Sq: query i sees keys j <= i + off when causal
@@ -94,8 +93,8 @@ struct ColstatsKernelParams {
 // weight exp((t + g) / tau) with g = -ln E equals exp(t / tau) E^(-1/tau); the in-kernel E lies in
 // [6e-8, 16.7], so for tau >= 0.25 the plain softmax's running maximum also stabilises the perturbed sum
 // (exponent <= (6 + 24) / tau <= 120) and no second maximum is tracked; tau == 1 needs 1 / E only.
-// kKfTensorLds: the noise tensor of kKfTensor, its tiles landing in LDS by direct-to-LDS loads a whole tile ahead
-// (16-byte aligned rows, Skv a multiple of 4, a (b, h) slice below 2 GiB; kKfTensor reads any layout into registers)
+// kKfTensor / kKfTensorLds: noise from a tensor, its tiles landing in LDS by direct-to-LDS loads a whole tile ahead, 4 or 16 bytes a
+// lane (16: rows of whole aligned chunks, a (b, h) slice below 2 GiB)
 enum KfMode { kKfNone = 0, kKfTensor = 1, kKfSeeded = 2, kKfSoftcap = 3, kKfSeededTau1 = 4, kKfSeededFast = 5, kKfTensorLds = 6 };
 // kStatCormRule: thresholds 1 / (i + 1) per query row i; kStatCormTensor: thresholds read from a tensor
 enum StatMode {
