@@ -62,18 +62,24 @@ hipError_t launch_attn_teams_kf_bf16(const AttnKernelParams& p, int D, int kf, u
 // workgroups a CU holds two, from five tiles on: H8 S1000 14.9 -> 12.0).  Shorter plain calls have 2 us at most to gain
 // (S500 14.0 -> 12.3) and keep to the forms whose results agree bit for bit; soft-capped ones, whose waves are slow
 // enough alone, take it from four tiles on (S300 13.4 -> 12.2, S500 19.4 -> 14.9, S130 9.6 -> 9.8).
-// With up to two workgroups for every CU: D64 gains under the causal mask, whose blocks differ in length (B1 H16 S2048
-// 25.2 -> 22.8; without the mask 28.6 -> 30.5; plain prompts beyond 32 tiles again keep to the bit-equal forms); D128 does not
-// (128 KB of LDS, and two in turn: H16 S2048 37.1 -> 38.7) but for soft-capped logits over twelve tiles or more (H16 S2048
-// 59.2 -> 47.8, H32 S777 26.8 -> 24.6, but B2 H32 S500 20.5 -> 23.0).
+// Under the causal mask, whose blocks differ in length, with more of them: D128 up to three for two CUs (H8 S3000 48 -> 40, H16 S1500
+// 28.5 -> 25.8; H16 S2048, four for two, 36.6 -> 35.8 and H32 S777 17.7 -> 20.8), D64 up to two for every CU (H8 S3000 33.5 -> 27.2, B2
+// H32 S500 10.7 -> 9.4) or, over more than 32 tiles, five for two (H16 S2500 31.7 -> 26.9, S3000 36 -> 38), longer ones than 48 again keeping to the bit-equal
+// forms; soft-capped D128 over twelve tiles or more up to
+// two for every CU (H32 S777 28.7 -> 26.0, B2 H32 S500 21.8 -> 23.4), over more than 32 five for two (H16 S2500 89 -> 81, S3000
+// 97 -> 107), D64 up to thirteen for four CUs (H16 S3000 85 -> 66, H32 S1500 47 -> 37, B2 H32 S777 28.6 -> 27.4, S1000 32 -> 36).
 static bool use_teams(const AttnKernelParams& p, int D, bool causal, bool cap, int64_t grid) {
   const int forced = attn_form_override();
   if (forced || attn_split_override()) return (forced & 16) != 0;
   const int64_t cus = device_cu_count();
   const int tiles = (p.Skv + 63) / 64;
-  if (tiles <= (cap ? 3 : D == 64 ? 5 : 10) || grid > 2 * cus) return false;
+  if (tiles <= (cap ? 3 : D == 64 ? 5 : 10)) return false;
   if (grid <= cus) return true;
-  return causal && (D == 64 ? cap || tiles <= 32 : cap && tiles > 11);
+  if (!causal) return false;
+  if (D == 128 && !cap) return 2 * grid <= 3 * cus;
+  if (D == 64 && cap) return 4 * grid <= 13 * cus;
+  if (D == 64 && tiles > 48) return false;
+  return (D == 64 || tiles > 11) && 2 * grid <= (tiles > 32 ? 5 : 4) * cus;
 }
 
 // KeyFormer's passes do two to four times the vector work per tile, so the chain of a block's tiles bounds launches of more

@@ -933,34 +933,52 @@ hipError_t launch_one(const AttnKernelParams& p0, hipStream_t stream) {
   p.head_major = 0;
   const int forced = attn_form_override();
   const int64_t BH = (int64_t)p.B * p.H;
-  // 256-row workgroups (8 waves) halve the K/V staging per row (measured 148 vs 158 us at B1 H32 S4096), but
-  // there are half as many of them: used on the pipelined paths once they still fill the chip twice
-  // (noise from a tensor: its slices in flight through LDS leave a CU room for one workgroup of either form at D = 128, and the
-  // 256-row one is used from five for every four CUs on, H32 S2527 315 -> 297 us, S2091 214 -> 222; at D = 64 two of the 128-row
-  // form fit, and it takes seven for four, H32 S3543 423 -> 408, S2527 226 -> 253)
-  constexpr bool kNoiseTensor = KF == kKfTensor || KF == kKfTensorLds;
-  constexpr bool kHas8 = KF == kKfNone || KF == kKfSoftcap || KF == kKfSeededTau1 || KF == kKfSeededFast || kNoiseTensor;
+  const int64_t cus = device_cu_count();
+  const int nMB = (p.Sq + 127) / 128, nMB8 = (p.Sq + 255) / 256;
+  const int64_t n4 = nMB * BH, n8 = nMB8 * BH, pairs = (int64_t)((nMB8 + 1) / 2) * BH;
+  // 256-row workgroups (8 waves) stage K and V once for twice the rows, but round every prompt up to 256 rows and are half as many:
+  // under the causal mask the 128-row form is the faster one nearly everywhere (attention, B4 H32 D128 S777 53.5 -> 42.2 us, S1024
+  // 55.5 -> 51.3, S2600 321 -> 278, B2 S2600 151 -> 135; D64 B4 S1300 61 -> 51; soft-capped B4 S777 75 -> 59).
+  // - plain, soft-cap, causal: where hardly a row is padding and the blocks pair up, heaviest with lightest, into whole rounds of
+  //   the chip: one round (B1 H32 S4096 151.9 -> 148.5), or three and more, for which an XCD finishes a pair's blocks before it
+  //   starts the next pair's (B8 H32 S1536 229 -> 214, S2048 387 -> 373, B3 S4096 453 -> 443; two rounds B2 H32 S4096 292.5 and
+  //   293.7, B4 S2048 166 and 169).  D64 and soft-capped logits from four rounds on (B4 H32 S4096 360 -> 351, soft-capped 941 ->
+  //   893; three rounds 204 and 211, 521 and 528), D64 at one round (89.5 -> 88.5; soft-capped 218 -> 229).
+  // - no mask: D128 up to 127 (b, h) pairs (B2 H32 S3600 477 -> 463; B4 S1024 86 -> 90; D64 B2 S2048 86 -> 98).
+  // - KeyFormer, seeded: D128 from two workgroups per CU on (B1 H32 S4096 345 -> 340 us whole; D64 260 -> 269).
+  // - KeyFormer, noise from a tensor: its slices in flight leave a CU room for one workgroup of either form at D128: from five for
+  //   every four CUs on (H32 S2527 315 -> 297, S2091 214 -> 222); at D64 two of the 128-row form fit: from seven for four on (H32
+  //   S3543 423 -> 408, S2527 226 -> 253).
+  constexpr bool kNoiseTensor = KF == kKfTensor || KF == kKfTensorLds, kPlain = KF == kKfNone || KF == kKfSoftcap;
+  constexpr bool kHas8 = kPlain || KF == kKfSeededTau1 || KF == kKfSeededFast || kNoiseTensor;
   if constexpr (kHas8) {
-    const int nMB8 = (p.Sq + 255) / 256;
-    const int64_t n8 = (int64_t)nMB8 * BH;
-    const int64_t cus = device_cu_count();
-    if ((forced & 7) ? (forced & 7) >= 2 : n8 >= (kNoiseTensor ? (D == 128 ? 5 : 7) * cus / 4 : 2 * cus)) {
-      // causal: pair the heaviest block with the lightest inside one workgroup when the pairs come out as whole
-      // rounds of the chip (or as many rounds that a ragged last one does not matter)
-      const int64_t pairs = (int64_t)((nMB8 + 1) / 2) * BH;
-      constexpr bool kCanPair = kAttnTwoBlocks && (KF == kKfNone || KF == kKfSoftcap) && CAUSAL;
-      p.two_blocks = kCanPair && nMB8 >= 2 && ((forced & 7) ? (forced & 7) == 3 : (pairs % cus == 0 || pairs >= 8 * cus));
+    const bool pair_up = kAttnTwoBlocks && kPlain && CAUSAL && nMB8 >= 2;
+    const int64_t rounds = pairs / cus;
+    bool eight;
+    if constexpr (kPlain && CAUSAL)
+      eight = pair_up && pairs % cus == 0 && (int64_t)nMB8 * 256 * 100 <= (int64_t)p.Sq * 103 &&
+              ((rounds == 1 && KF == kKfNone) || rounds >= (D == 128 && KF == kKfNone ? 3 : 4));
+    else if constexpr (kPlain)
+      eight = D == 128 && BH < 128 && 4 * n8 >= 7 * cus;
+    else if constexpr (kNoiseTensor)
+      eight = 4 * n8 >= (D == 128 ? 5 : 7) * cus;
+    else
+      eight = D == 128 && n8 >= 2 * cus;
+    if ((forced & 7) ? (forced & 7) >= 2 : eight) {
+      p.two_blocks = pair_up && ((forced & 7) ? (forced & 7) == 3 : 1);
       const int64_t grid = p.two_blocks ? pairs : n8;
-      // equal workgroups in several rounds: let an XCD finish a pair's blocks before it starts the next pair's
-      p.head_major = BH % 8 == 0 && (forced ? (forced & 8) != 0 : (p.two_blocks && grid >= 3 * cus));
+      p.head_major = BH % 8 == 0 && (forced ? (forced & 8) != 0 : (p.two_blocks && rounds >= 3));
       hipLaunchKernelGGL((attn_fwd_kernel<T, D, CAUSAL, EMU, KF, 8>), dim3((unsigned)grid), dim3(512), 0, stream, p);
       return hipGetLastError();
     }
   }
-  const int nMB = (p.Sq + 127) / 128;
-  dim3 grid((unsigned)(nMB * BH));
-  p.pair_order = CAUSAL && (int64_t)grid.x <= 2 * (int64_t)device_cu_count();  // two workgroups of this form per CU
-  p.head_major = BH % 8 == 0 && (forced & 8) != 0 && !p.pair_order;
+  dim3 grid((unsigned)n4);
+  p.pair_order = CAUSAL && (int64_t)grid.x <= 2 * cus;  // two workgroups of this form per CU
+  // Head-major where the K and V of all pairs together are beyond every cache: with the mask from 256 pairs and nine rounds on (B8
+  // H32 S2304 475 -> 445 us, S2600 645 -> 570, soft-capped 934 -> 849; S2048 374, paired 256-row blocks 373), without from 128 pairs
+  // (256 at D64) and two and a half rounds on (D128 B4 H32 S2600 518 -> 491, B8 S1024 193 -> 165, D64 99.5 -> 93; B4 D128 S513 38.6 -> 41.5).
+  const bool far = BH >= (CAUSAL || D == 64 ? 256 : 128) && n4 >= (CAUSAL ? 18 * cus : 5 * cus);
+  p.head_major = BH % 8 == 0 && !p.pair_order && (forced ? (forced & 8) != 0 : kPlain && far);
   hipLaunchKernelGGL((attn_fwd_kernel<T, D, CAUSAL, EMU, KF, 4>), grid, dim3(256), 0, stream, p);
   return hipGetLastError();
 }
