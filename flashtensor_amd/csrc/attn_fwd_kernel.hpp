@@ -979,7 +979,9 @@ hipError_t launch_one(const AttnKernelParams& p0, hipStream_t stream) {
   // (256 at D64) and two and a half rounds on (D128 B4 H32 S2600 518 -> 491, B8 S1024 193 -> 165, D64 99.5 -> 93; B4 D128 S513 38.6 -> 41.5).
   const bool far = BH >= (CAUSAL || D == 64 ? 256 : 128) && n4 >= (CAUSAL ? 18 * cus : 5 * cus);
   p.head_major = BH % 8 == 0 && !p.pair_order && (forced ? (forced & 8) != 0 : kPlain && far);
-  hipLaunchKernelGGL((attn_fwd_kernel<T, D, CAUSAL, EMU, KF, 4>), grid, dim3(256), 0, stream, p);
+  // no more workgroups than CUs: room for one in each (the dispatcher puts two on some otherwise, and leaves others idle)
+  const unsigned pad = kPlain && n4 <= cus ? 88 * 1024 - 4 * kAttnBN * 2 * D : 0;
+  hipLaunchKernelGGL((attn_fwd_kernel<T, D, CAUSAL, EMU, KF, 4>), grid, dim3(256), pad, stream, p);
   return hipGetLastError();
 }
 

@@ -205,78 +205,103 @@ __device__ __forceinline__ int shares_of_block(const AttnKernelParams& p, int mb
   return ((n_end + kAttnBN - 1) / kAttnBN + p.chunk_tiles - 1) / p.chunk_tiles;
 }
 
-// Folds the shares of a row, eight loads at a time: running maximum and sum, and what `f(share, weight)` adds up;
-// `scale` multiplies that when the maximum moves.  slot0: the row's wave in the first share, n: the row in the wave; every
-// `step`-th share is taken.  A share that shows the row no finite logit has m = kNoMax, l = 0.
-template <typename L, typename F, typename S>
-__device__ __forceinline__ void fold_shares(const AttnKernelParams& p, int D, int64_t slot0, int n, int nch, int step, float& M, float& sum, L load, F f, S scale) {
-  constexpr int U = 8;
+// Folds the shares of a row, U at a time: running maximum and sum, and Q pieces of four channels (Q = 0: none) of the shares'
+// accumulators.  slot0: the row's wave in the first share, n: the row in the wave; every `step`-th share is taken, nch of them.
+// A share that shows the row no finite logit has m = kNoMax, l = 0.
+template <int U, int Q, typename L>
+__device__ __forceinline__ void fold_shares(const AttnKernelParams& p, int D, int64_t slot0, int n, int nch, int step, float& M, float& sum, float4v (&acc)[Q ? Q : 1], L load) {
   M = kNoMax, sum = 0.f;
+#pragma unroll
+  for (int q = 0; q < Q; ++q) acc[q] = float4v{0.f, 0.f, 0.f, 0.f};
   for (int c0 = 0; c0 < nch; c0 += U) {
     float m[U], l[U];
-    float4v o[U];
+    float4v o[U][Q ? Q : 1];
 #pragma unroll
     for (int u = 0; u < U; ++u) {  // shares past the last one re-read it, with weight 0
       const SplitPartial s = split_partial(p.part, D, slot0 + (int64_t)min(c0 + u, nch - 1) * step * p.part_waves);
       m[u] = s.m[n];
       l[u] = s.l[n];
-      load(s, o[u]);
+#pragma unroll
+      for (int q = 0; q < Q; ++q) o[u][q] = load(s, q);
     }
     float M1 = M;
 #pragma unroll
     for (int u = 0; u < U; ++u) M1 = fmaxf(M1, m[u]);
     const float move = __builtin_amdgcn_exp2f(M - M1);
     sum *= move;
-    scale(move);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) acc[q] *= move;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const float w = c0 + u < nch ? __builtin_amdgcn_exp2f(m[u] - M1) : 0.f;
       sum = __builtin_fmaf(w, l[u], sum);
-      f(o[u], w);
+#pragma unroll
+      for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[q][e] = __builtin_fmaf(w, o[u][q][e], acc[q][e]);
     }
     M = M1;
   }
 }
 
-// One workgroup per (wave of 32 rows of a shared block, 32 channels), a wave for four of a lane's 16 channels: weights of
-// the shares from their row maxima, then the shares' accumulators in their own register layout (every load is 1 KB
-// contiguous).  Bound by the latency of its loads.
-template <typename T, int D>
-__device__ __forceinline__ void combine_rows(const AttnKernelParams& p, int first_shared, int i) {
+// A wave takes Q of the four pieces of (32 rows of a shared block, 32 channels); every load is up to 1 KB contiguous, in the
+// accumulators' own register layout.  Bound by the latency of its loads, over many rows by their bytes.
+// Q = 1: up to 16 rows (a generation step's) the lanes that have no row take every SUB-th share of the others' and meet by lane
+// exchanges, so that eighty shares of four rows are one round of loads and not ten (whole calls: B1 H16/4 Sq1 Skv5195 16.6 -> 10.6
+// us, H32/8 Sq1 Skv4000 15.4 -> 11.7, soft-capped B2 H16/4 Sq1 Skv3058 18.6 -> 13.0); eight shares or fewer are one round anyway.
+// Q = 4: whole waves of rows with up to four shares, a quarter of the waves with four times the loads in flight (B1 H32/8 Sq501
+// Skv5760 8.7 -> 6.5 us; sixteen shares, Sq172 Skv4918, 5.1 -> 8.0).
+template <typename T, int D, int Q>
+__device__ __forceinline__ void combine_rows(const AttnKernelParams& p, int first_shared, int unit) {
   constexpr int DB = D / 32;
   const int rows = p.Sq * p.group, Hkv = p.H / p.group;
   const int nshared = (rows + 127) / 128 - first_shared;
+  const int q0 = Q == 1 ? unit % 4 : 0;
+  int i = Q == 1 ? unit / 4 : unit;
   const int db = i % DB;
   i /= DB;
   const int wv = i % p.part_waves;
   i /= p.part_waves;
   const int mb = first_shared + i % nshared, bh = i / nshared;
-  const int lane = lane_id(), q4 = wave_id(), g = lane >> 5, n = lane & 31;
-  const int row = mb * 128 + wv * 32 + n;
-  if (row >= rows) return;
+  if (bh >= p.B * Hkv) return;
+  const int lane = lane_id(), g = lane >> 5;
+  int n = lane & 31, sub = 0, rp = 32;  // row in the wave; which shares
+  if (Q == 1) {
+    rp = 1;
+    while (rp < 32 && (rp < rows || 32 / rp >= 2 * ((shares_of_block(p, mb) + 7) / 8))) rp *= 2;
+    sub = n / rp;
+    n &= rp - 1;
+  }
+  const int row = mb * 128 + wv * 32 + n, slots = 32 / rp;
   const int64_t slot0 = ((int64_t)bh * p.nitems + p.first_item[mb]) * p.part_waves + wv;
+  const int nch = shares_of_block(p, mb), rc = min(row, rows - 1) - (row - n);  // (lanes without a row repeat the last one)
   float M, L;
-  float4v acc = {0.f, 0.f, 0.f, 0.f};
-  fold_shares(p, D, slot0, n, shares_of_block(p, mb), 1, M, L,
-              [&](const SplitPartial& s, float4v& o) { o = *reinterpret_cast<const float4v*>(s.o + ((db * 4 + q4) * 64 + lane) * 4); },
-              [&](const float4v& o, float w) {
+  float4v acc[Q];
+  fold_shares<Q == 4 ? 4 : 8, Q>(p, D, slot0 + (int64_t)sub * p.part_waves, max(rc, 0), (nch - sub + slots - 1) / slots, slots, M, L, acc,
+                                 [&](const SplitPartial& s, int q) { return *reinterpret_cast<const float4v*>(s.o + ((db * 4 + q0 + q) * 64 + g * 32 + max(rc, 0)) * 4); });
+  if (Q == 1) {
+    for (int d = rp; d < 32; d *= 2) {
+      const float M2 = __shfl_xor(M, d), L2 = __shfl_xor(L, d), M1 = fmaxf(M, M2);
+      const float w = __builtin_amdgcn_exp2f(M - M1), w2 = __builtin_amdgcn_exp2f(M2 - M1);
+      L = __builtin_fmaf(L2, w2, L * w);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) acc[e] = __builtin_fmaf(w, o[e], acc[e]);
-              },
-              [&](float move) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) acc[e] *= move;
-              });
+      for (int e = 0; e < 4; ++e) acc[0][e] = __builtin_fmaf(__shfl_xor(acc[0][e], d), w2, acc[0][e] * w);
+      M = M1;
+    }
+  }
+  if (row >= rows || sub > 0) return;
   const float inv = 1.f / L;
   const int b = bh / Hkv, h = (bh % Hkv) * p.group + row % p.group, qi = row / p.group;
   uint16_t* optr = p.o + b * p.so.b + (int64_t)qi * p.so.s + h * p.so.h;
-  *reinterpret_cast<uint2*>(optr + 32 * db + 8 * q4 + 4 * g) = make_uint2(T::pack2(acc[0] * inv, acc[1] * inv), T::pack2(acc[2] * inv, acc[3] * inv));
-  if (db == 0 && q4 == 0 && g == 0 && p.lse) p.lse[((int64_t)b * p.H + h) * p.Sq + qi] = M + __builtin_amdgcn_logf(L);
+#pragma unroll
+  for (int q = 0; q < Q; ++q)
+    *reinterpret_cast<uint2*>(optr + 32 * db + 8 * (q0 + q) + 4 * g) = make_uint2(T::pack2(acc[q][0] * inv, acc[q][1] * inv), T::pack2(acc[q][2] * inv, acc[q][3] * inv));
+  if (db == 0 && q0 == 0 && g == 0 && p.lse) p.lse[((int64_t)b * p.H + h) * p.Sq + qi] = M + __builtin_amdgcn_logf(L);
 }
 
-template <typename T, int D>
+template <typename T, int D, int Q>
 __global__ void __launch_bounds__(256) attn_combine_kernel(const AttnKernelParams p, int first_shared) {
-  combine_rows<T, D>(p, first_shared, blockIdx.x);
+  combine_rows<T, D, Q>(p, first_shared, blockIdx.x * 4 + wave_id());
 }
 
 // The column sums of few rows from their kept logits, and (the last `gridDim.x - ncol` workgroups) the folding of the
@@ -290,7 +315,7 @@ __host__ __device__ constexpr int stat_step(int pool) { return pool ? kStatTiles
 template <typename T, int D, bool SQ>
 __global__ void __launch_bounds__(256) split_stats_kernel(const AttnKernelParams p, const SplitStats st, int ncol) {
   if ((int)blockIdx.x >= ncol) {
-    combine_rows<T, D>(p, 0, blockIdx.x - ncol);
+    combine_rows<T, D, 1>(p, 0, (blockIdx.x - ncol) * 4 + wave_id());
     return;
   }
   constexpr int KT = kStatTiles * kAttnBN;
@@ -320,9 +345,9 @@ __global__ void __launch_bounds__(256) split_stats_kernel(const AttnKernelParams
     const int nch = shares_of_block(p, 0);
     if (nch > 1) {
       float M = kNoMax, L = 0.f;
+      float4v none[1];
       if (part < nch)
-        fold_shares(p, D, (int64_t)bh * p.nitems + part, rc, (nch - part + 7) >> 3, 8, M, L, [](const SplitPartial&, float4v&) {},
-                    [](const float4v&, float) {}, [](float) {});
+        fold_shares<8, 0>(p, D, (int64_t)bh * p.nitems + part, rc, (nch - part + 7) >> 3, 8, M, L, none, [](const SplitPartial&, int) { return float4v{}; });
       s_sum[0][t] = M;
       s_sum[1][t] = L;
       __syncthreads();
@@ -439,11 +464,21 @@ hipError_t launch_attn_split(const AttnKernelParams& p0, const SplitPlan& plan, 
 #undef FT_CASE
     return hipGetLastError();
   }
-  const dim3 cgrid((unsigned)ncomb), cblk(256);
-  if (D == 128 && bf16) hipLaunchKernelGGL((attn_combine_kernel<BF16, 128>), cgrid, cblk, 0, s, p, plan.first_shared);
-  else if (D == 128) hipLaunchKernelGGL((attn_combine_kernel<F16, 128>), cgrid, cblk, 0, s, p, plan.first_shared);
-  else if (bf16) hipLaunchKernelGGL((attn_combine_kernel<BF16, 64>), cgrid, cblk, 0, s, p, plan.first_shared);
-  else hipLaunchKernelGGL((attn_combine_kernel<F16, 64>), cgrid, cblk, 0, s, p, plan.first_shared);
+  // whole waves of rows and no more than four shares of a block (up to kSplitStatRows rows: as in the fold beside the column sums)
+  const int64_t rows = (int64_t)p.Sq * p.group;
+  const int most = (std::min<int64_t>(p.Skv, (rows - 1) / p.group + 1 + p.off) + kAttnBN - 1) / kAttnBN;
+  const bool few = rows <= kSplitStatRows || most > 4 * plan.chunk_tiles;
+  const dim3 cgrid((unsigned)(few ? ncomb : (ncomb + 3) / 4)), cblk(256);
+#define FT_CASE(T, DD)                                                                                                  \
+  {                                                                                                                     \
+    if (few) hipLaunchKernelGGL((attn_combine_kernel<T, DD, 1>), cgrid, cblk, 0, s, p, plan.first_shared);              \
+    else hipLaunchKernelGGL((attn_combine_kernel<T, DD, 4>), cgrid, cblk, 0, s, p, plan.first_shared);                  \
+  }
+  if (D == 128 && bf16) FT_CASE(BF16, 128)
+  else if (D == 128) FT_CASE(F16, 128)
+  else if (bf16) FT_CASE(BF16, 64)
+  else FT_CASE(F16, 64)
+#undef FT_CASE
   return hipGetLastError();
 }
 
