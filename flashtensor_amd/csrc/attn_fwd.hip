@@ -68,11 +68,11 @@ hipError_t launch_attn_teams_kf_bf16(const AttnKernelParams& p, int D, int kf, u
 // forms; soft-capped D128 over twelve tiles or more up to
 // two for every CU (H32 S777 28.7 -> 26.0, B2 H32 S500 21.8 -> 23.4), over more than 32 five for two (H16 S2500 89 -> 81, S3000
 // 97 -> 107), D64 up to thirteen for four CUs (H16 S3000 85 -> 66, H32 S1500 47 -> 37, B2 H32 S777 28.6 -> 27.4, S1000 32 -> 36).
-static bool use_teams(const AttnKernelParams& p, int D, bool causal, bool cap, int64_t grid) {
+bool use_teams(int Skv, int D, bool causal, bool cap, int64_t grid) {
   const int forced = attn_form_override();
   if (forced || attn_split_override()) return (forced & 16) != 0;
   const int64_t cus = device_cu_count();
-  const int tiles = (p.Skv + 63) / 64;
+  const int tiles = (Skv + 63) / 64;
   if (tiles <= (cap ? 3 : D == 64 ? 5 : 10)) return false;
   if (grid <= cus) return true;
   if (!causal) return false;
@@ -99,7 +99,7 @@ static bool use_kf_teams(const AttnKernelParams& p, int D, int kf, int64_t grid)
 
 hipError_t launch_attn_fwd(const AttnKernelParams& p, int D, bool bf16, bool causal, bool emu, int kf, hipStream_t s) {
   const int64_t rows = (int64_t)p.Sq * p.group, grid = (rows + 63) / 64 * p.B * (p.H / p.group);
-  if ((kf == kKfNone || kf == kKfSoftcap) && rows < 0x7fffffff - 64 && grid < 0x7fffffff && use_teams(p, D, causal, kf == kKfSoftcap, grid)) {
+  if ((kf == kKfNone || kf == kKfSoftcap) && rows < 0x7fffffff - 64 && grid < 0x7fffffff && use_teams(p.Skv, D, causal, kf == kKfSoftcap, grid)) {
     AttnKernelParams pp = p;
     if (!causal) pp.off = p.Skv;
     // (D = 64: two workgroups per CU; see the kernel)

@@ -11,6 +11,8 @@ namespace ft {
 hipError_t launch_attn_split_f16(const AttnKernelParams& p, int D, bool emu, int kf, unsigned grid, unsigned lds, hipStream_t s);
 hipError_t launch_attn_split_bf16(const AttnKernelParams& p, int D, bool emu, int kf, unsigned grid, unsigned lds, hipStream_t s);
 
+bool use_teams(int Skv, int D, bool causal, bool cap, int64_t grid);  // attn_fwd.hip
+
 namespace {
 
 struct SplitShape {
@@ -21,14 +23,15 @@ struct SplitShape {
   }
 };
 
-// Microseconds by which launches are compared, from timings of this kernel and of the unsplit one at 1 to 48 tiles per
-// workgroup, D = 128 (D = 64 takes 0.6 of a tile's time).  A workgroup takes 7 us for its first loads, its last stores
-// and the launch, then 0.9 per tile where it has its CU to itself and 2.2 where two share one: the second wave of a
-// SIMD hides little of the first one's work (soft-capped logits: 1.9 and 3.5; there it does).  Partial results are
-// written at 10 MB/us and folded at 7, by a kernel that takes 5.5 us to begin with, its launch included; K and V come from HBM at 5.
-// In a launch of more workgroups than fit at once each further one in a slot takes 1 us until its first tile has landed (set
-// from four generation shapes; left out of account, B5 H32 Sq3 Skv3329 soft-capped bf16 became 8480 workgroups of one tile: 126 us against 100 unsplit).
-constexpr double kLaunch = 7.0, kCombine = 5.5, kNext = 1.0, kPartWrite = 10e6, kPartRead = 7e6, kKvBytes = 5e6;
+// Microseconds by which launches are compared, fitted to 8000 calls of random shapes in every form, 1 to 96 shares a block, for
+// the least regret of the choice (and the least error of the time): a launch 5.2, a tile 0.98 where a workgroup has its CU to
+// itself and 1.8 where two share one (soft-capped logits 1.7 and 2.67; D = 64 takes 0.64 of a tile's time; blocks of one wave, whose
+// other waves only load, feel 0.38 of the difference), a step of two teams 1.41 (2.09; D = 64 0.65 of it).  Partial results are
+// written at 8.2 MB/us and folded at 9.6, by a kernel that takes 3.5 us to begin with and 0.9 for every further round of eight
+// shares; K and V come at 6.5.  In a launch of more workgroups than fit at once each further one in a slot takes 0.8 us until
+// its first tile has landed.  The form so chosen was 1.3 % slower than the best one on average (one call in ten 4 %); with
+// the figures of before, which did not know the teams either, 4.8 % (13 %).
+constexpr double kLaunch = 5.2, kCombine = 3.5, kFoldRound = 0.91, kNext = 0.81, kPartWrite = 8.2e6, kPartRead = 9.6e6, kKvBytes = 6.5e6, kMix = 0.186;
 
 // `count` shares of `len` tiles.
 struct ShareRun {
@@ -85,9 +88,10 @@ SplitPlan make_plan(const SplitShape& a) {
     total += tiles[mb];
   }
   const int most = tiles[nMB - 1], part_waves = std::min(4, (rows + 31) / 32);
-  const double size = a.D == 128 ? 1.0 : 0.6, alone = (a.cap ? 1.9 : 0.9) * size, shared_cu = (a.cap ? 3.5 : 2.2) * size;
+  const double size = a.D == 128 ? 1.0 : 0.64, alone = (a.cap ? 1.7 : 0.98) * size;
+  const double shared_cu = alone + ((a.cap ? 2.67 : 1.8) * size - alone) * (part_waves == 1 ? 0.38 : 1.0);
   const double kv_us = pairs * (double)a.Skv * a.D * 4 / kKvBytes;
-  auto launch_us = [&](double work) { return kLaunch + std::max(work, kv_us) + 0.25 * std::min(work, kv_us); };
+  auto launch_us = [&](double work) { return kLaunch + std::max(work, kv_us) + kMix * std::min(work, kv_us); };
   // second: tiles of the workgroup that shares a CU with the longest one, where all of them are resident at once
   auto resident_us = [&](int64_t wgs, int longest, int second) {
     return wgs <= cus ? longest * alone : second * shared_cu + (longest - second) * alone;
@@ -95,11 +99,25 @@ SplitPlan make_plan(const SplitShape& a) {
   // more than that: handed out in order (longest first) to the slots of an XCD as they become free
   const int slots = std::max(1, 2 * cus / 8);
   const int64_t per_xcd = (pairs + 7) / 8;
+  int lanes = 1;  // of a wave's 32 rows that have a share each to fold (combine_rows)
+  while (lanes < std::min(rows, 32)) lanes *= 2;
   // few rows: the column sums come from kept logits (2 bytes a pair each way against K once more and another launch)
   const bool keep = a.stats;
   double best = 1e30;
   int best_chunk = 0;
-  if (!keep) {  // the unsplit form: a workgroup per 128 queries of a head
+  const int64_t teams = (rows + 63) / 64 * pairs;
+  if (!keep && use_teams(a.Skv, a.D, a.causal, a.cap, teams)) {  // undivided: two teams of waves per 64 rows
+    const double step = (a.cap ? 2.09 : 1.41) * (a.D == 128 ? 1.0 : 0.65);
+    int64_t sum = 0;
+    int longest = 0;
+    for (int r = 64; r < rows + 64; r += 64) {
+      longest = ((std::min(a.Skv, (std::min(r, rows) - 1) / a.group + 1 + off) + 63) / 64 + 1) / 2;
+      sum += longest;
+    }
+    // all at once, or as many rounds of the average
+    const int64_t nteams = (rows + 63) / 64, rounds = (teams + cus - 1) / cus;
+    best = launch_us(teams <= (a.D == 128 ? 1 : 2) * cus ? longest * step : std::max((double)longest, (double)sum / nteams * rounds) * step);
+  } else if (!keep) {  // a workgroup per 128 queries of a head
     const int nq = (a.Sq + 127) / 128;
     int64_t sum = 0;
     for (int i = 0; i < nq; ++i) sum += (std::min(a.Skv, std::min(i * 128 + 128, a.Sq) + off) + 63) / 64;
@@ -108,6 +126,7 @@ SplitPlan make_plan(const SplitShape& a) {
     best = launch_us(wgs <= 2 * cus ? resident_us(wgs, most, (int)std::max<int64_t>(0, std::min<int64_t>(most, 2 * sum / nq - most)))
                                     : std::max(most * alone, (double)sum * a.B * a.H * shared_cu / (2.0 * cus) + 0.25 * most * alone));
   }
+  if (nMB > 1) best *= 0.98;  // (a workspace of tens of megabytes and a second launch for less than the figures can tell apart)
   for (int parts = 1; parts <= kSplitMaxItems; ++parts) {
     const int chunk = a.forced > 0 ? a.forced : (most + parts - 1) / parts;
     if (parts > 1 && chunk == (most + parts - 2) / (parts - 1) && !a.forced) continue;
@@ -128,7 +147,8 @@ SplitPlan make_plan(const SplitShape& a) {
     }
     if (items > kSplitMaxItems) break;
     const int64_t wgs = items * pairs;
-    const double fold = shared ? kCombine + (double)shared * pairs * std::min(rows, 128) * a.D * 4 * (1 / kPartWrite + 1 / kPartRead) : 0;
+    const int rounds = (((most + chunk - 1) / chunk + 7) / 8 * lanes + 31) / 32;
+    const double fold = shared ? kCombine + kFoldRound * (rounds - 1) + (double)shared * pairs * std::min(rows, 128) * a.D * 4 * (1 / kPartWrite + 1 / kPartRead) : 0;
     // The search ends where no further cut can win: smaller shares mean more of them, so the folding, and in a launch of
     // several rounds the least that the slots' work adds up to, only grow.
     const double least = wgs > 2 * cus ? (total * shared_cu + items * kNext) * per_xcd / slots : 0;
