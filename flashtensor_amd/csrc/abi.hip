@@ -301,15 +301,22 @@ int run_colstats(const FtAttnArgs* a, float* colsum, float* colsumsq, int pool, 
   }
   hipError_t e = run_attn(a, p, ft::kKfNone, ws, used, ws_bytes, stream);
   if (e != hipSuccess) return hip_fail(e, "attn_fwd launch");
+  // SnapKV's window over the sums inside the column pass, whose workgroups then overlap by the window (a sixteenth at most), where
+  // that costs less than a launch of its own (4.2 us; the pass takes 90 us for 2^28 pairs)
+  const double work = (double)a->B * a->H * a->Sq * (a->Skv - (causal ? (a->Sq - 1) * 0.5 : 0));
+  const bool windows = pool && pool <= 5 && work * (pool - 1) / 64 * (90.0 / (1 << 28)) < 4.0;
+  if (windows && group == 1) per_head = colsum;
   ft::ColstatsKernelParams c = col_params(a, emu, lse, per_head, colsumsq);
-  e = ft::launch_colstats(c, a->D, a->dtype == FT_BF16, causal, emu, colsumsq ? ft::kStatSumSq : ft::kStatSum,
+  c.pool = windows ? pool / 2 : 0;
+  e = ft::launch_colstats(c, a->D, a->dtype == FT_BF16, causal, emu,
+                          colsumsq ? ft::kStatSumSq : windows ? ft::kStatSumPool : ft::kStatSum,
                           (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(e, "colstats launch");
   if (group > 1) {
-    e = ft::launch_group_mean(per_head, (int64_t)a->B * a->Hkv, group, a->Skv, sums, (hipStream_t)stream);
+    e = ft::launch_group_mean(per_head, (int64_t)a->B * a->Hkv, group, a->Skv, windows ? colsum : sums, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "group mean launch");
   }
-  if (pool) {
+  if (pool && !windows) {
     e = ft::launch_avgpool1d(raw, (int64_t)a->B * (a->H / group), a->Skv, pool, colsum, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "avgpool1d launch");
   }

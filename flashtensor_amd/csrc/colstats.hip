@@ -22,7 +22,7 @@ static hipError_t launch_td(const ColstatsKernelParams& p, bool causal, bool emu
 #define FT_CASE(C, E, M) \
   if (causal == C && emu == E && mode == M) return launch_colstats_one<T, D, C, E, M, 2>(p, s);
 #define FT_MODES(C, E)                                                                                       \
-  FT_CASE(C, E, kStatSum) FT_CASE(C, E, kStatSumSq) FT_CASE(C, E, kStatKfTensor) FT_CASE(C, E, kStatKfSeeded) \
+  FT_CASE(C, E, kStatSum) FT_CASE(C, E, kStatSumPool) FT_CASE(C, E, kStatSumSq) FT_CASE(C, E, kStatKfTensor) FT_CASE(C, E, kStatKfSeeded) \
   FT_CASE(C, E, kStatCormRule) FT_CASE(C, E, kStatCormTensor)
   FT_MODES(true, true) FT_MODES(true, false) FT_MODES(false, true) FT_MODES(false, false)
   if constexpr (std::is_same<T, F16>::value) {  // packed KeyFormer modes: fp16 with reference rounding only

@@ -7,6 +7,9 @@
 // normaliser written by the attention pass.  No S x S tensor is written or read (KeyFormer's tensor mode
 // reads the noise input once more, as the reference's definition requires).
 //
+// SnapKV's window over the sums (narrow ones, in calls of up to a few 2^28 pairs) is taken here as well: workgroups overlap by the
+// window, which costs BK / (BK - width) of the pass against 4.2 us for a launch of its own (B1 H32 Sq64 Skv8000 58.3 -> 55.1 us, B2 H8/2 S1040 36.4 -> 33.8).
+//
 // Mapping.  Key-stationary: one workgroup owns 128 key columns of one (b, h), 4 waves x 32 keys, holds
 // their K fragment in registers as the MFMA B operand and streams 64-row Q tiles through double-buffered
 // LDS.  S = Q K^T as 16x16 blocks (v_mfma_f32_16x16x32: the same rate as the 32x32x16 shape for a quarter of
@@ -41,7 +44,7 @@ constexpr int kColThreads = 256;
 // (packed rounding, or logits kept in fp32) fit three
 template <typename T, bool CAUSAL, bool EMU, int MODE>
 constexpr int colstats_waves_per_simd() {
-  return (MODE == kStatSum || MODE == kStatSumSq) ? 3 : 2;
+  return (MODE == kStatSum || MODE == kStatSumPool || MODE == kStatSumSq) ? 3 : 2;
 }
 
 template <typename T, int D, bool CAUSAL, bool EMU, int MODE, int NKEYS = 2, int TEAMS = 1>
@@ -59,6 +62,7 @@ __global__ void __launch_bounds__(kColThreads * TEAMS, (TEAMS == 1 ? colstats_wa
   constexpr bool CORM = (MODE == kStatCormRule || MODE == kStatCormTensor);
   constexpr bool kPacked = __is_same(typename T::elem, _Float16) && EMU;  // packed-fp16 rounding chain
   constexpr bool kPlainF32 = !EMU;                                        // logits stay in fp32: one fma per element
+  constexpr bool kPool = MODE == kStatSumPool;                            // the sums' window means
   constexpr bool kTensor = MODE == kStatKfTensor || MODE == kStatCormTensor;
   constexpr bool k16 = !kTensor;            // 16x16x32 blocks; the tensor modes stay on 32x32x16
   static_assert(k16 || NKEYS == 2, "32 keys per wave");
@@ -73,6 +77,7 @@ __global__ void __launch_bounds__(kColThreads * TEAMS, (TEAMS == 1 ? colstats_wa
   __shared__ __align__(16) float s_lse[TEAMS * 2 * BQ];     // row normalisers of the current / next tile
   __shared__ __align__(16) uint32_t s_row[TEAMS * 2 * BQ];  // noise row terms (seeded KeyFormer)
   __shared__ float s_fold[TEAMS > 1 ? 2 * BK : 1];          // the second team's results
+  __shared__ float s_pool[kPool ? BK : 1];                  // the workgroup's sums, for the windows over them
 
   const int BH = p.B * p.H;
   // Low key blocks see the most rows under the causal mask: heaviest first, every (b, h) pair's block 0 before any
@@ -89,7 +94,9 @@ __global__ void __launch_bounds__(kColThreads * TEAMS, (TEAMS == 1 ? colstats_wa
     jb = jb < half ? jb : nJB - 1 - (jb - half);
   }
   const int b = bh / p.H, h = bh % p.H;
-  const int j0 = jb * BK;
+  // with windows over the sums the workgroup's outer keys are its neighbours' as well
+  const int half = kPool ? p.pool : 0;
+  const int j0 = jb * (BK - 2 * half) - half;
   const int lane = lane_id(), wave = wave_id() & 3;
   const int team = TEAMS > 1 ? wave_id() >> 2 : 0, tid = TEAMS > 1 ? threadIdx.x & (NT - 1) : threadIdx.x;
   char* const ldsQ0 = s_q0 + team * TILE_BYTES;
@@ -104,7 +111,7 @@ __global__ void __launch_bounds__(kColThreads * TEAMS, (TEAMS == 1 ? colstats_wa
 #pragma unroll
   for (int key = 0; key < NKEY; ++key) {
     kjs[key] = j0 + wave * WK + (k16 ? 16 * key + n16 : n);
-    kjs_c[key] = kjs[key] < p.Skv ? kjs[key] : p.Skv - 1;
+    kjs_c[key] = kPool ? min(max(kjs[key], 0), p.Skv - 1) : kjs[key] < p.Skv ? kjs[key] : p.Skv - 1;
   }
   const int kj_c = kjs_c[0];
   const float POS_INF = __builtin_inff();
@@ -585,10 +592,10 @@ __global__ void __launch_bounds__(kColThreads * TEAMS, (TEAMS == 1 ? colstats_wa
   }
   if (TEAMS > 1) {
     __syncthreads();
-    if (team == 1) return;
+    if (team == 1 && !kPool) return;
   }
 #pragma unroll
-  for (int key = 0; key < NKEY; ++key) {
+  for (int key = 0; key < NKEY && team == 0; ++key) {
     float tot = tots[key], totsq = totsqs[key], top = tops[key];
     if (TEAMS > 1 && writer) {
       const float other = s_fold[kjs[key] - j0];
@@ -596,7 +603,9 @@ __global__ void __launch_bounds__(kColThreads * TEAMS, (TEAMS == 1 ? colstats_wa
       top = fmaxf(top, other);
       if (MODE == kStatSumSq) totsq += s_fold[BK + kjs[key] - j0];
     }
-    if (writer && kjs[key] < p.Skv) {
+    if (kPool) {
+      if (writer) s_pool[kjs[key] - j0] = kjs[key] >= 0 && kjs[key] < p.Skv ? tot : 0.f;
+    } else if (writer && kjs[key] < p.Skv) {
       const int64_t idx = (int64_t)bh * p.Skv + kjs[key];
       if (CORM) {
         p.keep[idx] = top >= (MODE == kStatCormRule ? -kCormSlack * kLog2e : 0.f) ? 1 : 0;
@@ -607,6 +616,16 @@ __global__ void __launch_bounds__(kColThreads * TEAMS, (TEAMS == 1 ? colstats_wa
       }
     }
   }
+  if (kPool) {
+    // stride-1 means with zero padding, divided by the whole width
+    __syncthreads();
+    const int k = threadIdx.x, j = j0 + k;
+    if (k >= half && k < BK - half && j < p.Skv) {
+      float s = 0.f;
+      for (int u = -half; u <= half; ++u) s += s_pool[k + u];
+      p.colsum[(int64_t)bh * p.Skv + j] = s / (float)(2 * half + 1);
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -615,7 +634,7 @@ int device_cu_count();  // attn_fwd.hip
 
 template <typename T, int D, bool CAUSAL, bool EMU, int MODE, int NKEYS, int TEAMS = 1>
 hipError_t launch_colstats_one(const ColstatsKernelParams& p, hipStream_t stream) {
-  const int nJB = (p.Skv + 64 * NKEYS - 1) / (64 * NKEYS);
+  const int step = 64 * NKEYS - (MODE == kStatSumPool ? 2 * p.pool : 0), nJB = (p.Skv + step - 1) / step;
   dim3 grid((unsigned)(nJB * p.B * p.H));
   ColstatsKernelParams pp = p;
   const int64_t cus = device_cu_count();

@@ -7,7 +7,7 @@ template <typename T, int D>
 static hipError_t launch_narrow_td(const ColstatsKernelParams& p, bool causal, int mode, hipStream_t s) {
 #define FT_CASE(M) \
   if (mode == M) return causal ? launch_colstats_one<T, D, true, true, M, 1>(p, s) : launch_colstats_one<T, D, false, true, M, 1>(p, s);
-  FT_CASE(kStatSum) FT_CASE(kStatSumSq) FT_CASE(kStatKfSeeded) FT_CASE(kStatCormRule)
+  FT_CASE(kStatSum) FT_CASE(kStatSumPool) FT_CASE(kStatSumSq) FT_CASE(kStatKfSeeded) FT_CASE(kStatCormRule)
   if constexpr (std::is_same<T, F16>::value) {
     FT_CASE(kStatKfSeededTau1) FT_CASE(kStatKfSeededFast)
   }

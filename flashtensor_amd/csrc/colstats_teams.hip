@@ -8,7 +8,7 @@ template <typename T, int D>
 static hipError_t launch_teams_td(const ColstatsKernelParams& p, bool causal, int mode, hipStream_t s) {
 #define FT_CASE(M) \
   if (mode == M) return causal ? launch_colstats_one<T, D, true, true, M, 1, 2>(p, s) : launch_colstats_one<T, D, false, true, M, 1, 2>(p, s);
-  FT_CASE(kStatSum) FT_CASE(kStatSumSq) FT_CASE(kStatKfSeeded) FT_CASE(kStatCormRule)
+  FT_CASE(kStatSum) FT_CASE(kStatSumPool) FT_CASE(kStatSumSq) FT_CASE(kStatKfSeeded) FT_CASE(kStatCormRule)
 #undef FT_CASE
 #define FT_CASE(M) \
   if (mode == M) return causal ? launch_colstats_one<T, D, true, true, M, 2, 2>(p, s) : launch_colstats_one<T, D, false, true, M, 2, 2>(p, s);

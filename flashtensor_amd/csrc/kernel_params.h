@@ -85,6 +85,7 @@ struct ColstatsKernelParams {
   uint32_t pk_hi2, pk_lo2;  // as in AttnKernelParams
   float inv_tau;
   int group;  // query heads per k head
+  int pool;        // kStatSumPool: half the odd width of SnapKV's window over the sums, whose means go to colsum
   int pair_order;  // key-block order for launches of two workgroups per CU: heavy half descending, light half ascending (launcher)
 };
 
@@ -99,7 +100,8 @@ enum KfMode { kKfNone = 0, kKfTensor = 1, kKfSeeded = 2, kKfSoftcap = 3, kKfSeed
 // kStatCormRule: thresholds 1 / (i + 1) per query row i; kStatCormTensor: thresholds read from a tensor
 enum StatMode {
   kStatSum = 0, kStatSumSq = 1, kStatKfTensor = 2, kStatKfSeeded = 3, kStatCormRule = 4, kStatCormTensor = 5,
-  kStatKfSeededTau1 = 6, kStatKfSeededFast = 7  // seeded KeyFormer inside the packed fp16 path (see KfMode)
+  kStatKfSeededTau1 = 6, kStatKfSeededFast = 7, // seeded KeyFormer inside the packed fp16 path (see KfMode)
+  kStatSumPool = 8                              // kStatSum and SnapKV's window over the sums
 };
 
 }  // namespace ft
