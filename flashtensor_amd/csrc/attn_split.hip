@@ -266,18 +266,18 @@ __device__ __forceinline__ void fold_shares(const AttnKernelParams& p, int D, in
 
 // A wave takes Q of the four pieces of (32 rows of a shared block, 32 channels); every load is up to 1 KB contiguous, in the
 // accumulators' own register layout.  Bound by the latency of its loads, over many rows by their bytes.
-// Q = 1: up to 16 rows (a generation step's) the lanes that have no row take every SUB-th share of the others' and meet by lane
-// exchanges, so that eighty shares of four rows are one round of loads and not ten (whole calls: B1 H16/4 Sq1 Skv5195 16.6 -> 10.6
-// us, H32/8 Sq1 Skv4000 15.4 -> 11.7, soft-capped B2 H16/4 Sq1 Skv3058 18.6 -> 13.0); eight shares or fewer are one round anyway.
-// Q = 4: whole waves of rows with up to four shares, a quarter of the waves with four times the loads in flight (B1 H32/8 Sq501
-// Skv5760 8.7 -> 6.5 us; sixteen shares, Sq172 Skv4918, 5.1 -> 8.0).
-template <typename T, int D, int Q>
+// FEW (up to kSplitStatRows rows): up to 16 rows (a generation step's) the lanes that have no row take every SUB-th share of the
+// others' and meet by lane exchanges, so that eighty shares of four rows are one round of loads and not ten (whole calls: B1 H16/4 Sq1
+// Skv5195 16.6 -> 10.6 us, H32/8 Sq1 Skv4000 15.4 -> 11.7, soft-capped B2 H16/4 Sq1 Skv3058 18.6 -> 13.0); eight shares or fewer
+// are one round anyway.
+// More rows: Q = 2, four shares a round, or Q = 1, eight a round (as it was before); launch_attn_split says which.
+template <typename T, int D, int Q, bool FEW>
 __device__ __forceinline__ void combine_rows(const AttnKernelParams& p, int first_shared, int unit) {
   constexpr int DB = D / 32;
   const int rows = p.Sq * p.group, Hkv = p.H / p.group;
   const int nshared = (rows + 127) / 128 - first_shared;
-  const int q0 = Q == 1 ? unit % 4 : 0;
-  int i = Q == 1 ? unit / 4 : unit;
+  const int q0 = unit % (4 / Q) * Q;
+  int i = unit / (4 / Q);
   const int db = i % DB;
   i /= DB;
   const int wv = i % p.part_waves;
@@ -286,7 +286,7 @@ __device__ __forceinline__ void combine_rows(const AttnKernelParams& p, int firs
   if (bh >= p.B * Hkv) return;
   const int lane = lane_id(), g = lane >> 5;
   int n = lane & 31, sub = 0, rp = 32;  // row in the wave; which shares
-  if (Q == 1) {
+  if (FEW) {
     rp = 1;
     while (rp < 32 && (rp < rows || 32 / rp >= 2 * ((shares_of_block(p, mb) + 7) / 8))) rp *= 2;
     sub = n / rp;
@@ -297,9 +297,9 @@ __device__ __forceinline__ void combine_rows(const AttnKernelParams& p, int firs
   const int nch = shares_of_block(p, mb), rc = min(row, rows - 1) - (row - n);  // (lanes without a row repeat the last one)
   float M, L;
   float4v acc[Q];
-  fold_shares<Q == 4 ? 4 : 8, Q>(p, D, slot0 + (int64_t)sub * p.part_waves, max(rc, 0), (nch - sub + slots - 1) / slots, slots, M, L, acc,
+  fold_shares<8 / Q, Q>(p, D, slot0 + (int64_t)sub * p.part_waves, max(rc, 0), (nch - sub + slots - 1) / slots, slots, M, L, acc,
                                  [&](const SplitPartial& s, int q) { return *reinterpret_cast<const float4v*>(s.o + ((db * 4 + q0 + q) * 64 + g * 32 + max(rc, 0)) * 4); });
-  if (Q == 1) {
+  if (FEW) {
     for (int d = rp; d < 32; d *= 2) {
       const float M2 = __shfl_xor(M, d), L2 = __shfl_xor(L, d), M1 = fmaxf(M, M2);
       const float w = __builtin_amdgcn_exp2f(M - M1), w2 = __builtin_amdgcn_exp2f(M2 - M1);
@@ -319,9 +319,9 @@ __device__ __forceinline__ void combine_rows(const AttnKernelParams& p, int firs
   if (db == 0 && q0 == 0 && g == 0 && p.lse) p.lse[((int64_t)b * p.H + h) * p.Sq + qi] = M + __builtin_amdgcn_logf(L);
 }
 
-template <typename T, int D, int Q>
+template <typename T, int D, int Q, bool FEW>
 __global__ void __launch_bounds__(256) attn_combine_kernel(const AttnKernelParams p, int first_shared) {
-  combine_rows<T, D, Q>(p, first_shared, blockIdx.x * 4 + wave_id());
+  combine_rows<T, D, Q, FEW>(p, first_shared, blockIdx.x * 4 + wave_id());
 }
 
 // The column sums of few rows from their kept logits, and (the last `gridDim.x - ncol` workgroups) the folding of the
@@ -335,7 +335,7 @@ __host__ __device__ constexpr int stat_step(int pool) { return pool ? kStatTiles
 template <typename T, int D, bool SQ>
 __global__ void __launch_bounds__(256) split_stats_kernel(const AttnKernelParams p, const SplitStats st, int ncol) {
   if ((int)blockIdx.x >= ncol) {
-    combine_rows<T, D, 1>(p, 0, (blockIdx.x - ncol) * 4 + wave_id());
+    combine_rows<T, D, 1, true>(p, 0, (blockIdx.x - ncol) * 4 + wave_id());
     return;
   }
   constexpr int KT = kStatTiles * kAttnBN;
@@ -484,15 +484,19 @@ hipError_t launch_attn_split(const AttnKernelParams& p0, const SplitPlan& plan, 
 #undef FT_CASE
     return hipGetLastError();
   }
-  // whole waves of rows and no more than four shares of a block (up to kSplitStatRows rows: as in the fold beside the column sums)
+  // Up to kSplitStatRows rows: as in the fold beside the column sums, whose rows are the same bit for bit.  More of them, up to five
+  // shares of a block: two pieces a wave, four shares a round (B1 H32/8 Sq501 Skv5760, four shares, 7.9 -> 6.2 us; two pieces with
+  // eight a round 7.1, four pieces 6.5; soft-capped Sq777 Skv3000, five shares, 12.5 -> 12.3; six to eight shares 4.35..4.9 against
+  // 4.28..5.1, sixteen 4.7 against 5.4, thirty-one 5.8 against 7.7).
   const int64_t rows = (int64_t)p.Sq * p.group;
   const int most = (std::min<int64_t>(p.Skv, (rows - 1) / p.group + 1 + p.off) + kAttnBN - 1) / kAttnBN;
-  const bool few = rows <= kSplitStatRows || most > 4 * plan.chunk_tiles;
-  const dim3 cgrid((unsigned)(few ? ncomb : (ncomb + 3) / 4)), cblk(256);
-#define FT_CASE(T, DD)                                                                                                  \
-  {                                                                                                                     \
-    if (few) hipLaunchKernelGGL((attn_combine_kernel<T, DD, 1>), cgrid, cblk, 0, s, p, plan.first_shared);              \
-    else hipLaunchKernelGGL((attn_combine_kernel<T, DD, 4>), cgrid, cblk, 0, s, p, plan.first_shared);                  \
+  const bool few = rows <= kSplitStatRows, two = !few && most <= 5 * plan.chunk_tiles;
+  const dim3 cgrid((unsigned)(two ? (ncomb + 1) / 2 : ncomb)), cblk(256);
+#define FT_CASE(T, DD)                                                                                                       \
+  {                                                                                                                          \
+    if (few) hipLaunchKernelGGL((attn_combine_kernel<T, DD, 1, true>), cgrid, cblk, 0, s, p, plan.first_shared);             \
+    else if (two) hipLaunchKernelGGL((attn_combine_kernel<T, DD, 2, false>), cgrid, cblk, 0, s, p, plan.first_shared);       \
+    else hipLaunchKernelGGL((attn_combine_kernel<T, DD, 1, false>), cgrid, cblk, 0, s, p, plan.first_shared);                \
   }
   if (D == 128 && bf16) FT_CASE(BF16, 128)
   else if (D == 128) FT_CASE(F16, 128)
