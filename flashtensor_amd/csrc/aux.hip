@@ -130,7 +130,7 @@ __global__ void __launch_bounds__(NT) topk_kernel(const float* __restrict__ scor
 // key i of one and key 64 E - 1 - i of the other, a bitonic sequence, and one merge pass), log2 NW levels through LDS with
 // two barriers each, half of the waves dropping out at every level.  The network over the whole row has two barriers for
 // every step across waves and works on all keys to the end (k = S / 8 of 32 rows, per call: S = 512 7.5 -> 4.6 us, 1024
-// 7.3 -> 4.9, 2048 9.8 -> 8.4, 4096 19.1 -> 16.3, 8192 38.9 -> 34.9: bound by the chain of compare-exchanges of one CU).
+// 7.3 -> 4.9: bound by the chain of compare-exchanges of one CU, which is why longer rows go to topk_select_kernel).
 template <int E, int NW>
 __global__ void __launch_bounds__(64 * NW) topk_runs_kernel(const float* __restrict__ score, int S, int k, int64_t* __restrict__ idx) {
   constexpr int R = 64 * E;
@@ -170,117 +170,199 @@ __global__ void __launch_bounds__(64 * NW) topk_runs_kernel(const float* __restr
   }
 }
 
-// Rows longer than the register sort holds (S > 8192), k <= kTopkSelectMax: one workgroup per row
-//   1. radix select over the 32-bit order keys, most significant byte first (four passes over the row, a 256-bin
-//      histogram in LDS each): the key T of the k-th entry and the number of entries that sort before it;
-//   2. one more pass gathers the winners into LDS as the 64-bit (order key, index) words of the register sort: every
-//      entry before T, and of the entries equal to T the ones with the smallest indices (a workgroup-wide prefix count
-//      in index order), as the full sort would have ranked them;
-//   3. a bitonic network over those <= 16384 words in LDS, and the indices go out in rank order.
-// The same answers as the register sort, ties and NaNs included (a NaN of positive sign has the largest order key and
-// sorts first, as in torch.topk).
-constexpr int kTopkSelectMax = 16384;  // 128 KB of LDS for the winners: k = S / 8 up to S = 131072
-constexpr int kTopkSelectThreads = 1024;
+// The k first entries of a row by selection, then a sort of those alone: one workgroup per row, whose (score, index) words it
+// holds in registers, E per thread (E = 0: reads the row again in every pass, in its own order).
+//   1. The word of rank k, by its digits from the top, 11 bits at a time: a histogram in LDS of the entries that have the
+//      digits found so far, a prefix sum over its bins, and the bin in which rank k lies.  It ends as soon as that bin is wanted
+//      whole, after two or three passes for distinct scores; ties go on into the index, whose smallest values make the cut.
+//   2. The entries up to that word go to LDS in any order, and a bitonic network over NT W >= k keys ranks them.
+// The same answers as the register sort, ties and NaNs included (a NaN of positive sign has the largest order key and sorts
+// first, as in torch.topk).
+// Bound by latency: some ten barriers, the counting (64 lanes that hit one bin take 64 turns) and the sort's chain.  k = S / 8 of 32
+// rows, per call, scores with and without noise, against sorted runs and (S > 8192) a selection by bytes whose bins one thread
+// walked: S = 2048 8.3 -> 6.7, 4096 16.3 -> 8.9, 8192 34.9 -> 14, 16384 75..89 -> 25, 65536 212..251 -> 86..95.  Scores in
+// their own order instead of 0.618 of the row apart: falling ones 8.7, 11.6, 19.3.  First the leading bits that all keys share, to
+// begin below them, saved less than that extra barrier.
+__device__ __forceinline__ uint32_t wave_prefix_sum(uint32_t v) {
+  int x = (int)v;
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, true);   // row_shr:1, 2, 4, 8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, true);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);  // the last lane of a row to the next one: rows 1 and 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);  // lane 31 to the upper half
+  return (uint32_t)x;
+}
 
-__global__ void __launch_bounds__(kTopkSelectThreads) topk_select_kernel(const float* __restrict__ score, int S, int k,
-                                                                         int64_t* __restrict__ idx) {
-  constexpr int NT = kTopkSelectThreads, NW = NT / 64;
-  __shared__ uint64_t win[kTopkSelectMax];
-  __shared__ uint32_t hist[256];
-  __shared__ uint32_t wave_cnt[NW];
-  __shared__ uint32_t s_prefix, s_before, s_slot;
+constexpr int kTopkSelectMax = 16384;  // 128 KB of LDS for the winners: k = S / 8 up to S = 131072
+
+template <int NT, int E, int W>
+__global__ void __launch_bounds__(NT) topk_select_kernel(const float* __restrict__ score, int S, int k, int64_t* __restrict__ idx) {
+  constexpr int NW = NT / 64, kBins = 2048, kPer = kBins / NT, kAhead = E ? E : 8, kN = NT * kAhead;
+  __shared__ uint64_t win[E > 2 * W ? NT * E / 2 : NT * W];
+  __shared__ __align__(16) uint32_t hist[kBins];
+  __shared__ uint32_t wave_sum[NW];
+  __shared__ uint32_t s_digit, s_before, s_count, s_slot;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const float* row = score + (int64_t)blockIdx.x * S;
-
-  // ---- 1. the order key of rank k
-  uint32_t prefix = 0, before = 0;  // high bytes fixed so far; entries whose key is below every key with this prefix
-#pragma unroll 1
-  for (int shift = 24; shift >= 0; shift -= 8) {
-    if (t < 256) hist[t] = 0;
+  uint32_t key[kAhead];
+  auto load = [&](uint32_t i0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int e = 0; e < kAhead; ++e) key[e] = float_order_desc(row[min(i0 + e * NT + t, S - 1u)]);
+  };
+  // E > 0: neighbouring scores are often alike, and 64 lanes that count in one bin wait for each other: the lanes of a wave
+  // take entries 0.618 of the row apart (an odd step: each one once, no two lanes in a bank).
+  constexpr uint32_t kStep = (uint32_t)(kN * 0.618) | 1;
+  auto index = [&](uint32_t i0, int e) __attribute__((always_inline)) { return E ? (e * NT + t) * kStep % kN : i0 + e * NT + t; };
+  if (E) {
+    load(0);
+    uint32_t* all = reinterpret_cast<uint32_t*>(win);
+#pragma unroll
+    for (int e = 0; e < kAhead; ++e) all[e * NT + t] = key[e];
     __syncthreads();
-    const uint32_t mask = shift == 24 ? 0u : ~0u << (shift + 8);
-    for (int i = t; i < S; i += NT) {
-      const uint32_t h = float_order_desc(row[i]);
-      if ((h & mask) == prefix) atomicAdd(&hist[(h >> shift) & 255u], 1u);
-    }
-    __syncthreads();
-    if (t == 0) {
-      uint32_t cum = before, d = 0;
-      for (; d < 255; ++d) {
-        if (cum + hist[d] >= (uint32_t)k) break;
-        cum += hist[d];
-      }
-      s_prefix = prefix | (d << shift);
-      s_before = cum;
-    }
-    __syncthreads();
-    prefix = s_prefix;
-    before = s_before;
+#pragma unroll
+    for (int e = 0; e < kAhead; ++e) key[e] = all[index(0, e)];
   }
-  const uint32_t T = prefix;
-  const uint32_t need_eq = (uint32_t)k - before;  // entries equal to T that make the cut: those of smallest index
-
-  // ---- 2. gather
+#pragma unroll
+  for (int b = 0; b < kPer; ++b) hist[t * kPer + b] = 0;
   if (t == 0) s_slot = 0;
   __syncthreads();
-  uint32_t eq_seen = 0;  // entries equal to T in the tiles before this one (the same in every thread)
-#pragma unroll 1
-  for (int i0 = 0; i0 < S; i0 += NT) {
-    const int i = i0 + t;
-    const uint32_t h = i < S ? float_order_desc(row[i]) : ~0u;
-    const bool lt = i < S && h < T, eq = i < S && h == T;
-    const uint64_t bal = __ballot(eq);
-    if (lane == 0) wave_cnt[wave] = (uint32_t)__popcll(bal);
-    __syncthreads();
-    uint32_t rank = eq_seen + (uint32_t)__popcll(bal & ((1ull << lane) - 1ull)), tile_eq = 0;
+
+  // ---- 1. the word of rank k
+  int ks = 32;  // bits of the key that are open still, and of the index
+  int is = S <= 1 << 21 ? 21 : 32;
+  uint32_t T = 0, I = 0;        // the others
+  uint32_t want = (uint32_t)k;  // rank among the entries that have these
+  while (true) {
+    const bool by_key = ks > 0;
+    const int bits = by_key ? min(11, ks) : is == 10 ? 10 : 11, next = (by_key ? ks : is) - bits;
+    const uint32_t mask = (1u << bits) - 1;
+    for (int64_t i0 = 0; i0 < S; i0 += kAhead * NT) {
+      if (!E) load((uint32_t)i0);
 #pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      if (w < wave) rank += wave_cnt[w];
-      tile_eq += wave_cnt[w];
-    }
-    if (lt || (eq && rank < need_eq)) win[atomicAdd(&s_slot, 1u)] = ((uint64_t)h << 32) | (uint32_t)i;
-    eq_seen += tile_eq;
-    __syncthreads();
-  }
-  // ---- 3. sort the k winners (padding sorts last)
-  int n2 = 2;
-  while (n2 < k) n2 <<= 1;
-  for (int i = k + t; i < n2; i += NT) win[i] = ~0ull;
-  __syncthreads();
-#pragma unroll 1
-  for (int size = 2; size <= n2; size <<= 1)
-#pragma unroll 1
-    for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      for (int p = t; p < (n2 >> 1); p += NT) {
-        const int lo = ((p & ~(stride - 1)) << 1) | (p & (stride - 1)), hi = lo | stride;
-        const bool up = (lo & size) == 0;
-        const uint64_t a = win[lo], b = win[hi];
-        if ((a > b) == up) {
-          win[lo] = b;
-          win[hi] = a;
+      for (int e = 0; e < kAhead; ++e) {
+        const uint32_t i = index((uint32_t)i0, e);
+        const bool open = by_key ? ks == 32 || key[e] >> ks == T : key[e] == T && (is == 32 || i >> is == I);
+        const bool on = open && i < (uint32_t)S;
+        const uint32_t digit = (by_key ? key[e] : i) >> next & mask;
+        if (E == 0) {  // the wave's first digit at once, the others one by one (k = S / 8, falling scores: 16384 32.5 -> 24.6 us)
+          const uint64_t m = __ballot(on);
+          if (m == 0) continue;
+          const int lead = __builtin_ctzll(m);
+          const uint32_t d0 = __builtin_amdgcn_readlane(digit, lead);
+          const uint64_t same = __ballot(on && digit == d0);
+          if (lane == lead) atomicAdd(&hist[d0], (uint32_t)__popcll(same));
+          if (on && digit != d0) atomicAdd(&hist[digit], 1u);
+        } else if (on) {
+          atomicAdd(&hist[digit], 1u);
         }
       }
-      __syncthreads();
     }
+    __syncthreads();
+    uint32_t h[kPer], sum = 0;
+#pragma unroll
+    for (int b = 0; b < kPer; ++b) {
+      h[b] = hist[t * kPer + b];
+      hist[t * kPer + b] = 0;
+      sum += h[b];
+    }
+    const uint32_t upto = wave_prefix_sum(sum);
+    if (lane == 63) wave_sum[wave] = upto;
+    __syncthreads();
+    uint32_t cum = upto - sum;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) cum += w < wave ? wave_sum[w] : 0;
+    if (cum < want && want <= cum + sum) {
+#pragma unroll
+      for (int b = 0; b < kPer; ++b) {
+        if (cum < want && want <= cum + h[b]) {
+          s_digit = t * kPer + b;
+          s_before = cum;
+          s_count = h[b];
+        }
+        cum += h[b];
+      }
+    }
+    __syncthreads();
+    want -= s_before;
+    if (by_key) {
+      T = T << bits | s_digit;
+      ks = next;
+    } else {
+      I = I << bits | s_digit;
+      is = next;
+    }
+    if (s_count == want || is == 0) break;  // (at the index's last digit the count is 1)
+  }
+
+  // ---- 2. the winners, and their order
+  if (ks > 0 || is == (S <= 1 << 21 ? 21 : 32)) {  // (the key decided)
+    is = 0;
+    I = ~0u;
+  }
+  for (int64_t i0 = 0; i0 < S; i0 += kAhead * NT) {
+    if (!E) load((uint32_t)i0);
+    uint64_t in[kAhead];
+    uint32_t total = 0, slot = 0;
+#pragma unroll
+    for (int e = 0; e < kAhead; ++e) {
+      const uint32_t i = index((uint32_t)i0, e), top = key[e] >> ks;
+      in[e] = __ballot(i < (uint32_t)S && (top < T || (top == T && i >> is <= I)));
+      total += (uint32_t)__popcll(in[e]);
+    }
+    if (lane == 0 && total) slot = atomicAdd(&s_slot, total);
+    slot = __builtin_amdgcn_readfirstlane(slot);
+#pragma unroll
+    for (int e = 0; e < kAhead; ++e) {
+      if (in[e] >> lane & 1) win[slot + (uint32_t)__popcll(in[e] & ((1ull << lane) - 1ull))] = (uint64_t)key[e] << 32 | index((uint32_t)i0, e);
+      slot += (uint32_t)__popcll(in[e]);
+    }
+  }
+  for (int i = k + t; i < NT * W; i += NT) win[i] = ~0ull;  // padding sorts last
+  __syncthreads();
+  uint64_t best[W];
+#pragma unroll
+  for (int e = 0; e < W; ++e) best[e] = win[e * NT + t];  // (the slots that this thread's keys take in the network's exchanges)
+  bitonic_sort<W, NT, 2>(best, win, t);
   int64_t* out = idx + (int64_t)blockIdx.x * k;
-  for (int i = t; i < k; i += NT) out[i] = (int64_t)(uint32_t)win[i];
+#pragma unroll
+  for (int e = 0; e < W; ++e) {
+    const int i = t * W + e;
+    if (i < k) out[i] = (int64_t)(uint32_t)best[e];
+  }
 }
 
 hipError_t launch_topk(const float* score, int64_t rows, int S, int k, int64_t* idx, hipStream_t s) {
   const dim3 grid((unsigned)rows);
-  if (S > 8192) {
-    if (k > kTopkSelectMax) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(topk_select_kernel, grid, dim3(kTopkSelectThreads), 0, s, score, S, k, idx);
-    return hipGetLastError();
-  }
-  // eight runs (sixteen of half the length where k allows it and the row is long)
+  // Runs where they are two barriers a level and little else (k = S / 8 of 32 rows, S = 1024: 4.8 us, selection 5.7).  Selection with
+  // S / 8 threads above (figures at the kernel).  The network over the whole row where most of it is wanted (k = 3 S / 4: 2048 9.8,
+  // 4096 20, 8192 40; selection at k = S / 2 takes 10.4..11, 15 and 26, so it has S <= 2048 up to a quarter only), or it is short.
 #define FT_RUNS(MAX_S, E, NW)                                                                                    \
   if (S <= MAX_S && k <= 64 * E) {                                                                               \
     hipLaunchKernelGGL((topk_runs_kernel<E, NW>), grid, dim3(64 * NW), 0, s, score, S, k, idx);                  \
     return hipGetLastError();                                                                                    \
   }
-  FT_RUNS(512, 1, 8) FT_RUNS(1024, 2, 8) FT_RUNS(2048, 4, 8) FT_RUNS(4096, 4, 16) FT_RUNS(4096, 8, 8) FT_RUNS(8192, 8, 16) FT_RUNS(8192, 16, 8)
+#define FT_SELECT(MAX_S, NT, E, W)                                                                               \
+  if (S <= MAX_S && k <= NT * W) {                                                                               \
+    hipLaunchKernelGGL((topk_select_kernel<NT, E, W>), grid, dim3(NT), 0, s, score, S, k, idx);                  \
+    return hipGetLastError();                                                                                    \
+  }
+  FT_RUNS(512, 1, 8) FT_RUNS(1024, 2, 8)
+  if (S > 8192) {
+    if (k > kTopkSelectMax) return hipErrorInvalidValue;
+    FT_SELECT(INT32_MAX, 1024, 0, 1) FT_SELECT(INT32_MAX, 1024, 0, 2) FT_SELECT(INT32_MAX, 1024, 0, 4)
+    FT_SELECT(INT32_MAX, 1024, 0, 8) FT_SELECT(INT32_MAX, 1024, 0, 16)
+  } else if (S > 4096) {
+    FT_SELECT(8192, 1024, 8, 1) FT_SELECT(8192, 1024, 8, 2) FT_SELECT(8192, 1024, 8, 4)
+  } else if (S > 2048) {
+    FT_SELECT(4096, 512, 8, 1) FT_SELECT(4096, 512, 8, 2) FT_SELECT(4096, 512, 8, 4)
+  } else if (S > 1024) {
+    FT_SELECT(2048, 256, 8, 1) FT_SELECT(2048, 256, 8, 2)
+  } else if (S > 512) {
+    FT_SELECT(1024, 256, 4, 1)
+  }
 #undef FT_RUNS
+#undef FT_SELECT
   if (S <= 512)
     hipLaunchKernelGGL((topk_kernel<2, 256>), grid, dim3(256), 0, s, score, S, k, idx);
   else if (S <= 1024)
