@@ -189,6 +189,17 @@ SplitPlan make_plan(const SplitShape& a) {
   return plan;
 }
 
+// Whether the column sums of few rows come from kept logits.  Up to 32 rows always; up to kSplitStatRows where the column pass would
+// read K once per query head of a group, and a launch take the mean (130 random calls of 33 to 64 rows: H32/8 Sq16 Skv8966 D128
+// B4 92 -> 46 us, Sq12 Skv16000 52 -> 27, H16/2 Sq5 Skv10808 D64 25.9 -> 16.2), and for heads of their own where the logits'
+// 4 bytes a pair, there and back, cost less than the 2 D bytes a key of K again and a launch (D128 H16 Sq40 Skv16372 46 -> 38,
+// Sq48 Skv2524 22.8 -> 18.7, H8 Sq64 Skv10574 24.7 -> 24.3, but H32 Sq64 Skv8000 55.1 -> 57.7; D64 H8 Sq40 Skv5543 17.2 -> 15.1,
+// H16 Sq48 Skv10507 25.6 -> 25.8, 64 rows -0.9 to 0.5 us either way).
+bool keep_logits(int64_t pairs, int group, int64_t rows, int Skv, int D) {
+  if (rows <= 32 || group > 1) return rows <= kSplitStatRows;
+  return rows <= (D == 128 ? kSplitStatRows : 48) && (double)pairs * Skv * (rows - (D == 128 ? 44 : 30)) < 2.5e6;
+}
+
 }  // namespace
 
 // stats: column sums of rounded logits are wanted too.  The reference holds until the thread's next call.
@@ -212,7 +223,7 @@ const SplitPlan& split_plan(int B, int H, int group, int Sq, int Skv, int D, boo
   // One row block: Skv matters through its tiles only, and a generation loop, whose Skv grows with every step, makes a plan
   // once in 64 steps.
   if (rows <= 128) Skv = (Skv + 63) / 64 * 64;
-  const SplitShape shape{B, H, group, Sq, Skv, D, forced, cus, causal, cap, stats && rows <= kSplitStatRows};
+  const SplitShape shape{B, H, group, Sq, Skv, D, forced, cus, causal, cap, stats && keep_logits(pairs, group, rows, Skv, D)};
   Entry& e = kept[(unsigned)(B * 31 + H * 7 + group * 3 + Sq * 5 + Skv / 64 + D + cap + 2 * shape.stats) % kEntries];
   if (!(e.shape == shape)) e = Entry{shape, make_plan(shape)};
   return e.plan;
@@ -266,7 +277,7 @@ __device__ __forceinline__ void fold_shares(const AttnKernelParams& p, int D, in
 
 // A wave takes Q of the four pieces of (32 rows of a shared block, 32 channels); every load is up to 1 KB contiguous, in the
 // accumulators' own register layout.  Bound by the latency of its loads, over many rows by their bytes.
-// FEW (up to kSplitStatRows rows): up to 16 rows (a generation step's) the lanes that have no row take every SUB-th share of the
+// FEW (up to 32 rows): up to 16 rows (a generation step's) the lanes that have no row take every SUB-th share of the
 // others' and meet by lane exchanges, so that eighty shares of four rows are one round of loads and not ten (whole calls: B1 H16/4 Sq1
 // Skv5195 16.6 -> 10.6 us, H32/8 Sq1 Skv4000 15.4 -> 11.7, soft-capped B2 H16/4 Sq1 Skv3058 18.6 -> 13.0); eight shares or fewer
 // are one round anyway.
@@ -332,15 +343,17 @@ __global__ void __launch_bounds__(256) attn_combine_kernel(const AttnKernelParam
 constexpr int kStatTiles = 8;
 __host__ __device__ constexpr int stat_step(int pool) { return pool ? kStatTiles - 1 : kStatTiles; }  // half a tile on either side for the window
 
-template <typename T, int D, bool SQ>
+// WIDE: more than 32 rows.
+template <typename T, int D, bool SQ, bool WIDE>
 __global__ void __launch_bounds__(256) split_stats_kernel(const AttnKernelParams p, const SplitStats st, int ncol) {
   if ((int)blockIdx.x >= ncol) {
-    combine_rows<T, D, 1, true>(p, 0, (blockIdx.x - ncol) * 4 + wave_id());
+    combine_rows<T, D, 1, !WIDE>(p, 0, (blockIdx.x - ncol) * 4 + wave_id());
     return;
   }
   constexpr int KT = kStatTiles * kAttnBN;
   constexpr bool kF16 = __is_same(typename T::elem, _Float16);
-  __shared__ float s_nlse[kSplitStatRows];
+  constexpr int kRows = WIDE ? kSplitStatRows : 32;
+  __shared__ float s_nlse[kRows];
   __shared__ __align__(16) float s_sum[4][KT];
   __shared__ __align__(16) float s_sq[SQ ? 4 : 1][SQ ? KT : 4];
   const int rows = p.Sq * p.group, Hkv = p.H / p.group, pairs = p.B * Hkv;
@@ -360,26 +373,28 @@ __global__ void __launch_bounds__(256) split_stats_kernel(const AttnKernelParams
       const int r = min(wave * per + min(i, per - 1), rows - 1);
       w[i] = *reinterpret_cast<const uint4v*>(col + (int64_t)r * stride);
     }
-    // eight threads a row for its shares: one round of loads up to 64 shares
-    const int row = t & 31, part = t >> 5, rc = min(row, rows - 1);
+    // eight threads a row for its shares (WIDE: four): one round of loads up to 64 shares (32)
+    constexpr int parts = 256 / kRows;
+    const int row = t & (kRows - 1), part = t / kRows, rc = min(row, rows - 1);
     const int nch = shares_of_block(p, 0);
     if (nch > 1) {
       float M = kNoMax, L = 0.f;
       float4v none[1];
       if (part < nch)
-        fold_shares<8, 0>(p, D, (int64_t)bh * p.nitems + part, rc, (nch - part + 7) >> 3, 8, M, L, none, [](const SplitPartial&, int) { return float4v{}; });
+        fold_shares<8, 0>(p, D, ((int64_t)bh * p.nitems + part) * p.part_waves + rc / 32, rc % 32, (nch - part + parts - 1) / parts, parts, M, L, none,
+                          [](const SplitPartial&, int) { return float4v{}; });
       s_sum[0][t] = M;
       s_sum[1][t] = L;
       __syncthreads();
-      if (t < 32) {
+      if (t < kRows) {
 #pragma unroll
-        for (int u = 1; u < 8; ++u) M = fmaxf(M, s_sum[0][32 * u + t]);
+        for (int u = 1; u < parts; ++u) M = fmaxf(M, s_sum[0][kRows * u + t]);
         L = 0.f;
 #pragma unroll
-        for (int u = 0; u < 8; ++u) L = __builtin_fmaf(__builtin_amdgcn_exp2f(s_sum[0][32 * u + t] - M), s_sum[1][32 * u + t], L);
+        for (int u = 0; u < parts; ++u) L = __builtin_fmaf(__builtin_amdgcn_exp2f(s_sum[0][kRows * u + t] - M), s_sum[1][kRows * u + t], L);
         s_nlse[t] = -(M + __builtin_amdgcn_logf(L));
       }
-    } else if (t < 32) {
+    } else if (t < kRows) {
       s_nlse[t] = -p.lse[((int64_t)(bh / Hkv) * p.H + (bh % Hkv) * p.group + rc % p.group) * p.Sq + rc / p.group];
     }
     __syncthreads();
@@ -399,12 +414,18 @@ __global__ void __launch_bounds__(256) split_stats_kernel(const AttnKernelParams
       }
     }
   };
-  if (per <= 1)
-    rows_of_wave(std::integral_constant<int, 1>{});
-  else if (per <= 3)
-    rows_of_wave(std::integral_constant<int, 3>{});
-  else
-    rows_of_wave(std::integral_constant<int, kSplitStatRows / 4>{});
+  if constexpr (!WIDE) {
+    if (per <= 1)
+      rows_of_wave(std::integral_constant<int, 1>{});
+    else if (per <= 3)
+      rows_of_wave(std::integral_constant<int, 3>{});
+    else
+      rows_of_wave(std::integral_constant<int, 8>{});
+  } else if (per <= 12) {
+    rows_of_wave(std::integral_constant<int, 12>{});
+  } else {
+    rows_of_wave(std::integral_constant<int, kRows / 4>{});
+  }
 #pragma unroll
   for (int hf = 0; hf < 2; ++hf) {
     *reinterpret_cast<float4v*>(&s_sum[wave][k0 + 4 * hf]) = float4v{sum[4 * hf], sum[4 * hf + 1], sum[4 * hf + 2], sum[4 * hf + 3]};
@@ -469,28 +490,33 @@ hipError_t launch_attn_split(const AttnKernelParams& p0, const SplitPlan& plan, 
     const int step = stat_step(stats->pool) * kAttnBN;
     const int64_t ncol = pairs * ((p.Skv + (stats->pool ? kAttnBN / 2 : 0) + step - 1) / step);
     const dim3 g((unsigned)(ncol + ncomb)), blk(256);
-#define FT_CASE(T, DD, SQ) hipLaunchKernelGGL((split_stats_kernel<T, DD, SQ>), g, blk, 0, s, p, *stats, (int)ncol)
+    const bool wide = (int64_t)p.Sq * p.group > 32;
+#define FT_CASE(T, DD, SQ)                                                                                               \
+  {                                                                                                                      \
+    if (wide) hipLaunchKernelGGL((split_stats_kernel<T, DD, SQ, true>), g, blk, 0, s, p, *stats, (int)ncol);             \
+    else hipLaunchKernelGGL((split_stats_kernel<T, DD, SQ, false>), g, blk, 0, s, p, *stats, (int)ncol);                 \
+  }
     if (stats->colsumsq) {
-      if (D == 128 && bf16) FT_CASE(BF16, 128, true);
-      else if (D == 128) FT_CASE(F16, 128, true);
-      else if (bf16) FT_CASE(BF16, 64, true);
-      else FT_CASE(F16, 64, true);
+      if (D == 128 && bf16) FT_CASE(BF16, 128, true)
+      else if (D == 128) FT_CASE(F16, 128, true)
+      else if (bf16) FT_CASE(BF16, 64, true)
+      else FT_CASE(F16, 64, true)
     } else {
-      if (D == 128 && bf16) FT_CASE(BF16, 128, false);
-      else if (D == 128) FT_CASE(F16, 128, false);
-      else if (bf16) FT_CASE(BF16, 64, false);
-      else FT_CASE(F16, 64, false);
+      if (D == 128 && bf16) FT_CASE(BF16, 128, false)
+      else if (D == 128) FT_CASE(F16, 128, false)
+      else if (bf16) FT_CASE(BF16, 64, false)
+      else FT_CASE(F16, 64, false)
     }
 #undef FT_CASE
     return hipGetLastError();
   }
-  // Up to kSplitStatRows rows: as in the fold beside the column sums, whose rows are the same bit for bit.  More of them, up to five
+  // Up to kSplitStatRows rows: as in the folds beside the column sums, whose rows are the same bit for bit.  More of them, up to five
   // shares of a block: two pieces a wave, four shares a round (B1 H32/8 Sq501 Skv5760, four shares, 7.9 -> 6.2 us; two pieces with
   // eight a round 7.1, four pieces 6.5; soft-capped Sq777 Skv3000, five shares, 12.5 -> 12.3; six to eight shares 4.35..4.9 against
   // 4.28..5.1, sixteen 4.7 against 5.4, thirty-one 5.8 against 7.7).
   const int64_t rows = (int64_t)p.Sq * p.group;
   const int most = (std::min<int64_t>(p.Skv, (rows - 1) / p.group + 1 + p.off) + kAttnBN - 1) / kAttnBN;
-  const bool few = rows <= kSplitStatRows, two = !few && most <= 5 * plan.chunk_tiles;
+  const bool few = rows <= 32, two = rows > kSplitStatRows && most <= 5 * plan.chunk_tiles;
   const dim3 cgrid((unsigned)(two ? (ncomb + 1) / 2 : ncomb)), cblk(256);
 #define FT_CASE(T, DD)                                                                                                       \
   {                                                                                                                          \

@@ -66,7 +66,7 @@ struct SplitStats {
   float *colsum, *colsumsq;
   int pool;
 };
-constexpr int kSplitMaxPool = 65, kSplitStatRows = 32;
+constexpr int kSplitMaxPool = 65, kSplitStatRows = 64;
 
 struct ColstatsKernelParams {
   const uint16_t* q;
