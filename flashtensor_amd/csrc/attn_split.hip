@@ -148,7 +148,9 @@ SplitPlan make_plan(const SplitShape& a) {
     if (items > kSplitMaxItems) break;
     const int64_t wgs = items * pairs;
     const int rounds = (((most + chunk - 1) / chunk + 7) / 8 * lanes + 31) / 32;
-    const double fold = shared ? kCombine + kFoldRound * (rounds - 1) + (double)shared * pairs * std::min(rows, 128) * a.D * 4 * (1 / kPartWrite + 1 / kPartRead) : 0;
+    // (where logits are kept the second launch is made anyway: H8 Sq2 Skv230 D128 13.2 -> 9.6 us, B4 H32 Sq1 Skv574 18.5 -> 15.9; not
+    // where undivided blocks are a workgroup per CU: B8 H32 Sq1 Skv700 23.2 -> 27.0, B16 H16 Sq1 Skv133 12.1 -> 14.5)
+    const double fold = shared ? (keep && pairs * nMB < cus ? 0 : kCombine) + kFoldRound * (rounds - 1) + (double)shared * pairs * std::min(rows, 128) * a.D * 4 * (1 / kPartWrite + 1 / kPartRead) : 0;
     // The search ends where no further cut can win: smaller shares mean more of them, so the folding, and in a launch of
     // several rounds the least that the slots' work adds up to, only grow.
     const double least = wgs > 2 * cus ? (total * shared_cu + items * kNext) * per_xcd / slots : 0;
