@@ -32,7 +32,7 @@ namespace ft {
 
 constexpr int kSbThreads = 512, kSbWaves = 8, kSbStrip = 32;
 constexpr int kSbPart = 32 * 32 + 3 * 32;  // per (batch, chunk, head): KV [d][e], then m or unused, l or sum|K|, sum|Q|
-constexpr int kSbMaxChunks = 4;
+constexpr int kSbMaxChunks = 64;  // their weights stand in LDS while pass 2 merges (in the x tiles, not yet in use)
 
 struct SmallBlockParams {
   const void* x;
@@ -394,8 +394,11 @@ __global__ void __launch_bounds__(kSbThreads) linblk_out_kernel(const SmallBlock
   __shared__ __align__(16) float s_bq[C];
   __shared__ __align__(16) float s_bo[C];
   __shared__ __align__(16) uint4v s_kv[H][2][2][64];      // [head][hi, lo][step][lane]: operand of O^T = KVn^T Qs^T
-  __shared__ float s_wgt[H][kSbMaxChunks][32];           // weight of chunk c in row d of the merged matrix
   __shared__ float s_winv[H];
+  __shared__ float s_gmax[kSbWaves];
+  // weight of chunk c in row d of head h's merged matrix: [H][kSbMaxChunks][32]
+  static_assert(H * kSbMaxChunks * 32 * sizeof(float) <= sizeof(s_x), "the merge's weights outgrow the x tiles");
+  float* const s_wgt = reinterpret_cast<float*>(s_x);
 
   const int b = blockIdx.x % p.B, ch = blockIdx.x / p.B;
   const int lane = lane_id(), wave = wave_id();
@@ -414,80 +417,121 @@ __global__ void __launch_bounds__(kSbThreads) linblk_out_kernel(const SmallBlock
   stage_bias<T, IN32>(s_bq, p.b_qkv, 0, C);
   stage_bias<T, IN32>(s_bo, p.b_out, 0, C);
 
-  // ---- merge this batch's chunk matrices: wave h takes head h
-  if (wave < H) {
-    const int h = wave;
+  // ---- merge this batch's chunk matrices: WPH waves to a head, each with its share of the contraction slots and the entries of STEP
+  // chunks in flight at one time (two heads: four chunks, so that two workgroups fit a CU's registers).  One wave, which meets no barrier, for up
+  // to four chunks (B64 S784 fp16: two waves +0.4 us).
+  auto merge = [&](auto step, auto wph) __attribute__((always_inline)) {
+    constexpr int STEP = decltype(step)::value, WPH = decltype(wph)::value, E = 16 / WPH;  // E: entries per lane and chunk
+    const int h = wave / WPH, k0 = wave % WPH * E;
+    auto meet = [&] {
+      if constexpr (WPH > 1) {
+        __syncthreads();
+      } else {
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // the wave's own LDS writes have landed (lgkmcnt(0))
+      }
+    };
     const float* part = p.part + ((int64_t)b * p.nch * H + h) * kSbPart;  // chunk c: + c * H * kSbPart
-    const int64_t cstride = (int64_t)H * kSbPart;
-    // (loops over all kSbMaxChunks slots, the ones past nch re-reading the last chunk with weight 0: every load of
-    // the merge is then independent of the others, and the matrix entries are requested before the statistics that
-    // weigh them are worked on: one memory latency for the whole merge)
-    // lane (e = n, g): slots i of step s are rows d = 16 s + 8 (i / 4) + 4 g + i % 4
-    float raw[16][kSbMaxChunks];
+    constexpr int64_t cstride = (int64_t)H * kSbPart;
+    // lane (e = n, g): slot k = 8 s + i is row d = 16 s + 8 (i / 4) + 4 g + i % 4
+    auto row = [&](int k) { return 16 * (k >> 3) + 8 * ((k >> 2) & 1) + 4 * g + (k & 3); };
+    // (slots past nch re-read the last chunk with weight 0, so that all loads of a step are in flight together; the first step's
+    // entries are requested before the statistics that weigh them are worked on: one memory latency for up to STEP chunks)
+    float raw[E][STEP];
+    auto request = [&](int c0) {
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const int d = 16 * (k >> 3) + 8 * ((k >> 2) & 1) + 4 * g + (k & 3);
+      for (int k = 0; k < E; ++k)
 #pragma unroll
-      for (int c = 0; c < kSbMaxChunks; ++c) raw[k][c] = part[min(c, p.nch - 1) * cstride + d * 32 + n];
-    }
-    if (g == 0) {  // row d = n: weights of the chunks
-      float mc[kSbMaxChunks], lc[kSbMaxChunks], qc[kSbMaxChunks];
-#pragma unroll
-      for (int c = 0; c < kSbMaxChunks; ++c) {
-        const float* st = part + min(c, p.nch - 1) * cstride + 1024 + n;
-        mc[c] = st[0];
-        lc[c] = st[32];
-        qc[c] = st[64];
-      }
+        for (int c = 0; c < STEP; ++c) raw[k][c] = part[min(c0 + c, p.nch - 1) * cstride + row(k0 + k) * 32 + n];
+    };
+    request(0);
+    const int nslots = WPH == 1 ? STEP : (p.nch + STEP - 1) / STEP * STEP;
+    if (k0 == 0) {  // the head's first wave: row d = n; the two half waves take the chunks in turn
       float M = NEG_INF, L = 0.f, NQs = 0.f;
+      float* wgt = s_wgt + (h * kSbMaxChunks) * 32 + n;
+      auto weight = [&](float m, float to) { return m == NEG_INF ? 0.f : __builtin_amdgcn_exp2f((m - to) * kLog2e); };
+      for (int c0 = 0; c0 < nslots; c0 += STEP) {
+        float mc[STEP / 2], lc[STEP / 2], qc[STEP / 2];
 #pragma unroll
-      for (int c = 0; c < kSbMaxChunks; ++c)
-        if (EA && c < p.nch) M = fmaxf(M, mc[c]);
-      float w[kSbMaxChunks];
+        for (int c = 0; c < STEP / 2; ++c) {
+          const float* st = part + min(c0 + 2 * c + g, p.nch - 1) * cstride + 1024 + n;
+          mc[c] = st[0];
+          lc[c] = st[32];
+          qc[c] = st[64];
+        }
+        float m_new = M;
 #pragma unroll
-      for (int c = 0; c < kSbMaxChunks; ++c) {
-        w[c] = c >= p.nch ? 0.f : EA ? (mc[c] == NEG_INF ? 0.f : __builtin_amdgcn_exp2f((mc[c] - M) * kLog2e)) : 1.f;
-        L += w[c] * lc[c];
-        NQs += c < p.nch ? qc[c] : 0.f;
+        for (int c = 0; c < STEP / 2; ++c) {
+          if (c0 + 2 * c + g >= p.nch) mc[c] = NEG_INF;
+          m_new = fmaxf(m_new, mc[c]);
+          if (EA) wgt[(c0 + 2 * c + g) * 32] = mc[c];  // its weight once the largest of all is known
+        }
+        if (EA) L *= weight(M, m_new);
+        M = m_new;
+#pragma unroll
+        for (int c = 0; c < STEP / 2; ++c) {
+          const bool in = c0 + 2 * c + g < p.nch;
+          L += EA ? weight(mc[c], M) * lc[c] : in ? lc[c] : 0.f;
+          NQs += in ? qc[c] : 0.f;
+        }
       }
+      const float all = fmaxf(M, xchg32(M));
+      if (EA) L *= weight(M, all);
+      L += xchg32(L);
+      NQs += xchg32(NQs);
       const float inv = 1.f / (!EA && p.normalize_q ? L * NQs : L);
-#pragma unroll
-      for (int c = 0; c < kSbMaxChunks; ++c) s_wgt[h][c][n] = w[c] * inv;
+#pragma unroll STEP / 2
+      for (int cc = g; cc < nslots; cc += 2) wgt[cc * 32] = EA ? weight(wgt[cc * 32], all) * inv : cc < p.nch ? inv : 0.f;  // (the lane's own)
     }
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // the wave's own LDS writes have landed (lgkmcnt(0))
-    float val[16];
+    meet();
+    float val[E];
+#pragma unroll
+    for (int k = 0; k < E; ++k) val[k] = 0.f;
+    for (int c0 = 0;;) {
+#pragma unroll
+      for (int k = 0; k < E; ++k)
+#pragma unroll
+        for (int c = 0; c < STEP; ++c) val[k] += s_wgt[(h * kSbMaxChunks + c0 + c) * 32 + row(k0 + k)] * raw[k][c];
+      c0 += STEP;
+      if (c0 >= p.nch) break;
+      request(c0);
+    }
     float gmax = 0.f;
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const int d = 16 * (k >> 3) + 8 * ((k >> 2) & 1) + 4 * g + (k & 3);
-      float v = 0.f;
-#pragma unroll
-      for (int c = 0; c < kSbMaxChunks; ++c) v += s_wgt[h][c][d] * raw[k][c];
-      val[k] = v;
-      gmax = fmaxf(gmax, __builtin_fabsf(v));
-    }
+    for (int k = 0; k < E; ++k) gmax = fmaxf(gmax, __builtin_fabsf(val[k]));
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) gmax = fmaxf(gmax, __shfl_xor(gmax, o));
+    if constexpr (WPH > 1) {
+      if (lane == 0) s_gmax[wave] = gmax;
+      __syncthreads();
+#pragma unroll
+      for (int w = 0; w < WPH; ++w) gmax = fmaxf(gmax, s_gmax[h * WPH + w]);
+    }
     // power-of-two scale that puts the largest entry in [2^13, 2^14): SimA's entries are ~1 / S^2
     int ex = 0;
     if (gmax > 0.f && gmax < __builtin_inff()) ex = 13 - (int)__builtin_floorf(__builtin_log2f(gmax));
     ex = max(-100, min(100, ex));
     const float scale = __builtin_ldexpf(1.f, ex);
-    uint32_t hi[8], lo[8];
+    uint32_t hi[E / 2], lo[E / 2];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < E / 2; ++j) {
       const float a0 = val[2 * j] * scale, a1 = val[2 * j + 1] * scale;
       hi[j] = T::pack2(a0, a1);
       lo[j] = T::pack2((a0 - T::lo(hi[j])) * (float)(1 << kSbLoShift<T>), (a1 - T::hi(hi[j])) * (float)(1 << kSbLoShift<T>));
     }
+    // slot k of a head: word k % 8 / 2 of step k / 8's operand
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      s_kv[h][0][s][lane] = uint4v{hi[4 * s], hi[4 * s + 1], hi[4 * s + 2], hi[4 * s + 3]};
-      s_kv[h][1][s][lane] = uint4v{lo[4 * s], lo[4 * s + 1], lo[4 * s + 2], lo[4 * s + 3]};
+    for (int j = 0; j < E / 2; ++j) {
+      const int k = k0 + 2 * j;
+      reinterpret_cast<uint32_t*>(&s_kv[h][0][k >> 3][lane])[(k & 7) >> 1] = hi[j];
+      reinterpret_cast<uint32_t*>(&s_kv[h][1][k >> 3][lane])[(k & 7) >> 1] = lo[j];
     }
-    if (lane == 0) s_winv[h] = __builtin_ldexpf(1.f, -ex);
-  }
+    if (k0 == 0 && lane == 0) s_winv[h] = __builtin_ldexpf(1.f, -ex);
+  };
+  if (p.nch > 4)
+    merge(std::integral_constant<int, 2 * H>(), std::integral_constant<int, kSbWaves / H>());
+  else if (wave < H)
+    merge(std::integral_constant<int, 4>(), std::integral_constant<int, 1>());
   __syncthreads();
 
   for (; strip < strip_end; strip += kSbWaves) {
@@ -607,25 +651,29 @@ __global__ void __launch_bounds__(kSbThreads) linblk_out_kernel(const SmallBlock
 int device_cu_count();  // attn_fwd.hip
 
 // Chunking of the token axis, or nch = 0 where this path does not apply: heads of 32 channels, 2 or 4 of them, in at
-// most kSbMaxChunks chunks per batch (every workgroup of pass 2 merges all chunks of its batch, holding one entry per
-// chunk and matrix row in registers).
+// most kSbMaxChunks chunks per batch (every workgroup of pass 2 merges all chunks of its batch).
+// Up to four chunks a workgroup may have waves without a strip; more are made where its waves then have fewer each and a single round
+// of the chip holds them, since a strip costs a wave about 6 us in each pass and four further chunks to merge about 0.7 (four chunks
+// against many, EA, 4 heads: fp16 B7 S7292 - and the library form, whose K = 128 products alone take 42 of its 72 us - 36 us, fp32 B28
+// S2296 48 -> 43).  Tensors of 16 bits take it at any length (against the library form, 4 heads, B1 S4096 27.7 -> 25.1 us, S16384
+// 43.2 -> 40.3, S65536 88 -> 74, B16 S4096 59 -> 32; 2 heads B1 S8192 28.2 -> 18.4, S131072 117 -> 59).  fp32 tensors, whose x and weights
+// this form rounds to fp16 (2.3e-4 of the result's norm from the exact one, the library form 0.7e-4), leave long calls that four chunks
+// would not spread over a quarter of the chip to the library's fp32 products.
 void small_block_plan(const FtLinBlockArgs& a, int* nch, int* strips_per_chunk) {
   *nch = 0;
   *strips_per_chunk = 0;
   if (a.D != 32 || (a.H != 2 && a.H != 4)) return;
-  const int nstrips = (a.S + kSbStrip - 1) / kSbStrip;
-  const int cus = device_cu_count();
-  const int want = (int)std::min<int64_t>(std::min(nstrips, kSbMaxChunks), std::max<int64_t>(1, ((int64_t)cus + a.B - 1) / a.B));
-  const int spc = (nstrips + want - 1) / want;
-  const int n = (nstrips + spc - 1) / spc;
-  // Short calls are launch-bound and two launches beat the library form's five whatever the size (B1 S784: 21 against
-  // 33 us); with more than two strips per wave the workgroups must also cover a good part of the chip, or the
-  // library GEMMs, which spread any token count over all of it, do better (B4 S4096: 55 against 44 us; B16: 57
-  // against 68).
-  const int strips_per_wave = (spc + kSbWaves - 1) / kSbWaves;
-  if (strips_per_wave > 2 && (int64_t)a.B * n * 4 < cus) return;
-  *nch = n;
-  *strips_per_chunk = spc;
+  const int64_t nstrips = ((int64_t)a.S + kSbStrip - 1) / kSbStrip, cus = device_cu_count();
+  const int64_t few = std::min<int64_t>(std::min<int64_t>(nstrips, 4), std::max<int64_t>(1, (cus + a.B - 1) / a.B));
+  const int64_t many = std::min<int64_t>(std::min<int64_t>(cus / a.B, kSbMaxChunks), (nstrips + kSbWaves - 1) / kSbWaves);
+  auto per_wave = [&](int64_t chunks) { return ((nstrips + chunks - 1) / chunks + kSbWaves - 1) / kSbWaves; };
+  const int64_t want = many > few && per_wave(many) < per_wave(few) ? many : few;
+  const int64_t spc = (nstrips + want - 1) / want;
+  const int64_t n = (nstrips + spc - 1) / spc;
+  const int64_t few_spc = (nstrips + few - 1) / few, few_n = (nstrips + few_spc - 1) / few_spc;
+  if (a.dtype == FT_F32 && few_spc > 2 * kSbWaves && a.B * few_n * 4 < cus) return;
+  *nch = (int)n;
+  *strips_per_chunk = (int)spc;
 }
 
 size_t small_block_workspace_bytes(const FtLinBlockArgs& a) {
