@@ -444,10 +444,35 @@ __global__ void __launch_bounds__(64 * WAVES * TEAMS, ((KF == kKfTensor || KF ==
         if (STORE)
           store_logits(it * 4 + blk, __builtin_bit_cast(uint32_t, t2[0]), __builtin_bit_cast(uint32_t, t2[1]),
                        __builtin_bit_cast(uint32_t, t2[2]), __builtin_bit_cast(uint32_t, t2[3]));
+        if constexpr (kCap) {
+          // Gemma2's soft-cap (below), bound by the vector pipe: a product with an fp16 operand and its rounding in one instruction
+          // (the sum with 0 makes it v_fma_mix{lo,hi}_f16, or v_fma_mix_f32 for the exponential's argument), in place of a
+          // conversion, a product and half a conversion of two.  tanh, whose operand is fp32, is rounded two at a time instead
+          // (1 - 1 / (e / 2 + 1 / 2) has the bits of tanh_exp_form and is no sum of a product, which the compiler would round singly:
+          // 436.9 against 432.3 us for the first call here).  418 vector instructions a mask-free tile for 546, the same
+          // results; B8 H32/8 S1885 D128 450 -> 432 us, B5 H16 S904 D64 40.9 -> 35.5, H32/8 Sq777 Skv3000 D128 80.1 -> 77.5.
+          auto mul = [](_Float16 a, float f) __attribute__((always_inline)) { return __builtin_fmaf((float)a, f, 0.f); };
+          half2v c2[4];
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-          x[i] = kCap ? (float)t2[i >> 1][i & 1] * (rcp_cap * 0.125f)  // logit / cap, rounded below
-                      : __builtin_fmaf((float)t2[i >> 1][i & 1], kLog2e / 8.f, neg_m);
+          for (int i = 0; i < 4; ++i) {
+            float2v z;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+              const _Float16 y = (_Float16)mul(t2[i][e], rcp_cap * 0.125f);
+              z[e] = 1.f - __builtin_amdgcn_rcpf(__builtin_fmaf(__builtin_amdgcn_exp2f(mul(y, 2.f * kLog2e)), 0.5f, 0.5f));  // tanh_exp_form
+            }
+            uint32_t zw = T::pack2(z[0], z[1]);
+            asm("" : "+v"(zw));  // one conversion of two, which the compiler would split otherwise
+            const half2v z2 = __builtin_bit_cast(half2v, zw);
+#pragma unroll
+            for (int e = 0; e < 2; ++e) c2[i][e] = (_Float16)mul(z2[e], p.softcap);
+          }
+#pragma unroll
+          for (int i = 0; i < 8; ++i) x[i] = __builtin_fmaf((float)c2[i >> 1][i & 1], kLog2e, neg_m);
+        } else {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) x[i] = __builtin_fmaf((float)t2[i >> 1][i & 1], kLog2e / 8.f, neg_m);
+        }
       } else if constexpr (EMU) {
         // bf16: round QK^T, multiply by the tuned constant (== dividing by sqrt(D) in bf16), round again; the
         // conversions handle two elements each, unpacking a half is a shift or a mask
@@ -466,7 +491,7 @@ __global__ void __launch_bounds__(64 * WAVES * TEAMS, ((KF == kKfTensor || KF ==
         for (int i = 0; i < 8; ++i)
           x[i] = kCap ? s[mbk][rb + i] * (p.logit_mul * (1.f / kLog2e) * rcp_cap) : __builtin_fmaf(s[mbk][rb + i], p.logit_mul, neg_m);
       }
-      if constexpr (kCap) {
+      if constexpr (kCap && !(EMU && kIsF16)) {
         // Gemma2's soft-cap, cap * tanh(logit / cap): three 16-bit tensor ops in the reference
         // (cases/kernels/gemma2.py:31-33), each rounded when the reference's rounding is reproduced
 #pragma unroll
