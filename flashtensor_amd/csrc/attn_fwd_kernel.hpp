@@ -559,43 +559,60 @@ __global__ void __launch_bounds__(64 * WAVES * TEAMS, ((KF == kKfTensor || KF ==
   // MASKED: some key of the half is hidden from some query of the wave (the diagonal, the end of K).
   auto softmax_half = [&](auto masked_tag, const float16v& s, vec8 (&pb)[2], int n0h, int buf, int mbk, const float (&er)[16]) __attribute__((always_inline)) {
     constexpr bool MASKED = decltype(masked_tag)::value;
-    // ---- logits in the log2 domain, with the reference's rounding points when EMU (the same chains as the
-    // pipelined path: two elements per conversion)
-    float x[16];
-    if constexpr (EMU && kIsF16) {
+    // ---- logits with the reference's rounding points when EMU (the same chains as the pipelined path: two elements per
+    // conversion), and their row maximum in the log2 domain.  fp16 logits stay packed, times 8: the log2 domain's factor rides in the
+    // v_fma_mix_f32 that subtract the noise and the maximum, and the maximum is taken two elements at a time: 11 registers and a
+    // tenth of the vector instructions less (noise tensor, tau 1.5, whole call: H32 S4096 D128 516 -> 507 us, S3000 329 -> 324; D64 as before).
+    constexpr bool kHalves = EMU && kIsF16;
+    float x[kHalves ? 1 : 16];
+    half2v x2[kHalves ? 8 : 1];
+    // local key index of register r is 8 (r / 4) + 4 g + r % 4; it is visible iff <= lim + 4 g
+    const int lim = (CAUSAL ? min(qi + off, Skv - 1) : Skv - 1) - n0h - 4 * g;
+    float rowmax;
+    if constexpr (kHalves) {
       const half2v pk_hi = __builtin_bit_cast(half2v, p.pk_hi2), pk_lo = __builtin_bit_cast(half2v, p.pk_lo2);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const float2v a2 = {s[2 * i], s[2 * i + 1]};
         const half2v h2 = __builtin_convertvector(a2, half2v);  // QK^T is an fp16 tensor in the reference
-        // ... divided by sqrt(D) in fp16: t2 = 8 * f16(h / sqrt(D)), exact for D = 64, two packed ops for D = 128
-        const half2v t2 = D == 64 ? h2 : __builtin_elementwise_fma(h2, pk_hi, h2 * pk_lo);
-        x[2 * i] = (float)t2[0] * (kLog2e / 8.f);
-        x[2 * i + 1] = (float)t2[1] * (kLog2e / 8.f);
-      }
-    } else if constexpr (EMU) {
+        // ... divided by sqrt(D) in fp16: 8 * f16(h / sqrt(D)), exact for D = 64, two packed ops for D = 128
+        x2[i] = D == 64 ? h2 : __builtin_elementwise_fma(h2, pk_hi, h2 * pk_lo);
+        if (MASKED) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const uint32_t h2 = T::pack2(s[2 * i], s[2 * i + 1]);
-        const uint32_t t2 = T::pack2(T::lo(h2) * p.logit_mul, T::hi(h2) * p.logit_mul);
-        x[2 * i] = T::lo(t2) * kLog2e;
-        x[2 * i + 1] = T::hi(t2) * kLog2e;
+          for (int e = 0; e < 2; ++e) x2[i][e] = (8 * (i >> 1) + 2 * (i & 1) + e > lim) ? (_Float16)NEG_INF : x2[i][e];
+        }
       }
+      half2v m2 = x2[0];
+#pragma unroll
+      for (int i = 1; i < 8; ++i) m2 = __builtin_elementwise_max(m2, x2[i]);
+      rowmax = fmaxf((float)m2[0], (float)m2[1]);
+      rowmax = fmaxf(rowmax, xchg32(rowmax)) * (kLog2e / 8.f);
     } else {
+      if constexpr (EMU) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) x[r] = s[r] * p.logit_mul;
+        for (int i = 0; i < 8; ++i) {
+          const uint32_t h2 = T::pack2(s[2 * i], s[2 * i + 1]);
+          const uint32_t t2 = T::pack2(T::lo(h2) * p.logit_mul, T::hi(h2) * p.logit_mul);
+          x[2 * i] = T::lo(t2) * kLog2e;
+          x[2 * i + 1] = T::hi(t2) * kLog2e;
+        }
+      } else {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) x[r] = s[r] * p.logit_mul;
+      }
+      if (MASKED) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) x[r] = (8 * (r >> 2) + (r & 3) > lim) ? NEG_INF : x[r];
+      }
+      rowmax = max3(x[0], x[1], x[2]);
+#pragma unroll
+      for (int r = 3; r < 15; r += 2) rowmax = max3(rowmax, x[r], x[r + 1]);
+      rowmax = fmaxf(rowmax, x[15]);
+      rowmax = fmaxf(rowmax, xchg32(rowmax));
     }
-    if (MASKED) {
-      // local key index of register r is 8 (r / 4) + 4 g + r % 4; it is visible iff <= lim + 4 g
-      const int lim = (CAUSAL ? min(qi + off, Skv - 1) : Skv - 1) - n0h - 4 * g;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) x[r] = (8 * (r >> 2) + (r & 3) > lim) ? NEG_INF : x[r];
-    }
-    float rowmax = max3(x[0], x[1], x[2]);
-#pragma unroll
-    for (int r = 3; r < 15; r += 2) rowmax = max3(rowmax, x[r], x[r + 1]);
-    rowmax = fmaxf(rowmax, x[15]);
-    rowmax = fmaxf(rowmax, xchg32(rowmax));
+    auto less = [&](int r, float by) __attribute__((always_inline)) -> float {  // the logit in the log2 domain less `by`
+      return kHalves ? __builtin_fmaf((float)x2[kHalves ? r >> 1 : 0][r & 1], kLog2e / 8.f, -by) : x[kHalves ? 0 : r] - by;
+    };
 
     // ---- KeyFormer: running normaliser of softmax((logit + gumbel) / tau), gumbel = -ln(E)
     {
@@ -610,7 +627,7 @@ __global__ void __launch_bounds__(64 * WAVES * TEAMS, ((KF == kKfTensor || KF ==
           const float u = noise_uniform(a_i, ldsCol[buf * BN + jl]);
           log2E = __builtin_amdgcn_logf(-kLn2 * __builtin_amdgcn_logf(u));
         }
-        z[r] = (x[r] - log2E) * p.inv_tau;
+        z[r] = less(r, log2E);  // times tau
       }
       float zmax = max3(z[0], z[1], z[2]);
 #pragma unroll
@@ -618,10 +635,10 @@ __global__ void __launch_bounds__(64 * WAVES * TEAMS, ((KF == kKfTensor || KF ==
       zmax = fmaxf(zmax, z[15]);
       zmax = fmaxf(zmax, xchg32(zmax));
       // (finite: a half that is hidden entirely, zmax = -inf, adds exp2(-inf) = 0)
-      const float mk_new = fmaxf(m_kf, zmax);
+      const float mk_new = fmaxf(m_kf, zmax * p.inv_tau);
       float zs = 0.f;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) zs += __builtin_amdgcn_exp2f(z[r] - mk_new);
+      for (int r = 0; r < 16; ++r) zs += __builtin_amdgcn_exp2f(__builtin_fmaf(z[r], p.inv_tau, -mk_new));
       l_kf = l_kf * __builtin_amdgcn_exp2f(m_kf - mk_new) + zs;
       m_kf = mk_new;
     }
@@ -630,7 +647,7 @@ __global__ void __launch_bounds__(64 * WAVES * TEAMS, ((KF == kKfTensor || KF ==
     uint4v pw[2];
 #pragma unroll
     for (int r = 0; r < 16; r += 2) {
-      const uint32_t w = T::pack2(__builtin_amdgcn_exp2f(x[r] - m_run), __builtin_amdgcn_exp2f(x[r + 1] - m_run));
+      const uint32_t w = T::pack2(__builtin_amdgcn_exp2f(less(r, m_run)), __builtin_amdgcn_exp2f(less(r + 1, m_run)));
       l_run = T::add2(w, l_run);  // row sum of the 16-bit P the MFMA consumes
       pw[r >> 3][(r & 7) >> 1] = w;
     }

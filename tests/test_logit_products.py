@@ -1,5 +1,6 @@
-"""The fp16 logits' chain that reads and rounds halves inside its products (soft cap) against the oracle: caps that fp16 does not hold,
-caps that saturate tanh or leave it linear, in both launch forms, on row lengths around the tile."""
+"""The fp16 logits' chains that read and round halves inside their products (soft cap, KeyFormer with noise from a tensor) against
+the oracle: caps that fp16 does not hold, caps that saturate tanh or leave it linear, temperatures on both sides of 1, in every
+launch form, on row lengths around the tile."""
 import pytest
 import torch
 
@@ -23,3 +24,20 @@ def test_soft_cap(monkeypatch, form, S, D, cap):
   out = ops.gemma2(q.cuda(), k.cuda(), v.cuda(), softcap=cap)
   torch.cuda.synchronize()
   assert (out.float().cpu() - oracle.gemma2_forward(q, k, v, softcap=cap).float()).abs().max().item() <= O_BAR
+
+
+@pytest.mark.parametrize("form", ["4", "8", "t"])
+@pytest.mark.parametrize("S,D", SIZES)
+@pytest.mark.parametrize("tau", [0.5, 4.0])
+def test_keyformer_tensor(monkeypatch, form, S, D, tau):
+  q, k, v = oracle.prepare_inputs(2, S, 2, D, seed=S)
+  er = oracle.prepare_exp_rand(2, 2, S, S, seed=S)
+  monkeypatch.setenv("FT_ATTN_FORM", form)
+  out, score = ops.keyformer(q.cuda(), k.cuda(), v.cuda(), er.cuda(), tau=tau)
+  torch.cuda.synchronize()
+  ref_out, ref_score = oracle.keyformer_forward(q, k, v, er, tau=tau)
+  assert (out.float().cpu() - ref_out.float()).abs().max().item() <= O_BAR
+  # one ulp of a logit below 4 (2^-9) moves a probability by that share over tau, and a key seen by n rows by 1 / n of it
+  n = torch.arange(S, 0, -1, dtype=torch.float32)
+  rel = ((score.cpu() - ref_score).abs() / ref_score).amax(dim=(0, 1))
+  assert (rel <= (1e-3 + 4e-3 / n) / min(tau, 1.0)).all(), rel.max().item()
