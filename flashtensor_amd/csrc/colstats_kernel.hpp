@@ -323,7 +323,7 @@ __global__ void __launch_bounds__(kColThreads * TEAMS, (TEAMS == 1 ? colstats_wa
             x[e] = __builtin_fmaf(T::lo(t2), kLog2e, nlse4[e]);
             x[e + 1] = __builtin_fmaf(T::hi(t2), kLog2e, nlse4[e + 1]);
           }
-        } else if (kPacked && !KFM) {
+        } else if (kPacked && MODE != kStatKfSeeded) {
 #pragma unroll
           for (int e = 0; e < 4; e += 2) {
             const float2v a2 = {sval(s, blk, key, e), sval(s, blk, key, e + 1)};
@@ -337,6 +337,11 @@ __global__ void __launch_bounds__(kColThreads * TEAMS, (TEAMS == 1 ? colstats_wa
               const float l1 = __builtin_amdgcn_logf(-__builtin_amdgcn_logf(noise_uniform(row4[e + 1], b_j[key])));
               x[e] = __builtin_fmaf(__builtin_fmaf((float)t2[0], kLog2e / 8.f, -l0), p.inv_tau, nlse4[e]);
               x[e + 1] = __builtin_fmaf(__builtin_fmaf((float)t2[1], kLog2e / 8.f, -l1), p.inv_tau, nlse4[e + 1]);
+            } else if (MODE == kStatKfTensor) {
+              // (E <= 0 and infinite E as in the attention pass: log2 E is what the instruction gives)
+#pragma unroll
+              for (int u = 0; u < 2; ++u)
+                x[e + u] = __builtin_fmaf(__builtin_fmaf((float)t2[u], kLog2e / 8.f, -__builtin_amdgcn_logf(er[blk >> 2][4 * (blk & 3) + e + u])), p.inv_tau, nlse4[e + u]);
             } else {
               x[e] = __builtin_fmaf((float)t2[0], kLog2e / 8.f, nlse4[e]);
               x[e + 1] = __builtin_fmaf((float)t2[1], kLog2e / 8.f, nlse4[e + 1]);
