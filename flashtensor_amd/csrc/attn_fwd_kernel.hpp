@@ -445,27 +445,29 @@ __global__ void __launch_bounds__(64 * WAVES * TEAMS, ((KF == kKfTensor || KF ==
           store_logits(it * 4 + blk, __builtin_bit_cast(uint32_t, t2[0]), __builtin_bit_cast(uint32_t, t2[1]),
                        __builtin_bit_cast(uint32_t, t2[2]), __builtin_bit_cast(uint32_t, t2[3]));
         if constexpr (kCap) {
-          // Gemma2's soft-cap (below), bound by the vector pipe: a product with an fp16 operand and its rounding in one instruction
-          // (the sum with 0 makes it v_fma_mix{lo,hi}_f16, or v_fma_mix_f32 for the exponential's argument), in place of a
-          // conversion, a product and half a conversion of two.  tanh, whose operand is fp32, is rounded two at a time instead
-          // (1 - 1 / (e / 2 + 1 / 2) has the bits of tanh_exp_form and is no sum of a product, which the compiler would round singly:
-          // 436.9 against 432.3 us for the first call here).  418 vector instructions a mask-free tile for 546, the same
-          // results; B8 H32/8 S1885 D128 450 -> 432 us, B5 H16 S904 D64 40.9 -> 35.5, H32/8 Sq777 Skv3000 D128 80.1 -> 77.5.
-          auto mul = [](_Float16 a, float f) __attribute__((always_inline)) { return __builtin_fmaf((float)a, f, 0.f); };
+          // Gemma2's soft-cap (below), bound by the vector pipe: a product reads its half by itself (the sum with 0 makes it
+          // v_fma_mix_f32), in place of a conversion and a product, and two products are rounded by one conversion.  A product is an
+          // fp32 number first, as in the reference: rounded straight to a half (v_fma_mix{lo,hi}_f16) some logits are another half
+          // where the cap has many bits (44.8: one in 50, 33.3: one in 500), and it is slower, since the two halves of a word wait for each
+          // other.  450 vector instructions a mask-free tile; in turn with conversions of their own (546) and with the straight
+          // rounding (418): B8 H32/8 S1885 D128 425 us, 460 and 436, B5 H16 S904 D64 34.2, 40.4 and 35.2, H32/8 Sq777 Skv3000 D128
+          // 80.0, 84.3 and 81.4.
+          auto mul = [](uint32_t w, float f) __attribute__((always_inline)) {
+            const half2v h = __builtin_bit_cast(half2v, w);
+            return float2v{__builtin_fmaf((float)h[0], f, 0.f), __builtin_fmaf((float)h[1], f, 0.f)};
+          };
+          auto round2 = [](float2v f) __attribute__((always_inline)) {
+            uint32_t w = T::pack2(f[0], f[1]);
+            asm("" : "+v"(w));  // one conversion of two, which the compiler would split (and join with the products) otherwise
+            return w;
+          };
           half2v c2[4];
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            float2v z;
+            float2v z = mul(round2(mul(__builtin_bit_cast(uint32_t, t2[i]), rcp_cap * 0.125f)), 2.f * kLog2e);
 #pragma unroll
-            for (int e = 0; e < 2; ++e) {
-              const _Float16 y = (_Float16)mul(t2[i][e], rcp_cap * 0.125f);
-              z[e] = 1.f - __builtin_amdgcn_rcpf(__builtin_fmaf(__builtin_amdgcn_exp2f(mul(y, 2.f * kLog2e)), 0.5f, 0.5f));  // tanh_exp_form
-            }
-            uint32_t zw = T::pack2(z[0], z[1]);
-            asm("" : "+v"(zw));  // one conversion of two, which the compiler would split otherwise
-            const half2v z2 = __builtin_bit_cast(half2v, zw);
-#pragma unroll
-            for (int e = 0; e < 2; ++e) c2[i][e] = (_Float16)mul(z2[e], p.softcap);
+            for (int e = 0; e < 2; ++e) z[e] = 1.f - __builtin_amdgcn_rcpf(__builtin_fmaf(__builtin_amdgcn_exp2f(z[e]), 0.5f, 0.5f));  // tanh_exp_form
+            c2[i] = __builtin_bit_cast(half2v, round2(mul(round2(z), p.softcap)));
           }
 #pragma unroll
           for (int i = 0; i < 8; ++i) x[i] = __builtin_fmaf((float)c2[i >> 1][i & 1], kLog2e, neg_m);

@@ -1,6 +1,9 @@
 """The fp16 logits' chains that read and round halves inside their products (soft cap, KeyFormer with noise from a tensor) against
 the oracle: caps that fp16 does not hold, caps that saturate tanh or leave it linear, temperatures on both sides of 1, in every
 launch form, on row lengths around the tile."""
+import math
+
+import numpy as np
 import pytest
 import torch
 
@@ -41,3 +44,42 @@ def test_keyformer_tensor(monkeypatch, form, S, D, tau):
   n = torch.arange(S, 0, -1, dtype=torch.float32)
   rel = ((score.cpu() - ref_score).abs() / ref_score).amax(dim=(0, 1))
   assert (rel <= (1e-3 + 4e-3 / n) / min(tau, 1.0)).all(), rel.max().item()
+
+
+def _capped(D, cap, singly=False):
+  """Every positive finite half as a product of q and k, and its capped logit by the oracle's chain of halves, the last product an fp32
+  number first (singly: rounded once, straight to a half), for those whose other roundings are no matter of a unit in the last places."""
+  x = torch.arange(1, 0x7c00, dtype=torch.int16).view(torch.float16)
+  t = x / math.sqrt(D)
+  y = t / cap
+  z = torch.tanh(y)
+  c = torch.from_numpy((z.numpy().astype("f8") * float(np.float32(cap))).astype("f2")) if singly else z * cap
+  ulp = lambda h: torch.from_numpy(np.spacing(h.numpy())).double()
+  clear = ((t.double() / cap - y.double()).abs() < 0.47 * ulp(y)) & ((torch.tanh(y.double()) - z.double()).abs() < 0.47 * ulp(z))
+  return x, c, clear
+
+
+@pytest.mark.parametrize("form", ["4", "8", "t", "s1"])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("cap", [57.6, 44.8, 22.4])
+def test_soft_cap_rounds_the_product_twice(monkeypatch, form, D, cap):
+  """Heads of one query and two keys whose capped logits c and c - 1 the output shows as exp(-1), over logits from 8 on that a product
+  rounded straight to a half would move by a unit, 2^-7 or more.  The bar is that of four half units of fp16: the two
+  probabilities in front of the second product, the two outputs."""
+  x, c, clear = _capped(D, cap)
+  other = _capped(D, cap, singly=True)[1]
+  pick = ((c != other) & clear & (c >= 8)).nonzero()[:, 0]
+  plain = ((c == other) & clear).nonzero()[:, 0]
+  beside = plain[(c[plain].double() - (c[pick].double()[:, None] - 1)).abs().argmin(1)]
+  H, bar = len(pick), 4 * 2**-11
+  assert H > 50
+  q, k, v = (torch.zeros(1, s, H, D, dtype=torch.float16) for s in (1, 2, 2))
+  q[..., 0] = 1
+  k[0, 0, :, 0], k[0, 1, :, 0] = x[pick], x[beside]
+  v[0, 0, :, 0] = v[0, 1, :, 1] = 1
+  monkeypatch.setenv("FT_ATTN_FORM", form)
+  out = ops.gemma2(q.cuda(), k.cuda(), v.cuda(), softcap=cap)[0, 0].double().cpu()
+  ratio = out[:, 0].log() - out[:, 1].log()
+  want = lambda to: to[pick].double() - c[beside].double()
+  assert ((want(c) - want(other)).abs() > 3 * bar).all()
+  assert ((ratio - want(c)).abs() <= bar).all(), (ratio - want(c)).abs().max().item()
