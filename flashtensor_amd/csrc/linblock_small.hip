@@ -11,8 +11,8 @@
 //     KV^T[e][d] += sum_t V[t][e] Ks[t][d]: the lane of the result holds column d, so EA's running maximum of
 //     K[:, d] (softmax over the tokens) rescales the lane's own registers, nothing crosses lanes.
 //     The waves are folded through LDS and the chunk's matrix, maxima and sums go to the workspace.
-//   pass 2 (linblk_out_kernel), same grid: every workgroup first merges its batch's chunk matrices (a wave per head)
-//     into normalised hi + lo 16-bit operand pairs, then per strip: Q^T = Wq x^T + bq with the tokens as MFMA
+//   pass 2 (linblk_out_kernel), same grid: every workgroup first merges its batch's chunk matrices (up to four of them a
+//     wave per head, else all eight waves) into normalised hi + lo 16-bit operand pairs, then per strip: Q^T = Wq x^T + bq with the tokens as MFMA
 //     columns (a lane holds one token and 16 channels of a head: EA's softmax over the head's channels is in-lane
 //     plus one exchange), O^T = KVn^T Qs^T, y^T = Wo O^T + bo, again feeding accumulators straight back as operands.
 //
@@ -419,7 +419,8 @@ __global__ void __launch_bounds__(kSbThreads) linblk_out_kernel(const SmallBlock
 
   // ---- merge this batch's chunk matrices: WPH waves to a head, each with its share of the contraction slots and the entries of STEP
   // chunks in flight at one time (two heads: four chunks, so that two workgroups fit a CU's registers).  One wave, which meets no barrier, for up
-  // to four chunks (B64 S784 fp16: two waves +0.4 us).
+  // to four chunks (B64 S784 fp16: two waves +0.4 us; two heads, all eight: fp16 B1 S784 11.9 -> 12.1), but for fp32 tensors of two heads,
+  // whose x in flight leaves one wave too few registers for the loads of all four at once (EA B1 S257 12.1 -> 11.7, B64 S784 15.6 -> 15.3).
   auto merge = [&](auto step, auto wph) __attribute__((always_inline)) {
     constexpr int STEP = decltype(step)::value, WPH = decltype(wph)::value, E = 16 / WPH;  // E: entries per lane and chunk
     const int h = wave / WPH, k0 = wave % WPH * E;
@@ -530,6 +531,8 @@ __global__ void __launch_bounds__(kSbThreads) linblk_out_kernel(const SmallBlock
   };
   if (p.nch > 4)
     merge(std::integral_constant<int, 2 * H>(), std::integral_constant<int, kSbWaves / H>());
+  else if (H == 2 && IN32)
+    merge(std::integral_constant<int, 4>(), std::integral_constant<int, kSbWaves / H>());
   else if (wave < H)
     merge(std::integral_constant<int, 4>(), std::integral_constant<int, 1>());
   __syncthreads();
