@@ -60,7 +60,9 @@ hipError_t launch_attn_teams_kf_bf16(const AttnKernelParams& p, int D, int kf, u
 
 // A form of the attention pass as launches are compared by: rows and teams of a workgroup, how many of them a CU holds, and the
 // microseconds that one takes to begin and end and per key tile (of each team), alone on its CU and beside another.  Fitted to
-// the differences between forms in 1900 random calls (some of them: tests/test_launch_forms.py).
+// the differences between forms in 1900 random calls (some of them: tests/test_launch_forms.py).  Soft-capped ones by both types alike,
+// since when fp16 has become shorter, two teams of D = 128 by 1 %, the other forms by 5 to 9: the form chosen is 0.7 % slower than the best
+// one in the mean over the test's fp16 calls (0.8 % before), 0.6 % over its bf16 ones.
 struct Form {
   int rows, teams, per_cu;
   double first, tile, shared;
@@ -91,13 +93,14 @@ static double form_us(const Form& f, int64_t pairs, int group, int Sq, int Skv, 
 // ten key tiles on (attention calls, same process: B1 H8 D128 S1000 21.1 -> 18.1 us, S2048 35.6 -> 29.3; D64, of whose
 // workgroups a CU holds two, from five tiles on: H8 S1000 14.9 -> 12.0).  Shorter plain calls have 2 us at most to gain
 // (S500 14.0 -> 12.3) and keep to the forms whose results agree bit for bit; soft-capped ones, whose waves are slow
-// enough alone, take it from four tiles on (S300 13.4 -> 12.2, S500 19.4 -> 14.9, S130 9.6 -> 9.8).
+// enough alone, take it from four tiles on (fp16 S300 13.0 -> 11.9, S500 19.2 -> 15.3, S130 9.2 -> 9.9).
 // Under the causal mask with more of them too, where the blocks differ in length enough that the second round fills the gaps of the
 // first.  D64: up to two for every CU (H8 S3000 33.5 -> 27.2, B2 H32 S500 10.7 -> 9.4) or, over more than 32 tiles, five for two (H16
 // S2500 31.7 -> 26.9, S3000 36 -> 38), longer ones than 48 again keeping to the bit-equal forms; soft-capped up to thirteen for four
-// CUs (H16 S3000 85 -> 66, H32 S1500 47 -> 37, B2 H32 S777 28.6 -> 27.4, S1000 32 -> 36).  D128: up to three for two CUs (H8 S3000 48 ->
-// 40; H16 S2048, four for two, 36.6 -> 35.8, H32 S777 17.7 -> 20.8), soft-capped over twelve tiles or more four for two (H32 S777 28.7
-// -> 26.0) and over more than 32 five (H16 S2500 89 -> 81, S3000 97 -> 107), where the two launches' times say so too: chunks
+// CUs (fp16 H16 S3000 70 -> 58, H32 S1500 39.6 -> 34.0, B2 H32 S777 25.8 -> 24.2, S1000 28.7 -> 31.5).  D128: up to three for two CUs (H8 S3000
+// 48 -> 40; H16 S2048, four for two, 36.6 -> 35.8, H32 S777 17.7 -> 20.8), soft-capped over twelve tiles or more four for two (bf16 H32 S777
+// 29.4 -> 26.8, fp16 25.7 either way) and over more than 32 five (bf16 H16 S2500 89.7 -> 86.6, S3000 98 -> 112; fp16, of which four waves'
+// tiles have become shorter since and two teams' have not, 76.5 -> 80.4), where the two launches' times say so too: chunks
 // over many more keys than queries, whose blocks are nearly alike, take the second round in full (attention of H16/2 Sq1101 Skv12131
 // 189 -> 265 us; over 200 random calls 7 % of the time, 53 % at most).
 bool use_teams(int64_t pairs, int group, int Sq, int Skv, int D, bool causal, bool cap) {
@@ -115,20 +118,20 @@ bool use_teams(int64_t pairs, int group, int Sq, int Skv, int D, bool causal, bo
 
 // 256-row workgroups (8 waves) stage K and V once for twice the rows, but round every prompt up to 256 rows and are half as many:
 // under the causal mask the 128-row form is the faster one nearly everywhere (attention, B4 H32 D128 S777 53.5 -> 42.2 us, S1024
-// 55.5 -> 51.3, S2600 321 -> 278, B2 S2600 151 -> 135; D64 B4 S1300 61 -> 51; soft-capped B4 S777 75 -> 59).
+// 55.5 -> 51.3, S2600 321 -> 278, B2 S2600 151 -> 135; D64 B4 S1300 61 -> 51; soft-capped fp16 B4 S777 68 -> 52).
 // - plain, soft-cap, causal: where hardly a row is padding and the blocks pair up, heaviest with lightest, into whole rounds of
 //   the chip: one round (B1 H32 S4096 151.9 -> 148.5), or three and more, for which an XCD finishes a pair's blocks before it
 //   starts the next pair's (B8 H32 S1536 229 -> 214, S2048 387 -> 373, B3 S4096 453 -> 443; two rounds B2 H32 S4096 292.5 and
-//   293.7, B4 S2048 166 and 169).  D64 and soft-capped logits from four rounds on (B4 H32 S4096 360 -> 351, soft-capped 941 ->
-//   893; three rounds 204 and 211, 521 and 528), D64 at one round (89.5 -> 88.5; soft-capped 218 -> 229).  Over half as many keys
+//   293.7, B4 S2048 166 and 169).  D64 and soft-capped logits from four rounds on (B4 H32 S4096 360 -> 351, soft-capped fp16 860 ->
+//   834, bf16 927 -> 896; three rounds 204 and 211, fp16 604 and 615), D64 at one round (89.5 -> 88.5; soft-capped bf16 218 and 221, fp16 199 either way).  Over half as many keys
 //   again as queries the blocks are nearly alike, and D128 pairs them up at any whole number of rounds, soft-capped from four
-//   blocks on (B8 H32 S1024 Skv2924 452 -> 364, B2 S2048 Skv5645 319 -> 311; soft-capped B8 H32/4 S1024 Skv10041 2165 -> 1877,
-//   B4 H16 S2048 Skv4098 328 -> 311, B8 H32 S512 Skv1050 106 and 111).
+//   blocks on (B8 H32 S1024 Skv2924 452 -> 364, B2 S2048 Skv5645 319 -> 311; soft-capped fp16 B8 H32/4 S1024 Skv10041 1893 -> 1752,
+//   B4 H16 S2048 Skv4098 298 -> 293, B8 H32 S512 Skv1050 100 either way).
 // - no mask: D128 up to 127 (b, h) pairs (B2 H32 S3600 477 -> 463; B4 S1024 86 -> 90; D64 B2 S2048 86 -> 98), where the last round, of
 //   one workgroup a CU, is three quarters full or one of many (H24 B3 S2048 Skv5231, two rounds and a quarter, 436 against 486, soft-capped
-//   B2 S2600 280 against 410).
+//   fp16 B2 S2600 250 against 346).
 // Head-major where the K and V of all pairs together are beyond every cache: with the mask from 256 pairs and nine rounds on (B8
-// H32 S2304 475 -> 445 us, S2600 645 -> 570, soft-capped 934 -> 849; S2048 374, paired 256-row blocks 373), without from 128 pairs
+// H32 S2304 475 -> 445 us, S2600 645 -> 570, soft-capped fp16 839 -> 762; S2048 374, paired 256-row blocks 373), without from 128 pairs
 // (256 at D64) and two and a half rounds on (D128 B4 H32 S2600 518 -> 491, B8 S1024 193 -> 165, D64 99.5 -> 93; B4 D128 S513 38.6 -> 41.5).
 // And where K and V outgrow the memory-side cache and blocks are alike in length: without the mask over 256 MB (B8 H32 S512 Skv6690
 // D128 651 -> 492 us), over half as many keys again as queries over 400 (B8 H32 S1437 Skv3859 984 -> 710, S689 Skv7010 D64 509 ->

@@ -30,6 +30,9 @@ struct SplitShape {
 //   A tile 0.98 where a workgroup has its CU to itself and 1.74 where two share one, whose second one starts 0.6 late (soft-capped
 //   logits 1.72 and 2.9); D = 64 takes 0.72 of that (soft-capped, whose chain is not shorter for it, 0.82); blocks of one wave, whose
 //   other waves only load, feel 0.18 of the difference; a tile whose logits are kept takes a quarter more.
+//   (Soft-capped logits by bf16; fp16's tiles, whose chain is shorter, take 0.93 to 0.97 of that in every form, and the choice is as
+//   good for them: 0.9 % slower than the best form in the mean over the test's calls, of either type.  Figures a tenth lower change
+//   the form of 227 of 3496 random calls, fp16 1.1 % faster in the mean, 0.81 to 1.16, but bf16 1.7 % slower, 0.92 to 1.17.)
 //   A step of two teams 1.44 (2.1; D = 64 0.65 and 0.82 of it), and 1.45 times that where two workgroups share a CU (D = 64), unless
 //   a team has one wave of rows.
 //   Partial results are written and folded at 7.2 MB/us (0.55 of that time beside the column sums), by a kernel that takes 3.5 to
