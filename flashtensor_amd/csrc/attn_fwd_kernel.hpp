@@ -407,7 +407,9 @@ __global__ void __launch_bounds__(64 * WAVES * TEAMS, ((KF == kKfTensor || KF ==
     const float other = xchg32(amax);
     amax = max3(amax, other, other);
     // soft-cap: the cap is monotonic as well (a product with a positive constant, tanh, roundings), so the
-    // maximum of the capped logits is the capped maximum
+    // maximum of the capped logits is the capped maximum (fp16: to a unit in its last place, since the compiler rounds a product here
+    // straight to a half; a stabiliser has no need to be the logit itself, and products rounded on their own, dependent on each other,
+    // took two teams of D = 128 0.5 to 0.9 % longer)
     auto r16 = [](float x) { return T::to_float(T::from_float(x)); };
     if (EMU) {
       float t = r16(r16(amax) * p.logit_mul);
