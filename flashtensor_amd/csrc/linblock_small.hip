@@ -658,10 +658,13 @@ int device_cu_count();  // attn_fwd.hip
 // Up to four chunks a workgroup may have waves without a strip; more are made where its waves then have fewer each and a single round
 // of the chip holds them, since a strip costs a wave about 6 us in each pass and four further chunks to merge about 0.7 (four chunks
 // against many, EA, 4 heads: fp16 B7 S7292 - and the library form, whose K = 128 products alone take 42 of its 72 us - 36 us, fp32 B28
-// S2296 48 -> 43).  Tensors of 16 bits take it at any length (against the library form, 4 heads, B1 S4096 27.7 -> 25.1 us, S16384
+// S2296 48 -> 43).  As many then as the round holds: with the fewest that leave a wave as many strips, more waves of a workgroup have that
+// many (52 random calls take 0.98 of the fewest's time in the mean, four heads 0.96, two 1.00; from 0.88, B40 S3423 four heads 44.8 against
+// 51.1 us, to 1.15, B1 S20082 two heads 26.3 against 22.8).  Tensors of 16 bits take it at any length (against the library form, 4 heads, B1 S4096 27.7 -> 25.1 us, S16384
 // 43.2 -> 40.3, S65536 88 -> 74, B16 S4096 59 -> 32; 2 heads B1 S8192 28.2 -> 18.4, S131072 117 -> 59).  fp32 tensors, whose x and weights
-// this form rounds to fp16 (2.3e-4 of the result's norm from the exact one, the library form 0.7e-4), leave long calls that four chunks
-// would not spread over a quarter of the chip to the library's fp32 products.
+// this form rounds to fp16 (EA 2.4e-4 to 4.1e-4 of the norm of the result in 64 bits, the library form 0.6e-4 to 1.0e-4; SimA over the raw
+// Q 5.5e-4 to 6.4e-4 and 2.1e-4 to 2.2e-4), leave long calls that four chunks would not spread over a quarter of the chip to the
+// library's fp32 products.
 void small_block_plan(const FtLinBlockArgs& a, int* nch, int* strips_per_chunk) {
   *nch = 0;
   *strips_per_chunk = 0;
