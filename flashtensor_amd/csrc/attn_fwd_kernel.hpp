@@ -783,6 +783,11 @@ __global__ void __launch_bounds__(64 * WAVES * TEAMS, ((KF == kKfTensor || KF ==
   if constexpr (kTailPairs) {
     auto tail_tile = [&](int it, auto odd_tag) __attribute__((always_inline)) {
       constexpr bool odd = decltype(odd_tag)::value;
+      // Behind all of the pair's first tile: nothing in the fp16 soft cap's chain keeps the compiler from raising this barrier to that
+      // tile's last operand read, and waves with both tiles then stand in the middle of the first one until those whose last tile it is
+      // have done theirs (H8 fp16, D64 S65 to S128 7.4 to 7.8 -> 6.7 to 7.1 us, D128 S128 9.2 -> 8.7, S200 10.9 -> 10.3; mask-free pairs,
+      // which all waves walk together, are no faster for it).
+      if constexpr (odd && kCap && EMU && kIsF16) __builtin_amdgcn_sched_barrier(0);
       sync_and_stage(it, odd ? ldsK1 : ldsK0, odd ? ldsV0 : ldsV1);
       fast_tile(std::true_type{}, std::true_type{}, std::false_type{}, S0, S1, odd ? ldsK0 : ldsK1, odd ? ldsV1 : ldsV0, it * BN, it, nullptr, nullptr);
 #pragma unroll
