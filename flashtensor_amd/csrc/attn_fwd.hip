@@ -61,8 +61,8 @@ hipError_t launch_attn_teams_kf_bf16(const AttnKernelParams& p, int D, int kf, u
 // A form of the attention pass as launches are compared by: rows and teams of a workgroup, how many of them a CU holds, and the
 // microseconds that one takes to begin and end and per key tile (of each team), alone on its CU and beside another.  Fitted to
 // the differences between forms in 1900 random calls (some of them: tests/test_launch_forms.py).  Soft-capped ones by both types alike,
-// since when fp16 has become shorter, two teams of D = 128 by 1 %, the other forms by 5 to 9: the form chosen is 0.7 % slower than the best
-// one in the mean over the test's fp16 calls (0.8 % before), 0.6 % over its bf16 ones.
+// since when fp16 has become shorter, two teams of D = 128 by 1 %, the other forms by 5 to 9, few tiles under the mask by up to 7 more:
+// the form chosen is 0.6 % slower than the best one in the mean over the test's calls of either type (fp16 0.8 % before).
 struct Form {
   int rows, teams, per_cu;
   double first, tile, shared;
@@ -93,14 +93,14 @@ static double form_us(const Form& f, int64_t pairs, int group, int Sq, int Skv, 
 // ten key tiles on (attention calls, same process: B1 H8 D128 S1000 21.1 -> 18.1 us, S2048 35.6 -> 29.3; D64, of whose
 // workgroups a CU holds two, from five tiles on: H8 S1000 14.9 -> 12.0).  Shorter plain calls have 2 us at most to gain
 // (S500 14.0 -> 12.3) and keep to the forms whose results agree bit for bit; soft-capped ones, whose waves are slow
-// enough alone, take it from four tiles on (fp16 S300 13.0 -> 11.9, S500 19.2 -> 15.3, S130 9.2 -> 9.9).
+// enough alone, take it from four tiles on (fp16 S300 13.1 -> 11.8, S500 18.8 -> 15.0, S130 9.2 either way).
 // Under the causal mask with more of them too, where the blocks differ in length enough that the second round fills the gaps of the
 // first.  D64: up to two for every CU (H8 S3000 33.5 -> 27.2, B2 H32 S500 10.7 -> 9.4) or, over more than 32 tiles, five for two (H16
 // S2500 31.7 -> 26.9, S3000 36 -> 38), longer ones than 48 again keeping to the bit-equal forms; soft-capped up to thirteen for four
-// CUs (fp16 H16 S3000 70 -> 58, H32 S1500 39.6 -> 34.0, B2 H32 S777 25.8 -> 24.2, S1000 28.7 -> 31.5).  D128: up to three for two CUs (H8 S3000
+// CUs (fp16 H16 S3000 67 -> 55, H32 S1500 37.6 -> 33.0, B2 H32 S777 23.8 either way, S1000 26.8 -> 30.9).  D128: up to three for two CUs (H8 S3000
 // 48 -> 40; H16 S2048, four for two, 36.6 -> 35.8, H32 S777 17.7 -> 20.8), soft-capped over twelve tiles or more four for two (bf16 H32 S777
-// 29.4 -> 26.8, fp16 25.7 either way) and over more than 32 five (bf16 H16 S2500 89.7 -> 86.6, S3000 98 -> 112; fp16, of which four waves'
-// tiles have become shorter since and two teams' have not, 76.5 -> 80.4), where the two launches' times say so too: chunks
+// 29.4 -> 26.8, fp16 25.7 -> 24.7) and over more than 32 five (bf16 H16 S2500 89.7 -> 86.6, S3000 98 -> 112; fp16, of which four waves'
+// tiles have become shorter since and two teams' have not, 73.5 -> 76.9), where the two launches' times say so too: chunks
 // over many more keys than queries, whose blocks are nearly alike, take the second round in full (attention of H16/2 Sq1101 Skv12131
 // 189 -> 265 us; over 200 random calls 7 % of the time, 53 % at most).
 bool use_teams(int64_t pairs, int group, int Sq, int Skv, int D, bool causal, bool cap) {
@@ -118,7 +118,7 @@ bool use_teams(int64_t pairs, int group, int Sq, int Skv, int D, bool causal, bo
 
 // 256-row workgroups (8 waves) stage K and V once for twice the rows, but round every prompt up to 256 rows and are half as many:
 // under the causal mask the 128-row form is the faster one nearly everywhere (attention, B4 H32 D128 S777 53.5 -> 42.2 us, S1024
-// 55.5 -> 51.3, S2600 321 -> 278, B2 S2600 151 -> 135; D64 B4 S1300 61 -> 51; soft-capped fp16 B4 S777 68 -> 52).
+// 55.5 -> 51.3, S2600 321 -> 278, B2 S2600 151 -> 135; D64 B4 S1300 61 -> 51; soft-capped fp16 B4 S777 67 -> 51).
 // - plain, soft-cap, causal: where hardly a row is padding and the blocks pair up, heaviest with lightest, into whole rounds of
 //   the chip: one round (B1 H32 S4096 151.9 -> 148.5), or three and more, for which an XCD finishes a pair's blocks before it
 //   starts the next pair's (B8 H32 S1536 229 -> 214, S2048 387 -> 373, B3 S4096 453 -> 443; two rounds B2 H32 S4096 292.5 and
